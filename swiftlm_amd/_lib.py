@@ -1,5 +1,6 @@
 """ctypes binding of libdflash_hip.so, the C ABI declared in include/dflash_hip.h
-and include/dflash_cache.h (plus the measurement hooks of include/dflash_profile.h).
+and include/dflash_cache.h (plus the measurement hooks of include/dflash_profile.h), and
+``native``, the compiled binding of the calls a host makes once per layer (csrc/py_native.cpp).
 
 There is no CPU or PyTorch fallback anywhere in this package: if the library is
 not built, or the device is not a gfx950, loading fails with an error.
@@ -96,6 +97,24 @@ def load() -> C.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+class _Native:
+    """The compiled binding, loaded on first use.  After that its functions are plain attributes of this object."""
+
+    def __getattr__(self, name):
+        load()
+        try:
+            from . import _native
+        except ImportError as e:
+            raise DFlashError(f"the compiled binding swiftlm_amd/_native.so does not load ({e}): build it with "
+                              "`make -C swiftlm_amd/csrc` (or __graft_entry__.build()); there is no fallback path") from e
+        _native.set_errors(DFlashError, DFlashUnsupported)
+        self.__dict__.update({k: v for k, v in vars(_native).items() if not k.startswith("__")})
+        return getattr(_native, name)
+
+
+native = _Native()
 
 
 def last_error() -> str:

@@ -16,14 +16,13 @@ from typing import Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from ._lib import DFlashError, DFlashUnsupported  # noqa: F401  (re-exported)
+from ._lib import DFlashError, DFlashUnsupported, native as _native  # noqa: F401  (errors re-exported)
 
 _DT = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16,
        torch.uint8: _lib.U8, torch.bool: _lib.U8}
 
 
-# arrival counters of gdn_layer's in-launch gated norm: int32 zeros per (device, stream, B*Hv), left zero by every call
-_ARRIVALS = {}
+_GATE_KINDS = {"sigmoid": 0, "silu": 1}
 
 
 def _code(t: torch.Tensor) -> int:
@@ -38,7 +37,7 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(_native.current_stream())
 
 
 def _dev(*ts: Optional[torch.Tensor]) -> None:
@@ -66,20 +65,7 @@ class DFlashKernels:
         tape [B,T,Hv,Dv], k [B,T,Hk,Dk], g [B,T,Hv] or [B,T,Hv,Dk], state
         [B,Hv,Dv,Dk], mask [B,T]; returns the replayed state (same dtype as ``state``).
         """
-        _dev(tape, k, g, state, mask)
-        tape, k, g, state = (t.contiguous() for t in (tape, k, g, state))
-        if g.dtype != k.dtype:
-            g = g.to(k.dtype)
-        mask = None if mask is None else mask.contiguous()
-        B, T, Hk, Dk = k.shape
-        Hv, Dv = tape.shape[2], tape.shape[3]
-        out = torch.empty_like(state)
-        rc = _lib.load().dflash_tape_replay(
-            _stream(), _ptr(tape), _code(tape), _ptr(k), _ptr(g), _code(k), g.dim(),
-            _ptr(state), _ptr(out), _code(state), _ptr(mask), _code(mask) if mask is not None else 0,
-            B, T, Hk, Hv, Dk, Dv)
-        _lib.check(rc, "tape_replay_kernel")
-        return out
+        return _native.tape_replay(tape, k, g, state, mask)
 
     @staticmethod
     def tape_replay_batched(tapes: Sequence[torch.Tensor], ks: Sequence[torch.Tensor], gs: Sequence[torch.Tensor],
@@ -118,23 +104,7 @@ class DFlashKernels:
         innovation tape [B,T,Hv,Dv] float32).  ``want_state=False`` (no counterpart in the reference) leaves the
         post-block state out -- None is returned in its place -- for a caller that replays the tape whatever is
         accepted; only the verify-block form supports it (``DFlashUnsupported`` otherwise)."""
-        _dev(q, k, v, g, beta, state, mask)
-        q, k, v, g, beta, state = (t.contiguous() for t in (q, k, v, g, beta, state))
-        for name, t in (("k", k), ("v", v), ("g", g), ("beta", beta)):
-            if t.dtype != q.dtype:
-                raise DFlashUnsupported(f"gated_delta_kernel_with_tape: {name} dtype {t.dtype} differs from q's {q.dtype}")
-        mask = None if mask is None else mask.contiguous()
-        B, T, Hk, Dk = k.shape
-        Hv, Dv = v.shape[2], v.shape[3]
-        y = torch.empty((B, T, Hv, Dv), dtype=q.dtype, device=q.device)
-        tape = torch.empty((B, T, Hv, Dv), dtype=torch.float32, device=q.device)
-        out = torch.empty_like(state) if want_state else None
-        rc = _lib.load().dflash_gated_delta_tape(
-            _stream(), _ptr(q), _ptr(k), _ptr(v), _ptr(g), g.dim(), _ptr(beta), _code(q),
-            _ptr(state), _ptr(out), _code(state), _ptr(y), _ptr(tape),
-            _ptr(mask), _code(mask) if mask is not None else 0, B, T, Hk, Hv, Dk, Dv)
-        _lib.check(rc, "gated_delta_kernel_with_tape")
-        return y, out, tape
+        return _native.gated_delta(q, k, v, g, beta, state, mask, want_state)
 
     # -- block-causal SDPA -------------------------------------------------------
     @staticmethod
@@ -190,7 +160,7 @@ class DFlashKernels:
         out = torch.empty_like(y)
         rc = _lib.load().dflash_gdn_finish(_stream(), _ptr(y), _ptr(gate.to(y.dtype).contiguous()),
                                            _ptr(norm_weight.to(y.dtype).contiguous()), _ptr(out), _code(y), float(eps),
-                                           {"sigmoid": 0, "silu": 1}[gate_kind], B, T, Hv, Dv)
+                                           _GATE_KINDS[gate_kind], B, T, Hv, Dv)
         _lib.check(rc, "gdn_finish")
         return out
 
@@ -214,71 +184,9 @@ class DFlashKernels:
         it is None, an array this module keeps per device, stream and size.  ``one_launch=False`` runs the gated
         norm as a second launch instead.  ``out`` (optional, [B,T,Hv,Dv] in the input type) receives the gated norm
         instead of a fresh tensor; it may be ``gate`` itself (the library then takes the second launch)."""
-        _dev(mixed_qkv, conv_state, conv_weight, a_logits, b_logits, a_log, dt_bias, state, gate, norm_weight)
-        B, T, C = mixed_qkv.shape
-        if C != 2 * Hk * Dk + Hv * Dv:
-            raise DFlashError(f"gdn_layer: {C} channels, expected 2*{Hk}*{Dk} + {Hv}*{Dv}")
-        if a_logits.dim() != 3:
-            raise DFlashUnsupported("gdn_layer: one decay per head and step only (a_logits [B,T,Hv])")
-        if state.dtype != torch.float32:
-            raise DFlashUnsupported("gdn_layer: float32 state only")
-        K = int(conv_weight.shape[1])
-        dt = mixed_qkv.dtype
-        dv = mixed_qkv.device
-        x = mixed_qkv.contiguous()
-        w = conv_weight.to(dt).contiguous()
-        st = None if conv_state is None else conv_state.to(dt).contiguous()
-        a = a_logits.to(dt).contiguous()
-        bl = b_logits.to(dt).contiguous()
-        al = a_log.float().contiguous()
-        db = dt_bias.float().contiguous().reshape(-1)
-        state = state.contiguous()
-        k = torch.empty(B, T, Hk, Dk, dtype=dt, device=dv)
-        g = torch.empty(B, T, Hv, dtype=dt, device=dv)
-        y = torch.empty(B, T, Hv, Dv, dtype=dt, device=dv)
-        tape = torch.empty(B, T, Hv, Dv, dtype=torch.float32, device=dv)
-        new_state = torch.empty_like(state)
-        new_conv = torch.empty(B, K - 1, C, dtype=dt, device=dv)
-        q = torch.empty_like(k) if want_intermediates else None
-        v = torch.empty_like(y) if want_intermediates else None
-        beta = torch.empty_like(g) if want_intermediates else None
-        zg = nw = None
-        if gate is None:
-            out = None
-        if gate is not None:
-            if norm_weight is None or gate.shape != y.shape or norm_weight.shape != (Dv,):
-                raise DFlashError("gdn_layer: gate must be [B,T,Hv,Dv] and come with norm_weight [Dv]")
-            zg, nw = gate.to(dt).contiguous(), norm_weight.to(dt).contiguous()
-            if out is None:
-                out = torch.empty_like(y)
-            elif out.shape != y.shape or out.dtype != dt or not out.is_contiguous() or not out.is_cuda:
-                raise DFlashError("gdn_layer: out must be a contiguous device tensor [B,T,Hv,Dv] of the input type")
-            if not one_launch:
-                arrivals = None
-            elif arrivals is None:
-                key = (dv.index, torch.cuda.current_stream().cuda_stream, B * Hv)
-                arrivals = _ARRIVALS.get(key)
-                if arrivals is None:
-                    if torch.cuda.is_current_stream_capturing():
-                        # zeros created here would only be RECORDED (and live in the graph's private pool): an eager call
-                        # on this stream before the first replay would count into uninitialised memory
-                        raise DFlashError("gdn_layer: first use on this stream happens inside a graph capture; pass "
-                                          "`arrivals` (int32 zeros [B*Hv]) or call gdn_layer once on this stream beforehand")
-                    arrivals = _ARRIVALS[key] = torch.zeros(B * Hv, dtype=torch.int32, device=dv)
-            elif arrivals.dtype != torch.int32 or arrivals.numel() < B * Hv or not arrivals.is_contiguous():
-                raise DFlashError("gdn_layer: arrivals must be a contiguous int32 tensor of at least B*Hv elements")
-        else:
-            arrivals = None
-        rc = _lib.load().dflash_gdn_layer(
-            _stream(), _ptr(x), _ptr(st), _ptr(w), _ptr(a), _ptr(bl), _ptr(al), _ptr(db), _code(x),
-            float(q_scale), float(k_scale), float(eps), _ptr(state), _ptr(new_state), _ptr(k), _ptr(g), _ptr(tape),
-            _ptr(new_conv), _ptr(y), _ptr(zg), _ptr(nw), float(norm_eps), {"sigmoid": 0, "silu": 1}[gate_kind],
-            _ptr(out), _ptr(arrivals), _ptr(q), _ptr(v), _ptr(beta), B, T, Hk, Hv, Dk, Dv, K)
-        _lib.check(rc, "gdn_layer")
-        res = dict(out=out, y=y, state=new_state, tape=tape, k=k, g=g, conv_state=new_conv)
-        if want_intermediates:
-            res.update(q=q, v=v, beta=beta)
-        return res
+        return _native.gdn_layer(mixed_qkv, conv_state, conv_weight, a_logits, b_logits, a_log, dt_bias, state, Hk, Hv, Dk, Dv,
+                                 q_scale, k_scale, eps, gate, norm_weight, norm_eps, _GATE_KINDS[gate_kind], want_intermediates,
+                                 arrivals, one_launch, out)
 
     @staticmethod
     def batched_sdpa_2pass(queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, scale: float,
@@ -293,45 +201,17 @@ class DFlashKernels:
         shape/dtype).  ``return_lse`` additionally returns the
         float32 logsumexp [B,Hq,16]; ``kv_len`` (int32 [B] on the device) gives
         per-sequence key counts for ragged batches."""
-        if queries.dim() != 4 or keys.dim() != 4 or values.dim() != 4:
-            return None
-        _dev(queries, keys, values, kv_len, workspace, mask)
-        B, Hq, M, D = queries.shape
-        Hk, N = keys.shape[1], keys.shape[2]
         if mask is not None:
+            if queries.dim() != 4 or keys.dim() != 4 or values.dim() != 4:
+                return None
+            _dev(queries, keys, values, kv_len, workspace, mask)
             # additive [B,Hq,16,N] (anything that broadcasts to it), cast to the input type (:783-787)
+            shape = (*queries.shape[:3], keys.shape[2])
             try:
-                mask = mask.to(queries.dtype).expand(B, Hq, M, N).contiguous()
+                mask = mask.to(queries.dtype).expand(shape).contiguous()
             except RuntimeError:
-                raise DFlashError(f"batched_sdpa_2pass: mask {tuple(mask.shape)} does not broadcast to {(B, Hq, M, N)}")
-        if values.shape != keys.shape or values.shape[3] != D or keys.dtype != queries.dtype or values.dtype != queries.dtype:
-            return None
-        queries = queries.contiguous()
-        if keys.stride(3) != 1 or keys.stride(2) != D or keys.stride() != values.stride():
-            keys, values = keys.contiguous(), values.contiguous()
-        lib = _lib.load()
-        need = int(lib.dflash_sdpa_workspace_bytes(B, Hq, Hk, M, N, D))
-        if need == 0:
-            return None
-        if workspace is None:
-            workspace = torch.empty(need, dtype=torch.uint8, device=queries.device)
-        out = torch.empty_like(queries)
-        lse = torch.empty((B, Hq, M), dtype=torch.float32, device=queries.device) if return_lse else None
-        try:
-            code = _code(queries)
-        except DFlashUnsupported:
-            return None
-        tail = (code, float(scale), B, Hq, Hk, M, N, D, keys.stride(0), keys.stride(1), _ptr(kv_len), _ptr(workspace),
-                workspace.numel() * workspace.element_size())
-        if mask is None:
-            rc = lib.dflash_sdpa_block_causal(_stream(), _ptr(queries), _ptr(keys), _ptr(values), _ptr(out), _ptr(lse), *tail)
-        else:
-            rc = lib.dflash_sdpa_block_causal_masked(_stream(), _ptr(queries), _ptr(keys), _ptr(values), _ptr(mask),
-                                                     _ptr(out), _ptr(lse), *tail)
-        if rc == _lib.UNSUPPORTED:
-            return None
-        _lib.check(rc, "batched_sdpa_2pass")
-        return (out, lse) if return_lse else out
+                raise DFlashError(f"batched_sdpa_2pass: mask {tuple(mask.shape)} does not broadcast to {shape}")
+        return _native.sdpa(queries, keys, values, scale, mask, return_lse, kv_len, workspace)
 
     @staticmethod
     def batched_sdpa_2pass_append(queries: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -344,39 +224,7 @@ class DFlashKernels:
         tensor ``cache_len`` is given; ``n_keys`` is then the upper bound of cache_len + 16);
         ``k_new``/``v_new`` [B,Hk,16,D] are the block's rows, attended as keys n_keys-16 .. n_keys-1
         and written into those cache rows.  Returns None for unsupported shapes."""
-        _dev(queries, k_cache, v_cache, k_new, v_new, cache_len, workspace)
-        if queries.dim() != 4 or k_cache.dim() != 4 or k_cache.shape != v_cache.shape:
-            return None
-        B, Hq, M, D = queries.shape
-        Hk, cap = k_cache.shape[1], k_cache.shape[2]
-        if (k_new.shape != (B, Hk, M, D) or v_new.shape != (B, Hk, M, D) or k_cache.shape[3] != D
-                or any(t.dtype != queries.dtype for t in (k_cache, v_cache, k_new, v_new))):
-            return None
-        if not (M <= n_keys <= cap):
-            raise DFlashError(f"batched_sdpa_2pass_append: n_keys={n_keys} outside [{M}, capacity={cap}]")
-        if k_cache.stride(3) != 1 or k_cache.stride(2) != D or k_cache.stride() != v_cache.stride():
-            raise DFlashError("batched_sdpa_2pass_append: the caches must be row-contiguous and laid out alike")
-        queries, k_new, v_new = queries.contiguous(), k_new.contiguous(), v_new.contiguous()
-        lib = _lib.load()
-        need = int(lib.dflash_sdpa_workspace_bytes(B, Hq, Hk, M, n_keys, D))
-        if need == 0:
-            return None
-        if workspace is None:
-            workspace = torch.empty(need, dtype=torch.uint8, device=queries.device)
-        out = torch.empty_like(queries)
-        lse = torch.empty((B, Hq, M), dtype=torch.float32, device=queries.device) if return_lse else None
-        try:
-            code = _code(queries)
-        except DFlashUnsupported:
-            return None
-        rc = lib.dflash_sdpa_block_causal_append(
-            _stream(), _ptr(queries), _ptr(k_cache), _ptr(v_cache), _ptr(k_new), _ptr(v_new), _ptr(out), _ptr(lse),
-            code, float(scale), B, Hq, Hk, M, int(n_keys), D, k_cache.stride(0), k_cache.stride(1), _ptr(cache_len),
-            _ptr(workspace), workspace.numel() * workspace.element_size())
-        if rc == _lib.UNSUPPORTED:
-            return None
-        _lib.check(rc, "batched_sdpa_2pass_append")
-        return (out, lse) if return_lse else out
+        return _native.sdpa_append(queries, k_cache, v_cache, k_new, v_new, scale, n_keys, return_lse, cache_len, workspace)
 
     @staticmethod
     def batched_sdpa_2pass_paged(queries: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
@@ -392,48 +240,7 @@ class DFlashKernels:
         rows already cached, block excluded; the block's rows are stored into their pages).  The
         reference's cache is dense (``batchedSDPA2Pass``, DFlashKernels.swift:737-743, takes one
         [B,Hk,N,D] array), so paging has no counterpart there.  Returns None for unsupported shapes."""
-        _dev(queries, k_pool, v_pool, page_table, k_new, v_new, lengths, workspace)
-        if queries.dim() != 4 or k_pool.dim() != 4 or k_pool.shape != v_pool.shape or page_table.dim() != 2:
-            return None
-        B, Hq, M, D = queries.shape
-        num_pages, Hk, page_size = k_pool.shape[0], k_pool.shape[1], k_pool.shape[2]
-        if k_pool.shape[3] != D or k_pool.dtype != queries.dtype or v_pool.dtype != queries.dtype:
-            return None
-        if (k_new is None) != (v_new is None):
-            raise DFlashError("batched_sdpa_2pass_paged: k_new and v_new go together")
-        if k_new is not None and (k_new.shape != (B, Hk, M, D) or v_new.shape != (B, Hk, M, D)
-                                  or k_new.dtype != queries.dtype or v_new.dtype != queries.dtype):
-            return None
-        if page_table.dtype != torch.int32 or page_table.shape[0] != B or page_table.stride(1) != 1:
-            raise DFlashError("batched_sdpa_2pass_paged: page_table must be int32 [B, pages] with unit inner stride")
-        if k_pool.stride(3) != 1 or k_pool.stride(2) != D or k_pool.stride() != v_pool.stride():
-            raise DFlashError("batched_sdpa_2pass_paged: the pools must be row-contiguous and laid out alike")
-        if page_table.shape[1] * page_size < n_keys:
-            raise DFlashError(f"batched_sdpa_2pass_paged: {page_table.shape[1]} pages of {page_size} keys do not cover n_keys={n_keys}")
-        table_pitch = page_table.stride(0) if B > 1 else page_table.shape[1]      # a single row's stride means nothing
-        queries = queries.contiguous()
-        if k_new is not None:
-            k_new, v_new = k_new.contiguous(), v_new.contiguous()
-        lib = _lib.load()
-        need = int(lib.dflash_sdpa_workspace_bytes(B, Hq, Hk, M, n_keys, D))
-        if need == 0:
-            return None
-        if workspace is None:
-            workspace = torch.empty(need, dtype=torch.uint8, device=queries.device)
-        out = torch.empty_like(queries)
-        lse = torch.empty((B, Hq, M), dtype=torch.float32, device=queries.device) if return_lse else None
-        try:
-            code = _code(queries)
-        except DFlashUnsupported:
-            return None
-        rc = lib.dflash_sdpa_block_causal_paged(
-            _stream(), _ptr(queries), _ptr(k_pool), _ptr(v_pool), _ptr(page_table), table_pitch, page_size, num_pages,
-            k_pool.stride(0), k_pool.stride(1), _ptr(k_new), _ptr(v_new), _ptr(out), _ptr(lse), code, float(scale),
-            B, Hq, Hk, M, int(n_keys), D, _ptr(lengths), _ptr(workspace), workspace.numel() * workspace.element_size())
-        if rc == _lib.UNSUPPORTED:
-            return None
-        _lib.check(rc, "batched_sdpa_2pass_paged")
-        return (out, lse) if return_lse else out
+        return _native.sdpa_paged(queries, k_pool, v_pool, page_table, scale, n_keys, k_new, v_new, lengths, return_lse, workspace)
 
     @staticmethod
     def sdpa_fallback(queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, scale: float,
