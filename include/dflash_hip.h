@@ -347,6 +347,8 @@ int dflash_sdpa_block_causal_paged(void* stream,
  *   out[1] = commitCount   = 1 + acceptanceLen  (= steps to replay)
  *   out[2] = stagedFirstNext = posterior[acceptanceLen]
  *   out[3] = *start_inout += commitCount (start_inout may be NULL -> commitCount)
+ * out4 may also be pinned host memory: the four words are written at system scope, so a
+ * host that looks at them sees each as soon as the kernel has it.
  * ---------------------------------------------------------------------- */
 int dflash_match_acceptance_length(void* stream, const uint32_t* drafted, const uint32_t* posterior,
                                    int n, int32_t* out);

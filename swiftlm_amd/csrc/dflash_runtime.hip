@@ -30,14 +30,15 @@ __global__ void empty_kernel() {}
 
 static std::mutex g_init_mu;
 static int g_cus[64];
-static bool g_ready[64];
+static std::atomic<bool> g_ready[64];
 
 int ensure_init() {
     int dev = 0;
     DFLASH_HIP_TRY(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64) { set_error("device index %d out of range", dev); return DFLASH_INVALID; }
+    if (g_ready[dev].load(std::memory_order_acquire)) return 0;
     std::lock_guard<std::mutex> lock(g_init_mu);
-    if (g_ready[dev]) return 0;
+    if (g_ready[dev].load(std::memory_order_relaxed)) return 0;
     hipDeviceProp_t prop;
     DFLASH_HIP_TRY(hipGetDeviceProperties(&prop, dev));
     if (strncmp(prop.gcnArchName, "gfx950", 6) != 0) {
@@ -50,7 +51,7 @@ int ensure_init() {
     rc = gdn_device_setup();
     if (rc) return rc;
     g_cus[dev] = prop.multiProcessorCount;
-    g_ready[dev] = true;
+    g_ready[dev].store(true, std::memory_order_release);
     return 0;
 }
 
@@ -80,19 +81,22 @@ __global__ __launch_bounds__(64) void match_acceptance_kernel(const uint32_t* dr
     if (threadIdx.x == 0) out[0] = acc;
 }
 
+// One cycle's bookkeeping (DFlashRuntime.swift:544-571).  The words go out at system scope: out4 may be pinned host memory
+// that the host is looking at.
+__device__ __forceinline__ void store_accept(int acc, uint32_t staged, int32_t* start_inout, int32_t* out4) {
+    const int commit = 1 + acc;                           // :544
+    int start = commit;
+    if (start_inout) { start += *start_inout; *start_inout = start; }   // :571
+    const int32_t w[4] = {acc, commit, (int32_t)staged, start};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) __hip_atomic_store(out4 + i, w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ __launch_bounds__(64) void accept_commit_kernel(const uint32_t* verify_ids, const uint32_t* posterior, int V,
                                                            int32_t* start_inout, int32_t* out4) {
     // drafted = verify_ids[1:], posterior[:V-1]  (DFlashRuntime.swift:525-530)
     const int acc = V > 1 ? leading_matches(verify_ids + 1, posterior, V - 1) : 0;
-    if (threadIdx.x == 0) {
-        const int commit = 1 + acc;                       // :544
-        out4[0] = acc;
-        out4[1] = commit;
-        out4[2] = (int32_t)posterior[acc];                // :547
-        int start = commit;
-        if (start_inout) { start += *start_inout; *start_inout = start; }   // :571
-        out4[3] = start;
-    }
+    if (threadIdx.x == 0) store_accept(acc, posterior[acc], start_inout, out4);   // staged token: :547
 }
 
 // ---- greedy tokens over the verify logits, fused with the acceptance ---------
@@ -210,36 +214,43 @@ __global__ __launch_bounds__(kArgmaxThreads) void greedy_finish_kernel(GreedyArg
         __builtin_amdgcn_s_waitcnt(0xc07f);                       // lgkmcnt(0): this wave's LDS writes have landed
         __builtin_amdgcn_wave_barrier();
         const int acc = A.T > 1 ? leading_matches(A.verify_ids + 1, post_s, A.T - 1) : 0;
-        if (tid == 0) {
-            const int commit = 1 + acc;
-            A.out4[0] = acc;
-            A.out4[1] = commit;
-            A.out4[2] = (int32_t)post_s[acc];
-            int start = commit;
-            if (A.start_inout) { start += *A.start_inout; *A.start_inout = start; }
-            A.out4[3] = start;
-        }
+        if (tid == 0) store_accept(acc, post_s[acc], A.start_inout, A.out4);
     }
 }
 
 // ---- conv-state rebuild ----------------------------------------------------
 
-// out[b, j, :] = concat(snapshot [B,keep,C], qkv [B,T,C])[b, s + j, :], 16-byte pieces.
-__global__ __launch_bounds__(256) void rebuild_conv_kernel(const uint4* snap, const uint4* qkv, uint4* out, int keep,
-                                                           int T, int C16, int steps, const int32_t* steps_dev,
-                                                           int32_t* status) {
-    int s = steps_dev ? *steps_dev : steps;
-    if (status && (s < 0 || s > T) && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0)
-        atomicOr(status, DFLASH_STATUS_CONV_STEPS);
+// out[b, j, :] = concat(snapshot [B,keep,C], qkv [B,T,C])[b, s + j, :], 16-byte pieces, for every layer of the batch
+// (grid z = layer * B + b).  A hybrid stack rolls all its caches back at once: one launch for all windows, where a
+// launch per cache cost more than copying its 48 KB.
+template <int LAYERS> struct ConvBatch {
+    const uint4* snap[LAYERS];
+    const uint4* qkv[LAYERS];
+    uint4* out[LAYERS];
+};
+struct ConvArgs {
+    int B, keep, T, C16, steps;
+    const int32_t* steps_dev;
+    int32_t* status;
+};
+template <int LAYERS>
+__global__ __launch_bounds__(256) void rebuild_conv_kernel(ConvBatch<LAYERS> P, ConvArgs A) {
+    int s = A.steps_dev ? *A.steps_dev : A.steps;
+    if (A.status && (s < 0 || s > A.T) && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0)
+        atomicOr(A.status, DFLASH_STATUS_CONV_STEPS);
     s = s < 0 ? 0 : s;
-    const int b = blockIdx.z, j = blockIdx.y;
+    const int layer = LAYERS == 1 ? 0 : blockIdx.z / A.B;
+    const int b = LAYERS == 1 ? blockIdx.z : blockIdx.z - layer * A.B;
+    const uint4 *snap = P.snap[layer], *qkv = P.qkv[layer];
+    uint4* out = P.out[layer];
+    const int j = blockIdx.y;
     const int src = s + j;
-    if (src >= keep + T) return;     // clamped slice end (RecurrentRollbackCache.swift:156)
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < C16; i += gridDim.x * blockDim.x) {
+    if (src >= A.keep + A.T) return;     // clamped slice end (RecurrentRollbackCache.swift:156)
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < A.C16; i += gridDim.x * blockDim.x) {
         uint4 val;
-        if (src < keep) val = snap ? snap[((size_t)b * keep + src) * C16 + i] : make_uint4(0, 0, 0, 0);
-        else val = qkv[((size_t)b * T + (src - keep)) * C16 + i];
-        out[((size_t)b * keep + j) * C16 + i] = val;
+        if (src < A.keep) val = snap ? snap[((size_t)b * A.keep + src) * A.C16 + i] : make_uint4(0, 0, 0, 0);
+        else val = qkv[((size_t)b * A.T + (src - A.keep)) * A.C16 + i];
+        out[((size_t)b * A.keep + j) * A.C16 + i] = val;
     }
 }
 
@@ -296,8 +307,7 @@ extern "C" int dflash_profile_empty_launch(void* stream, int grid_x, int grid_y,
     DFLASH_REQUIRE(threads >= 64 && threads <= 1024 && threads % 64 == 0, "empty launch: threads=%d is not a multiple of 64 in [64, 1024]", threads);
     DFLASH_REQUIRE(lds_bytes >= 0 && lds_bytes <= 160 * 1024, "empty launch: lds_bytes=%d outside [0, 160 KB]", lds_bytes);
     LaunchBracket br(DFLASH_KERNEL_EMPTY, (hipStream_t)stream);
-    br.launch(empty_kernel, dim3(grid_x, grid_y, grid_z), dim3(threads), (size_t)lds_bytes);
-    DFLASH_HIP_TRY(hipGetLastError());
+    DFLASH_HIP_TRY(br.launch(empty_kernel, dim3(grid_x, grid_y, grid_z), dim3(threads), (size_t)lds_bytes));
     return DFLASH_OK;
 }
 
@@ -306,8 +316,7 @@ extern "C" int dflash_match_acceptance_length(void* stream, const uint32_t* draf
     int rc = ensure_init();
     if (rc) return rc;
     DFLASH_REQUIRE(out && n >= 0 && (n == 0 || (drafted && posterior)), "match_acceptance_length: bad arguments");
-    hipLaunchKernelGGL(match_acceptance_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, drafted, posterior, n, out);
-    DFLASH_HIP_TRY(hipGetLastError());
+    DFLASH_HIP_TRY(launch_kernel(match_acceptance_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, drafted, posterior, n, out));
     return DFLASH_OK;
 }
 
@@ -316,9 +325,7 @@ extern "C" int dflash_accept_commit(void* stream, const uint32_t* verify_ids, co
     int rc = ensure_init();
     if (rc) return rc;
     DFLASH_REQUIRE(verify_ids && posterior && out4 && V >= 1, "accept_commit: bad arguments");
-    hipLaunchKernelGGL(accept_commit_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, verify_ids, posterior, V,
-                       start_inout, out4);
-    DFLASH_HIP_TRY(hipGetLastError());
+    DFLASH_HIP_TRY(launch_kernel(accept_commit_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, verify_ids, posterior, V, start_inout, out4));
     return DFLASH_OK;
 }
 
@@ -361,13 +368,11 @@ static int greedy_common(void* stream, const void* logits, int dtype, int T, int
     hipStream_t st = (hipStream_t)stream;
     {
         LaunchBracket br(DFLASH_KERNEL_GREEDY_PARTIAL, st);
-        if (dtype == DFLASH_F32) br.launch(greedy_partial_kernel<float>, grid, dim3(kArgmaxThreads), 0, A);
-        else if (dtype == DFLASH_BF16) br.launch(greedy_partial_kernel<bf16_t>, grid, dim3(kArgmaxThreads), 0, A);
-        else br.launch(greedy_partial_kernel<f16_t>, grid, dim3(kArgmaxThreads), 0, A);
+        DFLASH_HIP_TRY(br.launch(dtype == DFLASH_F32 ? greedy_partial_kernel<float> : dtype == DFLASH_BF16 ? greedy_partial_kernel<bf16_t>
+                                                                                                          : greedy_partial_kernel<f16_t>,
+                                 grid, dim3(kArgmaxThreads), 0, A));
     }
-    DFLASH_HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(greedy_finish_kernel, dim3(1), dim3(kArgmaxThreads), 0, st, A);
-    DFLASH_HIP_TRY(hipGetLastError());
+    DFLASH_HIP_TRY(launch_kernel(greedy_finish_kernel, dim3(1), dim3(kArgmaxThreads), 0, st, A));
     return DFLASH_OK;
 }
 
@@ -387,29 +392,37 @@ extern "C" int dflash_greedy_accept_commit(void* stream, const void* logits, int
                          workspace, workspace_bytes);
 }
 
-extern "C" int dflash_rebuild_conv_state(void* stream, const void* snapshot_conv, const void* tape_qkv, void* out, int B,
-                                         int keep, int T, int C, int elem_bytes, int accepted_steps,
-                                         const int32_t* steps_dev) {
+int dflash::rebuild_conv_batched(void* stream, int n, const void* const* snapshot_conv, const void* const* tape_qkv, void* const* out,
+                                 int B, int keep, int T, int C, int elem_bytes, int accepted_steps, const int32_t* steps_dev) {
     int rc = ensure_init();
     if (rc) return rc;
-    DFLASH_REQUIRE(tape_qkv && out && B > 0 && keep > 0 && T >= 0 && C > 0, "rebuild_conv_state: bad arguments");
+    DFLASH_REQUIRE(B > 0 && keep > 0 && T >= 0 && C > 0, "rebuild_conv_state: bad arguments");
     DFLASH_REQUIRE(elem_bytes == 2 || elem_bytes == 4, "rebuild_conv_state: element size must be 2 or 4");
     DFLASH_REQUIRE(accepted_steps >= 0, "rebuild_conv_state: negative accepted_steps");
     DFLASH_REQUIRE(((long)C * elem_bytes) % 16 == 0, "rebuild_conv_state: row of %d x %d bytes is not a multiple of 16", C, elem_bytes);
-    DFLASH_REQUIRE(((uintptr_t)snapshot_conv | (uintptr_t)tape_qkv | (uintptr_t)out) % 16 == 0, "rebuild_conv_state: pointers must be 16-byte aligned");
-    DFLASH_REQUIRE(keep <= 65535 && B <= 65535, "rebuild_conv_state: keep or B too large");
-    {
-        const size_t win = (size_t)B * keep * C * elem_bytes, tape_bytes = (size_t)B * T * C * elem_bytes;
-        const uintptr_t o = (uintptr_t)out, q = (uintptr_t)tape_qkv, sn = (uintptr_t)snapshot_conv;
+    DFLASH_REQUIRE(keep <= 65535 && (long)B * n <= 65535, "rebuild_conv_state: keep or B too large");
+    const size_t win = (size_t)B * keep * C * elem_bytes, tape_bytes = (size_t)B * T * C * elem_bytes;
+    ConvBatch<DFLASH_MAX_BATCHED_LAYERS> P;
+    for (int l = 0; l < n; ++l) {
+        DFLASH_REQUIRE(tape_qkv[l] && out[l], "rebuild_conv_state: bad arguments");
+        const uintptr_t o = (uintptr_t)out[l], q = (uintptr_t)tape_qkv[l], sn = (uintptr_t)snapshot_conv[l];
+        DFLASH_REQUIRE((sn | q | o) % 16 == 0, "rebuild_conv_state: pointers must be 16-byte aligned");
         DFLASH_REQUIRE(!(o < q + tape_bytes && q < o + win) && !(sn && o < sn + win && sn < o + win),
                        "rebuild_conv_state: out overlaps an input");
+        P.snap[l] = (const uint4*)snapshot_conv[l]; P.qkv[l] = (const uint4*)tape_qkv[l]; P.out[l] = (uint4*)out[l];
     }
-    const int C16 = (int)(((long)C * elem_bytes) / 16);
-    dim3 grid((C16 + 255) / 256, keep, B);
-    hipLaunchKernelGGL(rebuild_conv_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint4*)snapshot_conv,
-                       (const uint4*)tape_qkv, (uint4*)out, keep, T, C16, accepted_steps, steps_dev, status_word());
-    DFLASH_HIP_TRY(hipGetLastError());
+    const ConvArgs A = {B, keep, T, (int)(((long)C * elem_bytes) / 16), accepted_steps, steps_dev, status_word()};
+    dim3 grid((A.C16 + 255) / 256, keep, B * n);
+    hipStream_t st = (hipStream_t)stream;
+    if (n == 1) DFLASH_HIP_TRY(launch_kernel(rebuild_conv_kernel<1>, grid, dim3(256), 0, st, ConvBatch<1>{{P.snap[0]}, {P.qkv[0]}, {P.out[0]}}, A));
+    else DFLASH_HIP_TRY(launch_kernel(rebuild_conv_kernel<DFLASH_MAX_BATCHED_LAYERS>, grid, dim3(256), 0, st, P, A));
     return DFLASH_OK;
+}
+
+extern "C" int dflash_rebuild_conv_state(void* stream, const void* snapshot_conv, const void* tape_qkv, void* out, int B,
+                                         int keep, int T, int C, int elem_bytes, int accepted_steps,
+                                         const int32_t* steps_dev) {
+    return rebuild_conv_batched(stream, 1, &snapshot_conv, &tape_qkv, &out, B, keep, T, C, elem_bytes, accepted_steps, steps_dev);
 }
 
 extern "C" int dflash_kv_append(void* stream, void* k_cache, void* v_cache, const void* k_new, const void* v_new, int B,
@@ -429,9 +442,8 @@ extern "C" int dflash_kv_append(void* stream, void* k_cache, void* v_cache, cons
     DFLASH_REQUIRE((long)B * Hk <= 65535, "kv_append: B*Hk too large");
     const int D16 = (int)(((long)D * elem_bytes) / 16);
     dim3 grid((M * D16 + 255) / 256, B * Hk);
-    hipLaunchKernelGGL(kv_append_kernel, grid, dim3(256), 0, (hipStream_t)stream, (uint4*)k_cache, (uint4*)v_cache,
-                       (const uint4*)k_new, (const uint4*)v_new, Hk, M, D16, (long)(kv_batch_stride * elem_bytes / 16),
-                       (long)(kv_head_stride * elem_bytes / 16), offset, offset_dev, capacity, new_len_dev, status_word());
-    DFLASH_HIP_TRY(hipGetLastError());
+    DFLASH_HIP_TRY(launch_kernel(kv_append_kernel, grid, dim3(256), 0, (hipStream_t)stream, (uint4*)k_cache, (uint4*)v_cache,
+                                 (const uint4*)k_new, (const uint4*)v_new, Hk, M, D16, (long)(kv_batch_stride * elem_bytes / 16),
+                                 (long)(kv_head_stride * elem_bytes / 16), offset, offset_dev, capacity, new_len_dev, status_word()));
     return DFLASH_OK;
 }

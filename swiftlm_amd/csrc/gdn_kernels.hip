@@ -78,13 +78,16 @@ __device__ __forceinline__ float requant_rt(int dtype, float v) {      // v afte
 // Tape replay
 // ===========================================================================
 
-struct ReplayBatch {
-    const void* tape[DFLASH_MAX_BATCHED_LAYERS];
-    const void* k[DFLASH_MAX_BATCHED_LAYERS];
-    const void* g[DFLASH_MAX_BATCHED_LAYERS];
-    const void* state_in[DFLASH_MAX_BATCHED_LAYERS];
-    void* state_out[DFLASH_MAX_BATCHED_LAYERS];
+// The layers' pointers travel in the kernel arguments.  A launch copies its whole argument block to device memory, so a
+// call for one layer (a rollback cache on its own) takes the table of one: 48 bytes instead of 2.5 KB.
+template <int LAYERS> struct ReplayBatch {
+    const void* tape[LAYERS];
+    const void* k[LAYERS];
+    const void* g[LAYERS];
+    const void* state_in[LAYERS];
+    void* state_out[LAYERS];
 };
+typedef ReplayBatch<DFLASH_MAX_BATCHED_LAYERS> ReplayTable;
 
 struct ReplayArgs {
     const void* mask;        // [B,T_tape] or null
@@ -106,8 +109,8 @@ constexpr int kReplayChunk = 16;  // steps staged in LDS at a time (8 for Dk = 2
 // span a row, so a 256-thread workgroup covers RPP = floor(1024/DK) rows per pass
 // and NR passes (when DK/4 does not divide 256 the last few threads only help
 // with staging).  Grid: x = Dv tiles, y = b*Hv + hv, z = layer.
-template <typename StateT, bool VEC_G, int DK, int NR>
-__global__ __launch_bounds__(kThreads) void tape_replay_kernel(ReplayBatch P, ReplayArgs A) {
+template <typename StateT, bool VEC_G, int DK, int NR, int LAYERS>
+__global__ __launch_bounds__(kThreads) void tape_replay_kernel(ReplayBatch<LAYERS> P, ReplayArgs A) {
     constexpr int TPR = DK / 4;
     constexpr int RPP = kThreads / TPR;
     constexpr int ROWS = RPP * NR;
@@ -122,7 +125,7 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(ReplayBatch P, Re
     asm volatile("" ::"s"(A.mask), "s"(A.steps_dev), "s"(A.verify_ids), "s"(A.posterior), "s"(A.start_inout), "s"(A.out4),
                  "s"(A.V), "s"(A.mask_dtype), "s"(A.tape_dtype), "s"(A.in_dtype), "s"(A.steps), "s"(A.skip_if_full),
                  "s"(A.T_tape), "s"(A.Hk), "s"(A.Hv), "s"(A.Dv));
-    const int layer = blockIdx.z;
+    const int layer = LAYERS == 1 ? 0 : blockIdx.z;
     const int bh = blockIdx.y;
     const int b = bh / A.Hv, hv = bh % A.Hv;
     const int hk = hv / (A.Hv / A.Hk);
@@ -296,26 +299,29 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(ReplayBatch P, Re
     }
 }
 
+template <typename StateT, bool VEC_G, int DK, int NR>
+static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, const ReplayArgs& A, int B, int n_layers) {
+    constexpr int ROWS = kThreads / (DK / 4) * NR;
+    dim3 grid((A.Dv + ROWS - 1) / ROWS, B * A.Hv, n_layers);
+    if (n_layers > 1) return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, DFLASH_MAX_BATCHED_LAYERS>, grid, dim3(kThreads), 0, P, A);
+    const ReplayBatch<1> one = {{P.tape[0]}, {P.k[0]}, {P.g[0]}, {P.state_in[0]}, {P.state_out[0]}};
+    return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, 1>, grid, dim3(kThreads), 0, one, A);
+}
+
 template <typename StateT, bool VEC_G, int DK>
-static int launch_replay_nr(hipStream_t st, const ReplayBatch& P, const ReplayArgs& A, int B, int n_layers) {
+static int launch_replay_nr(hipStream_t st, const ReplayTable& P, const ReplayArgs& A, int B, int n_layers) {
     constexpr int RPP = kThreads / (DK / 4);
     // Fewer, fatter workgroups once the grid already covers the chip several times over.
     const long wg1 = (long)((A.Dv + RPP - 1) / RPP) * B * A.Hv * n_layers;
     const int cus = num_compute_units();
     LaunchBracket br(DFLASH_KERNEL_TAPE_REPLAY, st);
-    if (wg1 >= 16L * cus && A.Dv >= RPP * 4) {
-        dim3 grid((A.Dv + RPP * 4 - 1) / (RPP * 4), B * A.Hv, n_layers);
-        br.launch(tape_replay_kernel<StateT, VEC_G, DK, 4>, grid, dim3(kThreads), 0, P, A);
-    } else {
-        dim3 grid((A.Dv + RPP - 1) / RPP, B * A.Hv, n_layers);
-        br.launch(tape_replay_kernel<StateT, VEC_G, DK, 1>, grid, dim3(kThreads), 0, P, A);
-    }
-    DFLASH_HIP_TRY(hipGetLastError());
+    if (wg1 >= 16L * cus && A.Dv >= RPP * 4) DFLASH_HIP_TRY((launch_replay_layers<StateT, VEC_G, DK, 4>(br, P, A, B, n_layers)));
+    else DFLASH_HIP_TRY((launch_replay_layers<StateT, VEC_G, DK, 1>(br, P, A, B, n_layers)));
     return DFLASH_OK;
 }
 
 template <typename StateT>
-static int launch_replay_state(hipStream_t st, const ReplayBatch& P, const ReplayArgs& A, int B, int n_layers,
+static int launch_replay_state(hipStream_t st, const ReplayTable& P, const ReplayArgs& A, int B, int n_layers,
                                int g_ndim, int Dk) {
     const bool vec = g_ndim == 4;
 #define DFLASH_REPLAY_CASE(DKV)                                                              \
@@ -366,7 +372,7 @@ static int replay_common(hipStream_t st, int n_layers, const void* const* tape, 
     DFLASH_SUPPORTED(state_dtype == DFLASH_F32 || state_dtype == in_dtype, "tape replay: state dtype must be f32 or the input dtype");
     if (mask) DFLASH_REQUIRE(mask_dtype >= DFLASH_F32 && mask_dtype <= DFLASH_U8, "tape replay: bad mask dtype");
 
-    ReplayBatch P;
+    ReplayTable P;
     for (int l = 0; l < n_layers; ++l) {
         DFLASH_REQUIRE(state_in[l] && state_out[l], "tape replay: null state pointer (layer %d)", l);
         DFLASH_REQUIRE(state_in[l] != state_out[l], "tape replay: state_in aliases state_out (layer %d)", l);
@@ -1475,9 +1481,7 @@ static int launch_gdn_layer(hipStream_t st, const GdnArgs& A, const GdnPrep& P, 
     const size_t lds = sizeof(GdnChunkLds<DK>);
     dim3 grid(A.Dv / kChunkRows, A.Hv, B);
     LaunchBracket br(DFLASH_KERNEL_GDN_LAYER, st);
-    if (A.in_dtype == DFLASH_BF16) br.launch(gdn_layer_kernel<DK, true>, grid, dim3(kThreads), lds, A, P);
-    else br.launch(gdn_layer_kernel<DK, false>, grid, dim3(kThreads), lds, A, P);
-    DFLASH_HIP_TRY(hipGetLastError());
+    DFLASH_HIP_TRY(br.launch(A.in_dtype == DFLASH_BF16 ? gdn_layer_kernel<DK, true> : gdn_layer_kernel<DK, false>, grid, dim3(kThreads), lds, A, P));
     return DFLASH_OK;
 }
 
@@ -1488,11 +1492,9 @@ static int launch_gdn_chunk(hipStream_t st, const GdnArgs& A, int B) {
     LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);
     const bool bf = A.in_dtype == DFLASH_BF16;
     const uint32_t hv_dv = ((uint32_t)A.Hv << 16) | (uint32_t)A.Dv, hk_t = ((uint32_t)A.Hk << 16) | (uint32_t)A.T;   // each below 2^16, checked by the caller
-    if (A.mask && bf) br.launch(gated_delta_chunk_kernel<true, DK, true>, grid, dim3(kThreads), lds, A.state_in, A.k, A.q, A.v, A.g, A.beta, hv_dv, hk_t, A);
-    else if (A.mask) br.launch(gated_delta_chunk_kernel<true, DK, false>, grid, dim3(kThreads), lds, A.state_in, A.k, A.q, A.v, A.g, A.beta, hv_dv, hk_t, A);
-    else if (bf) br.launch(gated_delta_chunk_kernel<false, DK, true>, grid, dim3(kThreads), lds, A.state_in, A.k, A.q, A.v, A.g, A.beta, hv_dv, hk_t, A);
-    else br.launch(gated_delta_chunk_kernel<false, DK, false>, grid, dim3(kThreads), lds, A.state_in, A.k, A.q, A.v, A.g, A.beta, hv_dv, hk_t, A);
-    DFLASH_HIP_TRY(hipGetLastError());
+    auto kern = A.mask ? (bf ? gated_delta_chunk_kernel<true, DK, true> : gated_delta_chunk_kernel<true, DK, false>)
+                       : (bf ? gated_delta_chunk_kernel<false, DK, true> : gated_delta_chunk_kernel<false, DK, false>);
+    DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), lds, A.state_in, A.k, A.q, A.v, A.g, A.beta, hv_dv, hk_t, A));
     return DFLASH_OK;
 }
 
@@ -1522,11 +1524,9 @@ static int launch_gdn_state(hipStream_t st, const GdnArgs& A, int B, int g_ndim,
     case DKV: {                                                                                        \
         dim3 grid((A.Dv + (kThreads / LPRV) - 1) / (kThreads / LPRV), B * A.Hv);                       \
         LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);                                               \
-        if (vec && A.mask) br.launch(gated_delta_tape_kernel<StateT, true, true, DKV, LPRV>, grid, dim3(kThreads), 0, A);        \
-        else if (vec) br.launch(gated_delta_tape_kernel<StateT, true, false, DKV, LPRV>, grid, dim3(kThreads), 0, A);            \
-        else if (A.mask) br.launch(gated_delta_tape_kernel<StateT, false, true, DKV, LPRV>, grid, dim3(kThreads), 0, A);         \
-        else br.launch(gated_delta_tape_kernel<StateT, false, false, DKV, LPRV>, grid, dim3(kThreads), 0, A);                    \
-        DFLASH_HIP_TRY(hipGetLastError());                                                             \
+        auto kern = vec ? (A.mask ? gated_delta_tape_kernel<StateT, true, true, DKV, LPRV> : gated_delta_tape_kernel<StateT, true, false, DKV, LPRV>)    \
+                        : (A.mask ? gated_delta_tape_kernel<StateT, false, true, DKV, LPRV> : gated_delta_tape_kernel<StateT, false, false, DKV, LPRV>); \
+        DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), 0, A));                                   \
         return DFLASH_OK;                                                                              \
     }
     switch (Dk) {

@@ -197,10 +197,8 @@ extern "C" int dflash_gdn_finish(void* stream, const void* y, const void* gate, 
     dim3 grid((unsigned)((rows + 3) / 4));
     hipStream_t st = (hipStream_t)stream;
     LaunchBracket br(DFLASH_KERNEL_GDN_FINISH, st);
-    if (in_dtype == DFLASH_F32) br.launch(gdn_finish_kernel<float>, grid, dim3(256), 0, A);
-    else if (in_dtype == DFLASH_BF16) br.launch(gdn_finish_kernel<bf16_t>, grid, dim3(256), 0, A);
-    else br.launch(gdn_finish_kernel<f16_t>, grid, dim3(256), 0, A);
-    DFLASH_HIP_TRY(hipGetLastError());
+    DFLASH_HIP_TRY(br.launch(in_dtype == DFLASH_F32 ? gdn_finish_kernel<float> : in_dtype == DFLASH_BF16 ? gdn_finish_kernel<bf16_t> : gdn_finish_kernel<f16_t>,
+                             grid, dim3(256), 0, A));
     return DFLASH_OK;
 }
 
@@ -233,9 +231,7 @@ extern "C" int dflash_gdn_prepare(void* stream, const void* mixed_qkv, const voi
     dim3 grid(2 * Hk + Hv + (A.vec_gate ? Hv : 1), T, B);
     hipStream_t st = (hipStream_t)stream;
     LaunchBracket br(DFLASH_KERNEL_GDN_PREPARE, st);
-    if (in_dtype == DFLASH_F32) br.launch(gdn_prepare_kernel<float>, grid, dim3(threads), 0, A);
-    else if (in_dtype == DFLASH_BF16) br.launch(gdn_prepare_kernel<bf16_t>, grid, dim3(threads), 0, A);
-    else br.launch(gdn_prepare_kernel<f16_t>, grid, dim3(threads), 0, A);
-    DFLASH_HIP_TRY(hipGetLastError());
+    DFLASH_HIP_TRY(br.launch(in_dtype == DFLASH_F32 ? gdn_prepare_kernel<float> : in_dtype == DFLASH_BF16 ? gdn_prepare_kernel<bf16_t> : gdn_prepare_kernel<f16_t>,
+                             grid, dim3(threads), 0, A));
     return DFLASH_OK;
 }

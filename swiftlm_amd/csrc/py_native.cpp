@@ -14,15 +14,18 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/EmptyTensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <chrono>
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <vector>
 
 #include "../../include/dflash_cache.h"
 #include "../../include/dflash_hip.h"
@@ -113,12 +116,13 @@ at::Tensor fresh(at::IntArrayRef size, at::ScalarType st, const at::Tensor& like
 void* stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
 
 // Runs a library call without the interpreter lock.
-template <typename F> int enqueue(F f) {
-    int rc;
+struct Unlocked {
     PyThreadState* ts = PyEval_SaveThread();
-    rc = f();
-    PyEval_RestoreThread(ts);
-    return rc;
+    ~Unlocked() { PyEval_RestoreThread(ts); }
+};
+template <typename F> int enqueue(F f) {
+    Unlocked u;
+    return f();
 }
 void check(int rc, const char* what) {
     if (rc == DFLASH_OK) return;
@@ -440,6 +444,171 @@ PyObject* sdpa_paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- acceptance ----------------------------------------------------------------
+
+// Four words that a kernel leaves in pinned host memory, waited for by looking at them.  The device-to-host copy of 16
+// bytes this replaces is a call into the copy engine's path with a wait of its own, and the 4-byte upload of `start` ahead
+// of it was another; both together took longer than the kernels.  kUnset is a value that none of the words can take: they
+// are counts and token ids below 2^31.
+class AcceptWords {
+    static constexpr int32_t kUnset = INT32_MIN;
+    at::Tensor host = at::Tensor(at::detail::empty_cpu({4}, at::kInt, /*pin_memory=*/true, std::nullopt));
+    bool there() const {
+        for (int i = 0; i < 4; ++i)
+            if (__atomic_load_n(words() + i, __ATOMIC_ACQUIRE) == kUnset) return false;
+        return true;
+    }
+public:
+    AcceptWords() { for (int i = 0; i < 4; ++i) words()[i] = kUnset; }
+    int32_t* words() const { return host.mutable_data_ptr<int32_t>(); }
+    // Looks for up to two milliseconds, then lets the runtime wait for the stream (a long queue ahead of the kernel, an error).
+    void wait() const {
+        const c10::hip::HIPStream st = c10::hip::getCurrentHIPStream();
+        Unlocked u;
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+        for (unsigned i = 1; !there(); ++i) {
+            __builtin_ia32_pause();
+            if (i % 256 == 0 && std::chrono::steady_clock::now() > until) {
+                st.synchronize();
+                break;
+            }
+        }
+    }
+};
+
+PyObject* accept_tuple(const AcceptWords& w, int64_t start, at::Tensor&& posterior) {
+    const int32_t* v = w.words();
+    PyObject* post = wrap(std::move(posterior));
+    return Py_BuildValue("(iiiLN)", v[0], v[1], v[2], (long long)(start + v[1]), post);
+}
+
+// (logits, suppress mask, verify_ids, start) -> (acceptance_len, commit_count, staged_first_next, start, posterior)
+PyObject* greedy_accept(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 4, "greedy_accept");
+    const at::Tensor &logits_ = tensor(a[0], "logits"), &mask_ = tensor_or_none(a[1], "suppress_token_mask"), &ids_ = tensor(a[2], "verify_ids");
+    const int64_t start = integer(a[3]);
+    need_rank(logits_, 2, "greedy_accept_commit", "logits");
+    const Held logits = held(logits_), mask = held_as(mask_, at::kByte), ids = held_as(ids_, at::kInt);
+    const int64_t T = logits->size(0), V = logits->size(1);
+    if (ids->dim() < 1 || ids->size(0) != T) raise(g_error, "greedy_accept_commit: one logits row per verify position");
+    const int lc = code(*logits);
+    at::Tensor post = fresh({T}, at::kInt, *logits);
+    at::Tensor ws = fresh({(int64_t)dflash_greedy_workspace_bytes((int)T, (int)V)}, at::kByte, *logits);
+    const AcceptWords out;
+    void* st = stream();
+    check(enqueue([&] {
+              return dflash_greedy_accept_commit(st, ptr(*logits), lc, (int)T, (int)V, (const uint8_t*)ptr(*mask), (const uint32_t*)ptr(*ids),
+                                                 nullptr, out.words(), (uint32_t*)ptr(post), ptr(ws), (size_t)ws.numel());
+          }),
+          "greedy_accept_commit");
+    out.wait();
+    return accept_tuple(out, start, std::move(post));
+    END_HANDLE_TH_ERRORS
+}
+
+// (verify_ids, posterior, start) -> (acceptance_len, commit_count, staged_first_next, start, None)
+PyObject* accept_commit(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 3, "accept_commit");
+    const at::Tensor &ids_ = tensor(a[0], "verify_ids"), &post_ = tensor(a[1], "posterior");
+    const int64_t start = integer(a[2]);
+    const Held ids = held_as(ids_, at::kInt), post = held_as(post_, at::kInt);
+    const int64_t V = ids->dim() ? ids->size(0) : 0;
+    if (!post->dim() || post->size(0) < V) raise(g_error, "accept_commit: posterior must cover every verify position");
+    const AcceptWords out;
+    void* st = stream();
+    check(enqueue([&] {
+              return dflash_accept_commit(st, (const uint32_t*)ptr(*ids), (const uint32_t*)ptr(*post), (int)V, nullptr, out.words());
+          }),
+          "accept_commit");
+    out.wait();
+    return accept_tuple(out, start, at::Tensor());
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- rollback caches: the handle as an integer -----------------------------------
+
+dflash_cache_t* handle(PyObject* o) {
+    void* p = PyLong_AsVoidPtr(o);
+    if (!p && PyErr_Occurred()) throw python_error();
+    return (dflash_cache_t*)p;
+}
+
+// (handle, slot, tensor or None) -> data pointer
+PyObject* cache_set_slot(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 3, "cache_set_slot");
+    void* p = nullptr;
+    if (a[2] != Py_None) {
+        if (!THPVariable_Check(a[2])) raise(PyExc_TypeError, "cache slots hold tensors");
+        const at::Tensor& t = THPVariable_Unpack(a[2]);
+        if (!t.is_cuda() || !t.is_contiguous()) raise(g_error, "cache slots hold contiguous device tensors");
+        p = t.data_ptr();
+    }
+    check(dflash_cache_set_slot(handle(a[0]), (int)integer(a[1]), p), "cache_set_slot");
+    return PyLong_FromVoidPtr(p);
+    END_HANDLE_TH_ERRORS
+}
+// (handle, slot) -> data pointer
+PyObject* cache_get_slot(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 2, "cache_get_slot");
+    return PyLong_FromVoidPtr(dflash_cache_get_slot(handle(a[0]), (int)integer(a[1])));
+    END_HANDLE_TH_ERRORS
+}
+// (handle) -> whether the cache is armed
+PyObject* cache_is_armed(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 1, "cache_is_armed");
+    return PyBool_FromLong(dflash_cache_is_armed(handle(a[0])));
+    END_HANDLE_TH_ERRORS
+}
+// (handle, prefix_len)
+PyObject* cache_arm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 2, "cache_arm");
+    check(dflash_cache_arm_rollback(handle(a[0]), integer(a[1])), "arm_rollback");
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+// (handle, tape, k, g, qkv or None, state) -> the contiguous tensors whose pointers the handle now holds
+PyObject* cache_record_tape(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 6, "cache_record_tape");
+    const at::Tensor &tape_ = tensor(a[1], "tape"), &k_ = tensor(a[2], "k"), &g_ = tensor(a[3], "g"), &qkv_ = tensor_or_none(a[4], "qkv"),
+                     &state = tensor(a[5], "state");
+    need_rank(k_, 4, "record_tape", "k");
+    need_rank(tape_, 4, "record_tape", "tape");
+    const Held tape = held(tape_), k = held(k_), g = held(g_), qkv = held_or_none(qkv_);
+    const bool q = qkv->defined();
+    check(dflash_cache_record_tape(handle(a[0]), ptr(*tape), code(*tape), ptr(*k), ptr(*g), code(*k), (int)g->dim(), ptr(*qkv),
+                                   q ? (int)qkv->element_size() : 2, code(state), (int)k->size(0), (int)k->size(1), (int)k->size(2),
+                                   (int)tape->size(2), (int)k->size(3), (int)tape->size(3), q ? (int)qkv->size(-1) : 0),
+          "record_tape");
+    PyObject* r = PyTuple_New(4);
+    if (!r) throw python_error();
+    const Held* all[4] = {&tape, &k, &g, &qkv};
+    for (int i = 0; i < 4; ++i) PyTuple_SET_ITEM(r, i, wrap(at::Tensor(**all[i])));
+    return r;
+    END_HANDLE_TH_ERRORS
+}
+// (handles, target_len, acceptance_length, drafted_tokens) -> (status, nanoseconds)
+PyObject* restore(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 4, "restore");
+    if (!PyList_Check(a[0])) raise(PyExc_TypeError, "restore: a list of handles expected");
+    std::vector<dflash_cache_t*> h((size_t)PyList_GET_SIZE(a[0]));
+    for (size_t i = 0; i < h.size(); ++i) h[i] = handle(PyList_GET_ITEM(a[0], (Py_ssize_t)i));
+    const int64_t target = integer(a[1]);
+    const int acc = (int)integer(a[2]), drafted = (int)integer(a[3]);
+    int64_t ns = 0;
+    void* st = stream();
+    const int rc = enqueue([&] { return dflash_restore_target_cache_after_acceptance(h.data(), (int)h.size(), st, target, acc, drafted, &ns); });
+    return Py_BuildValue("(iL)", rc, (long long)ns);
+    END_HANDLE_TH_ERRORS
+}
+
 // () -> the current stream's handle
 PyObject* current_stream(PyObject*, PyObject* const*, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -464,7 +633,10 @@ PyObject* set_errors(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     FAST("set_errors", set_errors), FAST("tape_replay", tape_replay), FAST("gated_delta", gated_delta),
     FAST("gdn_layer", gdn_layer),   FAST("sdpa", sdpa),               FAST("sdpa_append", sdpa_append),
-    FAST("sdpa_paged", sdpa_paged), FAST("current_stream", current_stream), {nullptr, nullptr, 0, nullptr},
+    FAST("sdpa_paged", sdpa_paged), FAST("current_stream", current_stream),
+    FAST("greedy_accept", greedy_accept), FAST("accept_commit", accept_commit), FAST("cache_set_slot", cache_set_slot),
+    FAST("cache_get_slot", cache_get_slot), FAST("cache_record_tape", cache_record_tape), FAST("cache_is_armed", cache_is_armed), FAST("cache_arm", cache_arm), FAST("restore", restore),
+    {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -95,15 +95,35 @@ void restore_snapshot(dflash_cache* c, int n_accepted, bool need_replay, ReplayJ
     job->c = c; job->post_state = post1; job->post_conv = post0; job->steps = steps;
 }
 
-int finish_rollback(const ReplayJob& j, void* stream) {
-    dflash_cache* c = j.c;
-    c->slot[1] = j.post_state;                                    // :126, the replayed state
-    if (c->keep <= 0) { c->slot[0] = nullptr; return DFLASH_OK; } // :142
-    if (!c->qkv) return DFLASH_OK;                                // :140, keeps the restored window
-    int rc = dflash_rebuild_conv_state(stream, c->snap[0], c->qkv, j.post_conv, c->B, c->keep, c->T, c->C,
-                                       c->qkv_elem_bytes, j.steps, nullptr);
-    if (rc) return rc;
-    c->slot[0] = j.post_conv;                                     // :127
+// Whether the conv window of a replayed cache is rebuilt (RecurrentRollbackCache.swift:139-158).
+bool rebuilds_window(const dflash_cache* c) { return c->keep > 0 && c->qkv; }
+bool same_window(const ReplayJob& a, const ReplayJob& b) {
+    const dflash_cache *x = a.c, *y = b.c;
+    return a.steps == b.steps && x->B == y->B && x->keep == y->keep && x->T == y->T && x->C == y->C && x->qkv_elem_bytes == y->qkv_elem_bytes;
+}
+
+// The conv windows of all jobs, one launch per group of equal shapes, and the slots as they are after the rollback.
+int finish_rollbacks(const std::vector<ReplayJob>& jobs, void* stream) {
+    std::vector<char> done(jobs.size(), 0);
+    for (size_t i = 0; i < jobs.size(); ++i) {
+        dflash_cache* c = jobs[i].c;
+        c->slot[1] = jobs[i].post_state;                          // :126, the replayed state
+        if (c->keep <= 0) c->slot[0] = nullptr;                   // :142
+        if (done[i] || !rebuilds_window(c)) continue;             // :140, without qkv the restored window stays
+        const void *snap[DFLASH_MAX_BATCHED_LAYERS], *qkv[DFLASH_MAX_BATCHED_LAYERS];
+        void* out[DFLASH_MAX_BATCHED_LAYERS];
+        size_t member[DFLASH_MAX_BATCHED_LAYERS];
+        int n = 0;
+        for (size_t j = i; j < jobs.size() && n < DFLASH_MAX_BATCHED_LAYERS; ++j) {
+            if (done[j] || !rebuilds_window(jobs[j].c) || !same_window(jobs[i], jobs[j]) || (long)(n + 1) * c->B > 65535) continue;
+            done[j] = 1;
+            snap[n] = jobs[j].c->snap[0]; qkv[n] = jobs[j].c->qkv; out[n] = jobs[j].post_conv;
+            member[n++] = j;
+        }
+        int rc = dflash::rebuild_conv_batched(stream, n, snap, qkv, out, c->B, c->keep, c->T, c->C, c->qkv_elem_bytes, jobs[i].steps, nullptr);
+        if (rc) return rc;
+        for (int m = 0; m < n; ++m) jobs[member[m]].c->slot[0] = out[m];   // :127
+    }
     return DFLASH_OK;
 }
 
@@ -125,11 +145,7 @@ int replay_jobs(const std::vector<ReplayJob>& jobs, void* stream) {
                                             jobs[i].steps, nullptr, 0, a->B, a->T, a->Hk, a->Hv, a->Dk, a->Dv);
         if (rc) return rc;
     }
-    for (const ReplayJob& j : jobs) {
-        int rc = finish_rollback(j, stream);
-        if (rc) return rc;
-    }
-    return DFLASH_OK;
+    return finish_rollbacks(jobs, stream);
 }
 
 }  // namespace

@@ -11,12 +11,13 @@ give the caches the reference's names.  ``cache[0]`` is the conv window
 from __future__ import annotations
 
 import ctypes as C
-from typing import List, Optional
+from typing import Optional
 
 import torch
 
 from . import _lib
-from .dflash_kernels import _code, _stream
+from ._lib import native as _native
+from .dflash_kernels import _stream
 
 
 class _NativeCache:
@@ -26,27 +27,23 @@ class _NativeCache:
         self._h = C.c_void_p(_lib.load().dflash_cache_create(self.KIND, conv_kernel_size))
         if not self._h:
             raise _lib.DFlashError("cache_create: " + _lib.last_error())
-        self._slots: List[Optional[torch.Tensor]] = [None, None]
+        self._handle = self._h.value
         self._by_ptr = {}
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None
-        if h:
-            _lib.load().dflash_cache_destroy(h)
+        load = getattr(_lib, "load", None)          # None while the interpreter shuts down
+        if h and load:
+            load().dflash_cache_destroy(h)
 
     # slots -------------------------------------------------------------------
     def __getitem__(self, i: int) -> Optional[torch.Tensor]:
-        p = _lib.load().dflash_cache_get_slot(self._h, i)
-        return self._by_ptr.get(p) if p else None
+        return self._by_ptr.get(_native.cache_get_slot(self._handle, i))
 
     def __setitem__(self, i: int, t: Optional[torch.Tensor]) -> None:
+        p = _native.cache_set_slot(self._handle, i, t)
         if t is not None:
-            if not t.is_cuda or not t.is_contiguous():
-                raise _lib.DFlashError("cache slots hold contiguous device tensors")
-            self._by_ptr[t.data_ptr()] = t
-        _lib.check(_lib.load().dflash_cache_set_slot(self._h, i, C.c_void_p(t.data_ptr()) if t is not None else None),
-                   "cache_set_slot")
-        self._slots[i] = t
+            self._by_ptr[p] = t
         if not self._holds_snapshot():
             self._forget_dead()
 
@@ -54,8 +51,8 @@ class _NativeCache:
         return False
 
     def _forget_dead(self) -> None:
-        live = {_lib.load().dflash_cache_get_slot(self._h, i) for i in (0, 1)}
-        self._by_ptr = {p: t for p, t in self._by_ptr.items() if p in live}
+        held, h = self._by_ptr, self._handle
+        self._by_ptr = {p: held[p] for p in (_native.cache_get_slot(h, 0), _native.cache_get_slot(h, 1)) if p in held}
 
     @property
     def offset(self) -> int:
@@ -96,29 +93,19 @@ class _RollbackCache(_NativeCache):
 
     @property
     def is_armed(self) -> bool:
-        return bool(_lib.load().dflash_cache_is_armed(self._h))
+        return _native.cache_is_armed(self._handle)
 
     def _holds_snapshot(self) -> bool:
-        return self.is_armed
+        return _native.cache_is_armed(self._handle)
 
     def arm_rollback(self, prefix_len: int = 0) -> None:
-        _lib.check(_lib.load().dflash_cache_arm_rollback(self._h, int(prefix_len)), "arm_rollback")
+        _native.cache_arm(self._handle, prefix_len)
 
     def record_tape(self, tape: torch.Tensor, k: torch.Tensor, g: torch.Tensor, qkv: Optional[torch.Tensor]) -> None:
         state = self[1]
         if state is None:
             raise _lib.DFlashError("record_tape: slot 1 (recurrent state) is empty")
-        tape, k, g = tape.contiguous(), k.contiguous(), g.contiguous()
-        qkv = None if qkv is None else qkv.contiguous()
-        self._tape_refs = (tape, k, g, qkv)
-        B, T, Hk, Dk = k.shape
-        Hv, Dv = tape.shape[2], tape.shape[3]
-        rc = _lib.load().dflash_cache_record_tape(
-            self._h, C.c_void_p(tape.data_ptr()), _code(tape), C.c_void_p(k.data_ptr()), C.c_void_p(g.data_ptr()),
-            _code(k), g.dim(), C.c_void_p(qkv.data_ptr()) if qkv is not None else None,
-            qkv.element_size() if qkv is not None else 2, _code(state), B, T, Hk, Hv, Dk, Dv,
-            qkv.shape[-1] if qkv is not None else 0)
-        _lib.check(rc, "record_tape")
+        self._tape_refs = _native.cache_record_tape(self._handle, tape, k, g, qkv, state)
 
     def rollback(self, n_accepted: int) -> None:
         rc = _lib.load().dflash_cache_rollback(self._h, _stream(), int(n_accepted))

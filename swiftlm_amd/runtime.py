@@ -9,13 +9,13 @@ are the caller's.
 
 from __future__ import annotations
 
-import ctypes as C
 from dataclasses import dataclass
 from typing import List, Sequence
 
 import torch
 
 from . import _lib
+from ._lib import native as _native
 from .dflash_kernels import _code, _ptr, _stream
 from .rollback_cache import RecurrentRollbackCache, _NativeCache, _RollbackCache
 
@@ -27,21 +27,6 @@ class AcceptResult:
     commit_count: int
     staged_first_next: int
     start: int
-
-
-_greedy_ws = {}
-
-
-def _greedy_workspace(T: int, V: int, device) -> torch.Tensor:
-    """One scratch tensor per (T, V, device, stream): launches sharing it must not overlap, which
-    one stream guarantees."""
-    key = (T, V, str(device), int(_stream().value or 0))
-    ws = _greedy_ws.get(key)
-    if ws is None:
-        need = int(_lib.load().dflash_greedy_workspace_bytes(T, V))
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        _greedy_ws[key] = ws
-    return ws
 
 
 class DFlashRuntime:
@@ -67,7 +52,7 @@ class DFlashRuntime:
         T, V = logits.shape
         m = None if suppress_token_mask is None else suppress_token_mask.to(torch.uint8).contiguous()
         out = torch.empty(T, dtype=torch.int32, device=logits.device)
-        ws = _greedy_workspace(T, V, logits.device)
+        ws = torch.empty(int(_lib.load().dflash_greedy_workspace_bytes(T, V)), dtype=torch.uint8, device=logits.device)
         rc = _lib.load().dflash_greedy_tokens_with_mask(_stream(), _ptr(logits), _code(logits), T, V, _ptr(m), _ptr(out),
                                                         _ptr(ws), ws.numel())
         _lib.check(rc, "greedy_tokens_with_mask")
@@ -77,20 +62,7 @@ class DFlashRuntime:
     def greedy_accept_commit(logits: torch.Tensor, suppress_token_mask, verify_ids: torch.Tensor, start: int):
         """The cycle's greedy tokens, acceptance length and commit bookkeeping in one call
         (DFlashRuntime.swift:513-547): returns (AcceptResult, posterior int32 [T])."""
-        logits = logits.contiguous()
-        T, V = logits.shape
-        if int(verify_ids.shape[0]) != T:
-            raise _lib.DFlashError("greedy_accept_commit: one logits row per verify position")
-        m = None if suppress_token_mask is None else suppress_token_mask.to(torch.uint8).contiguous()
-        v = verify_ids.to(torch.int32).contiguous()
-        post = torch.empty(T, dtype=torch.int32, device=logits.device)
-        out = torch.empty(4, dtype=torch.int32, device=logits.device)
-        st = torch.tensor([start], dtype=torch.int32, device=logits.device)
-        ws = _greedy_workspace(T, V, logits.device)
-        rc = _lib.load().dflash_greedy_accept_commit(_stream(), _ptr(logits), _code(logits), T, V, _ptr(m), _ptr(v), _ptr(st),
-                                                     _ptr(out), _ptr(post), _ptr(ws), ws.numel())
-        _lib.check(rc, "greedy_accept_commit")
-        a, c, s, n = out.tolist()
+        a, c, s, n, post = _native.greedy_accept(logits, suppress_token_mask, verify_ids, start)
         return AcceptResult(a, c, s, n), post
 
     # -- acceptance ----------------------------------------------------------------
@@ -110,20 +82,10 @@ class DFlashRuntime:
 
     @staticmethod
     def accept_commit(verify_ids: torch.Tensor, posterior: torch.Tensor, start: int) -> AcceptResult:
-        """One cycle's integer bookkeeping done on the device and read back in a single
-        16-byte copy (the reference blocks on ``.item()`` at DFlashRuntime.swift:525-530
+        """One cycle's integer bookkeeping done on the device and left in 16 bytes of
+        pinned host memory (the reference blocks on ``.item()`` at DFlashRuntime.swift:525-530
         and then derives commitCount / stagedFirstNext / start on the host, :544-571)."""
-        V = int(verify_ids.shape[0])
-        v = verify_ids.to(torch.int32).contiguous()
-        p = posterior.to(torch.int32).contiguous()
-        if p.shape[0] < V:
-            raise _lib.DFlashError("accept_commit: posterior must cover every verify position")
-        out = torch.empty(4, dtype=torch.int32, device=v.device)
-        st = torch.tensor([start], dtype=torch.int32, device=v.device)
-        rc = _lib.load().dflash_accept_commit(_stream(), _ptr(v), _ptr(p), V, _ptr(st), _ptr(out))
-        _lib.check(rc, "accept_commit")
-        a, c, s, n = out.tolist()
-        return AcceptResult(a, c, s, n)
+        return AcceptResult(*_native.accept_commit(verify_ids, posterior, start)[:4])
 
     # -- caches ----------------------------------------------------------------------
     @staticmethod
@@ -139,17 +101,12 @@ class DFlashRuntime:
         """``restoreTargetCacheAfterAcceptance`` (DFlashRuntime.swift:188-223); returns the
         nanoseconds spent enqueuing the rollbacks.  Every tape cache's replay goes out in one
         launch instead of one launch per cache."""
-        n = len(cache_entries)
-        arr = (C.c_void_p * max(n, 1))(*[c._h.value for c in cache_entries])
-        ns = C.c_int64(0)
-        rc = _lib.load().dflash_restore_target_cache_after_acceptance(
-            C.cast(arr, _lib.vpp), n, _stream(), int(target_len), int(acceptance_length), int(drafted_tokens),
-            C.byref(ns))
+        rc, ns = _native.restore([c._handle for c in cache_entries], int(target_len), int(acceptance_length), int(drafted_tokens))
         for c in cache_entries:
             if isinstance(c, _RollbackCache):
                 c._after_rollback()
         _lib.check(rc, "restore_target_cache_after_acceptance")
-        return int(ns.value)
+        return ns
 
 
 class DFlashEngine:
