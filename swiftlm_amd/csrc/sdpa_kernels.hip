@@ -91,7 +91,6 @@ struct SdpaArgs {
     int64_t kv_batch_stride, kv_head_stride;
     float scale_log2;   // scale * log2(e)
     int Hq, Hk, G, N, S, groups_per_kv;
-    int rows_total;     // B*Hq*16
     int len_bias;       // added to kv_len_dev[b]: 0, or 16 when the device count excludes the block
     // Paged K/V (PAGED instantiations): key n of sequence b lives in page page_table[b * table_stride + (n >> page_shift)]
     // of the pool, at row n & (page_size - 1); k, v point at the pools, kv_batch_stride is the page pitch and
@@ -100,6 +99,8 @@ struct SdpaArgs {
     int page_shift, table_stride, num_pages;
     int32_t* status;         // device status word (dflash_set_status_word), or null
     uint32_t gpk_magic, S_magic;   // fast_div_magic of groups_per_kv and S
+    float* lse;              // S == 1: part_o is the output itself and this (or null) its logsumexp; no combine follows
+    int B, balance;          // balance: sequences of a ragged batch share the B * S splits by their lengths (RaggedShare)
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -206,6 +207,34 @@ template <int D> struct SdpaLds {
     static constexpr int BYTES = RING_END > EPI ? RING_END : EPI;
 };
 
+// Ragged batches.  With S splits for every sequence, a launch lasts as long as the longest sequence takes S workgroups,
+// while those of the shorter ones are done early and their compute units idle: four sequences of 8K to 64K keys ran at
+// 4.2 TB/s.  Instead the B * S workgroups of a (KV head, head group) are dealt to the sequences in proportion to their
+// key counts, which only the device knows: every wave loads the counts (one per lane, B <= 64), finds the smallest number
+// L of tiles per workgroup with sum(ceil(tiles_b / L)) <= B * S, and takes its place in that sequence of shares.  The
+// combine kernel repeats the computation for its row's sequence.
+struct RaggedShare {
+    int n_lane, s_lane;      // lane b: key count and splits of sequence b (0 beyond B)
+};
+__device__ __forceinline__ int wave_sum_int(int x) { return (int)butterfly_sum<64>((float)x); }   // exact below 2^24
+__device__ __forceinline__ RaggedShare ragged_share(const int32_t* len_dev, int bias, int N, int B, int W, int lane) {
+    int n = len_dev[lane < B ? lane : B - 1] + bias;
+    n = n < kM ? kM : (n > N ? N : n);
+    n = lane < B ? n : 0;
+    const int nt = (n + kBN - 1) / kBN;
+    const int total = wave_sum_int(nt), longest = (int)wave_max((float)nt);
+    int L = (total + W - 1) / W;
+    const int least = (longest + kMaxSplits - 1) / kMaxSplits;       // a sequence takes kMaxSplits splits at most
+    L = L < least ? least : L;
+    int s;
+    for (;;) {                                                       // ends: with L = longest every sequence takes one split, and B <= W
+        s = (nt + L - 1) / L;
+        if (L >= longest || wave_sum_int(s) <= W) break;
+        ++L;
+    }
+    return {n, s};
+}
+
 // The t-th tile of a split: tiles are dealt in rows of S neighbouring tiles, one per split.
 __device__ __forceinline__ int tile_index(int split, int t, int S) { return t * S + split; }
 
@@ -225,7 +254,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     asm volatile("" ::"s"(A.q), "s"(A.k), "s"(A.v), "s"(A.k_new), "s"(A.v_new), "s"(A.k_cache), "s"(A.v_cache), "s"(A.part_o),
                  "s"(A.part_m), "s"(A.part_l), "s"(A.kv_len_dev), "s"(A.mask), "s"(A.kv_batch_stride), "s"(A.kv_head_stride));
     asm volatile("" ::"s"(A.scale_log2), "s"(A.Hq), "s"(A.Hk), "s"(A.G), "s"(A.N), "s"(A.S), "s"(A.groups_per_kv),
-                 "s"(A.rows_total), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages),
+                 "s"(A.balance), "s"(A.B), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages),
                  "s"(A.status), "s"(A.gpk_magic), "s"(A.S_magic));
 
     const int tid = threadIdx.x;
@@ -233,10 +262,25 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool producer = wave >= 4;
     const int c = lane & 31, h = lane >> 5;
-    const int split = blockIdx.x;
     const int hk = (int)fast_div(blockIdx.y, (uint32_t)A.groups_per_kv, A.gpk_magic);
     const int hg0 = ((int)blockIdx.y - hk * A.groups_per_kv) * kHeadsPerWG;
-    const int b = blockIdx.z;
+    int split = blockIdx.x, b = blockIdx.z, S = A.S, Nb_share = 0;
+    if (A.balance) {                                         // uniform
+        const int W = A.B * A.S, w = (int)blockIdx.z * A.S + (int)blockIdx.x;
+        const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, W, lane);
+        if (A.status && w == 0 && blockIdx.y == 0 && wave == 0 && lane < A.B) {
+            const int n = A.kv_len_dev[lane] + A.len_bias;
+            if (n < kM || n > A.N) atomicOr(A.status, DFLASH_STATUS_SDPA_LEN);
+        }
+        int first = 0;
+        b = -1;
+        for (int i = 0; i < A.B; ++i) {
+            const int si = __builtin_amdgcn_readlane(sh.s_lane, i);
+            if (b < 0 && w < first + si) { b = i; split = w - first; S = si; Nb_share = __builtin_amdgcn_readlane(sh.n_lane, i); }
+            first += si;
+        }
+        if (b < 0) return;                                   // more workgroups than tiles
+    }
     const int hcount = (A.G - hg0) < kHeadsPerWG ? (A.G - hg0) : kHeadsPerWG;
 
     // Paged: each producer wave keeps the page-table entries of this workgroup's next 64 tiles in a register, one
@@ -248,7 +292,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     auto load_entries = [&](int base) -> int {
         // no branch and no arithmetic on the value here: the wait for it then sits at its first use, not at the load
         const int nt_max = (A.N + kBN - 1) / kBN;
-        int tile = tile_index(split, base + lane, A.S);
+        int tile = tile_index(split, base + lane, S);
         tile = tile < nt_max ? tile : nt_max - 1;
         return A.page_table[(size_t)b * A.table_stride + ((tile * kBN) >> A.page_shift)];
     };
@@ -311,7 +355,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     const unsigned char* knew = reinterpret_cast<const unsigned char*>(A.k_new) + ((size_t)b * A.Hk + hk) * kM * L::ROWB;
     const unsigned char* vnew = reinterpret_cast<const unsigned char*>(A.v_new) + ((size_t)b * A.Hk + hk) * kM * L::ROWB;
     asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(len_raw) : "s"(kbase), "s"(vbase), "s"(knew), "s"(vnew));
-    int Nb = A.kv_len_dev ? len_raw + A.len_bias : A.N;
+    int Nb = A.balance ? Nb_share : (A.kv_len_dev ? len_raw + A.len_bias : A.N);
     if (A.status && (Nb < kM || Nb > A.N) && split == 0 && blockIdx.y == 0 && tid == 0) atomicOr(A.status, DFLASH_STATUS_SDPA_LEN);
     Nb = Nb < kM ? kM : (Nb > A.N ? A.N : Nb);
     const int nt = (Nb + kBN - 1) / kBN;
@@ -320,10 +364,17 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     // apart, which the memory system serves faster.  Below, t counts this split's own tiles (0 .. t_end-1) and
     // key_of(t) is the first key of its t-th tile.
     const int t_begin = 0;
-    const int t_full = (int)fast_div((uint32_t)nt, (uint32_t)A.S, A.S_magic);    // rows of S tiles that every split takes part in
-    const int t_end = t_full + (tile_index(split, t_full, A.S) < nt ? 1 : 0);
+    const int t_full = A.balance ? nt / S : (int)fast_div((uint32_t)nt, (uint32_t)S, A.S_magic);    // rows of S tiles that every split takes part in
+    const int t_end = t_full + (tile_index(split, t_full, S) < nt ? 1 : 0);
     const int t_last = t_end - 1;
-    auto key_of = [&](int t) { return tile_index(split, t, A.S) * kBN; };
+    auto key_of = [&](int t) { return tile_index(split, t, S) * kBN; };
+    // Where the split's partial rows and statistics go: rows [slot][Hq * 16][D]; statistics [row][split], in a balanced
+    // launch [row of the sequence][workgroup], so that a sequence's splits are neighbours either way.
+    const int hqm = A.Hq * kM;
+    const int slot = A.balance ? (int)blockIdx.z * A.S + (int)blockIdx.x : split * A.B + b;
+    auto stat_at = [&](int row_in_seq) -> size_t {
+        return A.balance ? (size_t)row_in_seq * (A.B * A.S) + slot : ((size_t)b * hqm + row_in_seq) * A.S + split;
+    };
 
     // Byte offset of key n's row from kbase / vbase (the K and V pools share one layout), for the rows that are
     // looked up one by one: those of the fused append.  Paged: the page comes from the table, clamped to the pool.
@@ -348,7 +399,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
         // 16-byte pieces of the block's rows, dealt evenly over the splits of the KV head: a handful per workgroup,
         // read and written by the first compute wave in one round trip.
         const int pieces = kM * L::CPR;
-        const int per = (pieces + A.S - 1) / A.S;
+        const int per = (pieces + S - 1) / S;
         const u32x4_t* ksrc = reinterpret_cast<const u32x4_t*>(knew);
         const u32x4_t* vsrc = reinterpret_cast<const u32x4_t*>(vnew);
         for (int i0 = 0; i0 < per; i0 += 64) {
@@ -365,8 +416,9 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     if (t_begin >= t_end) {   // empty split: tell the combine kernel to ignore it
         wait_vmcnt<0>();                             // the Q requests must have landed before the wave ends
         if (row_valid && h == 0) {
-            A.part_m[row_id * A.S + split] = -INFINITY;
-            A.part_l[row_id * A.S + split] = 0.f;
+            const size_t at = stat_at(hq * kM + qi);
+            A.part_m[at] = -INFINITY;
+            A.part_l[at] = 0.f;
         }
         return;
     }
@@ -735,9 +787,14 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
 
     // ---- epilogue: partial statistics and O rows (through LDS for coalesced stores) ----
     const float l_tot = l_run + __shfl_xor(l_run, 32);
-    if (row_valid && h == 0) {      // written through like the partial rows: 4-byte fragments of lines shared with other splits
-        __hip_atomic_store(A.part_m + row_id * A.S + split, m_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(A.part_l + row_id * A.S + split, l_tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (row_valid && h == 0) {
+        if (A.S == 1) {             // the only split: this is the result
+            if (A.lse) A.lse[row_id] = (m_run + log2f(l_tot)) * 0.6931471805599453f;
+        } else {                    // written through like the partial rows: 4-byte fragments of lines shared with other splits
+            const size_t at = stat_at(hq * kM + qi);
+            __hip_atomic_store(A.part_m + at, m_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(A.part_l + at, l_tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
     if (wave_active) {
         const float inv_l = l_tot > 0.f ? 1.f / l_tot : 0.f;
@@ -754,11 +811,11 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_s_waitcnt(0xc07f);
         const int rows = (hcount - 2 * cw) >= 2 ? 32 : 16;
-        const size_t rid0 = ((size_t)b * A.Hq + hk * A.G + hg0 + 2 * cw) * kM;
+        const size_t rid0 = (size_t)slot * hqm + (size_t)(hk * A.G + hg0 + 2 * cw) * kM;
         constexpr int PER_ROW = D / 8;
         constexpr int RPP = 64 / PER_ROW;
         const int rsub = lane / PER_ROW, d = (lane % PER_ROW) * 8;
-        uint16_t* dst = A.part_o + ((size_t)split * A.rows_total + rid0) * D + d;
+        uint16_t* dst = A.part_o + rid0 * D + d;
 #pragma unroll
         for (int r0 = 0; r0 < 32; r0 += 8 * RPP) {
             u32x4_t o[8];
@@ -778,16 +835,34 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     }
 }
 
-// One workgroup per output row (b, hq, i): merges the S partials.
+// Merging the partials of a row (b, hq, i).  Where they are: row r of sequence b has its partial rows at
+// slot * Hq*16 + r for `S` consecutive slots and its statistics at stat .. stat + S - 1.
 struct CombineArgs {
     const uint16_t* part_o;
     const float* part_m;
     const float* part_l;
     uint16_t* out;
     float* lse;
-    int S;
+    int S, B, hqm;           // hqm = Hq * 16
+    int rows;                // B * hqm
+    int balance;             // ragged shares (RaggedShare): the fields below are theirs
+    const int32_t* kv_len_dev;
+    int len_bias, N;
 };
+struct RowParts { const float *m, *l; const uint16_t* o; int S; size_t pitch; };   // o: the first slot's row; pitch: elements from slot to slot
+__device__ __forceinline__ RowParts row_parts(const CombineArgs& A, int row, int D, int lane) {
+    if (!A.balance) {
+        const size_t stat = (size_t)row * A.S;
+        return {A.part_m + stat, A.part_l + stat, A.part_o + (size_t)row * D, A.S, (size_t)A.rows * D};
+    }
+    const int W = A.B * A.S, b = row / A.hqm, r = row - b * A.hqm;
+    const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, W, lane);
+    const int first = wave_sum_int(lane < b ? sh.s_lane : 0);
+    const size_t stat = (size_t)r * W + first;
+    return {A.part_m + stat, A.part_l + stat, A.part_o + ((size_t)first * A.hqm + r) * D, __builtin_amdgcn_readlane(sh.s_lane, b), (size_t)A.hqm * D};
+}
 
+// One workgroup per row, for many splits: up to 16 partial rows per thread, all in flight at once.
 template <typename Tag, int D>
 __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineArgs A) {
     constexpr int TPG = D / 8;                     // threads spanning one row, 8 elements (16 B) each
@@ -801,27 +876,27 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
     asm volatile("" ::"s"(A.part_o), "s"(A.part_m), "s"(A.part_l), "s"(A.out), "s"(A.lse), "s"(A.S));   // one burst of argument loads
     const size_t row = blockIdx.x;
     const int tid = threadIdx.x;
-    const float* pm = A.part_m + row * A.S;
-    const float* pl = A.part_l + row * A.S;
+    const RowParts R = row_parts(A, (int)row, D, tid & 63);
+    const int S = R.S;
     const int grp = tid / TPG, d8 = (tid % TPG) * 8;
-    const uint16_t* po = A.part_o + row * D + d8;
+    const uint16_t* po = R.o + d8;
 
     // Everything the row needs is requested in one go: the statistics of this thread's splits (tid and, beyond 256
     // splits, tid + 256; addresses clamped, values dropped) and the first UNROLL partial rows of its group.  Asked
     // for one after the other -- maxima, then sums, then rows -- they are three dependent trips to memory.
-    const int sa = tid < A.S ? tid : A.S - 1, sb = tid + kCombineThreads < A.S ? tid + kCombineThreads : A.S - 1;
-    float m0 = pm[sa], m1 = pm[sb];
-    const float l0 = pl[sa], l1 = pl[sb];
+    const int sa = tid < S ? tid : S - 1, sb = tid + kCombineThreads < S ? tid + kCombineThreads : S - 1;
+    float m0 = R.m[sa], m1 = R.m[sb];
+    const float l0 = R.l[sa], l1 = R.l[sb];
     u32x4_t raw[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
         const int sp = grp + u * NG;
         // Loaded without looking at the weight (a branch per load makes the loads wait for one another); the rows of
         // empty splits hold no data, whatever was read from them is dropped below.
-        raw[u] = *reinterpret_cast<const u32x4_t*>(po + (size_t)(sp < A.S ? sp : 0) * gridDim.x * D);
+        raw[u] = *reinterpret_cast<const u32x4_t*>(po + (size_t)(sp < S ? sp : 0) * R.pitch);
     }
-    if (tid >= A.S) m0 = -INFINITY;
-    if (tid + kCombineThreads >= A.S) m1 = -INFINITY;
+    if (tid >= S) m0 = -INFINITY;
+    if (tid + kCombineThreads >= S) m1 = -INFINITY;
 
     // global max
     float mx = wave_max(fmaxf(m0, m1));
@@ -831,8 +906,8 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
     // weights and denominator (the partial rows are O / l: weight by l)
     const float w0 = m0 == -INFINITY ? 0.f : fast_exp2(m0 - mx) * l0;
     const float w1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - mx) * l1;
-    if (tid < A.S) w_s[tid] = w0;
-    if (tid + kCombineThreads < A.S) w_s[tid + kCombineThreads] = w1;
+    if (tid < S) w_s[tid] = w0;
+    if (tid + kCombineThreads < S) w_s[tid + kCombineThreads] = w1;
     float lsum = butterfly_sum<64>(w0 + w1);
     if ((tid & 63) == 0) reds_s[tid >> 6] = lsum;
     __syncthreads();
@@ -842,13 +917,13 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-    for (int s0 = grp; s0 < A.S; s0 += NG * UNROLL) {
+    for (int s0 = grp; s0 < S; s0 += NG * UNROLL) {
         float w[UNROLL];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             const int sp = s0 + u * NG;
-            w[u] = sp < A.S ? w_s[sp] : 0.f;
-            if (s0 != grp) raw[u] = *reinterpret_cast<const u32x4_t*>(po + (size_t)(sp < A.S ? sp : 0) * gridDim.x * D);
+            w[u] = sp < S ? w_s[sp] : 0.f;
+            if (s0 != grp) raw[u] = *reinterpret_cast<const u32x4_t*>(po + (size_t)(sp < S ? sp : 0) * R.pitch);
         }
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
@@ -872,12 +947,86 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
     if (tid == 0 && A.lse) A.lse[row] = (mx + log2f(lsum)) * 0.6931471805599453f;
 }
 
+// One wave per row, for few splits (a batch or many KV heads fill the chip, a short context has few tiles): no LDS, no
+// barrier, U partial rows per lane in flight.  A workgroup per row would fetch 16 rows per thread whatever S is and run
+// thousands of workgroups: 13 us for 4096 rows of 4 splits (B=8, Hq=32, D=128), where this takes 4.
+template <typename Tag, int D, int U>
+__global__ __launch_bounds__(kCombineThreads) void sdpa_combine_wave_kernel(CombineArgs A) {
+    constexpr int TPG = D / 8;                     // lanes spanning one row, 8 elements each
+    constexpr int SG = 64 / TPG;                   // split groups of the wave
+    asm volatile("" ::"s"(A.part_o), "s"(A.part_m), "s"(A.part_l), "s"(A.out), "s"(A.lse), "s"(A.S));
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * (kCombineThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row >= A.rows) return;                     // whole waves; no barrier follows
+    const RowParts R = row_parts(A, row, D, lane);
+    const int S = R.S, grp = lane / TPG, d8 = (lane % TPG) * 8;
+    const uint16_t* po = R.o + d8;
+    // the statistics of split `lane` and the first U partial rows of the group in one round trip
+    float m0 = R.m[lane < S ? lane : S - 1];
+    const float l0 = R.l[lane < S ? lane : S - 1];
+    u32x4_t raw[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int sp = grp + u * SG;
+        raw[u] = *reinterpret_cast<const u32x4_t*>(po + (size_t)(sp < S ? sp : 0) * R.pitch);
+    }
+    if (lane >= S) m0 = -INFINITY;
+    float mx = m0;
+    for (int s0 = 64; s0 < S; s0 += 64) mx = fmaxf(mx, s0 + lane < S ? R.m[s0 + lane] : -INFINITY);   // rare: more than 64 splits
+    mx = wave_max(mx);
+
+    float acc[8], lpart = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    for (int s0 = 0; s0 < S; s0 += 64) {
+        if (s0) m0 = s0 + lane < S ? R.m[s0 + lane] : -INFINITY;
+        const float l = s0 == 0 ? l0 : (s0 + lane < S ? R.l[s0 + lane] : 0.f);
+        const float w0 = m0 == -INFINITY ? 0.f : fast_exp2(m0 - mx) * l;
+        lpart += w0;
+        for (int i0 = 0; i0 < 64 && s0 + i0 < S; i0 += SG * U) {
+            if (s0 + i0) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int sp = s0 + i0 + grp + u * SG;
+                    raw[u] = *reinterpret_cast<const u32x4_t*>(po + (size_t)(sp < S ? sp : 0) * R.pitch);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float w = __shfl(w0, i0 + grp + u * SG);      // 0 for splits at or beyond S
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t x = w == 0.f ? 0u : raw[u][e];    // the rows of empty splits hold no data
+                    acc[2 * e] = fmaf(w, Tag::to_f32((uint16_t)(x & 0xffffu)), acc[2 * e]);
+                    acc[2 * e + 1] = fmaf(w, Tag::to_f32((uint16_t)(x >> 16)), acc[2 * e + 1]);
+                }
+            }
+        }
+    }
+    const float lsum = butterfly_sum<64>(lpart);
+    // the split groups' sums: lanes TPG and 2 TPG .. apart
+#pragma unroll
+    for (int o = TPG; o < 64; o *= 2)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += __shfl_xor(acc[e], o);
+    const float inv = lsum == 0.f ? 1.f : 1.f / lsum;       // divide unless the sum is 0 (DFlashKernels.swift:711)
+    if (grp == 0) {
+        u32x4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (uint32_t)Tag::cvt(acc[2 * e] * inv) | ((uint32_t)Tag::cvt(acc[2 * e + 1] * inv) << 16);
+        *reinterpret_cast<u32x4_t*>(A.out + (size_t)row * D + d8) = o;
+    }
+    if (lane == 0 && A.lse) A.lse[row] = (mx + log2f(lsum)) * 0.6931471805599453f;
+}
+
 // ---- host side -------------------------------------------------------------
 
+constexpr int kDirectTiles = 4;
 static int choose_splits(int B, int Hk, int groups_per_kv, int N) {
     const int nt = (N + kBN - 1) / kBN;
     const int cus = num_compute_units();
     const int per = B * Hk * groups_per_kv;      // workgroups per split index
+    if (nt <= kDirectTiles) return 1;
     // How many workgroups W = per * S the key axis is spread over.  Every split pays a fixed price -- its partial rows,
     // written once and read back by the combine kernel, are as large as 4 tiles of K/V, and a launch drains them all at
     // once -- while a workgroup streams a tile in about 1.2 us.  Measured on split counts swept at 4K .. 100K keys
@@ -927,9 +1076,13 @@ static int launch_sdpa(hipStream_t st, const SdpaArgs& A, const CombineArgs& C, 
         LaunchBracket br(DFLASH_KERNEL_SDPA_PARTIAL, st);
         DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kPartialThreads), L::BYTES, A));
     }
-    {
+    if (A.S > 1) {
         LaunchBracket br(DFLASH_KERNEL_SDPA_COMBINE, st);
-        DFLASH_HIP_TRY(br.launch(sdpa_combine_kernel<Tag, D>, dim3(B * A.Hq * kM), dim3(kCombineThreads), 0, C));
+        const dim3 waves((C.rows + kCombineThreads / 64 - 1) / (kCombineThreads / 64)), threads(kCombineThreads);
+        const int groups = 64 / (D / 8);
+        if (A.S <= 4 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 4>, waves, threads, 0, C));
+        else if (A.S <= 16 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
+        else DFLASH_HIP_TRY(br.launch(sdpa_combine_kernel<Tag, D>, dim3(C.rows), threads, 0, C));
     }
     return DFLASH_OK;
 }
@@ -1050,7 +1203,7 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     A.mask = (const uint16_t*)mask;
     A.kv_batch_stride = kv_batch_stride; A.kv_head_stride = kv_head_stride;
     A.scale_log2 = scale * 1.4426950408889634f;
-    A.Hq = Hq; A.Hk = Hk; A.G = G; A.N = N; A.S = S; A.groups_per_kv = groups; A.rows_total = B * Hq * kM;
+    A.Hq = Hq; A.Hk = Hk; A.G = G; A.N = N; A.S = S; A.groups_per_kv = groups;
     A.gpk_magic = fast_div_magic((uint32_t)groups); A.S_magic = fast_div_magic((uint32_t)S);
     A.len_bias = k_new ? kM : 0;
     A.page_table = paged ? paged->table : nullptr;
@@ -1060,7 +1213,13 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     A.status = status_word();
     CombineArgs C;
     C.part_o = A.part_o; C.part_m = A.part_m; C.part_l = A.part_l;
-    C.out = (uint16_t*)out; C.lse = lse; C.S = S;
+    C.out = (uint16_t*)out; C.lse = lse; C.S = S; C.B = B; C.hqm = Hq * kM; C.rows = B * C.hqm;
+    // A single split writes the output itself.  Several sequences with device-side lengths share the splits by length (one
+    // lane of a wave per sequence; tile counts are summed as floats, exact below 2^24).
+    A.lse = lse; A.B = B;
+    if (S == 1) A.part_o = (uint16_t*)out;
+    A.balance = kv_len_dev && B > 1 && B <= 64 && S > 1 && (int64_t)B * ((N + kBN - 1) / kBN) < (1 << 24);
+    C.balance = A.balance; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
 
     hipStream_t st = (hipStream_t)stream;
 #define DFLASH_SDPA_CASE(MASKED, PAGED)                                                                              \
