@@ -444,14 +444,18 @@ constexpr int kGdnChunk = 16;  // steps staged in LDS at a time
 // LPR lanes share one state row; each keeps DK/LPR channels as float4 pieces
 // interleaved across the group (piece c of lane j covers channels
 // c*4*LPR + 4j .. +3) so that state loads and stores are fully coalesced.
-// Three row dot products are reduced together with DPP adds inside the 16-lane
-// row: S'k for the innovation, S'q for the read-out and k.q, because
+// Two row dot products are reduced with DPP adds and lane swaps: S'k for the
+// innovation and S'q for the read-out, because
 //   y = (S' + delta (x) k) q = S'q + delta * (k.q),
-// so only S'k sits on the step-to-step critical path.  The kernel is bound by
-// the latency of that serial chain (T dependent steps), not by bandwidth: each
-// step's operands are therefore fetched from LDS one step ahead, and the dot
-// products run as two half-length chains.
+// so only S'k sits on the step-to-step critical path; k.q is formed once per step
+// while the chunk is staged.  The kernel is bound by the latency of that serial chain
+// (T dependent steps) and by the instructions of a step, not by bandwidth: operands are
+// fetched from LDS several steps ahead, the dot products run as two half-length chains,
+// and a chunk of fewer than 16 steps takes the same pipelined loop (it had a loop of its
+// own, one step ahead: B=4, T=13, per-channel gate, bf16 state took 12.0 us, now 7.1).
 // Grid: x = Dv tiles of ROWS = 256/LPR rows, y = b*Hv + hv.
+__device__ __forceinline__ float dot4(float4 a, float4 b) { return fmaf(a.x, b.x, a.y * b.y) + fmaf(a.z, b.z, a.w * b.w); }
+
 template <int CH> struct GdnStepOps {
     float4 k[CH], q[CH], g[CH];
     float gs, v, beta, kq;
@@ -465,6 +469,9 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
     constexpr int TC = kGdnChunk;
     constexpr int TPR = DK / 4;                                   // threads spanning one step's q (or k) row, 4 channels each
     static_assert(CH >= 1, "row slice must hold at least one float4");
+    // k.q is one value per head and step.  The threads that stage a step's k and q form it on the way where they are a
+    // power of two (inside the steps, by every row group for itself, it was a sixth of their instructions).
+    constexpr bool KQ_AT_STAGING = (TPR & (TPR - 1)) == 0 && TPR >= 4 && TPR <= 64;
 
     __shared__ float q_s[TC][DK];
     __shared__ float k_s[TC][DK];
@@ -473,6 +480,7 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
     __shared__ float y_s[TC][ROWS];
     __shared__ float t_s[TC][ROWS];
     __shared__ float beta_s[TC];
+    __shared__ float kq_s[TC];
     __shared__ int on_s[TC];
 
     // every argument in one burst of scalar loads (fetched where first used they are several dependent trips to memory)
@@ -566,8 +574,13 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
         for (int u = 0; u < QI; ++u) {
             const int i = tid + u * kThreads, t = i / TPR, c = (i % TPR) * 4;
             if (t < tc) {
-                store4(&q_s[t][c], cvt4(q32[u], q16[u]));
-                store4(&k_s[t][c], cvt4(k32[u], k16[u]));
+                const float4 q4 = cvt4(q32[u], q16[u]), k4 = cvt4(k32[u], k16[u]);
+                store4(&q_s[t][c], q4);
+                store4(&k_s[t][c], k4);
+                if constexpr (KQ_AT_STAGING) {        // the TPR lanes of a step are all here or all not
+                    const float kq = butterfly_sum<TPR>(dot4(k4, q4));
+                    if (c == 0) kq_s[t] = kq;
+                }
                 if (VEC_G) store4(&g_s[t][c], cvt4(g32[VEC_G ? u : 0], g16[VEC_G ? u : 0]));
             }
         }
@@ -595,15 +608,7 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
         o.v = v_s[t][rloc];
         o.beta = beta_s[t];
         o.on = HAS_MASK ? on_s[t] : 1;
-        // k.q of the step (one value per head and step) from the lane's own channels; it does not depend on the
-        // state, so its reduction runs beside the step-to-step chain, not on it
-        float kq0 = 0.f, kq1 = 0.f;
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            kq0 = fmaf(o.k[c].x, o.q[c].x, kq0); kq1 = fmaf(o.k[c].y, o.q[c].y, kq1);
-            kq0 = fmaf(o.k[c].z, o.q[c].z, kq0); kq1 = fmaf(o.k[c].w, o.q[c].w, kq1);
-        }
-        o.kq = group_sum<LPR>(kq0 + kq1);
+        o.kq = kq_s[t];
     };
 
     if (A.T > 0) request_chunk(0, A.T < TC ? A.T : TC);
@@ -615,8 +620,19 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
         }
         park_chunk(tc);
         __syncthreads();
+        if constexpr (!KQ_AT_STAGING) {
+            for (int t = rloc; t < tc; t += ROWS) {
+                float kq = 0.f;
+#pragma unroll
+                for (int c = 0; c < CH; ++c)
+                    kq += dot4(*reinterpret_cast<const float4*>(&k_s[t][c * 4 * LPR + 4 * j]), *reinterpret_cast<const float4*>(&q_s[t][c * 4 * LPR + 4 * j]));
+                kq = butterfly_sum<LPR>(kq);
+                if (j == 0) kq_s[t] = kq;
+            }
+            __syncthreads();
+        }
 
-        // ---- serial steps, operands one step ahead (two operand sets, no register copies) ----
+        // ---- serial steps ----
         auto step = [&](int t, const GdnStepOps<CH>& cur) {
             float yv = 0.f, delta = 0.f;
             if (!HAS_MASK || cur.on) {                // uniform across the workgroup
@@ -631,8 +647,8 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
                     sq0 = fmaf(s[c].x, q4.x, sq0); sq1 = fmaf(s[c].y, q4.y, sq1);
                     sq0 = fmaf(s[c].z, q4.z, sq0); sq1 = fmaf(s[c].w, q4.w, sq1);
                 }
-                const float sk = group_sum<LPR>(sk0 + sk1);
-                const float sq = group_sum<LPR>(sq0 + sq1);
+                const float sk = butterfly_sum<LPR>(sk0 + sk1);
+                const float sq = butterfly_sum<LPR>(sq0 + sq1);
                 delta = (cur.v - sk) * cur.beta;
                 yv = fmaf(delta, cur.kq, sq);
 #pragma unroll
@@ -646,27 +662,22 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
             }
             if (j == 0) { y_s[t][rloc] = yv; t_s[t][rloc] = delta; }
         };
-        if (tc == TC) {
-            // A full chunk (the verify block) is straight-line code: operands are fetched kAhead steps ahead of their
-            // use, so no step waits for LDS.
-            constexpr int kAhead = 4;
-            GdnStepOps<CH> ops[TC];
+        {
+            // Operands are fetched ahead of their use, so no step waits for LDS, into sets of registers that the loop goes
+            // round: four sets, each refilled behind its step; with four float4 per operand (Dk = 256 on 16 lanes) three,
+            // refilled ahead of the step, which is what still fits the registers.
+            constexpr bool kWideSet = CH * (VEC_G ? 3 : 2) > 6;
+            constexpr int kSets = kWideSet ? 3 : 4;
+            GdnStepOps<CH> ops[kSets];
 #pragma unroll
-            for (int t = 0; t < kAhead; ++t) fetch(t, ops[t]);
+            for (int u = 0; u < kSets - (kWideSet ? 1 : 0); ++u) fetch(u, ops[u]);
+            for (int t0s = 0; t0s < tc; t0s += kSets) {
 #pragma unroll
-            for (int t = 0; t < TC; ++t) {
-                if (t + kAhead < TC) fetch(t + kAhead, ops[t + kAhead]);
-                step(t, ops[t]);
-            }
-        } else {
-            GdnStepOps<CH> opa, opb;
-            fetch(0, opa);
-            for (int t = 0; t < tc; t += 2) {
-                if (t + 1 < tc) fetch(t + 1, opb);
-                step(t, opa);
-                if (t + 1 < tc) {
-                    if (t + 2 < tc) fetch(t + 2, opa);
-                    step(t + 1, opb);
+                for (int u = 0; u < kSets; ++u) {
+                    const int t = t0s + u, next = t + kSets - (kWideSet ? 1 : 0), nl = next < TC ? next : TC - 1;
+                    if (kWideSet) fetch(nl, ops[(u + kSets - 1) % kSets]);
+                    if (t < tc) step(t, ops[u]);      // uniform
+                    if (!kWideSet) fetch(nl, ops[u]);
                 }
             }
         }
@@ -1517,30 +1528,36 @@ int gdn_device_setup() {
     return rc;
 }
 
+template <typename StateT, int DK, int LPR>
+static int launch_gdn_steps(hipStream_t st, const GdnArgs& A, int B, bool vec) {
+    dim3 grid((A.Dv + (kThreads / LPR) - 1) / (kThreads / LPR), B * A.Hv);
+    LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);
+    auto kern = vec ? (A.mask ? gated_delta_tape_kernel<StateT, true, true, DK, LPR> : gated_delta_tape_kernel<StateT, true, false, DK, LPR>)
+                    : (A.mask ? gated_delta_tape_kernel<StateT, false, true, DK, LPR> : gated_delta_tape_kernel<StateT, false, false, DK, LPR>);
+    DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), 0, A));
+    return DFLASH_OK;
+}
+
 template <typename StateT>
 static int launch_gdn_state(hipStream_t st, const GdnArgs& A, int B, int g_ndim, int Dk) {
     const bool vec = g_ndim == 4;
-#define DFLASH_GDN_CASE(DKV, LPRV)                                                                     \
-    case DKV: {                                                                                        \
-        dim3 grid((A.Dv + (kThreads / LPRV) - 1) / (kThreads / LPRV), B * A.Hv);                       \
-        LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);                                               \
-        auto kern = vec ? (A.mask ? gated_delta_tape_kernel<StateT, true, true, DKV, LPRV> : gated_delta_tape_kernel<StateT, true, false, DKV, LPRV>)    \
-                        : (A.mask ? gated_delta_tape_kernel<StateT, false, true, DKV, LPRV> : gated_delta_tape_kernel<StateT, false, false, DKV, LPRV>); \
-        DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), 0, A));                                   \
-        return DFLASH_OK;                                                                              \
-    }
+    // Lanes per row: a step is a chain of dependent instructions whose length is set by the channels a lane holds, so a row
+    // is spread over as many lanes as still leave every workgroup a compute unit to itself (sharing one is slower: 180 against
+    // 146 us at T=300, 32 heads, Dk=256).
+    const long rows = (long)B * A.Hv * A.Dv, lanes = (long)num_compute_units() * kThreads;
+    const bool wide = rows * 32 <= lanes, widest = rows * 64 <= lanes;
     switch (Dk) {
-        DFLASH_GDN_CASE(32, 8)
-        DFLASH_GDN_CASE(64, 16)
-        DFLASH_GDN_CASE(96, 8)
-        DFLASH_GDN_CASE(128, 16)
-        DFLASH_GDN_CASE(160, 8)
-        DFLASH_GDN_CASE(192, 16)
-        DFLASH_GDN_CASE(224, 8)
-        DFLASH_GDN_CASE(256, 16)
+        case 32: return launch_gdn_steps<StateT, 32, 8>(st, A, B, vec);
+        case 64: return launch_gdn_steps<StateT, 64, 16>(st, A, B, vec);
+        case 96: return launch_gdn_steps<StateT, 96, 8>(st, A, B, vec);
+        case 128: return wide ? launch_gdn_steps<StateT, 128, 32>(st, A, B, vec) : launch_gdn_steps<StateT, 128, 16>(st, A, B, vec);
+        case 160: return launch_gdn_steps<StateT, 160, 8>(st, A, B, vec);
+        case 192: return launch_gdn_steps<StateT, 192, 16>(st, A, B, vec);
+        case 224: return launch_gdn_steps<StateT, 224, 8>(st, A, B, vec);
+        case 256: return widest ? launch_gdn_steps<StateT, 256, 64>(st, A, B, vec)
+                         : wide ? launch_gdn_steps<StateT, 256, 32>(st, A, B, vec) : launch_gdn_steps<StateT, 256, 16>(st, A, B, vec);
         default: break;
     }
-#undef DFLASH_GDN_CASE
     set_error("gated delta: Dk=%d is not a multiple of 32 in [32, 256]", Dk);
     return DFLASH_UNSUPPORTED;
 }

@@ -1,0 +1,85 @@
+"""GPU parity where the host picks another kernel or another split: shapes on both sides of each line, and the
+smallest and largest of what each variant takes, against the oracle.
+
+Tolerances are those of the dedicated tests and follow from the types: an fp32 state or tape is held to 1e-4 (a few
+hundred roundings of 6e-8), bf16/f16 outputs to 2e-2 (the rounding of weights, partial rows and output)."""
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import dflash_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def host(t):
+    return t.detach().float().cpu().numpy()
+
+
+def dev(a, dt=torch.float32):
+    return torch.from_numpy(np.ascontiguousarray(a)).to("cuda", dt)
+
+
+# step-by-step GatedDelta kernel: lanes per state row (16, 32 or 64) by B*Hv*Dv against 256 compute units
+@pytest.mark.parametrize("Dk,Hv,Dv", [(128, 16, 128), (128, 17, 128), (256, 8, 128), (256, 9, 128), (256, 16, 128), (256, 17, 120)],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("T", [1, 3, 4, 13, 17])
+def test_step_kernel_lanes_per_row(gpu_lib, Dk, Hv, Dv, T):
+    from swiftlm_amd import DFlashKernels as K
+
+    d = O.make_gdn_inputs(Dk + Hv + T, 1, T, 1, Hv, Dk, Dv, in_dtype="bf16", vec_gate=True)
+    mask = np.ones((1, T), np.float32)
+    mask[0, T // 2] = float(T == 1)
+    y, s, tape = K.gated_delta_kernel_with_tape(*[dev(d[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")], dev(d["state"]), dev(mask))
+    yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], mask, dtype=np.float64)
+    np.testing.assert_allclose(host(s), sw, rtol=1e-4, atol=1e-6)
+    np.testing.assert_allclose(host(tape), tw, rtol=1e-4, atol=1e-5)
+    np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
+
+
+def attend(q, k, v, lens, D, **kw):
+    from swiftlm_amd import DFlashKernels as K
+
+    out, lse = K.batched_sdpa_2pass(q, k, v, 1.0 / math.sqrt(D), return_lse=True, **kw)
+    torch.cuda.synchronize()
+    for b, n in enumerate(lens):
+        ow, lw = O.sdpa_block_causal(host(q[b:b + 1]), host(k[b:b + 1, :, :n]), host(v[b:b + 1, :, :n]), 1.0 / math.sqrt(D))
+        np.testing.assert_allclose(host(out[b]), ow[0], rtol=2e-2, atol=2e-2, err_msg=f"sequence {b} of {n} keys")
+        np.testing.assert_allclose(host(lse[b]), lw[0], rtol=2e-3, atol=2e-3, err_msg=f"sequence {b} of {n} keys")
+
+
+def tensors(seed, B, Hq, Hk, N, D, dt=torch.bfloat16):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return [torch.randn(B, h, n, D, generator=g, device="cuda").to(dt) for h, n in ((Hq, 16), (Hk, N), (Hk, N))]
+
+
+# one split writes the output itself (up to four tiles of 32 keys); with few splits a wave merges a row, with more a workgroup
+@pytest.mark.parametrize("N", [16, 17, 32, 33, 128, 129, 250, 1024, 1056, 2048, 2080])
+@pytest.mark.parametrize("Hq,Hk,D", [(3, 1, 256), (4, 2, 128)])
+def test_attention_split_counts(gpu_lib, N, Hq, Hk, D):
+    attend(*tensors(N + D, 1, Hq, Hk, N, D), [N], D)
+
+
+# ragged batches share the splits: one sequence beside many, equal lengths, all at the minimum, more sequences than one wave has lanes
+@pytest.mark.parametrize("lens", [[700, 16], [16, 17, 2000, 33], [500] * 5, [16] * 3 + [129], [40 + 3 * i for i in range(64)],
+                                  [40 + 3 * i for i in range(65)]], ids=lambda v: f"{len(v)}x{max(v)}")
+@pytest.mark.parametrize("D", [128, 256])
+def test_ragged_shares(gpu_lib, lens, D):
+    q, k, v = tensors(len(lens) + D, len(lens), 4, 2, max(lens), D)
+    attend(q, k, v, lens, D, kv_len=torch.tensor(lens, dtype=torch.int32, device="cuda"))
+
+
+def test_ragged_share_of_a_length_outside_the_bound_is_flagged_and_clamped(gpu_lib):
+    import ctypes as C
+
+    q, k, v = tensors(3, 3, 4, 2, 400, 128)
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    assert gpu_lib.dflash_set_status_word(C.c_void_p(status.data_ptr())) == 0
+    try:
+        attend(q, k, v, [400, 16, 200], 128, kv_len=torch.tensor([900, 3, 200], dtype=torch.int32, device="cuda"))
+        assert int(status) == 1
+    finally:
+        assert gpu_lib.dflash_set_status_word(None) == 0
