@@ -1,0 +1,86 @@
+// What the GatedDelta kernel files share: the argument block, the bf16 splitting of fp32 values and the
+// unit-triangular solve of a chunk.  Internal to the library.
+#pragma once
+
+#include "dflash_common.h"
+
+namespace dflash {
+
+struct GdnArgs {
+    const void *q, *k, *v, *g, *beta, *mask;
+    const void* state_in;
+    void* state_out;
+    void* y;
+    float* tape;
+    int in_dtype, mask_dtype;
+    int T, Hk, Hv, Dv;
+    // chunked kernels only: value heads per key head and ceil(2^32 / group), so that hv / group is one multiply
+    // (exact for hv, group < 2^16; group == 1 is handled apart, its reciprocal does not fit)
+    uint32_t group, group_magic;
+};
+
+constexpr int kChunkRows = 16;
+constexpr int kChunkSteps = 16;
+
+typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
+
+// The upper halves of two words as one: (a >> 16) | (b & 0xffff0000), one v_perm_b32.
+__device__ __forceinline__ uint32_t upper_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+// Four floats that are bf16 values -> their 4 x 16 bits.
+__device__ __forceinline__ uint2 pack4_bf16_exact(float4 v) {
+    return make_uint2(upper_halves(__float_as_uint(v.x), __float_as_uint(v.y)), upper_halves(__float_as_uint(v.z), __float_as_uint(v.w)));
+}
+// x = hi + mid + lo with each term a bf16, by truncation: hi = the upper 16 bits of x, mid = the upper 16 bits of
+// x - hi, lo = x - hi - mid.  hi takes 8 of x's 24 significand bits, mid the next 8 (or more, where zeros follow hi),
+// so lo has at most 8 left and is a bf16 as it stands; both subtractions are exact, and the three terms add up to x
+// bit for bit.  Four VALU operations per value and one v_perm per pair and term.
+__device__ __forceinline__ void split3_bf16(float x, float& r1, float& r2) {
+    r1 = x - __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+    r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+}
+__device__ __forceinline__ void split3_bf16(float x, uint16_t& hi, uint16_t& mid, uint16_t& lo) {
+    float r1, r2;
+    split3_bf16(x, r1, r2);
+    hi = (uint16_t)(__float_as_uint(x) >> 16); mid = (uint16_t)(__float_as_uint(r1) >> 16); lo = (uint16_t)(__float_as_uint(r2) >> 16);
+}
+__device__ __forceinline__ void split3_bf16(float4 v, uint2& hi, uint2& mid, uint2& lo) {
+    const float x[4] = {v.x, v.y, v.z, v.w};
+    float r1[4], r2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) split3_bf16(x[i], r1[i], r2[i]);
+    hi = make_uint2(upper_halves(__float_as_uint(x[0]), __float_as_uint(x[1])), upper_halves(__float_as_uint(x[2]), __float_as_uint(x[3])));
+    mid = make_uint2(upper_halves(__float_as_uint(r1[0]), __float_as_uint(r1[1])), upper_halves(__float_as_uint(r1[2]), __float_as_uint(r1[3])));
+    lo = make_uint2(upper_halves(__float_as_uint(r2[0]), __float_as_uint(r2[1])), upper_halves(__float_as_uint(r2[2]), __float_as_uint(r2[3])));
+}
+
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef float f32x2v __attribute__((ext_vector_type(2)));
+typedef float f32x16v __attribute__((ext_vector_type(16)));
+
+template <int QUAD_LANE> __device__ __forceinline__ float quad_broadcast(float x) {
+    constexpr int ctrl = QUAD_LANE | (QUAD_LANE << 2) | (QUAD_LANE << 4) | (QUAD_LANE << 6);
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, true));
+}
+
+// Steps S..15 of the unit-triangular solve for one state row held by a quad (lane q owns steps 4q..4q+3).
+// Every lane of the quad sees every delta; lane q keeps those of its own four steps in `mine` (a select per step,
+// no branch) for the store that follows.
+template <int S> struct SolveStep {
+    static __device__ __forceinline__ void run(float (&acc)[4], const float4 (&arow)[16], const float (&bet)[16],
+                                               float (&mine)[4], const int q) {
+        const float d = quad_broadcast<S / 4>(bet[S] * acc[S % 4]);
+        mine[S % 4] = q == S / 4 ? d : mine[S % 4];
+        acc[0] = fmaf(-arow[S].x, d, acc[0]);
+        acc[1] = fmaf(-arow[S].y, d, acc[1]);
+        acc[2] = fmaf(-arow[S].z, d, acc[2]);
+        acc[3] = fmaf(-arow[S].w, d, acc[3]);
+        if constexpr (S + 1 < 16) SolveStep<S + 1>::run(acc, arow, bet, mine, q);
+    }
+};
+
+// The chunked form for longer calls (gdn_long.hip)
+bool gdn_long_applies(const GdnArgs& A, int Dk);
+int launch_gdn_long(hipStream_t st, const GdnArgs& A, int B, int Dk);
+int gdn_long_device_setup();
+
+}  // namespace dflash

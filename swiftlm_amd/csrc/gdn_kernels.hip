@@ -12,7 +12,7 @@
 // Semantics follow Sources/DFlash/DFlashKernels.swift: Metal kernels :43-81 and
 // :122-199, ops restatements :371-407 and :409-466.
 
-#include "dflash_common.h"
+#include "gdn_common.h"
 
 namespace dflash {
 
@@ -397,19 +397,6 @@ static int replay_common(hipStream_t st, int n_layers, const void* const* tape, 
 // Gated delta forward with tape
 // ===========================================================================
 
-struct GdnArgs {
-    const void *q, *k, *v, *g, *beta, *mask;
-    const void* state_in;
-    void* state_out;
-    void* y;
-    float* tape;
-    int in_dtype, mask_dtype;
-    int T, Hk, Hv, Dv;
-    // chunked kernels only: value heads per key head and ceil(2^32 / group), so that hv / group is one multiply
-    // (exact for hv, group < 2^16; group == 1 is handled apart, its reciprocal does not fit)
-    uint32_t group, group_magic;
-};
-
 // Inputs of the layer's pre-ops when they run inside the forward kernel (gdn_layer_kernel): the short
 // conv + SiLU over q|k|v, the q/k normalisation and the gate formulas of dflash_gdn_prepare.
 struct GdnPrep {
@@ -721,9 +708,6 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
 // Workgroup: 16 state rows of one head (grid x = Dv/16, y = b*Hv + hv), 4 waves.
 // ---------------------------------------------------------------------------
 
-constexpr int kChunkRows = 16;
-constexpr int kChunkSteps = 16;
-
 template <int DK> struct GdnChunkLds {
     static constexpr int LD = DK + 4;      // row pitch in floats: 16-byte pad spreads rows over the banks
     float x[32][LD];                       // rows 0..15 state tile, rows 16..31 k_t
@@ -741,62 +725,6 @@ template <int DK> struct GdnChunkLds {
     static constexpr int LB = DK + 8;
     uint16_t xs[3][16][LB];
     uint16_t kb[16][LB], qb[16][LB];
-};
-
-typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
-
-// The upper halves of two words as one: (a >> 16) | (b & 0xffff0000), one v_perm_b32.
-__device__ __forceinline__ uint32_t upper_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
-// Four floats that are bf16 values -> their 4 x 16 bits.
-__device__ __forceinline__ uint2 pack4_bf16_exact(float4 v) {
-    return make_uint2(upper_halves(__float_as_uint(v.x), __float_as_uint(v.y)), upper_halves(__float_as_uint(v.z), __float_as_uint(v.w)));
-}
-// x = hi + mid + lo with each term a bf16, by truncation: hi = the upper 16 bits of x, mid = the upper 16 bits of
-// x - hi, lo = x - hi - mid.  hi takes 8 of x's 24 significand bits, mid the next 8 (or more, where zeros follow hi),
-// so lo has at most 8 left and is a bf16 as it stands; both subtractions are exact, and the three terms add up to x
-// bit for bit.  Four VALU operations per value and one v_perm per pair and term.
-__device__ __forceinline__ void split3_bf16(float x, float& r1, float& r2) {
-    r1 = x - __uint_as_float(__float_as_uint(x) & 0xffff0000u);
-    r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
-}
-__device__ __forceinline__ void split3_bf16(float x, uint16_t& hi, uint16_t& mid, uint16_t& lo) {
-    float r1, r2;
-    split3_bf16(x, r1, r2);
-    hi = (uint16_t)(__float_as_uint(x) >> 16); mid = (uint16_t)(__float_as_uint(r1) >> 16); lo = (uint16_t)(__float_as_uint(r2) >> 16);
-}
-__device__ __forceinline__ void split3_bf16(float4 v, uint2& hi, uint2& mid, uint2& lo) {
-    const float x[4] = {v.x, v.y, v.z, v.w};
-    float r1[4], r2[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) split3_bf16(x[i], r1[i], r2[i]);
-    hi = make_uint2(upper_halves(__float_as_uint(x[0]), __float_as_uint(x[1])), upper_halves(__float_as_uint(x[2]), __float_as_uint(x[3])));
-    mid = make_uint2(upper_halves(__float_as_uint(r1[0]), __float_as_uint(r1[1])), upper_halves(__float_as_uint(r1[2]), __float_as_uint(r1[3])));
-    lo = make_uint2(upper_halves(__float_as_uint(r2[0]), __float_as_uint(r2[1])), upper_halves(__float_as_uint(r2[2]), __float_as_uint(r2[3])));
-}
-
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-typedef float f32x2v __attribute__((ext_vector_type(2)));
-typedef float f32x16v __attribute__((ext_vector_type(16)));
-
-template <int QUAD_LANE> __device__ __forceinline__ float quad_broadcast(float x) {
-    constexpr int ctrl = QUAD_LANE | (QUAD_LANE << 2) | (QUAD_LANE << 4) | (QUAD_LANE << 6);
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, true));
-}
-
-// Steps S..15 of the unit-triangular solve for one state row held by a quad (lane q owns steps 4q..4q+3).
-// Every lane of the quad sees every delta; lane q keeps those of its own four steps in `mine` (a select per step,
-// no branch) for the store that follows.
-template <int S> struct SolveStep {
-    static __device__ __forceinline__ void run(float (&acc)[4], const float4 (&arow)[16], const float (&bet)[16],
-                                               float (&mine)[4], const int q) {
-        const float d = quad_broadcast<S / 4>(bet[S] * acc[S % 4]);
-        mine[S % 4] = q == S / 4 ? d : mine[S % 4];
-        acc[0] = fmaf(-arow[S].x, d, acc[0]);
-        acc[1] = fmaf(-arow[S].y, d, acc[1]);
-        acc[2] = fmaf(-arow[S].z, d, acc[2]);
-        acc[3] = fmaf(-arow[S].w, d, acc[3]);
-        if constexpr (S + 1 < 16) SolveStep<S + 1>::run(acc, arow, bet, mine, q);
-    }
 };
 
 // BF: the inputs are bf16 (fixed at compile time): the product then runs on bf16 MFMAs, exactly (see below).
@@ -1525,6 +1453,7 @@ int gdn_device_setup() {
     int rc = gdn_chunk_setup<64>();
     if (rc == DFLASH_OK) rc = gdn_chunk_setup<128>();
     if (rc == DFLASH_OK) rc = gdn_chunk_setup<256>();
+    if (rc == DFLASH_OK) rc = gdn_long_device_setup();
     return rc;
 }
 
@@ -1627,6 +1556,7 @@ extern "C" int dflash_gated_delta_tape(void* stream, const void* q, const void* 
     A.in_dtype = in_dtype; A.mask_dtype = mask_dtype; A.T = T; A.Hk = Hk; A.Hv = Hv; A.Dv = Dv;
     if (state_dtype == DFLASH_F32 && g_ndim == 3 && Dv % kChunkRows == 0 && T > 0 && T < 65536 && Dv < 65536 && chunk_index_setup(A, B, Dk)) {
         // fp32 state with one decay per head and step: chunked form
+        if (gdn_long_applies(A, Dk)) return launch_gdn_long((hipStream_t)stream, A, B, Dk);
         if (Dk == 64) return launch_gdn_chunk<64>((hipStream_t)stream, A, B);
         if (Dk == 128) return launch_gdn_chunk<128>((hipStream_t)stream, A, B);
         if (Dk == 256) return launch_gdn_chunk<256>((hipStream_t)stream, A, B);

@@ -1,0 +1,442 @@
+// GatedDelta forward over more than one chunk of 16 steps: the stretches of a prompt.
+//
+// Semantics follow Sources/DFlash/DFlashKernels.swift:122-199 (Metal kernel) and :409-466 (ops restatement).
+
+#include "gdn_common.h"
+
+namespace dflash {
+
+// ---------------------------------------------------------------------------
+// Chunked form for longer calls (bf16 inputs, fp32 state, one decay per head and step, more than one chunk); the algebra is
+// that of gated_delta_chunk_kernel.
+//
+// That kernel does a chunk as phases of one workgroup -- loads, product, tables, solve, read-out, update -- each of which
+// waits for the one before: 2.4 us per 16 steps, of which the state needs a small part.  Only S_0 k_t, delta and
+// the update depend on the chunk before; everything else (loads, k_s.k_t, k_s.q_t, decays, the solve's matrix, the
+// read-out) is done by other waves, ahead of or behind that chain:
+//
+//   waves 0-3 (chain)     own Dk/4 channels of the 16 state rows each, as MFMA accumulators that never leave the
+//                         registers.  Chunk m: add the four partial S_0 k_t, delta = T (v - gam S_0 k_t), update, split
+//                         the new state into three bf16 terms, partial S_0 k_t of chunk m+1 into LDS, barrier.
+//   waves 4-7 (producers) wave 4+p prepares chunks p, p+4, ...: interval m-2 k rows, k_s.k_t, k_s.q_t, decays; interval
+//                         m-1 T = (I + diag(beta) A)^-1 diag(beta) by substitution; interval m the loads of chunk m+4 and
+//                         k of chunk m+1 transposed; interval m+1 y and the tape of the chunk.
+//
+// One barrier per chunk, no wave waits for memory inside a chunk (loads are asked for two chunks ahead of their use), and
+// no operand crosses lanes: with S^T as the accumulator a lane holds row l%16 and channels 4*(l/16)+v, which is also how
+// the next product's b operand may be laid out, as the order of a contraction's indices is free.
+//
+// Bound by the length of an interval: 1,400 / 1,600 / 2,200 cycles at Dk = 64 / 128 / 256, of which the chain works 1,200 /
+// 1,400 / 1,900 (the split of the state on the VALU, the exchange of the partial sums through LDS, three groups of
+// dependent MFMAs) and the busiest producer about as long.  us, chunk by chunk kernel against this one: 1,003 steps,
+// 32 heads of 128x128 152 -> 44; 730 steps, 8 heads, Dk = 256 147 -> 45; two sequences of 1,000 steps, 32 heads, Dk = 256
+// 419 -> 123; 40 steps 8.3 -> 5.7.
+// ---------------------------------------------------------------------------
+
+typedef short s16x4v __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));   // (a select between two HIP uint4 is a select of addresses: the arrays end in scratch)
+
+template <int DK> struct GdnLongLds {
+    static constexpr int LB = DK + 8;      // row pitch: 16 bytes of pad spread 16-byte reads of a column of rows over the banks
+    // Every array is read at most one barrier after the interval that follows its writing, so two sets (the chunk's parity) do.
+    // k and q rows; inside each 32 channels position 8g + 4h + x holds channel 16h + 4g + x (what one lane of the product takes)
+    uint16_t k[2][16][LB], q[2][16][LB];
+    uint16_t kt[2][DK][16];                // k transposed: steps of a channel
+    float na[2][16][16];                   // na[t][s] = -beta_t G[s][t] k_s.k_t for s < t, else 0
+    float t2[2][64][4];                    // lane (g, n): T[t = n][s = 4g + i]
+    float v[2][64][4];                     // lane (g, n): v_s of row n, s = 4g + i
+    float pk[2][4][64][4], pq[2][4][64][4];// partial S_0 k_t and S_0 q_t of the four chain waves, as accumulators
+    float dl[2][64][4];                    // lane (g, n): delta_s of row n, s = 4g + i
+    float gam[2][16], w[2][16], beta[2][16];
+};
+
+// A barrier that orders LDS only: loads and stores of global memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ f32x4v lds4(const float* p) { return *reinterpret_cast<const f32x4v*>(p); }
+__device__ __forceinline__ void split3_bf16(f32x4v v, uint2& hi, uint2& mid, uint2& lo) {
+    split3_bf16(make_float4(v[0], v[1], v[2], v[3]), hi, mid, lo);
+}
+__device__ __forceinline__ bf16x8v as_bf16x8(uint2 a, uint2 b) { return __builtin_bit_cast(bf16x8v, make_uint4(a.x, a.y, b.x, b.y)); }
+__device__ __forceinline__ s16x4v as_s16x4(uint2 a) { return __builtin_bit_cast(s16x4v, a); }
+
+// Lane S of each 16-lane row to all lanes of the row.
+template <int S> __device__ __forceinline__ float row_broadcast(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + S, 0xf, 0xf, true));
+}
+template <int L0, int L1, int L2, int L3> __device__ __forceinline__ float quad_take(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), L0 | (L1 << 2) | (L2 << 4) | (L3 << 6), 0xf, 0xf, true));
+}
+// X = (I + A)^-1, A strictly lower: lane n of a 16-lane row holds A[n][.], negated, and four columns of X[n][.]; row S of X
+// is final when its turn comes and is taken off the rows below it.  One fused multiply-add per step and column, its first
+// factor broadcast from lane S of the row (DPP row_newbcast).  One block of assembly: a DPP operand may be read two wait
+// states after it was written, which the order of the columns gives; the s_nop is for what stands in front.
+#define DFLASH_INVERSE_STEP(S, A)                                              \
+    "v_fmac_f32_dpp %0, %0, " A " row_newbcast:" S " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %1, %1, " A " row_newbcast:" S " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %2, %2, " A " row_newbcast:" S " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %3, %3, " A " row_newbcast:" S " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ f32x4v unit_inverse(f32x4v x, const float (&na)[16]) {
+    float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+    asm volatile("s_nop 1\n\t" DFLASH_INVERSE_STEP("0", "%4") DFLASH_INVERSE_STEP("1", "%5") DFLASH_INVERSE_STEP("2", "%6")
+                 DFLASH_INVERSE_STEP("3", "%7") DFLASH_INVERSE_STEP("4", "%8") DFLASH_INVERSE_STEP("5", "%9")
+                 DFLASH_INVERSE_STEP("6", "%10") DFLASH_INVERSE_STEP("7", "%11") DFLASH_INVERSE_STEP("8", "%12")
+                 DFLASH_INVERSE_STEP("9", "%13") DFLASH_INVERSE_STEP("10", "%14") DFLASH_INVERSE_STEP("11", "%15")
+                 DFLASH_INVERSE_STEP("12", "%16") DFLASH_INVERSE_STEP("13", "%17") DFLASH_INVERSE_STEP("14", "%18")
+                 : "+&v"(x0), "+&v"(x1), "+&v"(x2), "+&v"(x3)
+                 : "v"(na[0]), "v"(na[1]), "v"(na[2]), "v"(na[3]), "v"(na[4]), "v"(na[5]), "v"(na[6]), "v"(na[7]), "v"(na[8]),
+                   "v"(na[9]), "v"(na[10]), "v"(na[11]), "v"(na[12]), "v"(na[13]), "v"(na[14]));
+    return f32x4v{x0, x1, x2, x3};
+}
+#undef DFLASH_INVERSE_STEP
+
+constexpr int kLongThreads = 512;
+
+template <int DK>
+__global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnArgs A) {
+    using Lds = GdnLongLds<DK>;
+    extern __shared__ __align__(16) unsigned char gdn_chunk_smem[];
+    Lds& L = *reinterpret_cast<Lds*>(gdn_chunk_smem);
+    constexpr int NB = DK / 64, NK = DK / 32;          // 16-channel blocks of a chain wave; contraction steps of 32 over all channels
+
+    const int lane = threadIdx.x % 64, w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int n = lane % 16, g = lane / 16;
+    const int b = blockIdx.z, hv = blockIdx.y, bh = b * A.Hv + hv, hk = (int)((uint32_t)hv / A.group);
+    const int row0 = blockIdx.x * kChunkRows;
+    const int chunks = (A.T + kChunkSteps - 1) / kChunkSteps;   // >= 2
+    // Intervals run from -2 (the producers' first chunk) to chunks (the last read-out), with a barrier behind each but the
+    // last: both halves of this function pass chunks + 2 of them.
+
+    if (w < 4) {
+        // ---- chain ----
+        __builtin_amdgcn_s_setprio(2);
+        const int cb = w * 16 * NB;                    // first channel of the wave
+        const size_t so = ((size_t)bh * A.Dv + row0 + n) * DK + cb + 4 * g;
+        f32x4v s[NB];
+        uint2 hi[NB], mid[NB], lo[NB];
+        const float* s_in = reinterpret_cast<const float*>(A.state_in) + so;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) s[i] = *reinterpret_cast<const f32x4v*>(s_in + 16 * i);
+
+        // S_0 x_t over the wave's channels, x = k or q of the chunk: rows t of the accumulator, columns = state rows.
+        // Exact products: x is bf16, the state enters as three bf16 terms that add up to it.
+        typedef uint32_t Rows __attribute__((ext_vector_type(NB == 1 ? 2 : 2 * NB)));      // the wave's channels of row n
+        auto rows = [&](const uint16_t (&x)[16][Lds::LB]) -> Rows {
+            Rows r;
+            if constexpr (NB == 1) {
+                r = *reinterpret_cast<const Rows*>(&x[n][32 * (w / 2) + 8 * g + 4 * (w & 1)]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < NB / 2; ++j) {
+                    const u32x4v c = *reinterpret_cast<const u32x4v*>(&x[n][cb + 32 * j + 8 * g]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) r[4 * j + e] = c[e];
+                }
+            }
+            return r;
+        };
+        auto product = [&](const Rows r) -> f32x4v {
+            f32x4v acc = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (NB == 1) {
+                const s16x4v xv = __builtin_bit_cast(s16x4v, r);
+                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xv, as_s16x4(lo[0]), acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xv, as_s16x4(mid[0]), acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xv, as_s16x4(hi[0]), acc, 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int j = 0; j < NB / 2; ++j) {
+                    const bf16x8v xv = __builtin_bit_cast(bf16x8v, u32x4v{r[4 * j], r[4 * j + 1], r[4 * j + 2], r[4 * j + 3]});
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, as_bf16x8(lo[2 * j], lo[2 * j + 1]), acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, as_bf16x8(mid[2 * j], mid[2 * j + 1]), acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, as_bf16x8(hi[2 * j], hi[2 * j + 1]), acc, 0, 0, 0);
+                }
+            }
+            return acc;
+        };
+
+        lds_barrier();                                 // interval -2
+#pragma unroll
+        for (int i = 0; i < NB; ++i) split3_bf16(s[i], hi[i], mid[i], lo[i]);
+        f32x4v own = product(rows(L.k[0]));
+        *reinterpret_cast<f32x4v*>(L.pk[0][w][lane]) = own;
+        lds_barrier();                                 // interval -1
+
+        for (int m = 0; m < chunks; ++m) {
+            const int par = m & 1;
+            const f32x4v pk1 = lds4(L.pk[par][w ^ 1][lane]), pk2 = lds4(L.pk[par][w ^ 2][lane]), pk3 = lds4(L.pk[par][w ^ 3][lane]);
+            const f32x4v vv = lds4(L.v[par][lane]), gm = lds4(&L.gam[par][4 * g]), t2 = lds4(L.t2[par][lane]);
+            // the same sum of pairs in every wave, so that all hold the same bits
+            const f32x4v pk = (own + pk1) + (pk2 + pk3);
+            f32x4v rhs, dl = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rhs[i] = fmaf(-gm[i], pk[i], vv[i]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dl = __builtin_amdgcn_mfma_f32_16x16x4f32(t2[i], rhs[i], dl, 0, 0, 0);
+            // the other reads, while the matrix pipe is on T
+            const Rows qrow = rows(L.q[par]);
+            const f32x4v wv = lds4(&L.w[par][4 * g]);
+            const float gam_end = L.gam[par][kChunkSteps - 1];
+            uint2 kt[NB];
+#pragma unroll
+            for (int i = 0; i < NB; ++i) kt[i] = *reinterpret_cast<const uint2*>(&L.kt[par][cb + 16 * i + n][4 * g]);
+            const Rows krow = rows(L.k[par ^ 1]);      // of the next chunk (behind the last one: not used)
+            // S_0 q_t, from the split state of before the update
+            const f32x4v pq = product(qrow);
+            // A product with T mixes all steps of a row: an infinity or NaN would reach the steps before it (0 * inf), and T may
+            // overflow where no delta does.  Then the deltas are substituted for one step after the other.
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(dl[0]) + fabsf(dl[1]) + fabsf(dl[2]) + fabsf(dl[3]) < __builtin_inff())) != 0, 0)) {
+                rhs *= lds4(&L.beta[par][4 * g]);
+                for (int tg = 0; tg < 4; ++tg)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int t = 4 * tg + i;
+                        const float d = __shfl(rhs[i], 16 * tg + n);
+                        if (g == tg) dl[i] = d;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            if (4 * g + j > t) rhs[j] = fmaf(L.na[par][4 * g + j][t], d, rhs[j]);
+                    }
+            }
+            if (w == 0) *reinterpret_cast<f32x4v*>(L.dl[par][lane]) = dl;
+            // S <- gam_15 S_0 + sum_s w_s delta_s (x) k_s, again as exact products of bf16 terms: hi and mid share one MFMA
+            uint2 dh, dm, dlo;
+            split3_bf16(dl * wv, dh, dm, dlo);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                s[i] = s[i] * gam_end;
+                s[i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as_s16x4(kt[i]), as_s16x4(dlo), s[i], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+                s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kt[i], kt[i]), as_bf16x8(dh, dm), s[i], 0, 0, 0);
+            *reinterpret_cast<f32x4v*>(L.pq[par][w][lane]) = pq;
+            if (m + 1 < chunks) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) split3_bf16(s[i], hi[i], mid[i], lo[i]);
+                own = product(krow);
+                *reinterpret_cast<f32x4v*>(L.pk[par ^ 1][w][lane]) = own;
+            }
+            lds_barrier();
+        }
+        if (A.state_out != nullptr) {
+            float* s_out = reinterpret_cast<float*>(A.state_out) + so;
+#pragma unroll
+            for (int i = 0; i < NB; ++i) *reinterpret_cast<f32x4v*>(s_out + 16 * i) = s[i];
+        }
+        return;
+    }
+
+    // ---- producers ----
+    const int p = w - 4;
+    const uint16_t* kp = reinterpret_cast<const uint16_t*>(A.k);
+    const uint16_t* qp = reinterpret_cast<const uint16_t*>(A.q);
+    const bf16_t* vp = reinterpret_cast<const bf16_t*>(A.v);
+    const bf16_t* gp = reinterpret_cast<const bf16_t*>(A.g);
+    const bf16_t* bp = reinterpret_cast<const bf16_t*>(A.beta);
+    const uint32_t k_step = (uint32_t)A.Hk * DK, step = (uint32_t)A.Hv * A.Dv;           // elements per step, below 2^24
+    u32x4v kr[NK], qr[NK];                              // rows n of k and q, channels 32j + 8g .. +7: both operands of the products
+    bf16_t vr[4], gr, br;
+    auto request = [&](int m) {
+        const int t0 = m * kChunkSteps, tc = min(A.T - t0, kChunkSteps);
+        const uint32_t bt0 = (uint32_t)b * A.T + t0;                                   // uniform, as are the products with it
+        const int tl = min(n, tc - 1);                 // clamped: always a valid address, selected away where it is used
+        const uint32_t o = (bt0 * A.Hk + hk) * DK + __umul24(tl, k_step) + 8 * g;
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+            kr[j] = *reinterpret_cast<const u32x4v*>(kp + o + 32 * j);
+            qr[j] = *reinterpret_cast<const u32x4v*>(qp + o + 32 * j);
+        }
+        const uint32_t vo = (bt0 * A.Hv + hv) * A.Dv + row0 + n;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vr[i] = vp[vo + __umul24(min(4 * g + i, tc - 1), step)];
+        const uint32_t go = bt0 * A.Hv + hv + __umul24(tl, A.Hv);
+        gr = gp[go];
+        br = bp[go];
+    };
+    // a row's 8 channels 32j + 8g .. +7 at their positions
+    auto park = [&](uint16_t* row, int j, u32x4v x) {
+        uint16_t* d = row + 32 * j + 4 * (g / 2) + 16 * (g & 1);
+        *reinterpret_cast<uint2*>(d) = make_uint2(x[0], x[1]);
+        *reinterpret_cast<uint2*>(d + 8) = make_uint2(x[2], x[3]);
+    };
+    const u32x4v none = {0u, 0u, 0u, 0u};
+    f32x4v av, cv, gam4;                               // of the chunk in hand: a and c columns, gam of steps 4g .. +3
+    float G[4], gam = 0.f, beta = 0.f;
+    f32x4v vf, yv, dl;                                 // v of the chunk in hand; y and tape of the one before, not yet stored
+    uint64_t on_bits = 0;
+    auto store_rows = [&](int m, int tc) {             // rows t = 4g + v, column = state row n
+        const uint32_t o = (((uint32_t)b * A.T + m * kChunkSteps) * A.Hv + hv) * A.Dv + row0 + n + __umul24(4 * g, step);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (4 * g + v < tc) {
+                reinterpret_cast<bf16_t*>(A.y)[o + v * step] = from_float<bf16_t>(yv[v]);
+                A.tape[o + v * step] = dl[v];
+            }
+    };
+    // k of chunk m transposed, two neighbouring channels per lane
+    auto transpose_k = [&](int par) {
+#pragma unroll
+        for (int c0 = 0; c0 < DK; c0 += 128) {
+            const int pos = c0 + 2 * lane;
+            if (DK >= 128 || lane < DK / 2) {
+                const int ch = (pos & ~31) + 16 * ((pos / 4) & 1) + 4 * ((pos % 32) / 8) + pos % 4;
+                uint32_t x[16], even[8], odd[8];
+#pragma unroll
+                for (int t = 0; t < 16; ++t) x[t] = *reinterpret_cast<const uint32_t*>(&L.k[par][t][pos]);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    even[t] = __builtin_amdgcn_perm(x[2 * t + 1], x[2 * t], 0x05040100u);
+                    odd[t] = upper_halves(x[2 * t], x[2 * t + 1]);
+                }
+                uint4* d = reinterpret_cast<uint4*>(L.kt[par][ch]);
+                d[0] = make_uint4(even[0], even[1], even[2], even[3]);
+                d[1] = make_uint4(even[4], even[5], even[6], even[7]);
+                d[2] = make_uint4(odd[0], odd[1], odd[2], odd[3]);
+                d[3] = make_uint4(odd[4], odd[5], odd[6], odd[7]);
+            }
+        }
+    };
+    if (p < chunks) request(p);
+    for (int j = 0; j < p; ++j) {                      // intervals -2 .. p - 3
+        if (j == 1 && p == 3) transpose_k(0);
+        lds_barrier();
+    }
+    for (int m = p; m < chunks; m += 4) {
+        const int par = m & 1, t0 = m * kChunkSteps, tc = min(A.T - t0, kChunkSteps);
+        {   // interval m - 2
+            f32x4v kk = {0.f, 0.f, 0.f, 0.f}, kq = {0.f, 0.f, 0.f, 0.f};
+            if (tc < kChunkSteps) {                    // the last chunk's missing steps are zeros
+#pragma unroll
+                for (int j = 0; j < NK; ++j) {
+                    kr[j] = n < tc ? kr[j] : none;
+                    qr[j] = n < tc ? qr[j] : none;
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) vr[v].bits = 4 * g + v < tc ? vr[v].bits : 0;
+            }
+#pragma unroll
+            for (int j = 0; j < NK; ++j) {
+                park(L.k[par][n], j, kr[j]);
+                const bf16x8v k8 = __builtin_bit_cast(bf16x8v, kr[j]);
+                kk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, k8, kk, 0, 0, 0);
+                kq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, __builtin_bit_cast(bf16x8v, qr[j]), kq, 0, 0, 0);
+            }
+            // decay products G[v] = g_{s+1} ... g_t of the lane's pairs (s, t) = (4g + v, n), 1 where s >= t
+            bool on = n < tc;
+            if (A.mask != nullptr) on = on && mask_on(A.mask, A.mask_dtype, (int)((uint32_t)b * A.T + t0 + min(n, tc - 1)));
+            const float gl = on ? to_float(gr) : 1.f;
+            beta = on ? to_float(br) : 0.f;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) vf[v] = to_float(vr[v]);
+            on_bits = __builtin_amdgcn_ballot_w64(on);
+            // steps in blocks of four: pre = the product from the block's first step up to the lane's, block products by broadcast
+            // (lane exchanges outside the selects: a select may become a branch, with the lanes that are read switched off)
+            const float left1 = quad_take<0, 0, 1, 2>(gl);
+            float pre = gl * (n % 4 >= 1 ? left1 : 1.f);
+            const float left2 = quad_take<0, 0, 0, 1>(pre);
+            pre *= n % 4 >= 2 ? left2 : 1.f;
+            const float b1 = row_broadcast<7>(pre), b2 = row_broadcast<11>(pre);
+            G[3] = n / 4 > g ? pre : 1.f;
+            G[3] *= g < 1 && n / 4 > 1 ? b1 : 1.f;
+            G[3] *= g < 2 && n / 4 > 2 ? b2 : 1.f;
+#pragma unroll
+            for (int v = 2; v >= 0; --v) {
+                const float gs = __shfl(gl, 4 * g + v + 1);
+                G[v] = G[v + 1] * (4 * g + v + 1 <= n ? gs : 1.f);
+            }
+            gam = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(gl), 0)) * G[0];      // of step n, in lanes g = 0
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int s = 4 * g + v;
+                av[v] = s < n ? -beta * (G[v] * kk[v]) : 0.f;
+                cv[v] = s <= n ? G[v] * kq[v] : 0.f;
+            }
+            asm volatile("" : "+v"(av), "+v"(cv), "+v"(gam), "+v"(G[0]), "+v"(G[1]), "+v"(G[2]), "+v"(G[3]));   // not sunk into the next interval
+        }
+        lds_barrier();
+        {   // interval m - 1
+            // T = (I + A)^-1 diag(beta), in the layout of the chain's a operand: lane (g, n) forms T[n][4g .. +3].  What other lanes
+            // of this wave wrote is read back without a wait: LDS serves a wave's accesses in order.
+            if (g == 0) { L.beta[par][n] = beta; L.gam[par][n] = gam; }
+            *reinterpret_cast<f32x4v*>(&L.na[par][n][4 * g]) = av;
+            float na[16];                              // row n of -A, the four lanes' pieces gathered
+            f32x4v x;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(av[v]), __float_as_uint(av[v]), false, false);   // g even, odd
+                const auto e = __builtin_amdgcn_permlane32_swap(r[0], r[0], false, false), o = __builtin_amdgcn_permlane32_swap(r[1], r[1], false, false);
+                na[v] = __uint_as_float(e[0]); na[8 + v] = __uint_as_float(e[1]);
+                na[4 + v] = __uint_as_float(o[0]); na[12 + v] = __uint_as_float(o[1]);
+            }
+            const f32x4v b4 = lds4(&L.beta[par][4 * g]);
+            gam4 = lds4(&L.gam[par][4 * g]);
+            *reinterpret_cast<f32x4v*>(L.v[par][lane]) = vf;
+            if (n == kChunkSteps - 1) *reinterpret_cast<float4*>(&L.w[par][4 * g]) = make_float4(G[0], G[1], G[2], G[3]);
+#pragma unroll
+            for (int j = 0; j < NK; ++j) park(L.q[par][n], j, qr[j]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = 4 * g + e == n ? 1.f : 0.f;
+            *reinterpret_cast<f32x4v*>(L.t2[par][lane]) = unit_inverse(x, na) * b4;
+        }
+        lds_barrier();
+        // interval m: this wave has no work on its own chunk.  Stores go ahead of the loads: the two are counted together, and
+        // the wait for the loads would include stores behind them (where loops join, the count is not exact).
+        if (m > p) store_rows(m - 4, kChunkSteps);
+        if (m + 4 < chunks) request(m + 4);
+        if (m + 1 < chunks) transpose_k(par ^ 1);
+        lds_barrier();
+        {   // interval m + 1: read-out and tape, rows t = 4g + v, column = state row n
+            const f32x4v pq = (lds4(L.pq[par][0][lane]) + lds4(L.pq[par][1][lane])) + (lds4(L.pq[par][2][lane]) + lds4(L.pq[par][3][lane]));
+            dl = lds4(L.dl[par][lane]);
+            yv = gam4 * pq;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) yv = __builtin_amdgcn_mfma_f32_16x16x4f32(cv[e], dl[e], yv, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) yv[v] = (on_bits >> (4 * g + v)) & 1 ? yv[v] : 0.f;
+            if (m + 4 >= chunks) store_rows(m, tc);
+            if (m + 1 == chunks) return;               // behind the last barrier
+        }
+        lds_barrier();
+    }
+    for (int i = p + (chunks - p + 3) / 4 * 4 - 2; i < chunks; ++i) lds_barrier();
+}
+
+template <int DK>
+static int launch_long(hipStream_t st, const GdnArgs& A, int B) {
+    dim3 grid(A.Dv / kChunkRows, A.Hv, B);
+    LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);
+    DFLASH_HIP_TRY(br.launch(gated_delta_long_kernel<DK>, grid, dim3(kLongThreads), sizeof(GdnLongLds<DK>), A));
+    return DFLASH_OK;
+}
+
+// More than one chunk, and k and q rows readable 16 bytes at a time.  The line lies at the second chunk as that is where
+// there is something to prepare ahead; this kernel is the faster one from there on (us, 17 and 32 steps: 32 heads of 128x128
+// 6.1 -> 5.3 and 6.3 -> 5.2, two such sequences 7.5 -> 6.3 and 7.9 -> 7.4, Dk = 256 17.0 -> 11.6 and 17.5 -> 12.3).  f16 inputs
+// stay with the chunk by chunk kernel: three f16 terms do not hold an fp32 state.
+bool gdn_long_applies(const GdnArgs& A, int Dk) {
+    return A.in_dtype == DFLASH_BF16 && A.T > kChunkSteps && (((uintptr_t)A.k | (uintptr_t)A.q) & 15) == 0 && (Dk == 64 || Dk == 128 || Dk == 256);
+}
+
+int launch_gdn_long(hipStream_t st, const GdnArgs& A, int B, int Dk) {
+    if (Dk == 64) return launch_long<64>(st, A, B);
+    if (Dk == 128) return launch_long<128>(st, A, B);
+    return launch_long<256>(st, A, B);
+}
+
+template <int DK>
+static int long_setup() {
+    DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gated_delta_long_kernel<DK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GdnLongLds<DK>)));
+    return DFLASH_OK;
+}
+
+int gdn_long_device_setup() {
+    int rc = long_setup<64>();
+    if (rc == DFLASH_OK) rc = long_setup<128>();
+    if (rc == DFLASH_OK) rc = long_setup<256>();
+    return rc;
+}
+
+}  // namespace dflash

@@ -40,6 +40,59 @@ def test_step_kernel_lanes_per_row(gpu_lib, Dk, Hv, Dv, T):
     np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
 
 
+# GatedDelta forward over more than one chunk of 16 steps: 2 to 9 chunks (the producer waves take every fourth), whole and ragged
+# last chunks, one and several row tiles
+@pytest.mark.parametrize("Dk,Dv", [(64, 16), (128, 128), (256, 32)], ids=lambda v: str(v))
+@pytest.mark.parametrize("T", [17, 32, 33, 48, 63, 65, 80, 97, 131])
+@pytest.mark.parametrize("masked", [False, True])
+def test_long_forward(gpu_lib, Dk, Dv, T, masked):
+    from swiftlm_amd import DFlashKernels as K
+
+    d = O.make_gdn_inputs(Dk + T, 2, T, 2, 4, Dk, Dv, in_dtype="bf16")
+    mask = None
+    if masked:
+        mask = np.ones((2, T), np.float32)
+        mask[0, 15:18] = 0
+        mask[1, T - 5:] = 0
+    ins = [dev(d[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")]
+    dmask = None if mask is None else dev(mask)
+    y, s, tape = K.gated_delta_kernel_with_tape(*ins, dev(d["state"]), dmask)
+    yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], mask, dtype=np.float64)
+    np.testing.assert_allclose(host(s), sw, rtol=1e-4, atol=1e-6)
+    np.testing.assert_allclose(host(tape), tw, rtol=1e-4, atol=1e-5)
+    np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
+    # the same rows 8 bytes off a 16-byte line take the chunk-by-chunk kernel: the same sums in another order
+    off = [torch.empty(t.numel() + 4, dtype=t.dtype, device="cuda")[4:].view(t.shape).copy_(t) if i < 2 else t for i, t in enumerate(ins)]
+    y2, s2, tape2 = K.gated_delta_kernel_with_tape(*off, dev(d["state"]), dmask)
+    np.testing.assert_allclose(host(s2), host(s), rtol=1e-4, atol=1e-6)
+    np.testing.assert_allclose(host(tape2), host(tape), rtol=1e-4, atol=1e-5)
+    np.testing.assert_allclose(host(y2), host(y), rtol=2e-2, atol=2e-2)
+
+
+# A value that is not finite stays in its row and in the steps from it on; a chunk whose solve matrix overflows (1e4^15) where no
+# delta does has the deltas that substitution gives.
+def test_long_forward_not_finite(gpu_lib):
+    from swiftlm_amd import DFlashKernels as K
+
+    T, row, step = 50, 5, 23
+    d = O.make_gdn_inputs(1, 1, T, 2, 4, 128, 32, in_dtype="bf16")
+    q, k, v, g, beta = [dev(d[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")]
+    y, s, tape = K.gated_delta_kernel_with_tape(q, k, v, g, beta, dev(d["state"]))
+    for bad in (float("inf"), float("nan")):
+        vb = v.clone()
+        vb[0, step, 1, row] = bad
+        yb, sb, tb = K.gated_delta_kernel_with_tape(q, k, vb, g, beta, dev(d["state"]))
+        np.testing.assert_allclose(host(tb[:, :step]), host(tape[:, :step]), rtol=1e-4, atol=1e-5)
+        assert not torch.isfinite(tb[0, step:, 1, row]).any() and not torch.isfinite(sb[0, 1, row]).any()
+        keep = torch.ones_like(tape, dtype=torch.bool)
+        keep[0, :, 1, row] = False
+        np.testing.assert_allclose(host(tb[keep]), host(tape[keep]), rtol=1e-4, atol=1e-5)
+        np.testing.assert_allclose(host(yb[keep]), host(y[keep]), rtol=2e-2, atol=2e-2)
+    big = torch.full_like(k, 10.0)                            # k.k = 12800
+    y, s, tape = K.gated_delta_kernel_with_tape(q, big, torch.zeros_like(v), torch.ones_like(g), torch.ones_like(beta), torch.zeros_like(s))
+    assert not y.any() and not s.any() and not tape.any()
+
+
 def attend(q, k, v, lens, D, **kw):
     from swiftlm_amd import DFlashKernels as K
 
