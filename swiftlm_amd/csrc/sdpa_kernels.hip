@@ -1080,8 +1080,12 @@ static int launch_sdpa(hipStream_t st, const SdpaArgs& A, const CombineArgs& C, 
         LaunchBracket br(DFLASH_KERNEL_SDPA_COMBINE, st);
         const dim3 waves((C.rows + kCombineThreads / 64 - 1) / (kCombineThreads / 64)), threads(kCombineThreads);
         const int groups = 64 / (D / 8);
+        // More than four splits per lane group are one wave's work up to 64 splits at D = 128, at D = 256 only where a workgroup per
+        // row would be more than the chip holds at once, and in a balanced launch half as many, as a long sequence takes more
+        // than S.  us per call, wave against workgroup: D=256, 256 rows of 14 splits 0.5 slower; D=128, 128 rows of 47 splits 8.3
+        // and 8.6, 512 rows of 32 splits 23.6 and 24.5; balanced, 256 rows of 64 splits 20.0 and 17.2.
         if (A.S <= 4 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 4>, waves, threads, 0, C));
-        else if (A.S <= 16 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
+        else if (A.S <= (C.balance ? 8 : 16) * groups && (D == 128 || C.rows > 4 * num_compute_units())) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
         else DFLASH_HIP_TRY(br.launch(sdpa_combine_kernel<Tag, D>, dim3(C.rows), threads, 0, C));
     }
     return DFLASH_OK;
@@ -1218,7 +1222,11 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     // lane of a wave per sequence; tile counts are summed as floats, exact below 2^24).
     A.lse = lse; A.B = B;
     if (S == 1) A.part_o = (uint16_t*)out;
-    A.balance = kv_len_dev && B > 1 && B <= 64 && S > 1 && (int64_t)B * ((N + kBN - 1) / kBN) < (1 << 24);
+    // The dealing costs both kernels a dependent trip to the counts and a few wave-wide sums and saves a part of the longest
+    // split's tiles: it is done from 8 tiles per split on (us, dealt and not: D=256, 2 x 12,000 keys, 6 tiles 17.3 and 15.7,
+    // 8 x 3,000 keys, 3 tiles 15.3 and 14.1; D=128, 4 x 9,000 keys, 9 tiles 13.4 and 14.4).
+    const int64_t tiles = (N + kBN - 1) / kBN;
+    A.balance = kv_len_dev && B > 1 && B <= 64 && S > 1 && tiles >= 8 * (int64_t)S && B * tiles < (1 << 24);
     C.balance = A.balance; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
 
     hipStream_t st = (hipStream_t)stream;

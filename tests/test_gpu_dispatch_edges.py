@@ -125,6 +125,26 @@ def test_ragged_shares(gpu_lib, lens, D):
     attend(q, k, v, lens, D, kv_len=torch.tensor(lens, dtype=torch.int32, device="cuda"))
 
 
+# ... which is done from 8 tiles per split on: eight sequences of eight KV heads take four splits each
+@pytest.mark.parametrize("D,N", [(256, 992), (256, 1024), (128, 992), (128, 1024), (128, 2200)])
+def test_ragged_shares_line(gpu_lib, D, N):
+    import ctypes as C
+
+    lens = [N, 16, N // 2, 17, 33, N, 700, 129]
+    q, k, v = tensors(N + D, 8, 8, 8, N, D)
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    assert gpu_lib.dflash_set_status_word(C.c_void_p(status.data_ptr())) == 0
+    try:
+        given = torch.tensor(lens, dtype=torch.int32, device="cuda")
+        attend(q, k, v, lens, D, kv_len=given)
+        assert int(status) == 0
+        given[5], given[1] = 9000, 3                # outside the bounds: flagged, and read as N and 16
+        attend(q, k, v, lens, D, kv_len=given)
+        assert int(status) == 1
+    finally:
+        assert gpu_lib.dflash_set_status_word(None) == 0
+
+
 def test_ragged_share_of_a_length_outside_the_bound_is_flagged_and_clamped(gpu_lib):
     import ctypes as C
 
