@@ -156,3 +156,59 @@ def test_ragged_share_of_a_length_outside_the_bound_is_flagged_and_clamped(gpu_l
         assert int(status) == 1
     finally:
         assert gpu_lib.dflash_set_status_word(None) == 0
+
+
+# A tile of 32 keys that a row sees nothing of leaves the row alone, whatever its V rows hold: in one split that writes the output
+# itself and as the first, a middle and the last tile of a longer one.  Tolerances as above: the tile adds nothing to these rows.
+def same_rows(out, lse, ow, lw):
+    np.testing.assert_allclose(host(out), ow, rtol=2e-2, atol=2e-2)
+    np.testing.assert_allclose(host(lse), lw, rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("N", [33, 47, 97, 110, 129, 2049, 2063])
+@pytest.mark.parametrize("Hq,Hk,D", [(3, 1, 256), (8, 8, 128)])
+def test_last_tile_hidden_by_the_causal_rule(gpu_lib, N, Hq, Hk, D, bad):
+    from swiftlm_amd import DFlashKernels as K
+
+    q, k, v = tensors(N + D, 1, Hq, Hk, N, D)
+    keys = N % 32                                             # of the last tile; row r sees keys up to N - 16 + r
+    want = O.sdpa_block_causal(host(q), host(k), host(v), 0.1)
+    v[:, :, N - keys:] = bad
+    out, lse = K.batched_sdpa_2pass(q, k, v, 0.1, return_lse=True)
+    same_rows(out[:, :, :16 - keys], lse[:, :, :16 - keys], want[0][:, :, :16 - keys], want[1][:, :, :16 - keys])
+    assert not torch.isfinite(out[:, :, 15]).any()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("N,tiles", [(64, [1]), (100, [0, 2]), (128, [0]), (128, [1, 3]), (2048, [0]), (2048, [16, 33]), (2048, [48]), (2048, [0, 16, 47])],
+                         ids=str)
+@pytest.mark.parametrize("Hq,Hk,D", [(8, 8, 128), (32, 8, 256)])
+def test_tiles_hidden_by_the_mask(gpu_lib, N, tiles, Hq, Hk, D, dt):
+    from swiftlm_amd import DFlashKernels as K
+
+    q, k, v = tensors(N + D, 1, Hq, Hk, N, D, dt)
+    mask = 0.1 * torch.randn(1, Hq, 16, N, generator=torch.Generator(device="cuda").manual_seed(N), device="cuda")
+    for t in tiles:
+        mask[..., 32 * t:32 * t + 32] = float("-inf")
+    mask[0, 1, 5] = float("-inf")                             # a row without any key
+    mask[0, 2, 3] = 0.0                                       # a row that sees the values that are not finite
+    mask = mask.to(dt)
+    seen = torch.ones(1, Hq, 16, dtype=torch.bool)
+    seen[0, 2, 3] = False
+    want = O.sdpa_block_causal(host(q), host(k), host(v), 0.1, host(mask).astype(np.float64))
+    for t in tiles:
+        v[:, :, 32 * t:32 * t + 32] = float("nan")
+    out, lse = K.batched_sdpa_2pass(q, k, v, 0.1, mask, return_lse=True)
+    same_rows(out[seen], lse[seen], want[0][seen], want[1][seen])
+    assert not out[0, 1, 5].any() and torch.isneginf(lse[0, 1, 5])
+    assert torch.isnan(out[0, 2, 3]).all()
+
+
+def test_tile_with_only_a_nan_score_is_not_hidden(gpu_lib):
+    from swiftlm_amd import DFlashKernels as K
+
+    q, k, v = tensors(1, 1, 4, 2, 33, 128)
+    k[:, :, 32] = float("nan")                                # seen by the last row alone
+    nan = torch.isnan(K.batched_sdpa_2pass(q, k, v, 0.1))
+    assert nan[:, :, 15].all() and not nan[:, :, :15].any()
