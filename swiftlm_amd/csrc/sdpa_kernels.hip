@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "dflash_common.h"
+#include "sdpa_shares.h"
 
 namespace dflash {
 
@@ -75,6 +76,7 @@ struct F16Tag {
     static __device__ __forceinline__ float to_f32(uint16_t x) { return (float)__builtin_bit_cast(_Float16, x); }
 };
 
+struct ShareDivide { uint32_t W_magic, rest_magic; };       // fast_div_magic of W = B * S and of W - B (RaggedShare)
 struct SdpaArgs {
     const uint16_t* q;
     const uint16_t* k;
@@ -101,6 +103,7 @@ struct SdpaArgs {
     uint32_t gpk_magic, S_magic;   // fast_div_magic of groups_per_kv and S
     float* lse;              // S == 1: part_o is the output itself and this (or null) its logsumexp; no combine follows
     int B, balance;          // balance: sequences of a ragged batch share the B * S splits by their lengths (RaggedShare)
+    ShareDivide share_div;
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -211,28 +214,30 @@ template <int D> struct SdpaLds {
 // while those of the shorter ones are done early and their compute units idle: four sequences of 8K to 64K keys ran at
 // 4.2 TB/s.  Instead the B * S workgroups of a (KV head, head group) are dealt to the sequences in proportion to their
 // key counts, which only the device knows: every wave loads the counts (one per lane, B <= 64), finds the smallest number
-// L of tiles per workgroup with sum(ceil(tiles_b / L)) <= B * S, and takes its place in that sequence of shares.  The
-// combine kernel repeats the computation for its row's sequence.
+// L of tiles per workgroup with sum(ceil(tiles_b / L)) <= B * S (tiles_per_share), and takes its place in that sequence of
+// shares.  The combine kernel repeats the computation once per workgroup.  us per call, not dealt, L searched one by one in every
+// wave, now (16 sequences, 8 KV heads of 8 query heads, D = 128, two splits each): 8K to 64K keys 706, 707, 522; 16K to 32K 418,
+// 569, 422, as lengths this close and two splits leave nothing to gain; one sequence of 102,400 beside 15 of 83,200 1218, 1597, 1224.
 struct RaggedShare {
     int n_lane, s_lane;      // lane b: key count and splits of sequence b (0 beyond B)
 };
 __device__ __forceinline__ int wave_sum_int(int x) { return (int)butterfly_sum<64>((float)x); }   // exact below 2^24
-__device__ __forceinline__ RaggedShare ragged_share(const int32_t* len_dev, int bias, int N, int B, int W, int lane) {
+__device__ __forceinline__ RaggedShare ragged_share(const int32_t* len_dev, int bias, int N, int B, int W, ShareDivide div, int lane) {
     int n = len_dev[lane < B ? lane : B - 1] + bias;
     n = n < kM ? kM : (n > N ? N : n);
     n = lane < B ? n : 0;
-    const int nt = (n + kBN - 1) / kBN;
-    const int total = wave_sum_int(nt), longest = (int)wave_max((float)nt);
-    int L = (total + W - 1) / W;
+    const float nt = (float)((n + kBN - 1) / kBN);
+    const int total = __builtin_amdgcn_readfirstlane((int)butterfly_sum<64>(nt)), longest = __builtin_amdgcn_readfirstlane((int)wave_max(nt));
     const int least = (longest + kMaxSplits - 1) / kMaxSplits;       // a sequence takes kMaxSplits splits at most
-    L = L < least ? least : L;
-    int s;
-    for (;;) {                                                       // ends: with L = longest every sequence takes one split, and B <= W
-        s = (nt + L - 1) / L;
-        if (L >= longest || wave_sum_int(s) <= W) break;
-        ++L;
-    }
-    return {n, s};
+    const int even = (int)fast_div((uint32_t)(total + W - 1), (uint32_t)W, div.W_magic);
+    const int loose = (int)fast_div((uint32_t)total, (uint32_t)(W - B), div.rest_magic) + 1;
+    auto splits = [&](int L) -> float {
+        return floorf(share_quotient(nt, __builtin_amdgcn_rcpf((float)L))) + 1.f;       // 0 beyond B
+    };
+    const int L = tiles_per_share(even < least ? least : even, longest < loose ? longest : loose, [&](int l) {
+        return __builtin_amdgcn_readfirstlane((int)butterfly_sum<64>(splits(l))) <= W;
+    });
+    return {n, (int)splits(L)};
 }
 
 // The t-th tile of a split: tiles are dealt in rows of S neighbouring tiles, one per split.
@@ -254,7 +259,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     asm volatile("" ::"s"(A.q), "s"(A.k), "s"(A.v), "s"(A.k_new), "s"(A.v_new), "s"(A.k_cache), "s"(A.v_cache), "s"(A.part_o),
                  "s"(A.part_m), "s"(A.part_l), "s"(A.kv_len_dev), "s"(A.mask), "s"(A.kv_batch_stride), "s"(A.kv_head_stride));
     asm volatile("" ::"s"(A.scale_log2), "s"(A.Hq), "s"(A.Hk), "s"(A.G), "s"(A.N), "s"(A.S), "s"(A.groups_per_kv),
-                 "s"(A.balance), "s"(A.B), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages),
+                 "s"(A.balance), "s"(A.B), "s"(A.share_div.W_magic), "s"(A.share_div.rest_magic), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages),
                  "s"(A.status), "s"(A.gpk_magic), "s"(A.S_magic));
 
     const int tid = threadIdx.x;
@@ -267,7 +272,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     int split = blockIdx.x, b = blockIdx.z, S = A.S, Nb_share = 0;
     if (A.balance) {                                         // uniform
         const int W = A.B * A.S, w = (int)blockIdx.z * A.S + (int)blockIdx.x;
-        const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, W, lane);
+        const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, W, A.share_div, lane);
         if (A.status && w == 0 && blockIdx.y == 0 && wave == 0 && lane < A.B) {
             const int n = A.kv_len_dev[lane] + A.len_bias;
             if (n < kM || n > A.N) atomicOr(A.status, DFLASH_STATUS_SDPA_LEN);
@@ -914,18 +919,27 @@ struct CombineArgs {
     int balance;             // ragged shares (RaggedShare): the fields below are theirs
     const int32_t* kv_len_dev;
     int len_bias, N;
+    ShareDivide share_div;
 };
 struct RowParts { const float *m, *l; const uint16_t* o; int S; size_t pitch; };   // o: the first slot's row; pitch: elements from slot to slot
-__device__ __forceinline__ RowParts row_parts(const CombineArgs& A, int row, int D, int lane) {
+__device__ __forceinline__ RowParts row_parts(const CombineArgs& A, int row, int D) {
     if (!A.balance) {
         const size_t stat = (size_t)row * A.S;
         return {A.part_m + stat, A.part_l + stat, A.part_o + (size_t)row * D, A.S, (size_t)A.rows * D};
     }
+    // The rows of a workgroup belong to one sequence (hqm is a multiple of 16): one wave looks its share up for all.
+    __shared__ int share_s[2];
     const int W = A.B * A.S, b = row / A.hqm, r = row - b * A.hqm;
-    const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, W, lane);
-    const int first = wave_sum_int(lane < b ? sh.s_lane : 0);
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, W, A.share_div, lane);
+        const int before = wave_sum_int(lane < b ? sh.s_lane : 0);
+        if (lane == b) { share_s[0] = before; share_s[1] = sh.s_lane; }
+    }
+    __syncthreads();
+    const int first = __builtin_amdgcn_readfirstlane(share_s[0]);
     const size_t stat = (size_t)r * W + first;
-    return {A.part_m + stat, A.part_l + stat, A.part_o + ((size_t)first * A.hqm + r) * D, __builtin_amdgcn_readlane(sh.s_lane, b), (size_t)A.hqm * D};
+    return {A.part_m + stat, A.part_l + stat, A.part_o + ((size_t)first * A.hqm + r) * D, __builtin_amdgcn_readfirstlane(share_s[1]), (size_t)A.hqm * D};
 }
 
 // One workgroup per row, for many splits: up to 16 partial rows per thread, all in flight at once.
@@ -942,7 +956,7 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
     asm volatile("" ::"s"(A.part_o), "s"(A.part_m), "s"(A.part_l), "s"(A.out), "s"(A.lse), "s"(A.S));   // one burst of argument loads
     const size_t row = blockIdx.x;
     const int tid = threadIdx.x;
-    const RowParts R = row_parts(A, (int)row, D, tid & 63);
+    const RowParts R = row_parts(A, (int)row, D);
     const int S = R.S;
     const int grp = tid / TPG, d8 = (tid % TPG) * 8;
     const uint16_t* po = R.o + d8;
@@ -1013,8 +1027,8 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
     if (tid == 0 && A.lse) A.lse[row] = (mx + log2f(lsum)) * 0.6931471805599453f;
 }
 
-// One wave per row, for few splits (a batch or many KV heads fill the chip, a short context has few tiles): no LDS, no
-// barrier, U partial rows per lane in flight.  A workgroup per row would fetch 16 rows per thread whatever S is and run
+// One wave per row, for few splits (a batch or many KV heads fill the chip, a short context has few tiles): no exchange
+// between waves, U partial rows per lane in flight.  A workgroup per row would fetch 16 rows per thread whatever S is and run
 // thousands of workgroups: 13 us for 4096 rows of 4 splits (B=8, Hq=32, D=128), where this takes 4.
 template <typename Tag, int D, int U>
 __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_wave_kernel(CombineArgs A) {
@@ -1023,8 +1037,7 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_wave_kernel(Comb
     asm volatile("" ::"s"(A.part_o), "s"(A.part_m), "s"(A.part_l), "s"(A.out), "s"(A.lse), "s"(A.S));
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * (kCombineThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (row >= A.rows) return;                     // whole waves; no barrier follows
-    const RowParts R = row_parts(A, row, D, lane);
+    const RowParts R = row_parts(A, row, D);       // (A.rows is a multiple of 16: every wave has a row)
     const int S = R.S, grp = lane / TPG, d8 = (lane % TPG) * 8;
     const uint16_t* po = R.o + d8;
     // the statistics of split `lane` and the first U partial rows of the group in one round trip
@@ -1144,7 +1157,7 @@ static int launch_sdpa(hipStream_t st, const SdpaArgs& A, const CombineArgs& C, 
     }
     if (A.S > 1) {
         LaunchBracket br(DFLASH_KERNEL_SDPA_COMBINE, st);
-        const dim3 waves((C.rows + kCombineThreads / 64 - 1) / (kCombineThreads / 64)), threads(kCombineThreads);
+        const dim3 waves(C.rows / (kCombineThreads / 64)), threads(kCombineThreads);
         const int groups = 64 / (D / 8);
         // More than four splits per lane group are one wave's work up to 64 splits at D = 128, at D = 256 only where a workgroup per
         // row would be more than the chip holds at once, and in a balanced launch half as many, as a long sequence takes more
@@ -1285,15 +1298,16 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     C.part_o = A.part_o; C.part_m = A.part_m; C.part_l = A.part_l;
     C.out = (uint16_t*)out; C.lse = lse; C.S = S; C.B = B; C.hqm = Hq * kM; C.rows = B * C.hqm;
     // A single split writes the output itself.  Several sequences with device-side lengths share the splits by length (one
-    // lane of a wave per sequence; tile counts are summed as floats, exact below 2^24).
+    // lane of a wave per sequence; tile counts are summed as floats, exact below 2^24; share_quotient holds below 2^20).
     A.lse = lse; A.B = B;
     if (S == 1) A.part_o = (uint16_t*)out;
     // The dealing costs both kernels a dependent trip to the counts and a few wave-wide sums and saves a part of the longest
     // split's tiles: it is done from 8 tiles per split on (us, dealt and not: D=256, 2 x 12,000 keys, 6 tiles 17.3 and 15.7,
     // 8 x 3,000 keys, 3 tiles 15.3 and 14.1; D=128, 4 x 9,000 keys, 9 tiles 13.4 and 14.4).
     const int64_t tiles = (N + kBN - 1) / kBN;
-    A.balance = kv_len_dev && B > 1 && B <= 64 && S > 1 && tiles >= 8 * (int64_t)S && B * tiles < (1 << 24);
-    C.balance = A.balance; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
+    A.balance = kv_len_dev && B > 1 && B <= 64 && S > 1 && tiles >= 8 * (int64_t)S && tiles < (1 << 20) && B * tiles < (1 << 24);
+    A.share_div = {fast_div_magic((uint32_t)(B * S)), fast_div_magic((uint32_t)(B * (S - 1)))};
+    C.balance = A.balance; C.share_div = A.share_div; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
 
     hipStream_t st = (hipStream_t)stream;
 #define DFLASH_SDPA_CASE(MASKED, PAGED)                                                                              \

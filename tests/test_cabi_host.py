@@ -204,3 +204,28 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert r.returncode != 0
     assert "one GPU" in (r.stdout + r.stderr)
+
+
+def test_ragged_shares_are_found_in_few_sums(tmp_path):
+    """How many tiles a workgroup of a ragged attention batch takes: the smallest number that leaves enough workgroups, found by
+    halving (at most 2 + log2 of the range), also where a search one by one takes hundreds of sums; tile counts up to 2^20."""
+    import math
+    import random
+    import subprocess
+
+    exe = tmp_path / "shares_check"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", os.path.join(ROOT, "tests", "shares", "shares_check.cpp"), "-o", str(exe)])
+    rng = random.Random(0)
+    sets = [(2, [3200] + [2600] * 15), (2, [512 + 32 * i for i in range(16)]), (2, [1] * 63 + [3200]), (2, [1, 1]), (64, [300, 1, 7]),
+            (255, [1 << 19, (1 << 20) - 1]), (2, [(1 << 18) - i for i in range(64)])]
+    for _ in range(400):
+        top = rng.choice([8, 300, 3200, 1 << 18])
+        sets.append((rng.choice([2, 2, 3, 4, 8, 32, 128]), [rng.randint(1, top) for _ in range(rng.randint(2, 64))]))
+    text = "".join(f"{len(t)} {s} {' '.join(map(str, t))}\n" for s, t in sets)
+    lines = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.split("\n")
+    slowest = 0
+    for (s, tiles), line in zip(sets, lines):
+        _, sums, linear = map(int, line.split())
+        assert sums <= 2 + math.log2(max(tiles)), (s, tiles)
+        slowest = max(slowest, linear)
+    assert slowest > 200
