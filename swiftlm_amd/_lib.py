@@ -108,7 +108,7 @@ class _Native:
             from . import _native
         except ImportError as e:
             raise DFlashError(f"the compiled binding swiftlm_amd/_native.so does not load ({e}): build it with "
-                              "`make -C swiftlm_amd/csrc` (or __graft_entry__.build()); there is no fallback path") from e
+                              "`make -C swiftlm_amd/csrc native` (or __graft_entry__.build()); there is no fallback path") from e
         _native.set_errors(DFlashError, DFlashUnsupported)
         self.__dict__.update({k: v for k, v in vars(_native).items() if not k.startswith("__")})
         return getattr(_native, name)

@@ -229,3 +229,15 @@ def test_ragged_shares_are_found_in_few_sums(tmp_path):
         assert sums <= 2 + math.log2(max(tiles)), (s, tiles)
         slowest = max(slowest, linear)
     assert slowest > 200
+
+
+def test_library_builds_without_python():
+    """The library and its plain-C clients are what `make` builds by default, on a machine without Python or PyTorch too; the
+    Python package's binding is a target of its own."""
+    import subprocess
+
+    make = ["make", "-n", "-B", "-C", os.path.join(ROOT, "swiftlm_amd", "csrc"), "PYTHON=/nonexistent"]
+    r = subprocess.run(make, capture_output=True, text=True)
+    assert r.returncode == 0 and not r.stderr, r.stderr
+    assert "libdflash_hip.so" in r.stdout and "step_check" in r.stdout and "_native.so" not in r.stdout
+    assert "_native.so" in subprocess.run(make[:-1] + ["native"], capture_output=True, text=True).stdout
