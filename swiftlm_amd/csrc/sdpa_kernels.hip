@@ -76,7 +76,7 @@ struct F16Tag {
     static __device__ __forceinline__ float to_f32(uint16_t x) { return (float)__builtin_bit_cast(_Float16, x); }
 };
 
-struct ShareDivide { uint32_t W_magic, rest_magic; };       // fast_div_magic of W = B * S and of W - B (RaggedShare)
+struct ShareOut { int W; uint32_t W_magic, rest_magic; };       // workgroups to share out (RaggedShare), fast_div_magic of W and of W - B
 struct SdpaArgs {
     const uint16_t* q;
     const uint16_t* k;
@@ -102,8 +102,8 @@ struct SdpaArgs {
     int32_t* status;         // device status word (dflash_set_status_word), or null
     uint32_t gpk_magic, S_magic;   // fast_div_magic of groups_per_kv and S
     float* lse;              // S == 1: part_o is the output itself and this (or null) its logsumexp; no combine follows
-    int B, balance;          // balance: sequences of a ragged batch share the B * S splits by their lengths (RaggedShare)
-    ShareDivide share_div;
+    int B, balance;          // balance: sequences of a ragged batch share the splits by their lengths (RaggedShare)
+    ShareOut deal;
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -163,7 +163,7 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 }
 
 // ---------------------------------------------------------------------------
-// The partial kernel.  Grid: x = split, y = kv head * groups_per_kv + head group, z = batch.
+// The partial kernel.  Grid: x = split, y = kv head * groups_per_kv + head group, z = batch (dealt: x = share, z = 1).
 //
 // Roles.  A wave that issues HBM -> LDS loads is held at each load until the memory pipeline takes it; in the
 // streaming steady state that is most of a tile's transfer time, and a wave that is held cannot feed its
@@ -212,30 +212,41 @@ template <int D> struct SdpaLds {
 
 // Ragged batches.  With S splits for every sequence, a launch lasts as long as the longest sequence takes S workgroups,
 // while those of the shorter ones are done early and their compute units idle: four sequences of 8K to 64K keys ran at
-// 4.2 TB/s.  Instead the B * S workgroups of a (KV head, head group) are dealt to the sequences in proportion to their
-// key counts, which only the device knows: every wave loads the counts (one per lane, B <= 64), finds the smallest number
-// L of tiles per workgroup with sum(ceil(tiles_b / L)) <= B * S (tiles_per_share), and takes its place in that sequence of
-// shares.  The combine kernel repeats the computation once per workgroup.  us per call, not dealt, L searched one by one in every
-// wave, now (16 sequences, 8 KV heads of 8 query heads, D = 128, two splits each): 8K to 64K keys 706, 707, 522; 16K to 32K 418,
-// 569, 422, as lengths this close and two splits leave nothing to gain; one sequence of 102,400 beside 15 of 83,200 1218, 1597, 1224.
+// 4.2 TB/s.  Instead W workgroups of a (KV head, head group) -- its B * S, or as many as the chip holds at once, as all of them
+// take the same time -- are dealt to the sequences in proportion to their key counts, which only the device knows: every wave
+// loads the counts (one per lane, B <= 64), finds the smallest number L of tiles per workgroup with sum(ceil(tiles_b / L)) <= W
+// (tiles_per_share), and takes its place in that sequence of shares.  The combine kernel repeats the computation once per
+// workgroup.  us per call, not dealt, L searched one by one in every wave, now (16 sequences, 8 KV heads of 8 query heads,
+// D = 128, two splits each): 8K to 64K keys 670, 673, 530; 16K to 32K 436, 574, 438, as lengths this close and two splits leave
+// nothing to gain; one sequence of 102,400 beside 15 of 83,200 1239, 1542, 1245.
 struct RaggedShare {
     int n_lane, s_lane;      // lane b: key count and splits of sequence b (0 beyond B)
 };
 __device__ __forceinline__ int wave_sum_int(int x) { return (int)butterfly_sum<64>((float)x); }   // exact below 2^24
-__device__ __forceinline__ RaggedShare ragged_share(const int32_t* len_dev, int bias, int N, int B, int W, ShareDivide div, int lane) {
+// Sum over the lanes up to and including this one: shifts inside rows of 16 lanes, then a row's last lane to the rows behind.
+__device__ __forceinline__ int wave_prefix_sum(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return x;
+}
+__device__ __forceinline__ RaggedShare ragged_share(const int32_t* len_dev, int bias, int N, int B, ShareOut deal, int lane) {
     int n = len_dev[lane < B ? lane : B - 1] + bias;
     n = n < kM ? kM : (n > N ? N : n);
     n = lane < B ? n : 0;
     const float nt = (float)((n + kBN - 1) / kBN);
     const int total = __builtin_amdgcn_readfirstlane((int)butterfly_sum<64>(nt)), longest = __builtin_amdgcn_readfirstlane((int)wave_max(nt));
     const int least = (longest + kMaxSplits - 1) / kMaxSplits;       // a sequence takes kMaxSplits splits at most
-    const int even = (int)fast_div((uint32_t)(total + W - 1), (uint32_t)W, div.W_magic);
-    const int loose = (int)fast_div((uint32_t)total, (uint32_t)(W - B), div.rest_magic) + 1;
+    const int even = (int)fast_div((uint32_t)(total + deal.W - 1), (uint32_t)deal.W, deal.W_magic);
+    const int loose = (int)fast_div((uint32_t)total, (uint32_t)(deal.W - B), deal.rest_magic) + 1;
     auto splits = [&](int L) -> float {
         return floorf(share_quotient(nt, __builtin_amdgcn_rcpf((float)L))) + 1.f;       // 0 beyond B
     };
     const int L = tiles_per_share(even < least ? least : even, longest < loose ? longest : loose, [&](int l) {
-        return __builtin_amdgcn_readfirstlane((int)butterfly_sum<64>(splits(l))) <= W;
+        return __builtin_amdgcn_readfirstlane((int)butterfly_sum<64>(splits(l))) <= deal.W;
     });
     return {n, (int)splits(L)};
 }
@@ -259,7 +270,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     asm volatile("" ::"s"(A.q), "s"(A.k), "s"(A.v), "s"(A.k_new), "s"(A.v_new), "s"(A.k_cache), "s"(A.v_cache), "s"(A.part_o),
                  "s"(A.part_m), "s"(A.part_l), "s"(A.kv_len_dev), "s"(A.mask), "s"(A.kv_batch_stride), "s"(A.kv_head_stride));
     asm volatile("" ::"s"(A.scale_log2), "s"(A.Hq), "s"(A.Hk), "s"(A.G), "s"(A.N), "s"(A.S), "s"(A.groups_per_kv),
-                 "s"(A.balance), "s"(A.B), "s"(A.share_div.W_magic), "s"(A.share_div.rest_magic), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages),
+                 "s"(A.balance), "s"(A.B), "s"(A.deal.W), "s"(A.deal.W_magic), "s"(A.deal.rest_magic), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages),
                  "s"(A.status), "s"(A.gpk_magic), "s"(A.S_magic));
 
     const int tid = threadIdx.x;
@@ -271,20 +282,18 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     const int hg0 = ((int)blockIdx.y - hk * A.groups_per_kv) * kHeadsPerWG;
     int split = blockIdx.x, b = blockIdx.z, S = A.S, Nb_share = 0;
     if (A.balance) {                                         // uniform
-        const int W = A.B * A.S, w = (int)blockIdx.z * A.S + (int)blockIdx.x;
-        const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, W, A.share_div, lane);
+        const int w = blockIdx.x;
+        const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, A.deal, lane);
         if (A.status && w == 0 && blockIdx.y == 0 && wave == 0 && lane < A.B) {
             const int n = A.kv_len_dev[lane] + A.len_bias;
             if (n < kM || n > A.N) atomicOr(A.status, DFLASH_STATUS_SDPA_LEN);
         }
-        int first = 0;
-        b = -1;
-        for (int i = 0; i < A.B; ++i) {
-            const int si = __builtin_amdgcn_readlane(sh.s_lane, i);
-            if (b < 0 && w < first + si) { b = i; split = w - first; S = si; Nb_share = __builtin_amdgcn_readlane(sh.n_lane, i); }
-            first += si;
-        }
-        if (b < 0) return;                                   // more workgroups than tiles
+        const int end = wave_prefix_sum(sh.s_lane);          // lane i: the first workgroup behind sequence i
+        b = __builtin_popcountll(__builtin_amdgcn_ballot_w64(end <= w));      // beyond B: `end` is that of the last sequence
+        if (b >= A.B) return;                                // more workgroups than shares
+        S = __builtin_amdgcn_readlane(sh.s_lane, b);
+        split = w - (__builtin_amdgcn_readlane(end, b) - S);
+        Nb_share = __builtin_amdgcn_readlane(sh.n_lane, b);
     }
     const int hcount = (A.G - hg0) < kHeadsPerWG ? (A.G - hg0) : kHeadsPerWG;
 
@@ -376,7 +385,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
     // Where the split's partial rows and statistics go: rows [slot][Hq * 16][D]; statistics [row][split], in a balanced
     // launch [row of the sequence][workgroup], so that a sequence's splits are neighbours either way.
     const int hqm = A.Hq * kM;
-    const int slot = A.balance ? (int)blockIdx.z * A.S + (int)blockIdx.x : split * A.B + b;
+    const int slot = A.balance ? (int)blockIdx.x : split * A.B + b;
     auto stat_at = [&](int row_in_seq) -> size_t {
         return A.balance ? (size_t)row_in_seq * (A.B * A.S) + slot : ((size_t)b * hqm + row_in_seq) * A.S + split;
     };
@@ -919,7 +928,7 @@ struct CombineArgs {
     int balance;             // ragged shares (RaggedShare): the fields below are theirs
     const int32_t* kv_len_dev;
     int len_bias, N;
-    ShareDivide share_div;
+    ShareOut deal;
 };
 struct RowParts { const float *m, *l; const uint16_t* o; int S; size_t pitch; };   // o: the first slot's row; pitch: elements from slot to slot
 __device__ __forceinline__ RowParts row_parts(const CombineArgs& A, int row, int D) {
@@ -932,7 +941,7 @@ __device__ __forceinline__ RowParts row_parts(const CombineArgs& A, int row, int
     const int W = A.B * A.S, b = row / A.hqm, r = row - b * A.hqm;
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x;
-        const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, W, A.share_div, lane);
+        const RaggedShare sh = ragged_share(A.kv_len_dev, A.len_bias, A.N, A.B, A.deal, lane);
         const int before = wave_sum_int(lane < b ? sh.s_lane : 0);
         if (lane == b) { share_s[0] = before; share_s[1] = sh.s_lane; }
     }
@@ -1150,7 +1159,7 @@ static int launch_sdpa(hipStream_t st, const SdpaArgs& A, const CombineArgs& C, 
     typedef SdpaLds<D> L;
     static_assert(L::BYTES <= 160 * 1024, "Q and the tile rings must fit the 160 KB LDS of a gfx950 CU");
     auto kern = sdpa_partial_kernel<Tag, D, MASKED, PAGED>;     // its dynamic-LDS limit is set per device by sdpa_device_setup()
-    dim3 grid(A.S, A.Hk * A.groups_per_kv, B);
+    const dim3 grid(A.balance ? A.deal.W : A.S, A.Hk * A.groups_per_kv, A.balance ? 1 : B);
     {
         LaunchBracket br(DFLASH_KERNEL_SDPA_PARTIAL, st);
         DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kPartialThreads), L::BYTES, A));
@@ -1301,13 +1310,27 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     // lane of a wave per sequence; tile counts are summed as floats, exact below 2^24; share_quotient holds below 2^20).
     A.lse = lse; A.B = B;
     if (S == 1) A.part_o = (uint16_t*)out;
-    // The dealing costs both kernels a dependent trip to the counts and a few wave-wide sums and saves a part of the longest
-    // split's tiles: it is done from 8 tiles per split on (us, dealt and not: D=256, 2 x 12,000 keys, 6 tiles 17.3 and 15.7,
-    // 8 x 3,000 keys, 3 tiles 15.3 and 14.1; D=128, 4 x 9,000 keys, 9 tiles 13.4 and 14.4).
-    const int64_t tiles = (N + kBN - 1) / kBN;
-    A.balance = kv_len_dev && B > 1 && B <= 64 && S > 1 && tiles >= 8 * (int64_t)S && tiles < (1 << 20) && B * tiles < (1 << 24);
-    A.share_div = {fast_div_magic((uint32_t)(B * S)), fast_div_magic((uint32_t)(B * (S - 1)))};
-    C.balance = A.balance; C.share_div = A.share_div; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
+    // W workgroups per (KV head, head group): one for every split, but no more than fit the chip at once, one on a compute unit.
+    // The dealing costs both kernels a dependent trip to the counts, the search and the look-up, 1 to 2 us, and takes off the
+    // longest split what the others have too little: with lengths spread evenly a share of its tiles that grows with
+    // (B - 1) / B.  us, not dealt and dealt, lengths from an eighth of N up, at x = (B - 1) * tiles / W:
+    //   more than eight splits per sequence   2 sequences, Hk=2, D=256: x = 8 33.4 34.3, x = 12 42.6 42.6, x = 16 52.3 50.5
+    //                                         64 sequences of 4 splits, D=128: x = 12 18.0 18.7, x = 16 20.8 20.2
+    //   three to eight, up to 16 sequences    8 of 4 splits, Hk=8, D=128: x = 7 13.3 14.2, x = 9 14.3 14.4, x = 14 18.0 17.3
+    //                                         4 of 8 splits, Hk=8, D=256: x = 6 22.8 21.9, x = 9 28.1 25.7
+    //   less than three (halves to deal)      16 of 2 splits, Hk=8, G=8, D=128: x = 22 29.1 30.8, x = 30 34.0 34.4, x = 45 44.3 42.4
+    //   more splits than fit at once          5 sequences, Hk=8, D=128: x = 7 13.8 12.3, x = 42 37.1 28.7 (equal lengths 62.4 41.1)
+    //                                         6 sequences, Hk=2, D=256: x = 7 26.8 26.8, x = 41 68.9 57.9 (equal lengths 116.7 84.8)
+    A.balance = 0;
+    A.deal = {0, 0, 0};
+    if (kv_len_dev && B > 1 && B <= 64 && S > 1) {
+        const int64_t tiles = (N + kBN - 1) / kBN;
+        const int fit = num_compute_units() / (Hk * groups), W = fit < B * S ? fit : B * S;
+        const int line = B * S > fit || (W >= 3 * B && W <= 8 * B && B <= 16) ? 7 : W < 3 * B ? 30 : 12;
+        A.balance = W > B && (B - 1) * tiles >= (int64_t)line * W && tiles < (1 << 20) && B * tiles < (1 << 24);
+        if (A.balance) A.deal = {W, fast_div_magic((uint32_t)W), fast_div_magic((uint32_t)(W - B))};
+    }
+    C.balance = A.balance; C.deal = A.deal; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
 
     hipStream_t st = (hipStream_t)stream;
 #define DFLASH_SDPA_CASE(MASKED, PAGED)                                                                              \

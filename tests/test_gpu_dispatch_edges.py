@@ -102,6 +102,7 @@ def attend(q, k, v, lens, D, **kw):
         ow, lw = O.sdpa_block_causal(host(q[b:b + 1]), host(k[b:b + 1, :, :n]), host(v[b:b + 1, :, :n]), 1.0 / math.sqrt(D))
         np.testing.assert_allclose(host(out[b]), ow[0], rtol=2e-2, atol=2e-2, err_msg=f"sequence {b} of {n} keys")
         np.testing.assert_allclose(host(lse[b]), lw[0], rtol=2e-3, atol=2e-3, err_msg=f"sequence {b} of {n} keys")
+    return out, lse
 
 
 def tensors(seed, B, Hq, Hk, N, D, dt=torch.bfloat16):
@@ -116,20 +117,105 @@ def test_attention_split_counts(gpu_lib, N, Hq, Hk, D):
     attend(*tensors(N + D, 1, Hq, Hk, N, D), [N], D)
 
 
-# ragged batches share the splits: one sequence beside many, equal lengths, all at the minimum, more sequences than one wave has lanes
+# ragged batches of short sequences, every one with its own splits: one beside many, equal lengths, all at the minimum, 64 and 65
 @pytest.mark.parametrize("lens", [[700, 16], [16, 17, 2000, 33], [500] * 5, [16] * 3 + [129], [40 + 3 * i for i in range(64)],
                                   [40 + 3 * i for i in range(65)]], ids=lambda v: f"{len(v)}x{max(v)}")
 @pytest.mark.parametrize("D", [128, 256])
-def test_ragged_shares(gpu_lib, lens, D):
+def test_ragged_short(gpu_lib, lens, D):
+    assert not dealt(len(lens), 4, 2, max(lens), D)
     q, k, v = tensors(len(lens) + D, len(lens), 4, 2, max(lens), D)
     attend(q, k, v, lens, D, kv_len=torch.tensor(lens, dtype=torch.int32, device="cuda"))
 
 
-# ... which is done from 8 tiles per split on: eight sequences of eight KV heads take four splits each
+# From a line on, in tiles of 32 keys per workgroup and with up to 64 sequences, a lane each, the workgroups are dealt by length.
+def splits(B, Hq, Hk, N, D):
+    from swiftlm_amd import DFlashKernels as K
+
+    return K.sdpa_workspace_bytes(B, Hq, Hk, 16, N, D) // (B * Hq * 16 * (2 * D + 8))
+
+
+def dealt(B, Hq, Hk, N, D, most=64):
+    S = splits(B, Hq, Hk, N, D)
+    fit = torch.cuda.get_device_properties(0).multi_processor_count // (Hk * -(-(Hq // Hk) // 8))
+    W = min(fit, B * S)
+    line = 7 if B * S > fit or (3 * B <= W <= 8 * B and B <= 16) else 30 if W < 3 * B else 12
+    return B <= most and W > B and (B - 1) * -(-N // 32) >= line * W
+
+
+# Every form of the call, each with a sequence of more than 64 splits beside short ones: one wave merges a row at D = 128, a
+# workgroup at D = 256.  Paged and fused calls give the bits of the dense one (the same shares, the same order).
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("lens", [[16384, 16, 17, 40], [33, 16384, 16383, 16], [9000, 8999, 16, 16382]], ids=str)
+def test_ragged_shares_every_form(gpu_lib, lens, D, dt):
+    from swiftlm_amd import DFlashKernels as K
+
+    B, Hq, Hk, N, P, scale = 4, 4, 2, 16384, 64, 1.0 / math.sqrt(D)
+    assert dealt(B, Hq, Hk, N, D) and splits(B, Hq, Hk, N, D) == 32
+    q, k, v = tensors(sum(lens) + D, B, Hq, Hk, N, D, dt)
+    n = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out, lse = attend(q, k, v, lens, D, kv_len=n)
+    mask = 0.1 * torch.randn(B, Hq, 16, N, generator=torch.Generator(device="cuda").manual_seed(N), device="cuda")
+    mask[:, :, :, 32:64] = float("-inf")                      # a hidden tile among others, with values that are not finite
+    mask = mask.to(dt)
+    vm = v.clone()
+    vm[:, :, 32:64] = float("nan")
+    om, lm = K.batched_sdpa_2pass(q, k, vm, scale, mask, return_lse=True, kv_len=n)
+    for b, m in enumerate(lens):
+        want = O.sdpa_block_causal(host(q[b:b + 1]), host(k[b:b + 1, :, :m]), host(v[b:b + 1, :, :m]), scale, host(mask[b:b + 1, :, :, :m]).astype(np.float64))
+        same_rows(om[b], lm[b], want[0][0], want[1][0])
+    # fused append: the block's rows come from apart and end up in the cache
+    kc, vc = k.clone(), v.clone()
+    k_new, v_new = (torch.stack([t[b, :, m - 16:m] for b, m in enumerate(lens)]).contiguous() for t in (k, v))
+    for b, m in enumerate(lens):
+        kc[b, :, m - 16:m] = vc[b, :, m - 16:m] = 9.0
+    oa, la = K.batched_sdpa_2pass_append(q, kc, vc, k_new, v_new, scale, N, cache_len=n - 16, return_lse=True)
+    assert torch.equal(oa, out) and torch.equal(la, lse) and torch.equal(kc, k) and torch.equal(vc, v)
+    # pages in any order
+    order = torch.randperm(B * N // P, generator=torch.Generator().manual_seed(D))
+    table = order.view(B, N // P).to(torch.int32).cuda()
+    kp, vp = (torch.empty(B * N // P, Hk, P, D, dtype=dt, device="cuda") for _ in range(2))
+    for pool, t in ((kp, k), (vp, v)):
+        pool[order.cuda()] = t.view(B, Hk, N // P, P, D).transpose(1, 2).reshape(-1, Hk, P, D)
+    op, lp = K.batched_sdpa_2pass_paged(q, kp, vp, table, scale, N, lengths=n, return_lse=True)
+    assert torch.equal(op, out) and torch.equal(lp, lse)
+    for b, m in enumerate(lens):
+        for r in range(m - 16, m):
+            kp[table[b, r // P], :, r % P] = vp[table[b, r // P], :, r % P] = 9.0
+    op, lp = K.batched_sdpa_2pass_paged(q, kp, vp, table, scale, N, k_new=k_new, v_new=v_new, lengths=n - 16, return_lse=True)
+    assert torch.equal(op, out) and torch.equal(lp, lse)
+    for pool, t in ((kp, k), (vp, v)):
+        assert torch.equal(pool[order.cuda()].view(B, N // P, Hk, P, D).transpose(1, 2).reshape(B, Hk, N, D), t)
+
+
+# The combine kernels behind dealt splits: a wave with 4 or 16 rows in flight, a workgroup; as many sequences as a wave has lanes; a
+# workgroup for every split, and fewer, as no more fit the chip at once.
+@pytest.mark.parametrize("B,Hq,Hk,D,N,S", [(64, 2, 1, 128, 1600, 4), (64, 3, 1, 256, 1600, 4), (63, 1, 1, 128, 2000, 5), (16, 8, 1, 256, 6600, 16), (16, 2, 1, 256, 6600, 16),
+                                           (2, 1, 1, 128, 98304, 128), (2, 1, 1, 256, 98304, 128), (32, 8, 4, 128, 2000, 2),
+                                           (3, 16, 2, 128, 16512, 43), (3, 4, 2, 256, 16000, 43), (5, 8, 8, 128, 2000, 7), (12, 8, 8, 256, 900, 3), (50, 8, 1, 128, 2000, 6)])
+def test_ragged_shares_combine(gpu_lib, B, Hq, Hk, D, N, S):
+    assert dealt(B, Hq, Hk, N, D) and splits(B, Hq, Hk, N, D) == S
+    rng = np.random.default_rng(B + D)
+    lens = [int(n) for n in np.exp(rng.uniform(math.log(16), math.log(N), B))]
+    lens[B // 2] = N
+    q, k, v = tensors(B + D, B, Hq, Hk, N, D)
+    attend(q, k, v, lens, D, kv_len=torch.tensor(lens, dtype=torch.int32, device="cuda"))
+
+
+def test_ragged_batch_of_more_sequences_than_lanes(gpu_lib):
+    B, N, D = 65, 1600, 128
+    assert not dealt(B, 2, 1, N, D) and dealt(B, 2, 1, N, D, most=B)
+    lens = [16 + (N - 16) * i // (B - 1) for i in range(B)]
+    q, k, v = tensors(B, B, 2, 1, N, D)
+    attend(q, k, v, lens, D, kv_len=torch.tensor(lens, dtype=torch.int32, device="cuda"))
+
+
+# the line: eight sequences of eight KV heads take four splits each
 @pytest.mark.parametrize("D,N", [(256, 992), (256, 1024), (128, 992), (128, 1024), (128, 2200)])
 def test_ragged_shares_line(gpu_lib, D, N):
     import ctypes as C
 
+    assert dealt(8, 8, 8, N, D) == (N >= 1024)
     lens = [N, 16, N // 2, 17, 33, N, 700, 129]
     q, k, v = tensors(N + D, 8, 8, 8, N, D)
     status = torch.zeros(1, dtype=torch.int32, device="cuda")
@@ -145,7 +231,8 @@ def test_ragged_shares_line(gpu_lib, D, N):
         assert gpu_lib.dflash_set_status_word(None) == 0
 
 
-def test_ragged_share_of_a_length_outside_the_bound_is_flagged_and_clamped(gpu_lib):
+# (splits of its own; the test above has dealt ones)
+def test_ragged_short_length_outside_the_bound_is_flagged_and_clamped(gpu_lib):
     import ctypes as C
 
     q, k, v = tensors(3, 3, 4, 2, 400, 128)
