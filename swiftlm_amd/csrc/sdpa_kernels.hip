@@ -1109,6 +1109,12 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_wave_kernel(Comb
 
 // ---- host side -------------------------------------------------------------
 
+// Up to this many tiles one split does them all and writes the output itself: no partial rows, no second launch.  us on the GPU,
+// one split and one per tile:
+//     tiles          2           3           4           5           6
+//     D=128    5.3   7.2   5.7   7.0   6.3   7.0   6.9   7.1   7.4   7.1   (512 rows; 2,048 rows at four 6.3 7.9, at six 7.5 8.5)
+//     D=256    7.1   8.4   7.7   7.8   8.7   8.0   9.7   8.3  10.6   8.1   (256 rows; 1,024 rows at four 8.8 8.5, at five 9.8 9.0)
+// At four, what D=256 loses is less than what D=128 and the host gain; at five it is more.
 constexpr int kDirectTiles = 4;
 static int choose_splits(int B, int Hk, int groups_per_kv, int N) {
     const int nt = (N + kBN - 1) / kBN;
@@ -1168,12 +1174,16 @@ static int launch_sdpa(hipStream_t st, const SdpaArgs& A, const CombineArgs& C, 
         LaunchBracket br(DFLASH_KERNEL_SDPA_COMBINE, st);
         const dim3 waves(C.rows / (kCombineThreads / 64)), threads(kCombineThreads);
         const int groups = 64 / (D / 8);
-        // More than four splits per lane group are one wave's work up to 64 splits at D = 128, at D = 256 only where a workgroup per
-        // row would be more than the chip holds at once, and in a balanced launch half as many, as a long sequence takes more
-        // than S.  us per call, wave against workgroup: D=256, 256 rows of 14 splits 0.5 slower; D=128, 128 rows of 47 splits 8.3
-        // and 8.6, 512 rows of 32 splits 23.6 and 24.5; balanced, 256 rows of 64 splits 20.0 and 17.2.
+        // More than four splits per lane group: one wave per row, 16 partial rows per lane in flight, up to 64 splits at D = 128 (a
+        // dealt launch 32, as its long sequences take more than S), at D = 256 where a workgroup per row would be more than the
+        // chip holds at once.  us per call, wave against workgroup, rows x splits:
+        //   D=128  1,024 x 32 17.3 19.1   512 x 64 16.6 17.8   384 x 74 17.0 16.0   256 x 128 19.3 16.7
+        //   dealt    896 x 37 23.3 23.6   768 x 43 21.4 20.6   512 x 64 21.3 18.4
+        //   D=256  2,048 x 16 38.9 42.3  1,280 x 26 38.4 40.9  1,024 x 32 29.0 29.5  256 x 16 29.1 28.5  512 x 64 32.7 27.8
+        //   dealt  2,048 x 16 43.4 48.2  1,280 x 26 34.2 35.0  1,024 x 32 32.1 30.1
+        auto one_wave = [&]() { return D == 128 ? A.S <= (C.balance ? 32 : 64) : A.S <= 32 && C.rows > 4 * num_compute_units(); };
         if (A.S <= 4 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 4>, waves, threads, 0, C));
-        else if (A.S <= (C.balance ? 8 : 16) * groups && (D == 128 || C.rows > 4 * num_compute_units())) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
+        else if (one_wave()) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
         else DFLASH_HIP_TRY(br.launch(sdpa_combine_kernel<Tag, D>, dim3(C.rows), threads, 0, C));
     }
     return DFLASH_OK;

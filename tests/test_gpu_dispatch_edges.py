@@ -190,7 +190,7 @@ def test_ragged_shares_every_form(gpu_lib, lens, D, dt):
 
 # The combine kernels behind dealt splits: a wave with 4 or 16 rows in flight, a workgroup; as many sequences as a wave has lanes; a
 # workgroup for every split, and fewer, as no more fit the chip at once.
-@pytest.mark.parametrize("B,Hq,Hk,D,N,S", [(64, 2, 1, 128, 1600, 4), (64, 3, 1, 256, 1600, 4), (63, 1, 1, 128, 2000, 5), (16, 8, 1, 256, 6600, 16), (16, 2, 1, 256, 6600, 16),
+@pytest.mark.parametrize("B,Hq,Hk,D,N,S", [(64, 2, 1, 128, 1600, 4), (64, 3, 1, 256, 1600, 4), (63, 1, 1, 128, 2000, 5), (16, 8, 1, 256, 6600, 16), (16, 2, 1, 256, 6600, 16), (11, 8, 1, 256, 6600, 24),
                                            (2, 1, 1, 128, 98304, 128), (2, 1, 1, 256, 98304, 128), (32, 8, 4, 128, 2000, 2),
                                            (3, 16, 2, 128, 16512, 43), (3, 4, 2, 256, 16000, 43), (5, 8, 8, 128, 2000, 7), (12, 8, 8, 256, 900, 3), (50, 8, 1, 128, 2000, 6)])
 def test_ragged_shares_combine(gpu_lib, B, Hq, Hk, D, N, S):
