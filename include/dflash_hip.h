@@ -227,6 +227,11 @@ int dflash_gdn_layer(void* stream,
  *        0 .. N-M+i (:614).  hk = hq / (Hq/Hk) (:575).
  *   kv_len_dev  NULL, or device int32[B]: per-sequence key counts (ragged
  *        batches, or a count produced on the device); each must be in [M, N].
+ *        How the keys are split over workgroups follows from B, Hq, Hk, N and, in a
+ *        ragged batch, from all of its counts, and the splits' partial rows are rounded
+ *        to `dtype`: a sequence gives the same values in another batch, not the same bits
+ *        (they differ by a rounding of the partial rows, 4e-3 relative in bf16, 5e-4 in
+ *        f16).  The same call gives the same bits.
  *   out  [B, Hq, M, D] of `dtype`;  lse  NULL or float32 [B, Hq, M] receiving
  *        max + log(sum exp) of the scaled, masked scores (natural log).
  *   dtype DFLASH_BF16 or DFLASH_F16 (:756); D in {128, 256} (:757).
@@ -273,6 +278,8 @@ int dflash_sdpa_block_causal_static(void* stream,
  * is used when it passes the block-causal rule AND its mask value is at least the
  * lowest finite value of `dtype` (:551); the mask value is added to the scaled
  * score (:553).  A row without any usable key gets zeros (:711) and lse = -inf.
+ * V rows of a tile of 32 keys (32t .. 32t+31) that a row sees nothing of never reach that
+ * row, whatever they hold; in a tile that it sees a part of, hidden V rows must be finite.
  * ---------------------------------------------------------------------- */
 int dflash_sdpa_block_causal_masked(void* stream,
                                     const void* q, const void* k, const void* v, const void* mask,

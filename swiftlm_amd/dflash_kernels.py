@@ -200,7 +200,9 @@ class DFlashKernels:
         mask [B,Hq,16,N].  Returns None where the reference returns nil (unsupported
         shape/dtype).  ``return_lse`` additionally returns the
         float32 logsumexp [B,Hq,16]; ``kv_len`` (int32 [B] on the device) gives
-        per-sequence key counts for ragged batches."""
+        per-sequence key counts for ragged batches.  The keys are split by the sizes of the call and
+        all counts of the batch, and the splits' partial rows are rounded to the input type, so a
+        sequence gives the same values in another batch but not the same bits."""
         if mask is not None:
             if queries.dim() != 4 or keys.dim() != 4 or values.dim() != 4:
                 return None
