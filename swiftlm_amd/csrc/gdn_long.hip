@@ -31,6 +31,8 @@ namespace dflash {
 // dependent MFMAs) and the busiest producer about as long.  us, chunk by chunk kernel against this one: 1,003 steps,
 // 32 heads of 128x128 152 -> 44; 730 steps, 8 heads, Dk = 256 147 -> 45; two sequences of 1,000 steps, 32 heads, Dk = 256
 // 419 -> 123; 40 steps 8.3 -> 5.7.
+// 106 / 122 / 160 registers: two workgroups share a compute unit at Dk = 64 and 128 (two sequences of 1,000 steps 75 where one takes
+// 44), at 256 a second sequence waits for the first (62 for one).
 // ---------------------------------------------------------------------------
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));
