@@ -1323,20 +1323,26 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     // W workgroups per (KV head, head group): one for every split, but no more than fit the chip at once, one on a compute unit.
     // The dealing costs both kernels a dependent trip to the counts, the search and the look-up, 1 to 2 us, and takes off the
     // longest split what the others have too little: with lengths spread evenly a share of its tiles that grows with
-    // (B - 1) / B.  us, not dealt and dealt, lengths from an eighth of N up, at x = (B - 1) * tiles / W:
-    //   more than eight splits per sequence   2 sequences, Hk=2, D=256: x = 8 33.4 34.3, x = 12 42.6 42.6, x = 16 52.3 50.5
-    //                                         64 sequences of 4 splits, D=128: x = 12 18.0 18.7, x = 16 20.8 20.2
-    //   three to eight, up to 16 sequences    8 of 4 splits, Hk=8, D=128: x = 7 13.3 14.2, x = 9 14.3 14.4, x = 14 18.0 17.3
-    //                                         4 of 8 splits, Hk=8, D=256: x = 6 22.8 21.9, x = 9 28.1 25.7
-    //   less than three (halves to deal)      16 of 2 splits, Hk=8, G=8, D=128: x = 22 29.1 30.8, x = 30 34.0 34.4, x = 45 44.3 42.4
-    //   more splits than fit at once          5 sequences, Hk=8, D=128: x = 7 13.8 12.3, x = 42 37.1 28.7 (equal lengths 62.4 41.1)
-    //                                         6 sequences, Hk=2, D=256: x = 7 26.8 26.8, x = 41 68.9 57.9 (equal lengths 116.7 84.8)
+    // (B - 1) / B.  us, not dealt and dealt, K and V from memory, mean of six draws of lengths from an eighth of N up, at
+    // x = (B - 1) * tiles / W:
+    //   more than eight splits per sequence, or many sequences
+    //       4 sequences, Hk=2, D=256   x = 9 31.0 31.6   x = 12 35.9 35.4   x = 24 56.5 50.7
+    //       8 sequences, Hk=1, D=128   x = 10 18.4 18.9  x = 14 21.5 21.0   x = 28 32.8 29.2
+    //      64 sequences, Hk=1, D=128   x = 12 19.3 20.4  x = 16 22.5 22.9   x = 24 28.4 27.9
+    //   three to eight
+    //       4 of 8 splits, Hk=8, D=256 x = 6 23.4 23.4   x = 7.5 26.8 25.7  x = 12 34.4 31.3
+    //       8 of 4 splits, Hk=8, D=128 x = 10 16.5 16.9  x = 14 19.4 19.2   x = 28 29.3 26.8
+    //   less than three, which leave halves to deal
+    //      16 of 2 splits, Hk=8, D=256 x = 22 46.4 47.3  x = 30 55.7 55.7   (D=128 36.9 38.8)
+    //   more splits than fit at once, where not dealing takes two rounds
+    //       5 sequences, Hk=8, D=128   x = 7 14.5 13.2   x = 28 30.7 25.5   (equal lengths 48.8 33.9)
+    //       6 sequences, Hk=2, D=256   x = 7 25.8 27.0   x = 28 54.5 47.5   (equal lengths 93.2 62.1)
     A.balance = 0;
     A.deal = {0, 0, 0};
     if (kv_len_dev && B > 1 && B <= 64 && S > 1) {
         const int64_t tiles = (N + kBN - 1) / kBN;
         const int fit = num_compute_units() / (Hk * groups), W = fit < B * S ? fit : B * S;
-        const int line = B * S > fit || (W >= 3 * B && W <= 8 * B && B <= 16) ? 7 : W < 3 * B ? 30 : 12;
+        const int line = B * S > fit ? 6 : W < 3 * B ? 30 : D == 256 && W <= 8 * B && B <= 16 ? 7 : 12;
         A.balance = W > B && (B - 1) * tiles >= (int64_t)line * W && tiles < (1 << 20) && B * tiles < (1 << 24);
         if (A.balance) A.deal = {W, fast_div_magic((uint32_t)W), fast_div_magic((uint32_t)(W - B))};
     }

@@ -138,7 +138,7 @@ def dealt(B, Hq, Hk, N, D, most=64):
     S = splits(B, Hq, Hk, N, D)
     fit = torch.cuda.get_device_properties(0).multi_processor_count // (Hk * -(-(Hq // Hk) // 8))
     W = min(fit, B * S)
-    line = 7 if B * S > fit or (3 * B <= W <= 8 * B and B <= 16) else 30 if W < 3 * B else 12
+    line = 6 if B * S > fit else 30 if W < 3 * B else 7 if D == 256 and W <= 8 * B and B <= 16 else 12
     return B <= most and W > B and (B - 1) * -(-N // 32) >= line * W
 
 
@@ -211,11 +211,11 @@ def test_ragged_batch_of_more_sequences_than_lanes(gpu_lib):
 
 
 # the line: eight sequences of eight KV heads take four splits each
-@pytest.mark.parametrize("D,N", [(256, 992), (256, 1024), (128, 992), (128, 1024), (128, 2200)])
+@pytest.mark.parametrize("D,N", [(256, 992), (256, 1024), (128, 1728), (128, 1760), (128, 2200)])
 def test_ragged_shares_line(gpu_lib, D, N):
     import ctypes as C
 
-    assert dealt(8, 8, 8, N, D) == (N >= 1024)
+    assert dealt(8, 8, 8, N, D) == (N not in (992, 1728))
     lens = [N, 16, N // 2, 17, 33, N, 700, 129]
     q, k, v = tensors(N + D, 8, 8, 8, N, D)
     status = torch.zeros(1, dtype=torch.int32, device="cuda")
