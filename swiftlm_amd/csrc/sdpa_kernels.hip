@@ -30,137 +30,15 @@
 
 #include <type_traits>
 
-#include "dflash_common.h"
+#include "sdpa_common.h"
 #include "sdpa_shares.h"
 
 namespace dflash {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
-typedef __attribute__((ext_vector_type(8))) float f32x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4_t;
-typedef __attribute__((ext_vector_type(4))) _Float16 f16x4_t;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;   // one 16-byte global/LDS access
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
-
 constexpr int kCombineThreads = 256;
-constexpr int kBN = 32;             // keys per tile
-constexpr int kM = 16;              // block rows per head
 constexpr int kHeadsPerWG = 8;      // query heads sharing one K/V pass
 constexpr int kMaxSplits = 512;
 constexpr float kRescaleLog2 = 8.f;   // lazy-rescale threshold of the online softmax, log2 units
-
-struct Bf16Tag {
-    typedef bf16x8_t vec8;
-    static __device__ __forceinline__ f32x16_t mfma(vec8 a, vec8 b, f32x16_t c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ vec8 pack(f32x8_t x) { return __builtin_convertvector(x, vec8); }
-    static __device__ __forceinline__ bf16x4_t pack4(f32x4_t x) { return __builtin_convertvector(x, bf16x4_t); }
-    static __device__ __forceinline__ uint16_t cvt(float x) { return f32_to_bf16_bits(x); }
-    static __device__ __forceinline__ float to_f32(uint16_t x) { return __uint_as_float(((uint32_t)x) << 16); }
-};
-struct F16Tag {
-    typedef f16x8_t vec8;
-    static __device__ __forceinline__ f32x16_t mfma(vec8 a, vec8 b, f32x16_t c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ vec8 pack(f32x8_t x) { return __builtin_convertvector(x, vec8); }
-    static __device__ __forceinline__ f16x4_t pack4(f32x4_t x) { return __builtin_convertvector(x, f16x4_t); }
-    static __device__ __forceinline__ uint16_t cvt(float x) {
-        _Float16 hf = (_Float16)x;
-        return *reinterpret_cast<uint16_t*>(&hf);
-    }
-    static __device__ __forceinline__ float to_f32(uint16_t x) { return (float)__builtin_bit_cast(_Float16, x); }
-};
-
-struct ShareOut { int W; uint32_t W_magic, rest_magic; };       // workgroups to share out (RaggedShare), fast_div_magic of W and of W - B
-struct SdpaArgs {
-    const uint16_t* q;
-    const uint16_t* k;
-    const uint16_t* v;
-    const uint16_t* k_new;   // [B,Hk,16,D] rows standing for keys Nb-16 .. Nb-1, or null
-    const uint16_t* v_new;
-    uint16_t* k_cache;       // where the fused append stores those rows (== k, v), or null
-    uint16_t* v_cache;
-    uint16_t* part_o;   // [S, B*Hq*16, D]  partial O / l in the input type (DFlashKernels.swift:647 stores it unnormalised)
-    float* part_m;   // [B*Hq*16, S]   running max, log2 units
-    float* part_l;   // [B*Hq*16, S]   sum of exp2
-    const int32_t* kv_len_dev;
-    const uint16_t* mask;    // additive mask [B,Hq,16,N] in the input type (DFlashKernels.swift:548-553), or null
-    int64_t kv_batch_stride, kv_head_stride;
-    float scale_log2;   // scale * log2(e)
-    int Hq, Hk, G, N, S, groups_per_kv;
-    int len_bias;       // added to kv_len_dev[b]: 0, or 16 when the device count excludes the block
-    // Paged K/V (PAGED instantiations): key n of sequence b lives in page page_table[b * table_stride + (n >> page_shift)]
-    // of the pool, at row n & (page_size - 1); k, v point at the pools, kv_batch_stride is the page pitch and
-    // kv_head_stride the head pitch inside a page.
-    const int32_t* page_table;
-    int page_shift, table_stride, num_pages;
-    int32_t* status;         // device status word (dflash_set_status_word), or null
-    uint32_t gpk_magic, S_magic;   // fast_div_magic of groups_per_kv and S
-    float* lse;              // S == 1: part_o is the output itself and this (or null) its logsumexp; no combine follows
-    int B, balance;          // balance: sequences of a ragged batch share the splits by their lengths (RaggedShare)
-    ShareOut deal;
-};
-
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef __attribute__((ext_vector_type(4))) short s16x4_t;
-typedef __attribute__((ext_vector_type(8))) short s16x8_t;
-
-// 64 lanes x 16 B from HBM straight into LDS at lds_base + 16 * lane (lds_base is wave-uniform and
-// travels in M0).  Issued as inline assembly on purpose: the compiler then does not track these
-// loads, so it cannot force a full vmcnt(0) drain ahead of every LDS read or barrier; completion
-// is tracked by hand with wait_vmcnt<> below, which is what keeps several tiles in flight.
-// K/V rows are read once per call, so their loads carry the non-temporal hint: the stream (800 MB per verify step
-// at the benchmark's shape) then no longer pushes the recurrent state, the tapes and the split partials out of
-// the 256 MB memory-side cache -- worth 8 % of the whole step, most of it in the OTHER kernels.
-__device__ __forceinline__ void async_load_16B(const unsigned char* gbase, uint32_t goff, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-                 :
-                 : "v"(goff), "s"(gbase), "s"(__builtin_amdgcn_readfirstlane(lds_base))
-                 : "memory", "m0");
-}
-
-// The same without the non-temporal hint (Q, which every workgroup of the head re-reads).
-__device__ __forceinline__ void async_load_16B_plain(const unsigned char* gbase, uint32_t goff, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(goff), "s"(gbase), "s"(__builtin_amdgcn_readfirstlane(lds_base))
-                 : "memory", "m0");
-}
-
-// Tells the compiler a wave-uniform pointer is uniform (inline-assembly "s" operands need SGPRs).
-__device__ __forceinline__ const unsigned char* uniform_ptr(const unsigned char* p) {
-    const uint64_t u = (uint64_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-    return (const unsigned char*)(((uint64_t)hi << 32) | lo);
-}
-
-// Same, with a full per-lane 64-bit address (rows that come from different buffers).  STREAM: non-temporal, for
-// K/V rows; Q, which every workgroup of the head re-reads, is loaded without the hint.
-template <bool STREAM> __device__ __forceinline__ void async_load_16B_addr(const unsigned char* gptr, uint32_t lds_base) {
-    if constexpr (STREAM)
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
-                     :
-                     : "v"((uint64_t)gptr), "s"(__builtin_amdgcn_readfirstlane(lds_base))
-                     : "memory", "m0");
-    else
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                     :
-                     : "v"((uint64_t)gptr), "s"(__builtin_amdgcn_readfirstlane(lds_base))
-                     : "memory", "m0");
-}
-
-// s_waitcnt vmcnt(n) only (expcnt and lgkmcnt left alone), GFX9 encoding.
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-    __builtin_amdgcn_s_waitcnt(((N >> 4) << 14) | (0xF << 8) | (0x7 << 4) | (N & 0xF));
-}
 
 // ---------------------------------------------------------------------------
 // The partial kernel.  Grid: x = split, y = kv head * groups_per_kv + head group, z = batch (dealt: x = share, z = 1).
@@ -1109,7 +987,8 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_wave_kernel(Comb
 
 // ---- host side -------------------------------------------------------------
 
-// Up to this many tiles one split does them all and writes the output itself: no partial rows, no second launch.  us on the GPU,
+// Up to this many tiles one split does them all and writes the output itself: no partial rows, no second launch (for more query
+// heads than compute units; fewer take sdpa_short_kernel, the faster one there).  us on the GPU,
 // one split and one per tile:
 //     tiles          2           3           4           5           6
 //     D=128    5.3   7.2   5.7   7.0   6.3   7.0   6.9   7.1   7.4   7.1   (512 rows; 2,048 rows at four 6.3 7.9, at six 7.5 8.5)
@@ -1211,6 +1090,7 @@ int sdpa_device_setup() {
     if (rc == DFLASH_OK) rc = sdpa_partial_setup<Bf16Tag, 128>();
     if (rc == DFLASH_OK) rc = sdpa_partial_setup<F16Tag, 256>();
     if (rc == DFLASH_OK) rc = sdpa_partial_setup<F16Tag, 128>();
+    if (rc == DFLASH_OK) rc = sdpa_short_device_setup();
     if (rc != DFLASH_OK) return rc;
     int dev = 0;
     DFLASH_HIP_TRY(hipGetDevice(&dev));
@@ -1349,6 +1229,11 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     C.balance = A.balance; C.deal = A.deal; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
 
     hipStream_t st = (hipStream_t)stream;
+    // (the workspace asked for is that of the split form, whichever form runs)
+    if (sdpa_short_applies(B, Hq, N, D)) {
+        A.part_o = (uint16_t*)out;
+        return launch_sdpa_short(st, A, B, D, dtype, paged != nullptr);
+    }
 #define DFLASH_SDPA_CASE(MASKED, PAGED)                                                                              \
     do {                                                                                                             \
         if (dtype == DFLASH_BF16)                                                                                    \

@@ -1,0 +1,372 @@
+// Block-causal attention of the 16-token verify block over a short context, in one launch.
+//
+// Semantics follow Sources/DFlash/DFlashKernels.swift:737-815 (entry), :563-649 (causal rule :614, GQA mapping :575).
+
+#include <type_traits>
+
+#include "sdpa_common.h"
+
+namespace dflash {
+
+// ---------------------------------------------------------------------------
+// One workgroup per (query head, sequence); its eight waves take tiles of keys in turn, each with the running maximum, the sum and
+// O^T of its own tiles, and merge them through LDS at the end in fp32.  No partial rows in memory and no second launch; inside
+// the loop no barrier, as a wave brings its own tiles.  The price is that the query heads of a group each read their KV head's
+// rows (from the L2), so it is for contexts whose rows one compute unit can take in: see sdpa_short_applies().
+//
+// Bound by one launch and its first trip to memory (4.1 us) and, from some 200 keys on, by what a compute unit takes in, 64 bytes
+// per clock at best: that is reached by loads HBM -> LDS of 1 KB of whole rows.  K rows straight into the operand registers, where
+// neighbouring lanes hold different rows, come in at a quarter of it (16 query heads, D = 128, 512 keys: 8.5 us, and 6.1 as it
+// is; split over workgroups with a combine kernel behind them 8.1).  At D = 256 tiles of 16 keys, so that eight waves find room:
+// with four waves of 32 keys 700 keys took 14.1 us, now 11.2.
+//
+// MFMA 16x16x32, n = lane % 16, g = lane / 16: operands hold row (column) n, k-elements 8g .. 8g+7; the accumulator column n, rows
+// 4g .. 4g+3.  S^T = K Q^T, then O^T += V^T P^T, with P^T taken from the accumulators of S^T as they are: lane (n, g) holds keys
+// 4g .. 4g+3 of each 16 keys, and V^T is gathered in that order by the transposing LDS read (16x16x16 for a tile of 16 keys).
+// 16-byte piece p of row r stands at p ^ (r % 16) (K, Q) or p ^ 4 (r % 4) (V), which keeps the reads free of conflicts.  A wave's K
+// slot is asked for again behind its scores, its V slot behind the product.
+// ---------------------------------------------------------------------------
+template <int D> struct SdpaShortLds {
+    static constexpr int WAVES = 8;
+    static constexpr int NB = D == 128 ? 32 : 16;                   // keys of a tile
+    static constexpr int ROWB = D * 2;
+    struct Slot { unsigned char k[NB * ROWB], v[NB * ROWB]; };
+    unsigned char q[kM * ROWB];
+    union { Slot slot[WAVES]; float o[WAVES][kM * D]; };            // at the end the wave's O^T
+    uint32_t mask[WAVES][kM][NB];                                   // 16 bits each; 4 keys p of row r at p ^ (r % (NB / 4))
+    float m[WAVES][kM], l[WAVES][kM];
+    static_assert(sizeof(Slot) >= kM * D * 4, "the wave's O fits its slot");
+};
+
+// One 16-bit element per lane, zero-extended, HBM -> LDS at lds_base + 4 * lane.
+__device__ __forceinline__ void async_load_2B_addr(const uint16_t* gptr, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_ushort %0, off"
+                 :
+                 : "v"((uint64_t)gptr), "s"(__builtin_amdgcn_readfirstlane(lds_base))
+                 : "memory", "m0");
+}
+// At most N of the wave's loads still under way.
+template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+template <typename Tag, int D, bool MASKED, bool PAGED>
+__global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_kernel(SdpaArgs A) {
+    typedef typename Tag::vec8 vec8;
+    typedef SdpaShortLds<D> Lds;
+    constexpr int W = Lds::WAVES, NB = Lds::NB, NU = NB / 16, ROWB = D * 2, CPR = D / 8, RPI = 64 / CPR;       // bytes and 16-byte pieces of a row, rows per 1 KB load
+    constexpr int KSTEPS = D / 32, DB = D / 16;
+    constexpr int TILE_LOADS = NB / RPI, MASK_LOADS = MASKED ? kM * NB / 64 : 0, KM_LOADS = TILE_LOADS + MASK_LOADS;
+    static_assert(2 * TILE_LOADS + MASK_LOADS <= 63, "vmcnt is a 6-bit counter");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    Lds& L = *reinterpret_cast<Lds*>(smem);
+
+    asm volatile("" ::"s"(A.q), "s"(A.k), "s"(A.v), "s"(A.k_new), "s"(A.v_new), "s"(A.k_cache), "s"(A.v_cache), "s"(A.part_o), "s"(A.lse),
+                 "s"(A.kv_len_dev), "s"(A.mask), "s"(A.kv_batch_stride), "s"(A.kv_head_stride), "s"(A.scale_log2), "s"(A.Hq), "s"(A.Hk),
+                 "s"(A.G), "s"(A.N), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages), "s"(A.status));
+
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4;
+    const int hk = blockIdx.x, b = blockIdx.z, hq = hk * A.G + (int)blockIdx.y;
+    const size_t row0 = ((size_t)b * A.Hq + hq) * kM;               // first row of the head in q, out and lse
+    auto lds_addr = [](const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; };
+
+    int len_raw = 0;
+    if (A.kv_len_dev) len_raw = A.kv_len_dev[b];
+    // the page-table entries of the wave's tiles, one tile per lane: w, w + W, ... (clamped to the host-side bound, which the table spans)
+    const int nt_max = (A.N + NB - 1) / NB;
+    int entries = 0;
+    if constexpr (PAGED) {
+        const int tile = min(w + W * lane, nt_max - 1);
+        entries = A.page_table[(size_t)b * A.table_stride + ((tile * NB) >> A.page_shift)];
+    }
+    {
+        const unsigned char* qp = uniform_ptr(reinterpret_cast<const unsigned char*>(A.q) + row0 * ROWB);
+#pragma unroll
+        for (int j = w; j < kM / RPI; j += W) {
+            const int row = j * RPI + lane / CPR;
+            async_load_16B_plain(qp, (uint32_t)row * ROWB + (((lane % CPR) ^ (row & 15)) * 16), lds_addr(L.q) + j * 1024);
+        }
+    }
+    const size_t head_off = PAGED ? (size_t)hk * A.kv_head_stride * 2 : ((size_t)b * A.kv_batch_stride + (size_t)hk * A.kv_head_stride) * 2;
+    const unsigned char* kbase = reinterpret_cast<const unsigned char*>(A.k) + head_off;
+    const unsigned char* vbase = reinterpret_cast<const unsigned char*>(A.v) + head_off;
+    const unsigned char* knew = reinterpret_cast<const unsigned char*>(A.k_new) + ((size_t)b * A.Hk + hk) * kM * ROWB;
+    const unsigned char* vnew = reinterpret_cast<const unsigned char*>(A.v_new) + ((size_t)b * A.Hk + hk) * kM * ROWB;
+
+    int Nb = A.kv_len_dev ? len_raw + A.len_bias : A.N;
+    if (A.status && (Nb < kM || Nb > A.N) && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) atomicOr(A.status, DFLASH_STATUS_SDPA_LEN);
+    Nb = Nb < kM ? kM : (Nb > A.N ? A.N : Nb);
+    const int nt = (Nb + NB - 1) / NB;
+    const bool fused = A.k_new != nullptr;
+    const int cache_rows = fused ? Nb - kM : Nb;                    // keys below this index are read from the cache
+    const int page_mask = PAGED ? (1 << A.page_shift) - 1 : 0;
+
+    // bytes from kbase / vbase to a page and to the tile's first row (the K and V pools share one layout); a stale table cannot leave the pool
+    auto page_off = [&](int e) -> size_t {
+        e = e < 0 ? 0 : (e >= A.num_pages ? A.num_pages - 1 : e);
+        return (size_t)e * (size_t)A.kv_batch_stride * 2;
+    };
+    auto tile_off = [&](int t) -> size_t {
+        if constexpr (PAGED)
+            return page_off(__builtin_amdgcn_readlane(entries, t / W)) + (size_t)((t * NB) & page_mask) * ROWB;
+        else
+            return (size_t)t * NB * ROWB;
+    };
+    auto request_rows = [&](int t, const unsigned char* base, const unsigned char* nw, uint32_t lds, bool is_k) __attribute__((always_inline)) {
+        const unsigned char* tile = uniform_ptr(base + tile_off(t));
+        const int key0 = t * NB;
+        uint32_t l = lane;
+        asm volatile("" : "+v"(l));                                 // offsets are formed anew: kept across the loop they are dozens of registers
+        if (key0 + NB <= cache_rows || !fused) {                   // uniform
+            const int last = Nb - 1 - key0;                         // past the end the last key once more (dropped later)
+#pragma unroll
+            for (int j = 0; j < TILE_LOADS; ++j) {
+                const int row = (int)(j * RPI + l / CPR);
+                const int piece = (int)(l % CPR) ^ (is_k ? row & 15 : 4 * (row & 3));
+                async_load_16B_plain(tile, (uint32_t)(min(row, last) * ROWB + piece * 16), lds + j * 1024);
+            }
+        } else {                                                    // the block's own rows come from k_new / v_new
+#pragma unroll 4
+            for (int j = 0; j < TILE_LOADS; ++j) {
+                const int row = (int)(j * RPI + l / CPR), key = min(key0 + row, Nb - 1);
+                const int piece = (int)(l % CPR) ^ (is_k ? row & 15 : 4 * (row & 3));
+                const unsigned char* src = key < cache_rows ? tile + (uint32_t)((key - key0) * ROWB) : nw + (uint32_t)((key - cache_rows) * ROWB);
+                async_load_16B_addr<false>(src + piece * 16, lds + j * 1024);
+            }
+        }
+    };
+    auto request_k = [&](int t) __attribute__((always_inline)) {
+        request_rows(t, kbase, knew, lds_addr(L.slot[w].k), true);
+        if constexpr (MASKED) {
+#pragma unroll
+            for (int j = 0; j < MASK_LOADS; ++j) {                   // whole rows of the tile
+                const int row = j * (64 / NB) + lane / NB, key = t * NB + ((lane % NB) ^ (4 * (row & (NB / 4 - 1))));
+                async_load_2B_addr(A.mask + (row0 + row) * (size_t)A.N + min(key, A.N - 1), lds_addr(L.mask[w]) + j * 256);    // (keys past the end fail the causal rule)
+            }
+        }
+    };
+    auto request_v = [&](int t) __attribute__((always_inline)) { request_rows(t, vbase, vnew, lds_addr(L.slot[w].v), false); };
+
+    f32x4_t oacc[DB];
+#pragma unroll
+    for (int i = 0; i < DB; ++i) oacc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;
+    const int tj = n >> 2, tq = n & 3;                               // transposing read: this lane points at row 4g + tj, channels 4 tq .. +3
+    uint32_t koff[4], voff[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        koff[m] = (uint32_t)(n * ROWB + (((4 * m + g) ^ n) * 16));
+        voff[m] = (uint32_t)((4 * g + tj) * ROWB + (tq & 1) * 8 + (tq >> 1) * 16 + ((m ^ tj) * 64));
+    }
+    auto load_k = [&](const unsigned char* rows, int s) -> vec8 {    // row n, channels 32 s + 8 g .. +7
+        return *reinterpret_cast<const vec8*>(rows + koff[s & 3] + 256 * (s >> 2));
+    };
+    auto load_v = [&](int i) {                               // channel 16 i + n, keys 4g .. +3 and 16 + 4g .. +3
+        const unsigned char* p = L.slot[w].v + voff[(i >> 1) & 3] + 32 * (i & 1) + 256 * (i >> 3);
+        const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)p);
+        if constexpr (NU == 1) return lo;
+        else {
+            const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + 16 * ROWB));
+            return __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    };
+
+    auto pack_weights = [](const float (&p)[4 * NU]) {
+        if constexpr (NU == 2) return Tag::pack(f32x8_t{p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7]});
+        else return Tag::pack4(f32x4_t{p[0], p[1], p[2], p[3]});
+    };
+
+    // Q is in LDS when every wave has waited for its part of it; its first tile may still be under way.
+    if (w < nt) {
+        request_k(w);
+        request_v(w);
+        wait_loads<KM_LOADS + TILE_LOADS>();
+    } else {
+        wait_loads<0>();
+    }
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    vec8 qf[KSTEPS];
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) qf[s] = load_k(L.q, s);
+
+    // One tile; HIDE: some rows may see nothing of it.
+    auto tile = [&](int t, auto hide) __attribute__((always_inline)) {
+        constexpr bool HIDE = decltype(hide)::value;
+        const bool more = t + W < nt;                                // uniform
+        wait_loads<TILE_LOADS>();                                    // all but V
+        f32x4_t sacc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};      // NU == 1: two chains
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+            for (int u = 0; u < NU; ++u) sacc[NU == 2 ? u : s & 1] = Tag::mfma16(load_k(L.slot[w].k + 16 * u * ROWB, s), qf[s], sacc[NU == 2 ? u : s & 1]);
+        if constexpr (NU == 1) sacc[0] += sacc[1];
+        const int key0 = t * NB, last_visible = Nb - kM + n;        // row n sees keys 0 .. Nb-16+n
+        float x[4 * NU], mloc = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            u32x4_t mk;
+            if constexpr (MASKED) mk = *reinterpret_cast<const u32x4_t*>(&L.mask[w][n][4 * ((4 * u + g) ^ (n & (NB / 4 - 1)))]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float s = sacc[u][e] * A.scale_log2;
+                if constexpr (MASKED) {
+                    // -inf (or NaN) drops the key; a finite mask value, however low, keeps it in the softmax
+                    const float mv = Tag::to_f32((uint16_t)mk[e]);
+                    s = mv >= -3.4028234663852886e38f ? fmaxf(fmaf(mv, 1.4426950408889634f, s), -3.4028234663852886e38f) : -INFINITY;
+                }
+                s = key0 + 16 * u + 4 * g + e <= last_visible ? s : -INFINITY;
+                x[4 * u + e] = s;
+                mloc = fmaxf(mloc, s);
+            }
+        }
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // K and mask have been read
+            request_k(t + W);
+        }
+        {   // over the four lanes that share the row
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+            mloc = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+            const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+            mloc = fmaxf(__uint_as_float(r2[0]), __uint_as_float(r2[1]));
+        }
+        // A row that sees nothing of the tile has zeros for weights, and zero times a V row that is hidden from it is not zero where
+        // that holds an infinity or NaN: it keeps what it had.
+        const bool seen = MASKED ? mloc != -INFINITY : key0 <= last_visible;
+        const float m_new = fmaxf(m_run, mloc);
+        const float m_safe = m_new == -INFINITY ? 0.f : m_new, alpha = fast_exp2(m_run - m_safe);     // (0 while the row is empty: so is what it scales)
+        m_run = m_new;
+        l_run *= alpha;
+        float pf[4 * NU];
+#pragma unroll
+        for (int e = 0; e < 4 * NU; ++e) {
+            pf[e] = fast_exp2(x[e] - m_safe);
+            l_run += pf[e];
+        }
+        if (more) wait_loads<KM_LOADS>();                            // V
+        else wait_loads<0>();
+        decltype(pack_weights(pf)) pb = pack_weights(pf);
+        constexpr int kAhead = 4;
+        decltype(load_v(0)) va[DB];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) va[i] = load_v(i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < DB; ++i) {
+            if (i + kAhead < DB) va[i + kAhead] = load_v(i + kAhead);
+            oacc[i] *= alpha;
+            f32x4_t o;
+            if constexpr (NU == 2) o = Tag::mfma16(va[i], pb, oacc[i]);
+            else o = Tag::mfma16_16(va[i], pb, oacc[i]);
+            if constexpr (HIDE) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) oacc[i][v] = seen ? o[v] : oacc[i][v];
+            } else {
+                oacc[i] = o;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the slot has been read
+            request_v(t + W);
+        }
+    };
+    // Without a mask only the last tile can be hidden from a row, where it begins behind the first of the block's keys.
+    const int plain = !MASKED && (nt - 1) * NB > Nb - kM ? nt - 1 : nt;
+    for (int t = w; t < plain; t += W) tile(t, std::bool_constant<MASKED>{});
+    if (plain < nt && plain % W == w) tile(plain, std::true_type{});
+
+    // ---- the waves' results into one ----
+    {
+        auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
+        l_run = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        r = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
+        l_run = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    if (g == 0) { L.m[w][n] = m_run; L.l[w][n] = l_run; }
+    __syncthreads();
+    float M = -INFINITY, l_tot = 0.f;
+#pragma unroll
+    for (int i = 0; i < W; ++i) M = fmaxf(M, L.m[i][n]);
+#pragma unroll
+    for (int i = 0; i < W; ++i) l_tot += L.m[i][n] == -INFINITY ? 0.f : fast_exp2(L.m[i][n] - M) * L.l[i][n];
+    const int waves = nt < W ? nt : W;                               // those that had a tile
+    if (w < waves) {
+        const float f = m_run == -INFINITY ? 0.f : fast_exp2(m_run - M) * (l_tot > 0.f ? 1.f / l_tot : 0.f);
+        f32x4_t* o = reinterpret_cast<f32x4_t*>(L.o[w]) + n * (D / 4);     // 16-byte piece p of row n at p ^ n
+#pragma unroll
+        for (int i = 0; i < DB; ++i) o[(4 * i + g) ^ n] = oacc[i] * f;
+    }
+    if (w == 0 && g == 0 && A.lse) A.lse[row0 + n] = (M + log2f(l_tot)) * 0.6931471805599453f;
+    // the block's own K/V rows into the cache: the group's first head does it
+    if (fused && A.k_cache && blockIdx.y == 0) {
+        for (int i = tid; i < kM * CPR; i += 64 * W) {
+            const int key = cache_rows + i / CPR;
+            size_t off = head_off + (size_t)(i % CPR) * 16;
+            if constexpr (PAGED)
+                off += page_off(A.page_table[(size_t)b * A.table_stride + (key >> A.page_shift)]) + (size_t)(key & page_mask) * ROWB;
+            else
+                off += (size_t)key * ROWB;
+            const u32x4_t kx = reinterpret_cast<const u32x4_t*>(knew)[i], vx = reinterpret_cast<const u32x4_t*>(vnew)[i];
+            *reinterpret_cast<u32x4_t*>(reinterpret_cast<unsigned char*>(A.k_cache) + off) = kx;
+            *reinterpret_cast<u32x4_t*>(reinterpret_cast<unsigned char*>(A.v_cache) + off) = vx;
+        }
+    }
+    __syncthreads();
+    constexpr int PER = D / 4;                                       // threads x 4 channels of a row
+    for (int i = tid; i < kM * PER; i += 64 * W) {
+        const int r = i / PER, p = i % PER;
+        f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < waves; ++j) o += reinterpret_cast<const f32x4_t*>(L.o[j])[r * PER + (p ^ r)];
+        *reinterpret_cast<u32x2_t*>(A.part_o + (row0 + r) * D + 4 * p) = __builtin_bit_cast(u32x2_t, Tag::pack4(o));
+    }
+}
+
+// Where one workgroup per query head is the faster form: no more heads than compute units, as the workgroups of a second round
+// wait for the first, and few enough keys for the split form's second launch and its partial rows to cost more than the serial
+// tiles here; with many heads that form has longer splits to do, too.  us per call, split form against this one:
+//     heads, keys  D=128   128        600         800         1000        1200       D=256   128       350         500         600
+//     8 (Hk=1)          6.1 4.8   8.3 6.6     8.3 7.6     8.5 8.5     8.4 9.5           8.1 6.0   9.2 8.7     9.2 9.9     9.3 11.1
+//     16 (Hk=2)         6.1 4.8   8.2 6.6     8.3 7.7     8.5 8.6     8.7 9.6           8.2 6.0   9.3 8.7     9.4 10.0    9.4 11.1
+//     64 (B=2)          6.0 4.7   8.8 6.7     9.1 7.8     10.1 8.7    10.0 9.8          8.1 6.1   10.4 8.8    10.9 10.1   13.2 11.4
+//     128 (B=4)         6.1 4.8   10.2 7.0    11.0 8.1    11.0 9.3    11.5 10.5         8.2 6.2   11.3 9.1    12.5 10.7   12.2 11.9
+//     256 (B=8)         6.1 4.9   12.1 7.5    12.6 8.6    13.3 9.8    14.5 11.2         8.5 6.6   13.6 9.6    15.2 11.3   16.6 12.7
+//     512 (B=8)         6.4 7.0   14.2 12.9   15.5 15.1   16.5 17.4   17.9 20.2         9.0 11.6  16.5 17.3   18.5 20.3   19.6 23.0
+bool sdpa_short_applies(int B, int Hq, int N, int D) {
+    const int64_t heads = (int64_t)B * Hq;
+    const int cus = num_compute_units();
+    const bool few = heads < cus / 4;
+    return heads <= cus && N <= (D == 128 ? (few ? 896 : 1152) : (few ? 416 : 576));
+}
+
+template <typename Tag, int D, bool MASKED, bool PAGED>
+static int launch_short(hipStream_t st, const SdpaArgs& A, int B) {
+    LaunchBracket br(DFLASH_KERNEL_SDPA_PARTIAL, st);
+    DFLASH_HIP_TRY(br.launch(sdpa_short_kernel<Tag, D, MASKED, PAGED>, dim3(A.Hk, A.G, B), dim3(64 * SdpaShortLds<D>::WAVES), sizeof(SdpaShortLds<D>), A));
+    return DFLASH_OK;
+}
+template <typename Tag, int D> static int launch_short(hipStream_t st, const SdpaArgs& A, int B, bool paged) {
+    if (A.mask) return launch_short<Tag, D, true, false>(st, A, B);
+    return paged ? launch_short<Tag, D, false, true>(st, A, B) : launch_short<Tag, D, false, false>(st, A, B);
+}
+int launch_sdpa_short(hipStream_t st, const SdpaArgs& A, int B, int D, int dtype, bool paged) {
+    if (dtype == DFLASH_BF16) return D == 256 ? launch_short<Bf16Tag, 256>(st, A, B, paged) : launch_short<Bf16Tag, 128>(st, A, B, paged);
+    return D == 256 ? launch_short<F16Tag, 256>(st, A, B, paged) : launch_short<F16Tag, 128>(st, A, B, paged);
+}
+
+template <typename Tag, int D>
+static int short_setup() {
+    const int lds = sizeof(SdpaShortLds<D>);
+    DFLASH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(sdpa_short_kernel<Tag, D, false, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    DFLASH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(sdpa_short_kernel<Tag, D, true, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    DFLASH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(sdpa_short_kernel<Tag, D, false, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    return DFLASH_OK;
+}
+int sdpa_short_device_setup() {
+    int rc = short_setup<Bf16Tag, 256>();
+    if (rc == DFLASH_OK) rc = short_setup<Bf16Tag, 128>();
+    if (rc == DFLASH_OK) rc = short_setup<F16Tag, 256>();
+    if (rc == DFLASH_OK) rc = short_setup<F16Tag, 128>();
+    return rc;
+}
+
+}  // namespace dflash

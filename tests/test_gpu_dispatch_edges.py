@@ -117,6 +117,32 @@ def test_attention_split_counts(gpu_lib, N, Hq, Hk, D):
     attend(*tensors(N + D, 1, Hq, Hk, N, D), [N], D)
 
 
+# Short contexts in one launch, up to a line of keys that depends on the query heads (B * Hq), and the split forms behind it; more
+# heads than compute units take the split forms at once.  Tiles of 32 (D = 128) and 16 keys, eight waves, one tile a wave and more.
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("Hq,Hk,D,N", [(2, 1, 128, 31), (3, 1, 128, 256), (3, 1, 128, 257), (12, 2, 128, 600), (8, 1, 128, 896), (8, 1, 128, 897),
+                                       (32, 8, 128, 1152), (32, 8, 128, 1153), (2, 1, 256, 17), (3, 1, 256, 128), (3, 1, 256, 129),
+                                       (8, 1, 256, 416), (8, 1, 256, 417), (32, 8, 256, 576), (32, 8, 256, 577), (130, 2, 128, 100), (130, 2, 256, 129)])
+def test_short_contexts(gpu_lib, Hq, Hk, D, N, dt):
+    from swiftlm_amd import DFlashKernels as K
+
+    lens = [N, max(16, N // 2 + 1)]
+    q, k, v = tensors(N + D, 2, Hq, Hk, N, D, dt)
+    kv_len = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out, lse = attend(q, k, v, lens, D, kv_len=kv_len)
+    # masked and fused calls give the same bits
+    zero = torch.zeros(2, Hq, 16, N, dtype=dt, device="cuda")
+    masked = K.batched_sdpa_2pass(q, k, v, 1.0 / math.sqrt(D), zero, return_lse=True, kv_len=kv_len)
+    new = [torch.stack([x[b, :, n - 16:n] for b, n in enumerate(lens)]).contiguous() for x in (k, v)]
+    kc, vc = k.clone(), v.clone()
+    for b, n in enumerate(lens):
+        kc[b, :, n - 16:n], vc[b, :, n - 16:n] = float("nan"), float("nan")
+    fused = K.batched_sdpa_2pass_append(q, kc, vc, *new, 1.0 / math.sqrt(D), N, cache_len=kv_len - 16, return_lse=True)
+    for o, l in (masked, fused):
+        assert torch.equal(o, out) and torch.equal(l, lse)
+    assert torch.equal(kc, k) and torch.equal(vc, v)
+
+
 # ragged batches of short sequences, every one with its own splits: one beside many, equal lengths, all at the minimum, 64 and 65
 @pytest.mark.parametrize("lens", [[700, 16], [16, 17, 2000, 33], [500] * 5, [16] * 3 + [129], [40 + 3 * i for i in range(64)],
                                   [40 + 3 * i for i in range(65)]], ids=lambda v: f"{len(v)}x{max(v)}")
