@@ -67,8 +67,7 @@ constexpr float kRescaleLog2 = 8.f;   // lazy-rescale threshold of the online so
 //
 // MASKED adds the reference's optional additive mask: a key is used when it passes the causal rule and its mask
 // value is at least the lowest finite value of the input type, and the mask value is added to the scaled score
-// (DFlashKernels.swift:550-553, :614-623).  The mask is read with plain loads inside the softmax; that
-// instantiation is for signature parity, not for speed.  PAGED reads K/V through a page table.
+// (DFlashKernels.swift:550-553, :614-623); it is read by the compute waves, a tile ahead.  PAGED reads K/V through a page table.
 // ---------------------------------------------------------------------------
 constexpr int kPartialThreads = 384;    // 4 compute waves + 2 producer waves
 constexpr int kRingSlots = 3;           // tiles per ring
@@ -553,6 +552,34 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
         }
         return mloc;
     };
+    // The mask of tile t: 4 keys per load (8 bytes, at any even address, as rows may have an odd length), asked for ahead of the tile's
+    // scores (at D = 256 half a tile later: registers).  Loaded element by element inside the softmax, 64 requests per load with
+    // nothing to hide behind, the mask bound the kernel: Hq=32, Hk=8, 16,384 keys 51 us at D = 128, now 24 (18 without a mask), 60 and
+    // now 43 at D = 256 (19).
+    u32x2_t mask_raw[4];
+    const uint16_t* mask_rows = A.mask + ((size_t)b * A.Hq + hk * A.G + hg0 + 2 * cw) * kM * A.N;      // uniform: the wave's 32 rows
+    const uint32_t mask_off = ((row_valid ? (uint32_t)c : 0u) * (uint32_t)A.N + 4 * h) * 2;
+    auto request_mask = [&](int t) {
+        if constexpr (MASKED) {
+            struct __attribute__((packed, aligned(2))) Keys4 { u32x2_t x; };
+            const int key0 = key_of(t);
+            const unsigned char* p = reinterpret_cast<const unsigned char*>(mask_rows + key0) + mask_off;
+            if (key0 + kBN <= A.N) {                // uniform
+#pragma unroll
+                for (int j = 0; j < 4; ++j) mask_raw[j] = reinterpret_cast<const Keys4*>(p + 16 * j)->x;
+            } else {
+                const int most = A.N - 1 - key0 - 4 * h;       // keys past the end, which fail the causal rule, read the last one (below 0 for a lane without any)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const int i = 8 * j + 2 * e;
+                        mask_raw[j][e] = (uint32_t)reinterpret_cast<const uint16_t*>(p)[i < most ? i : most]
+                                         | ((uint32_t)reinterpret_cast<const uint16_t*>(p)[i + 1 < most ? i + 1 : most] << 16);
+                    }
+            }
+        }
+    };
     // Masks on x (tiles that reach the block's own keys: the causal rule; MASKED: the additive mask as well) and
     // the row maximum over both half-waves.  mloc is the maximum of the unmasked scores.
     auto mask_and_max = [&](int t, float mloc) -> float {
@@ -560,23 +587,13 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
         const bool need_mask = (key0 + kBN) > (Nb - kM);
         if (MASKED || need_mask) {                  // uniform
             const int last_visible = Nb - kM + qi;  // row qi sees keys 0 .. Nb-16+qi
-            float mk[16];
-            if constexpr (MASKED) {
-                const uint16_t* mrow = A.mask + row_id * (size_t)A.N;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    int key = key0 + 8 * (v >> 2) + 4 * h + (v & 3);
-                    key = key < A.N ? key : A.N - 1;               // keys past the end fail the causal rule anyway
-                    mk[v] = row_valid ? Tag::to_f32(mrow[key]) : 0.f;
-                }
-            }
             mloc = -INFINITY;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 if constexpr (MASKED) {
                     // -inf (or NaN) drops the key; a finite mask value, however low, keeps it in the softmax
-                    x[v] = mk[v] >= -3.4028234663852886e38f ? fmaxf(fmaf(mk[v], 1.4426950408889634f, x[v]), -3.4028234663852886e38f)
-                                                             : -INFINITY;
+                    const float mk = Tag::to_f32((uint16_t)(mask_raw[v / 4][v / 2 % 2] >> (16 * (v % 2))));
+                    x[v] = mk >= -3.4028234663852886e38f ? fmaxf(fmaf(mk, 1.4426950408889634f, x[v]), -3.4028234663852886e38f) : -INFINITY;
                 }
                 const int key = key0 + 8 * (v >> 2) + 4 * h + (v & 3);
                 x[v] = key <= last_visible ? x[v] : -INFINITY;
@@ -652,6 +669,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
         }
     };
 
+    if (wave_active) request_mask(t_begin);
     wait_vmcnt<0>();                                // this wave's Q rows have landed
     __builtin_amdgcn_s_barrier();                   // Q and K(t_begin) are in LDS
     if (wave_active) {
@@ -669,6 +687,7 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
         bool jumped = false;
         if (MASKED && hidden) {                     // outside the hot loop, like the rescale
             __builtin_amdgcn_s_barrier();
+            request_mask(t + 1);
             exp_qk(t);
             float mloc = -INFINITY;
 #pragma unroll
@@ -683,7 +702,9 @@ __global__ __launch_bounds__(kPartialThreads, 1) void sdpa_partial_kernel(SdpaAr
         for (; t < t_last && !(MASKED && (hidden || jumped)); ++t) {
             __builtin_amdgcn_s_barrier();           // V(t) and K(t+1) are in LDS; everyone is done with iteration t-1
             if (wave_active) {
+                if constexpr (D == 128) request_mask(t + 1);
                 exp_qk(t);
+                if constexpr (D == 256) request_mask(t + 1);    // here, for registers
                 const float mloc = pv_scale(t);
                 if (!accept_max(mask_and_max(t + 1, mloc))) {
                     jumped = true;

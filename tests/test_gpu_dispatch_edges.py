@@ -143,6 +143,22 @@ def test_short_contexts(gpu_lib, Hq, Hk, D, N, dt):
     assert torch.equal(kc, k) and torch.equal(vc, v)
 
 
+# The split form's mask, four keys per load: rows of odd and even length, a last tile of one key and of all but one.
+@pytest.mark.parametrize("N", [1185, 1186, 1187, 1189, 1215, 1216])
+@pytest.mark.parametrize("Hq,Hk,D", [(3, 1, 256), (10, 2, 128)])
+def test_mask_row_ends(gpu_lib, N, Hq, Hk, D):
+    from swiftlm_amd import DFlashKernels as K
+
+    q, k, v = tensors(N + D, 2, Hq, Hk, N, D)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    mask = torch.randn(2, Hq, 16, N, generator=g, device="cuda").masked_fill(torch.rand(2, Hq, 16, N, generator=g, device="cuda") < 0.3, float("-inf"))
+    mask = mask.to(torch.bfloat16)
+    out, lse = K.batched_sdpa_2pass(q, k, v, 1.0 / math.sqrt(D), mask, return_lse=True)
+    ow, lw = O.sdpa_block_causal(host(q), host(k), host(v), 1.0 / math.sqrt(D), host(mask).astype(np.float64))
+    np.testing.assert_allclose(host(out), ow, rtol=2e-2, atol=2e-2)
+    np.testing.assert_allclose(host(lse), lw, rtol=2e-3, atol=2e-3)
+
+
 # ragged batches of short sequences, every one with its own splits: one beside many, equal lengths, all at the minimum, 64 and 65
 @pytest.mark.parametrize("lens", [[700, 16], [16, 17, 2000, 33], [500] * 5, [16] * 3 + [129], [40 + 3 * i for i in range(64)],
                                   [40 + 3 * i for i in range(65)]], ids=lambda v: f"{len(v)}x{max(v)}")
