@@ -64,11 +64,11 @@ template <int QUAD_LANE> __device__ __forceinline__ float quad_broadcast(float x
 
 // Steps S..15 of the unit-triangular solve for one state row held by a quad (lane q owns steps 4q..4q+3).
 // Every lane of the quad sees every delta; lane q keeps those of its own four steps in `mine` (a select per step,
-// no branch) for the store that follows.
+// no branch) for the store that follows.  `bet` holds the betas of the lane's own steps: only the lane that owns a step scales it.
 template <int S> struct SolveStep {
-    static __device__ __forceinline__ void run(float (&acc)[4], const float4 (&arow)[16], const float (&bet)[16],
+    static __device__ __forceinline__ void run(float (&acc)[4], const float4 (&arow)[16], const float (&bet)[4],
                                                float (&mine)[4], const int q) {
-        const float d = quad_broadcast<S / 4>(bet[S] * acc[S % 4]);
+        const float d = quad_broadcast<S / 4>(bet[S % 4] * acc[S % 4]);
         mine[S % 4] = q == S / 4 ? d : mine[S % 4];
         acc[0] = fmaf(-arow[S].x, d, acc[0]);
         acc[1] = fmaf(-arow[S].y, d, acc[1]);

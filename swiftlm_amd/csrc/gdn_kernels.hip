@@ -725,10 +725,15 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
 // Workgroup: 16 state rows of one head (grid x = Dv/16, y = b*Hv + hv), 4 waves.
 // ---------------------------------------------------------------------------
 
-template <int DK> struct GdnChunkLds {
+// BF (bf16 inputs): the product's operands are bf16, the state tile as three bf16 terms, S_0 = hi + mid + lo exactly (3 x 8 = 24
+// significand bits), k_t and q_t as they came; fp32 is the state tile only, for the update.  Either form holds just its own
+// arrays, as their size decides how many workgroups share a compute unit (Dk = 128: 37 KB, four; with every array of both forms
+// 62 KB, two).  us per call before and after, T = 16, 32 value heads of 128: four sequences 9.4 -> 7.1, two at Dk = 256 10.3 -> 7.2,
+// four 19.2 -> 12.6; the layer in one launch 20.2 -> 15.2 (B = 4), Dk = 256 21.6 -> 15.5 (B = 2), 40.2 -> 26.8 (B = 4).
+template <int DK, bool BF> struct GdnChunkLds {
     static constexpr int LD = DK + 4;      // row pitch in floats: 16-byte pad spreads rows over the banks
-    float x[32][LD];                       // rows 0..15 state tile, rows 16..31 k_t
-    float y[32][LD];                       // rows 0..15 k_t, rows 16..31 q_t
+    float x[BF ? 16 : 32][LD];             // rows 0..15 state tile, rows 16..31 k_t
+    float y[BF ? 1 : 32][BF ? 4 : LD];     // rows 0..15 k_t, rows 16..31 q_t
     float p[16][33];                       // S_0 x [k | q]^T: p[r][t] = S_0 k_t, p[r][16 + t] = S_0 q_t of state row r
     float a[16][16];                       // a[s][t] = G[s][t] k_s.k_t for s < t, else 0
     float c[16][16];                       // c[s][t] = G[s][t] k_s.q_t for s <= t, else 0
@@ -736,18 +741,18 @@ template <int DK> struct GdnChunkLds {
     float v[16][16];                       // v_t of row r at v[t][r]
     float g[16], beta[16], gam[16], w[16]; // w[s] = G[s][15]: decay from step s to the end of the chunk
     int on[16];
-    // bf16 inputs: the product's operands as bf16 (x rows 16..31 and y rows 16..31 are then unused).  The state tile
-    // as three bf16 terms, S_0 = hi + mid + lo exactly (3 x 8 = 24 significand bits); k_t and q_t as they came.
     // Row pitch DK + 8: the 16 bytes of pad spread a column of rows over all banks for 16-byte reads.
-    static constexpr int LB = DK + 8;
-    uint16_t xs[3][16][LB];
-    uint16_t kb[16][LB], qb[16][LB];
+    static constexpr int LB = BF ? DK + 8 : 8, RB = BF ? 16 : 1;
+    uint16_t xs[3][RB][LB];
+    uint16_t kb[RB][LB], qb[RB][LB];
 };
 
 // BF: the inputs are bf16 (fixed at compile time): the product then runs on bf16 MFMAs, exactly (see below).
-template <bool HAS_MASK, int DK, bool FUSED, bool BF>
+// LOOP: more than one chunk.  The single chunk of a verify block, without the loop behind it, takes 102 registers at Dk = 128 where
+// the two together take 136: four waves per SIMD.
+template <bool HAS_MASK, int DK, bool FUSED, bool BF, bool LOOP>
 __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& P) {
-    using Lds = GdnChunkLds<DK>;
+    using Lds = GdnChunkLds<DK, BF>;
     extern __shared__ __align__(16) unsigned char gdn_chunk_smem[];
     Lds& L = *reinterpret_cast<Lds*>(gdn_chunk_smem);
     // Every kernel argument is asked for here, in one burst of scalar loads.  Left alone the compiler fetches
@@ -813,11 +818,11 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
         }
     };
     auto store_kq4 = [&](int t, int c4, float4 k4, float4 q4) {
-        store4(&L.y[t][c4], k4);
         if constexpr (BF) {
             *reinterpret_cast<uint2*>(&L.kb[t][c4]) = pack4_bf16_exact(k4);
             *reinterpret_cast<uint2*>(&L.qb[t][c4]) = pack4_bf16_exact(q4);
         } else {
+            store4(&L.y[t][c4], k4);
             store4(&L.x[16 + t][c4], k4);
             store4(&L.y[16 + t][c4], q4);
         }
@@ -880,8 +885,6 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             const int i = tid + u * kThreads, t = i / (DK / 4), c4 = (i % (DK / 4)) * 4;
             if constexpr (BF) {
                 const uint2 kr = t < tc ? kraw[u] : make_uint2(0u, 0u), qr = t < tc ? qraw[u] : make_uint2(0u, 0u);
-                store4(&L.y[t][c4], make_float4(__uint_as_float(kr.x << 16), __uint_as_float(kr.x & 0xffff0000u),
-                                                __uint_as_float(kr.y << 16), __uint_as_float(kr.y & 0xffff0000u)));
                 *reinterpret_cast<uint2*>(&L.kb[t][c4]) = kr;
                 *reinterpret_cast<uint2*>(&L.qb[t][c4]) = qr;
             } else {
@@ -1090,7 +1093,7 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
     // load and carries waits round the back edge.
     auto run_chunk = [&](const int t0) {
         const int tc = (A.T - t0) < kChunkSteps ? (A.T - t0) : kChunkSteps;
-        const bool last_chunk = t0 + kChunkSteps >= A.T;
+        const bool last_chunk = !LOOP || t0 + kChunkSteps >= A.T;
         if constexpr (FUSED) {
             if constexpr (BF) stage_fused(bf16_t{}, tc);
             else if (A.in_dtype == DFLASH_F16) stage_fused(f16_t{}, tc);
@@ -1243,18 +1246,15 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
         // betas, the LDS stores of delta) is kept off it.
         if (w == 0) {
             const int r = lane / 4, q = lane % 4;
-            float acc[4], bet[16], mine[4] = {0.f, 0.f, 0.f, 0.f};
+            float acc[4], bet[4], mine[4] = {0.f, 0.f, 0.f, 0.f};
             float4 arow[16];
             // every LDS read of the phase goes out before the first use (the compiler keeps the order written here:
             // with the start values first, the coefficient reads waited for them -- a second trip to LDS)
             float gm[4], pv[4], vv[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { gm[e] = L.gam[4 * q + e]; pv[e] = L.p[r][4 * q + e]; vv[e] = L.v[4 * q + e][r]; }
+            for (int e = 0; e < 4; ++e) { gm[e] = L.gam[4 * q + e]; pv[e] = L.p[r][4 * q + e]; vv[e] = L.v[4 * q + e][r]; bet[e] = L.beta[4 * q + e]; }
 #pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                arow[s] = *reinterpret_cast<const float4*>(&L.a[s][4 * q]);
-                bet[s] = L.beta[s];
-            }
+            for (int s = 0; s < 16; ++s) arow[s] = *reinterpret_cast<const float4*>(&L.a[s][4 * q]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] = fmaf(-gm[e], pv[e], vv[e]);
@@ -1309,9 +1309,18 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             for (int ks = 0; ks < 4; ++ks) {
                 const int s = 4 * ks + kk;
                 const float av = L.w[s] * L.dl[s][n];
+                float kv[E];
+                if constexpr (BF) {
+                    typedef uint16_t Bits __attribute__((ext_vector_type(E)));
+                    const Bits kx = *reinterpret_cast<const Bits*>(&L.kb[s][base]);
 #pragma unroll
-                for (int e = 0; e < E; ++e)
-                    cacc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, L.y[s][base + e], cacc[e], 0, 0, 0);
+                    for (int e = 0; e < E; ++e) kv[e] = __uint_as_float((uint32_t)kx[e] << 16);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < E; ++e) kv[e] = L.y[s][base + e];
+                }
+#pragma unroll
+                for (int e = 0; e < E; ++e) cacc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, kv[e], cacc[e], 0, 0, 0);
             }
             // first use of the pointer: down here (null when the caller does not want the post-block state)
             float* const s_out = A.state_out ? reinterpret_cast<float*>(A.state_out) + tile_off : nullptr;
@@ -1396,7 +1405,7 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
         }
     };
     run_chunk(0);
-    if constexpr (!FUSED)
+    if constexpr (LOOP)
         for (int t0 = kChunkSteps; t0 < A.T; t0 += kChunkSteps) run_chunk(t0);
 }
 
@@ -1404,21 +1413,21 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
 // is passed as leading scalar arguments: the command processor hands those over in SGPRs when the wave starts (kernarg
 // preload, 14 dwords at most, hence the sizes packed in pairs), so no load waits for a trip to the argument block.
 // The rest of the arguments (outputs, mask, types) follow in the struct and are fetched while the loads are in flight.
-template <bool HAS_MASK, int DK, bool BF>
-__global__ __launch_bounds__(kThreads) void gated_delta_chunk_kernel(const void* state_in, const void* k, const void* q, const void* v,
+template <bool HAS_MASK, int DK, bool BF, bool LOOP>
+__global__ __launch_bounds__(kThreads, DK == 256 || LOOP ? 2 : 4) void gated_delta_chunk_kernel(const void* state_in, const void* k, const void* q, const void* v,
                                                                      const void* g, const void* beta, uint32_t hv_dv, uint32_t hk_t,
                                                                      GdnArgs A) {
     A.state_in = state_in; A.k = k; A.q = q; A.v = v; A.g = g; A.beta = beta;
     A.Hv = (int)(hv_dv >> 16); A.Dv = (int)(hv_dv & 0xffffu); A.Hk = (int)(hk_t >> 16); A.T = (int)(hk_t & 0xffffu);
     A.group = (uint32_t)A.Hv / (uint32_t)A.Hk;
     A.group_magic = 0;                 // hk = hv / group is divided out below (scalar, once): the reciprocal did not fit the registers
-    gdn_chunk_body<HAS_MASK, DK, false, BF>(A, GdnPrep{});
+    gdn_chunk_body<HAS_MASK, DK, false, BF, LOOP>(A, GdnPrep{});
 }
 
 // One GatedDelta layer from its projections to the recurrence's outputs in one launch.
 template <int DK, bool BF>
-__global__ __launch_bounds__(kThreads) void gdn_layer_kernel(GdnArgs A, GdnPrep P) {
-    gdn_chunk_body<false, DK, true, BF>(A, P);
+__global__ __launch_bounds__(kThreads, DK == 256 ? 2 : BF ? 4 : 3) void gdn_layer_kernel(GdnArgs A, GdnPrep P) {
+    gdn_chunk_body<false, DK, true, BF, false>(A, P);
 }
 
 // Whether the chunked kernels' 32-bit element offsets and 24-bit per-step strides cover this shape, and the
@@ -1434,33 +1443,38 @@ static bool chunk_index_setup(GdnArgs& A, int B, int Dk) {
 
 template <int DK>
 static int launch_gdn_layer(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B) {
-    const size_t lds = sizeof(GdnChunkLds<DK>);
+    const bool bf = A.in_dtype == DFLASH_BF16;
+    const size_t lds = bf ? sizeof(GdnChunkLds<DK, true>) : sizeof(GdnChunkLds<DK, false>);
     dim3 grid(A.Dv / kChunkRows, A.Hv, B);
     LaunchBracket br(DFLASH_KERNEL_GDN_LAYER, st);
-    DFLASH_HIP_TRY(br.launch(A.in_dtype == DFLASH_BF16 ? gdn_layer_kernel<DK, true> : gdn_layer_kernel<DK, false>, grid, dim3(kThreads), lds, A, P));
+    DFLASH_HIP_TRY(br.launch(bf ? gdn_layer_kernel<DK, true> : gdn_layer_kernel<DK, false>, grid, dim3(kThreads), lds, A, P));
     return DFLASH_OK;
 }
 
 template <int DK>
 static int launch_gdn_chunk(hipStream_t st, const GdnArgs& A, int B) {
-    const size_t lds = sizeof(GdnChunkLds<DK>);     // the attribute that allows it is set per device by gdn_device_setup()
+    const bool bf = A.in_dtype == DFLASH_BF16;
+    // the attribute that allows it is set per device by gdn_device_setup()
+    const size_t lds = bf ? sizeof(GdnChunkLds<DK, true>) : sizeof(GdnChunkLds<DK, false>);
     dim3 grid(A.Dv / kChunkRows, A.Hv, B);
     LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);
-    const bool bf = A.in_dtype == DFLASH_BF16;
     const uint32_t hv_dv = ((uint32_t)A.Hv << 16) | (uint32_t)A.Dv, hk_t = ((uint32_t)A.Hk << 16) | (uint32_t)A.T;   // each below 2^16, checked by the caller
-    auto kern = A.mask ? (bf ? gated_delta_chunk_kernel<true, DK, true> : gated_delta_chunk_kernel<true, DK, false>)
-                       : (bf ? gated_delta_chunk_kernel<false, DK, true> : gated_delta_chunk_kernel<false, DK, false>);
+    auto kern = A.T <= kChunkSteps ? (A.mask ? (bf ? gated_delta_chunk_kernel<true, DK, true, false> : gated_delta_chunk_kernel<true, DK, false, false>)
+                                             : (bf ? gated_delta_chunk_kernel<false, DK, true, false> : gated_delta_chunk_kernel<false, DK, false, false>))
+                                   : (A.mask ? (bf ? gated_delta_chunk_kernel<true, DK, true, true> : gated_delta_chunk_kernel<true, DK, false, true>)
+                                             : (bf ? gated_delta_chunk_kernel<false, DK, true, true> : gated_delta_chunk_kernel<false, DK, false, true>));
     DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), lds, A.state_in, A.k, A.q, A.v, A.g, A.beta, hv_dv, hk_t, A));
     return DFLASH_OK;
 }
 
 template <int DK>
 static int gdn_chunk_setup() {
-    const int lds = (int)sizeof(GdnChunkLds<DK>);
-    DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gated_delta_chunk_kernel<true, DK, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gated_delta_chunk_kernel<true, DK, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gated_delta_chunk_kernel<false, DK, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gated_delta_chunk_kernel<false, DK, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    const int lds = (int)(sizeof(GdnChunkLds<DK, true>) > sizeof(GdnChunkLds<DK, false>) ? sizeof(GdnChunkLds<DK, true>) : sizeof(GdnChunkLds<DK, false>));
+    const void* kernels[] = {(const void*)gated_delta_chunk_kernel<true, DK, true, false>, (const void*)gated_delta_chunk_kernel<true, DK, false, false>,
+                             (const void*)gated_delta_chunk_kernel<false, DK, true, false>, (const void*)gated_delta_chunk_kernel<false, DK, false, false>,
+                             (const void*)gated_delta_chunk_kernel<true, DK, true, true>, (const void*)gated_delta_chunk_kernel<true, DK, false, true>,
+                             (const void*)gated_delta_chunk_kernel<false, DK, true, true>, (const void*)gated_delta_chunk_kernel<false, DK, false, true>};
+    for (const void* k : kernels) DFLASH_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gdn_layer_kernel<DK, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gdn_layer_kernel<DK, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     return DFLASH_OK;
