@@ -62,6 +62,11 @@ template <int QUAD_LANE> __device__ __forceinline__ float quad_broadcast(float x
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, true));
 }
 
+// Lane S of each 16-lane row to all lanes of the row.
+template <int S> __device__ __forceinline__ float row_broadcast(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + S, 0xf, 0xf, true));
+}
+
 // Steps S..15 of the unit-triangular solve for one state row held by a quad (lane q owns steps 4q..4q+3).
 // Every lane of the quad sees every delta; lane q keeps those of its own four steps in `mine` (a select per step,
 // no branch) for the store that follows.  `bet` holds the betas of the lane's own steps: only the lane that owns a step scales it.

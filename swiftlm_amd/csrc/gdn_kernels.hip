@@ -422,9 +422,10 @@ struct GdnPrep {
     int32_t* status;          // device status word (dflash_set_status_word), or null
     float fin_eps;
     int fin_silu;
+    int fin_wide;             // bf16, and y, fin_gate, fin_weight and fin_out 16-byte aligned
 };
-constexpr int kLayerTaps = 4;
-constexpr int kLayerFinishMaxDv = 256;   // head dim up to which the post-op runs inside the layer kernel  // conv kernel size the one-launch layer kernel is built for
+constexpr int kLayerTaps = 4;            // conv kernel size the one-launch layer kernel is built for
+constexpr int kLayerFinishMaxDv = 256;   // head dim up to which the post-op runs inside the layer kernel
 
 constexpr int kGdnChunk = 16;  // steps staged in LDS at a time
 
@@ -730,7 +731,7 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
 // arrays, as their size decides how many workgroups share a compute unit (Dk = 128: 37 KB, four; with every array of both forms
 // 62 KB, two).  us per call before and after, T = 16, 32 value heads of 128: four sequences 9.4 -> 7.1, two at Dk = 256 10.3 -> 7.2,
 // four 19.2 -> 12.6; the layer in one launch 20.2 -> 15.2 (B = 4), Dk = 256 21.6 -> 15.5 (B = 2), 40.2 -> 26.8 (B = 4).
-template <int DK, bool BF> struct GdnChunkLds {
+template <int DK, bool BF, bool FUSED> struct GdnChunkLds {
     static constexpr int LD = DK + 4;      // row pitch in floats: 16-byte pad spreads rows over the banks
     float x[BF ? 16 : 32][LD];             // rows 0..15 state tile, rows 16..31 k_t
     float y[BF ? 1 : 32][BF ? 4 : LD];     // rows 0..15 k_t, rows 16..31 q_t
@@ -745,6 +746,12 @@ template <int DK, bool BF> struct GdnChunkLds {
     static constexpr int LB = BF ? DK + 8 : 8, RB = BF ? 16 : 1;
     uint16_t xs[3][RB][LB];
     uint16_t kb[RB][LB], qb[RB][LB];
+    // The layer's conv taps (k, then q), four per channel, and its window rows (k and q channels of a row side by side).  The rows
+    // are used up before anything else of the arrays in front of v is written.
+    static constexpr int WIN_ROWS = kChunkSteps + kLayerTaps - 1;
+    static constexpr bool STAGED = BF && FUSED;
+    uint16_t taps[STAGED ? 2 * DK : 1][kLayerTaps];
+    __device__ uint2* win() { return reinterpret_cast<uint2*>(&x[0][0]); }
 };
 
 // BF: the inputs are bf16 (fixed at compile time): the product then runs on bf16 MFMAs, exactly (see below).
@@ -752,7 +759,8 @@ template <int DK, bool BF> struct GdnChunkLds {
 // the two together take 136: four waves per SIMD.
 template <bool HAS_MASK, int DK, bool FUSED, bool BF, bool LOOP>
 __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& P) {
-    using Lds = GdnChunkLds<DK, BF>;
+    using Lds = GdnChunkLds<DK, BF, FUSED>;
+    static_assert(!Lds::STAGED || offsetof(Lds, v) >= Lds::WIN_ROWS * 2 * DK * 2, "the window rows fit in front of v");
     extern __shared__ __align__(16) unsigned char gdn_chunk_smem[];
     Lds& L = *reinterpret_cast<Lds*>(gdn_chunk_smem);
     // Every kernel argument is asked for here, in one burst of scalar loads.  Left alone the compiler fetches
@@ -764,7 +772,7 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
                      "s"(P.dt_bias), "s"(P.q_out), "s"(P.k_out), "s"(P.v_out), "s"(P.g_out), "s"(P.beta_out), "s"(P.conv_out),
                      "s"(P.q_scale), "s"(P.k_scale), "s"(P.eps), "s"(P.C));
     if constexpr (FUSED)
-        asm volatile("" ::"s"(P.fin_gate), "s"(P.fin_weight), "s"(P.fin_out), "s"(P.arrivals), "s"(P.status), "s"(P.fin_eps), "s"(P.fin_silu));
+        asm volatile("" ::"s"(P.fin_gate), "s"(P.fin_weight), "s"(P.fin_out), "s"(P.arrivals), "s"(P.status), "s"(P.fin_eps), "s"(P.fin_silu), "s"(P.fin_wide));
     // (The plain forward gets what its first loads need -- the state pointer, k, q and the sizes in their addresses -- in
     //  SGPRs at wave start, as leading kernel arguments; the rest of its arguments are named in one such statement
     //  further down, behind those loads, so that the wait for the argument block does not stand in front of them.)
@@ -808,7 +816,7 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
     // Where the staged operands go: fp32 rows for the fp32 product (x = [S_0 ; k], y = [k ; q]); with bf16 inputs the
     // product reads the bf16 arrays instead, and only what the state update needs stays fp32 (S_0 and k).
     auto store_state4 = [&](int r, int c4, float4 s4) {
-        store4(&L.x[r][c4], s4);
+        if constexpr (!Lds::STAGED) store4(&L.x[r][c4], s4);
         if constexpr (BF) {
             uint2 hi, mid, lo;
             split3_bf16(s4, hi, mid, lo);
@@ -924,29 +932,50 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             const int rr = in_x ? r - keep : (cs ? r : 0);
             return (in_x ? x : csz) + __umul24(rr, C);
         };
-        float4 kw[NV][KT], qw[NV][KT], ktap[4], qtap[4], vtap;
+        // Steps of a thread.  STAGED: neighbours, which share window rows; every window row and tap is loaded once per workgroup, in
+        // whole lines, and shared through LDS, where each lane loaded 16 windows and 8 strided taps (32 value heads of 128, T = 16: B = 2
+        // 10.8 us without, 10.6 with; B = 4 14.7, 14.1; Dk = 256 15.1, 13.9 and 25.9, 23.9).
+        auto step_of = [&](int u) { return Lds::STAGED ? NV * (tid / LPT) + u : (tid + u * kThreads) / LPT; };
+        constexpr int QPR = DK / 2, WINS = Lds::WIN_ROWS * QPR, NW = (WINS + kThreads - 1) / kThreads, NT = (2 * DK + kThreads - 1) / kThreads;
+        constexpr int ER = Lds::STAGED ? NV + keep : NV * KT;
+        uint2 wraw[NW], traw[NT];
+        float4 kw[ER], qw[ER], ktap[4], qtap[4], vtap;             // kw[NV * KT]: [u * KT + j]; STAGED: rows of the first step's window on
         float vw[KT];
+        if constexpr (Lds::STAGED) {
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {               // [m] = the KT taps of channel c4 + m
-            ktap[m] = load4(wt + (uint32_t)((ck + c4 + m) * KT));
-            qtap[m] = load4(wt + (uint32_t)((cq + c4 + m) * KT));
-        }
+            for (int u = 0; u < NW; ++u) {
+                const int i = tid + u * kThreads, r = i / QPR, c = (i % QPR) * 4;
+                const int rl = r < tc + keep ? r : tc + keep - 1;
+                wraw[u] = *reinterpret_cast<const uint2*>(win_row(rl) + (c < DK ? ck + c : cq + c - DK));
+            }
 #pragma unroll
-        for (int u = 0; u < NV; ++u) {
-            const int t = (tid + u * kThreads) / LPT, tl = t < tc ? t : tc - 1;
+            for (int u = 0; u < NT; ++u) {
+                const int i = tid + u * kThreads, c = i < 2 * DK ? i : 0;
+                traw[u] = *reinterpret_cast<const uint2*>(wt + (uint32_t)((c < DK ? ck + c : cq + c - DK) * KT));
+            }
+        } else {
 #pragma unroll
-            for (int j = 0; j < KT; ++j) {
-                const Elem* src = win_row(tl + j);
-                kw[u][j] = load4(src + ck + c4);
-                qw[u][j] = load4(src + cq + c4);
+            for (int m = 0; m < 4; ++m) {               // [m] = the KT taps of channel c4 + m
+                ktap[m] = load4(wt + (uint32_t)((ck + c4 + m) * KT));
+                qtap[m] = load4(wt + (uint32_t)((cq + c4 + m) * KT));
+            }
+#pragma unroll
+            for (int u = 0; u < NV; ++u) {
+                const int t = step_of(u), tl = t < tc ? t : tc - 1;
+#pragma unroll
+                for (int j = 0; j < KT; ++j) {
+                    const Elem* src = win_row(tl + j);
+                    kw[u * KT + j] = load4(src + ck + c4);
+                    qw[u * KT + j] = load4(src + cq + c4);
+                }
             }
         }
         const int tvl = ts < tc ? ts : tc - 1;
 #pragma unroll
         for (int j = 0; j < KT; ++j) vw[j] = to_float(win_row(tvl + j)[cv + tt]);
         vtap = load4(wt + (uint32_t)((cv + tt) * KT));
-        // gate inputs: every thread reads them (step tid mod 16), so that no load sits inside a branch
-        const int tg = (tid % kChunkSteps) < tc ? (tid % kChunkSteps) : tc - 1;
+        // gate inputs: every thread reads them (those beyond the last step its values), so that no load sits inside a branch
+        const int tg = tid < tc ? tid : tc - 1;
         const uint32_t btg = ((uint32_t)b * A.T + tg) * A.Hv + hv;
         const float av = to_float(reinterpret_cast<const Elem*>(P.a)[btg]);
         const float bv = to_float(reinterpret_cast<const Elem*>(P.b)[btg]);
@@ -962,15 +991,41 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             store_state4(r, cc, sv0[u]);
         }
         const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (Lds::STAGED) {
+#pragma unroll
+            for (int u = 0; u < NW; ++u) {
+                const int i = tid + u * kThreads;
+                if (i < WINS) L.win()[i] = cs || i / QPR >= keep ? wraw[u] : make_uint2(0u, 0u);
+            }
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+                const int i = tid + u * kThreads;
+                if (i < 2 * DK) *reinterpret_cast<uint2*>(L.taps[i]) = traw[u];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                ktap[m] = load4(reinterpret_cast<const bf16_t*>(L.taps[c4 + m]));
+                qtap[m] = load4(reinterpret_cast<const bf16_t*>(L.taps[DK + c4 + m]));
+            }
+            const bf16_t* rows = reinterpret_cast<const bf16_t*>(L.win()) + (size_t)step_of(0) * 2 * DK + c4;
+#pragma unroll
+            for (int r = 0; r < ER; ++r) {
+                kw[r] = load4(rows + r * 2 * DK);
+                qw[r] = load4(rows + r * 2 * DK + DK);
+            }
+        }
         // Without a carried window the rows in front of the sequence are zeros: set once here, under a uniform branch
         // (selected tap by tap inside the conv it was a select per multiply on every call, carried window or not).
         if (!cs) {
+            if constexpr (!Lds::STAGED) {
 #pragma unroll
-            for (int u = 0; u < NV; ++u) {
-                const int t = (tid + u * kThreads) / LPT, tl = t < tc ? t : tc - 1;
+                for (int u = 0; u < NV; ++u) {
+                    const int t = step_of(u), tl = t < tc ? t : tc - 1;
 #pragma unroll
-                for (int j = 0; j < KT; ++j)
-                    if (tl + j < keep) { kw[u][j] = zero4; qw[u][j] = zero4; }
+                    for (int j = 0; j < KT; ++j)
+                        if (tl + j < keep) { kw[u * KT + j] = zero4; qw[u * KT + j] = zero4; }
+                }
             }
 #pragma unroll
             for (int j = 0; j < KT; ++j)
@@ -978,7 +1033,7 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
         }
         const bool first_tile = blockIdx.x == 0;
         const bool qk_owner = first_tile && (hv % (A.Hv / A.Hk)) == 0;
-        auto conv4 = [&](const float4 (&w)[KT], const float4 (&tap)[4], int tl) -> float4 {
+        auto conv4 = [&](const float4* w, const float4 (&tap)[4]) -> float4 {
             float o[4];
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
@@ -1003,8 +1058,9 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
         };
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
-            const int t = (tid + u * kThreads) / LPT, tl = t < tc ? t : tc - 1;
-            const float4 kc = conv4(kw[u], ktap, tl), qc = conv4(qw[u], qtap, tl);
+            const int t = step_of(u);
+            const float4 *kwu = &kw[Lds::STAGED ? u : u * KT], *qwu = &qw[Lds::STAGED ? u : u * KT];
+            const float4 kc = conv4(kwu, ktap), qc = conv4(qwu, qtap);
             const float4 k4 = round4(kc, head_scale(kc, P.k_scale)), q4 = round4(qc, head_scale(qc, P.q_scale));
             const bool live = t < tc;
             store_kq4(t, c4, live ? k4 : zero4, live ? q4 : zero4);
@@ -1016,8 +1072,8 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
                     Elem* dst = reinterpret_cast<Elem*>(P.conv_out) + (size_t)b * keep * C;
 #pragma unroll
                     for (int j = 1; j < KT; ++j) {
-                        store4(dst + (size_t)(j - 1) * C + ck + c4, kw[u][j]);
-                        store4(dst + (size_t)(j - 1) * C + cq + c4, qw[u][j]);
+                        store4(dst + (size_t)(j - 1) * C + ck + c4, kwu[j]);
+                        store4(dst + (size_t)(j - 1) * C + cq + c4, qwu[j]);
                     }
                 }
             }
@@ -1088,6 +1144,47 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
         }
     };
 
+    // The same for bf16 at 16-byte aligned rows, eight channels per load: element by element it is 64 loads per lane, each of which
+    // occupies the address unit of the compute unit as long as a wide one (32 heads of 128, T = 16: 9.6 us, now 9.0).  (f16 stays element by element: where the last
+    // product and its rounding to f16 are one instruction or two depends on how the compiler packs the results.)
+    auto finish_head_wide = [&](int tc) {
+        using Elem = bf16_t;
+        constexpr int MAXI = kLayerFinishMaxDv / 128;
+        const int t = ts < tc ? ts : tc - 1, tiles = (int)gridDim.x;
+        const size_t row = (((size_t)b * A.T + t) * A.Hv + hv) * A.Dv;
+        Elem* orow = reinterpret_cast<Elem*>(P.fin_out) + row;
+        union Eight { uint64_t u[2]; uint4 v; Elem e[8]; } y8[MAXI], z8[MAXI], w8[MAXI];
+#pragma unroll
+        for (int i = 0; i < MAXI; ++i) {
+            const int d = 8 * tt + 128 * i, dl = d < A.Dv ? d : 0;
+            const uint64_t* yp = reinterpret_cast<const uint64_t*>(reinterpret_cast<const Elem*>(A.y) + row + dl);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) y8[i].u[j] = __hip_atomic_load(yp + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            z8[i].v = *reinterpret_cast<const uint4*>(reinterpret_cast<const Elem*>(P.fin_gate) + row + dl);
+            w8[i].v = *reinterpret_cast<const uint4*>(reinterpret_cast<const Elem*>(P.fin_weight) + dl);
+        }
+        float part = load_agent(reinterpret_cast<const float*>(orow) + (tt < tiles ? tt : 0));
+        part = tt < tiles ? part : 0.f;
+        float ss = 0.f;                        // in tile order
+        auto add = [&](float x) { ss = __fadd_rn(ss, x); };
+        add(row_broadcast<0>(part)); add(row_broadcast<1>(part)); add(row_broadcast<2>(part)); add(row_broadcast<3>(part));
+        add(row_broadcast<4>(part)); add(row_broadcast<5>(part)); add(row_broadcast<6>(part)); add(row_broadcast<7>(part));
+        if (tiles > 8) {
+            add(row_broadcast<8>(part)); add(row_broadcast<9>(part)); add(row_broadcast<10>(part)); add(row_broadcast<11>(part));
+            add(row_broadcast<12>(part)); add(row_broadcast<13>(part)); add(row_broadcast<14>(part)); add(row_broadcast<15>(part));
+        }
+        const float inv = gdn_rms_inv(ss, A.Dv, P.fin_eps);
+#pragma unroll
+        for (int i = 0; i < MAXI; ++i) {
+            const int d = 8 * tt + 128 * i;
+            Eight o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                o.e[e] = from_float<Elem>(gdn_gated_out(to_float(y8[i].e[e]), inv, to_float(w8[i].e[e]), to_float(z8[i].e[e]), P.fin_silu != 0));
+            if (d < A.Dv && ts < tc) *reinterpret_cast<uint4*>(orow + d) = o.v;
+        }
+    };
+
     // One chunk of up to 16 steps.  The first chunk (the only one of a verify block) is straight-line code ahead of
     // the loop over the rest: inside the loop the compiler hoists every invariant of the whole body above the first
     // load and carries waits round the back edge.
@@ -1104,6 +1201,13 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             else stage(float{}, t0, tc, t0 == 0);
         }
         __syncthreads();
+        if constexpr (Lds::STAGED) {           // the fp32 tile goes where the window rows were; it is read behind the next barriers
+#pragma unroll
+            for (int u = 0; u < NV; ++u) {
+                const int i = tid + u * kThreads;
+                store4(&L.x[i / (DK / 4)][(i % (DK / 4)) * 4], sv0[u]);
+            }
+        }
 
         // ---- [S_0 ; k] x [k | q]^T: one 16x16 block per wave, over all DK channels ----
         //   wave 0: S_0 k_t -> p[r][t]     wave 1: S_0 q_t -> p[r][16+t]     wave 2: k_s.k_t -> a     wave 3: k_s.q_t -> c
@@ -1398,9 +1502,13 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
                 if (arrived >= (int)gridDim.x && P.status && tid == 0) atomicOr(P.status, DFLASH_STATUS_LAYER_ARRIVALS);
                 if (arrived != (int)gridDim.x - 1) return;
                 if (tid == 0) __hip_atomic_store(P.arrivals + bh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // as the next launch expects it
-                if (A.in_dtype == DFLASH_BF16) finish_head(bf16_t{}, tc);
-                else if (A.in_dtype == DFLASH_F16) finish_head(f16_t{}, tc);
-                else finish_head(float{}, tc);
+                if constexpr (BF) {
+                    if (P.fin_wide) finish_head_wide(tc);
+                    else finish_head(bf16_t{}, tc);
+                } else {
+                    if (A.in_dtype == DFLASH_F16) finish_head(f16_t{}, tc);
+                    else finish_head(float{}, tc);
+                }
             }
         }
     };
@@ -1444,7 +1552,7 @@ static bool chunk_index_setup(GdnArgs& A, int B, int Dk) {
 template <int DK>
 static int launch_gdn_layer(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B) {
     const bool bf = A.in_dtype == DFLASH_BF16;
-    const size_t lds = bf ? sizeof(GdnChunkLds<DK, true>) : sizeof(GdnChunkLds<DK, false>);
+    const size_t lds = bf ? sizeof(GdnChunkLds<DK, true, true>) : sizeof(GdnChunkLds<DK, false, true>);
     dim3 grid(A.Dv / kChunkRows, A.Hv, B);
     LaunchBracket br(DFLASH_KERNEL_GDN_LAYER, st);
     DFLASH_HIP_TRY(br.launch(bf ? gdn_layer_kernel<DK, true> : gdn_layer_kernel<DK, false>, grid, dim3(kThreads), lds, A, P));
@@ -1455,7 +1563,7 @@ template <int DK>
 static int launch_gdn_chunk(hipStream_t st, const GdnArgs& A, int B) {
     const bool bf = A.in_dtype == DFLASH_BF16;
     // the attribute that allows it is set per device by gdn_device_setup()
-    const size_t lds = bf ? sizeof(GdnChunkLds<DK, true>) : sizeof(GdnChunkLds<DK, false>);
+    const size_t lds = bf ? sizeof(GdnChunkLds<DK, true, false>) : sizeof(GdnChunkLds<DK, false, false>);
     dim3 grid(A.Dv / kChunkRows, A.Hv, B);
     LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);
     const uint32_t hv_dv = ((uint32_t)A.Hv << 16) | (uint32_t)A.Dv, hk_t = ((uint32_t)A.Hk << 16) | (uint32_t)A.T;   // each below 2^16, checked by the caller
@@ -1469,7 +1577,7 @@ static int launch_gdn_chunk(hipStream_t st, const GdnArgs& A, int B) {
 
 template <int DK>
 static int gdn_chunk_setup() {
-    const int lds = (int)(sizeof(GdnChunkLds<DK, true>) > sizeof(GdnChunkLds<DK, false>) ? sizeof(GdnChunkLds<DK, true>) : sizeof(GdnChunkLds<DK, false>));
+    const int lds = (int)(sizeof(GdnChunkLds<DK, true, true>) > sizeof(GdnChunkLds<DK, false, true>) ? sizeof(GdnChunkLds<DK, true, true>) : sizeof(GdnChunkLds<DK, false, true>));
     const void* kernels[] = {(const void*)gated_delta_chunk_kernel<true, DK, true, false>, (const void*)gated_delta_chunk_kernel<true, DK, false, false>,
                              (const void*)gated_delta_chunk_kernel<false, DK, true, false>, (const void*)gated_delta_chunk_kernel<false, DK, false, false>,
                              (const void*)gated_delta_chunk_kernel<true, DK, true, true>, (const void*)gated_delta_chunk_kernel<true, DK, false, true>,
@@ -1656,6 +1764,7 @@ extern "C" int dflash_gdn_layer(void* stream, const void* mixed_qkv, const void*
     P.status = status_word();
     P.fin_eps = out_norm_eps;
     P.fin_silu = gate_kind;
+    P.fin_wide = in_dtype == DFLASH_BF16 && (((uintptr_t)y_out | (uintptr_t)gate | (uintptr_t)out_norm_weight | (uintptr_t)out) & 15) == 0;
     hipStream_t st = (hipStream_t)stream;
     if (Dk == 64) rc = launch_gdn_layer<64>(st, A, P, B);
     else if (Dk == 128) rc = launch_gdn_layer<128>(st, A, P, B);

@@ -65,10 +65,6 @@ __device__ __forceinline__ void split3_bf16(f32x4v v, uint2& hi, uint2& mid, uin
 __device__ __forceinline__ bf16x8v as_bf16x8(uint2 a, uint2 b) { return __builtin_bit_cast(bf16x8v, make_uint4(a.x, a.y, b.x, b.y)); }
 __device__ __forceinline__ s16x4v as_s16x4(uint2 a) { return __builtin_bit_cast(s16x4v, a); }
 
-// Lane S of each 16-lane row to all lanes of the row.
-template <int S> __device__ __forceinline__ float row_broadcast(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + S, 0xf, 0xf, true));
-}
 template <int L0, int L1, int L2, int L3> __device__ __forceinline__ float quad_take(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), L0 | (L1 << 2) | (L2 << 4) | (L3 << 6), 0xf, 0xf, true));
 }
