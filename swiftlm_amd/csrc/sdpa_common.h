@@ -141,8 +141,9 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt(((N >> 4) << 14) | (0xF << 8) | (0x7 << 4) | (N & 0xF));
 }
 
-// The whole attention in one launch, for short contexts (sdpa_short.hip); `out` and `lse` are A.part_o and A.lse.
-bool sdpa_short_applies(int B, int Hq, int N, int D);
+// Attention by one workgroup per query head and split (sdpa_short.hip).  One split writes the output itself (A.part_o, A.lse).
+// How many splits, at most `most`: 0 where the form does not apply.
+int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most);
 int launch_sdpa_short(hipStream_t st, const SdpaArgs& A, int B, int D, int dtype, bool paged);
 int sdpa_short_device_setup();
 

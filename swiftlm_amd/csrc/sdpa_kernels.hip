@@ -1060,6 +1060,25 @@ static size_t ws_layout(int B, int Hq, int S, int D, size_t* off_m, size_t* off_
     return (o + 255) & ~(size_t)255;
 }
 
+template <typename Tag, int D>
+static int launch_combine(hipStream_t st, const CombineArgs& C) {
+    LaunchBracket br(DFLASH_KERNEL_SDPA_COMBINE, st);
+    const dim3 waves(C.rows / (kCombineThreads / 64)), threads(kCombineThreads);
+    const int groups = 64 / (D / 8);
+    // More than four splits per lane group: one wave per row, 16 partial rows per lane in flight, up to 64 splits at D = 128 (a
+    // dealt launch 32, as its long sequences take more than S), at D = 256 where a workgroup per row would be more than the
+    // chip holds at once.  us per call, wave against workgroup, rows x splits:
+    //   D=128  1,024 x 32 17.3 19.1   512 x 64 16.6 17.8   384 x 74 17.0 16.0   256 x 128 19.3 16.7
+    //   dealt    896 x 37 23.3 23.6   768 x 43 21.4 20.6   512 x 64 21.3 18.4
+    //   D=256  2,048 x 16 38.9 42.3  1,280 x 26 38.4 40.9  1,024 x 32 29.0 29.5  256 x 16 29.1 28.5  512 x 64 32.7 27.8
+    //   dealt  2,048 x 16 43.4 48.2  1,280 x 26 34.2 35.0  1,024 x 32 32.1 30.1
+    auto one_wave = [&]() { return D == 128 ? C.S <= (C.balance ? 32 : 64) : C.S <= 32 && C.rows > 4 * num_compute_units(); };
+    if (C.S <= 4 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 4>, waves, threads, 0, C));
+    else if (one_wave()) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
+    else DFLASH_HIP_TRY(br.launch(sdpa_combine_kernel<Tag, D>, dim3(C.rows), threads, 0, C));
+    return DFLASH_OK;
+}
+
 template <typename Tag, int D, bool MASKED, bool PAGED>
 static int launch_sdpa(hipStream_t st, const SdpaArgs& A, const CombineArgs& C, int B) {
     typedef SdpaLds<D> L;
@@ -1070,23 +1089,7 @@ static int launch_sdpa(hipStream_t st, const SdpaArgs& A, const CombineArgs& C, 
         LaunchBracket br(DFLASH_KERNEL_SDPA_PARTIAL, st);
         DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kPartialThreads), L::BYTES, A));
     }
-    if (A.S > 1) {
-        LaunchBracket br(DFLASH_KERNEL_SDPA_COMBINE, st);
-        const dim3 waves(C.rows / (kCombineThreads / 64)), threads(kCombineThreads);
-        const int groups = 64 / (D / 8);
-        // More than four splits per lane group: one wave per row, 16 partial rows per lane in flight, up to 64 splits at D = 128 (a
-        // dealt launch 32, as its long sequences take more than S), at D = 256 where a workgroup per row would be more than the
-        // chip holds at once.  us per call, wave against workgroup, rows x splits:
-        //   D=128  1,024 x 32 17.3 19.1   512 x 64 16.6 17.8   384 x 74 17.0 16.0   256 x 128 19.3 16.7
-        //   dealt    896 x 37 23.3 23.6   768 x 43 21.4 20.6   512 x 64 21.3 18.4
-        //   D=256  2,048 x 16 38.9 42.3  1,280 x 26 38.4 40.9  1,024 x 32 29.0 29.5  256 x 16 29.1 28.5  512 x 64 32.7 27.8
-        //   dealt  2,048 x 16 43.4 48.2  1,280 x 26 34.2 35.0  1,024 x 32 32.1 30.1
-        auto one_wave = [&]() { return D == 128 ? A.S <= (C.balance ? 32 : 64) : A.S <= 32 && C.rows > 4 * num_compute_units(); };
-        if (A.S <= 4 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 4>, waves, threads, 0, C));
-        else if (one_wave()) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
-        else DFLASH_HIP_TRY(br.launch(sdpa_combine_kernel<Tag, D>, dim3(C.rows), threads, 0, C));
-    }
-    return DFLASH_OK;
+    return A.S > 1 ? launch_combine<Tag, D>(st, C) : DFLASH_OK;
 }
 
 template <typename Tag, int D>
@@ -1250,10 +1253,16 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     C.balance = A.balance; C.deal = A.deal; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
 
     hipStream_t st = (hipStream_t)stream;
-    // (the workspace asked for is that of the split form, whichever form runs)
-    if (sdpa_short_applies(B, Hq, N, D)) {
-        A.part_o = (uint16_t*)out;
-        return launch_sdpa_short(st, A, B, D, dtype, paged != nullptr);
+    // (the workspace asked for is that of the form with shared K/V tiles, whichever form runs)
+    if (const int few = sdpa_short_splits(B, Hq, Hk, N, D, S)) {
+        A.S = C.S = few;
+        A.S_magic = fast_div_magic((uint32_t)few); A.gpk_magic = fast_div_magic((uint32_t)Hk);
+        C.balance = 0;
+        A.part_o = few == 1 ? (uint16_t*)out : (uint16_t*)workspace;
+        rc = launch_sdpa_short(st, A, B, D, dtype, paged != nullptr);
+        if (rc || few == 1) return rc;
+        if (dtype == DFLASH_BF16) return D == 256 ? launch_combine<Bf16Tag, 256>(st, C) : launch_combine<Bf16Tag, 128>(st, C);
+        return D == 256 ? launch_combine<F16Tag, 256>(st, C) : launch_combine<F16Tag, 128>(st, C);
     }
 #define DFLASH_SDPA_CASE(MASKED, PAGED)                                                                              \
     do {                                                                                                             \

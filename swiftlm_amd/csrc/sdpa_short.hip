@@ -1,4 +1,5 @@
-// Block-causal attention of the 16-token verify block over a short context, in one launch.
+// Block-causal attention of the 16-token verify block with a workgroup per query head: short contexts in one launch, those of some
+// thousand keys over a few splits.
 //
 // Semantics follow Sources/DFlash/DFlashKernels.swift:737-815 (entry), :563-649 (causal rule :614, GQA mapping :575).
 
@@ -9,10 +10,11 @@
 namespace dflash {
 
 // ---------------------------------------------------------------------------
-// One workgroup per (query head, sequence); its eight waves take tiles of keys in turn, each with the running maximum, the sum and
-// O^T of its own tiles, and merge them through LDS at the end in fp32.  No partial rows in memory and no second launch; inside
-// the loop no barrier, as a wave brings its own tiles.  The price is that the query heads of a group each read their KV head's
-// rows (from the L2), so it is for contexts whose rows one compute unit can take in: see sdpa_short_applies().
+// One workgroup per (query head, sequence) and split of the keys; its eight waves take tiles of keys in turn, each with the running
+// maximum, the sum and O^T of its own tiles, and merge them through LDS at the end in fp32.  One split, for short contexts: no
+// partial rows in memory and no second launch.  Inside the loop no barrier, as a wave brings its own tiles.  The price is that the
+// query heads of a group each read their KV head's rows (from the L2), so it is for contexts whose rows one compute unit, or a
+// few, can take in: see sdpa_short_splits().
 //
 // Bound by one launch and its first trip to memory (4.1 us) and, from some 200 keys on, by what a compute unit takes in, 64 bytes
 // per clock at best: that is reached by loads HBM -> LDS of 1 KB of whole rows.  K rows straight into the operand registers, where
@@ -61,21 +63,24 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 
     asm volatile("" ::"s"(A.q), "s"(A.k), "s"(A.v), "s"(A.k_new), "s"(A.v_new), "s"(A.k_cache), "s"(A.v_cache), "s"(A.part_o), "s"(A.lse),
                  "s"(A.kv_len_dev), "s"(A.mask), "s"(A.kv_batch_stride), "s"(A.kv_head_stride), "s"(A.scale_log2), "s"(A.Hq), "s"(A.Hk),
-                 "s"(A.G), "s"(A.N), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages), "s"(A.status));
+                 "s"(A.G), "s"(A.N), "s"(A.len_bias), "s"(A.page_table), "s"(A.page_shift), "s"(A.table_stride), "s"(A.num_pages), "s"(A.status),
+                 "s"(A.S), "s"(A.B), "s"(A.gpk_magic), "s"(A.S_magic), "s"(A.part_m), "s"(A.part_l));
 
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
-    const int hk = blockIdx.x, b = blockIdx.z, hq = hk * A.G + (int)blockIdx.y;
+    // x = KV head + Hk * split, y = head of the group: the heads that share rows are Hk * S apart, on one XCD where that is a multiple of 8
+    const int S = A.S, split = (int)fast_div(blockIdx.x, (uint32_t)A.Hk, A.gpk_magic);
+    const int hk = (int)blockIdx.x - split * A.Hk, b = blockIdx.z, hq = hk * A.G + (int)blockIdx.y;
     const size_t row0 = ((size_t)b * A.Hq + hq) * kM;               // first row of the head in q, out and lse
     auto lds_addr = [](const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; };
 
     int len_raw = 0;
     if (A.kv_len_dev) len_raw = A.kv_len_dev[b];
-    // the page-table entries of the wave's tiles, one tile per lane: w, w + W, ... (clamped to the host-side bound, which the table spans)
+    // the page-table entries of the wave's tiles, one tile per lane (clamped to the host-side bound, which the table spans)
     const int nt_max = (A.N + NB - 1) / NB;
     int entries = 0;
     if constexpr (PAGED) {
-        const int tile = min(w + W * lane, nt_max - 1);
+        const int tile = min(split + S * (w + W * lane), nt_max - 1);
         entries = A.page_table[(size_t)b * A.table_stride + ((tile * NB) >> A.page_shift)];
     }
     {
@@ -95,7 +100,9 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
     int Nb = A.kv_len_dev ? len_raw + A.len_bias : A.N;
     if (A.status && (Nb < kM || Nb > A.N) && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) atomicOr(A.status, DFLASH_STATUS_SDPA_LEN);
     Nb = Nb < kM ? kM : (Nb > A.N ? A.N : Nb);
-    const int nt = (Nb + NB - 1) / NB;
+    // the split's tiles: split, split + S, ...; below, t counts them (0 .. nt-1) and tile t begins at key (split + S * t) * NB
+    const int nt_all = (Nb + NB - 1) / NB;
+    const int nt = (int)fast_div((uint32_t)(nt_all - split + S - 1), (uint32_t)S, A.S_magic);      // (S <= the tiles of 16 keys: not negative)
     const bool fused = A.k_new != nullptr;
     const int cache_rows = fused ? Nb - kM : Nb;                    // keys below this index are read from the cache
     const int page_mask = PAGED ? (1 << A.page_shift) - 1 : 0;
@@ -105,32 +112,35 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
         e = e < 0 ? 0 : (e >= A.num_pages ? A.num_pages - 1 : e);
         return (size_t)e * (size_t)A.kv_batch_stride * 2;
     };
+    auto first_key = [&](int t) { return (split + S * t) * NB; };
     auto tile_off = [&](int t) -> size_t {
         if constexpr (PAGED)
-            return page_off(__builtin_amdgcn_readlane(entries, t / W)) + (size_t)((t * NB) & page_mask) * ROWB;
+            return page_off(__builtin_amdgcn_readlane(entries, t / W)) + (size_t)(first_key(t) & page_mask) * ROWB;
         else
-            return (size_t)t * NB * ROWB;
+            return (size_t)first_key(t) * ROWB;
     };
     auto request_rows = [&](int t, const unsigned char* base, const unsigned char* nw, uint32_t lds, bool is_k) __attribute__((always_inline)) {
         const unsigned char* tile = uniform_ptr(base + tile_off(t));
-        const int key0 = t * NB;
+        const int key0 = first_key(t);
         uint32_t l = lane;
         asm volatile("" : "+v"(l));                                 // offsets are formed anew: kept across the loop they are dozens of registers
-        if (key0 + NB <= cache_rows || !fused) {                   // uniform
-            const int last = Nb - 1 - key0;                         // past the end the last key once more (dropped later)
+        const int last = Nb - 1 - key0, cut = fused ? cache_rows - key0 : NB;      // past `last` the last key once more (dropped later)
+        if (cut <= 0 || cut >= NB) {                                // uniform: all rows from one place
+            const unsigned char* from = cut > 0 ? tile : uniform_ptr(nw - (ptrdiff_t)cut * ROWB);
 #pragma unroll
             for (int j = 0; j < TILE_LOADS; ++j) {
                 const int row = (int)(j * RPI + l / CPR);
                 const int piece = (int)(l % CPR) ^ (is_k ? row & 15 : 4 * (row & 3));
-                async_load_16B_plain(tile, (uint32_t)(min(row, last) * ROWB + piece * 16), lds + j * 1024);
+                async_load_16B_plain(from, (uint32_t)(min(row, last) * ROWB + piece * 16), lds + j * 1024);
             }
-        } else {                                                    // the block's own rows come from k_new / v_new
-#pragma unroll 4
+        } else {                                                    // from row `cut` on the block's own rows, in k_new / v_new
+            const uint64_t here = (uint64_t)tile, there = (uint64_t)(nw - (ptrdiff_t)cut * ROWB);
+#pragma unroll
             for (int j = 0; j < TILE_LOADS; ++j) {
-                const int row = (int)(j * RPI + l / CPR), key = min(key0 + row, Nb - 1);
+                const int row = (int)(j * RPI + l / CPR), r = min(row, last);
                 const int piece = (int)(l % CPR) ^ (is_k ? row & 15 : 4 * (row & 3));
-                const unsigned char* src = key < cache_rows ? tile + (uint32_t)((key - key0) * ROWB) : nw + (uint32_t)((key - cache_rows) * ROWB);
-                async_load_16B_addr<false>(src + piece * 16, lds + j * 1024);
+                async_load_16B_addr<false>((const unsigned char*)((r < cut ? here : there) + (uint32_t)(r * ROWB + piece * 16)), lds + j * 1024);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
@@ -139,7 +149,7 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
         if constexpr (MASKED) {
 #pragma unroll
             for (int j = 0; j < MASK_LOADS; ++j) {                   // whole rows of the tile
-                const int row = j * (64 / NB) + lane / NB, key = t * NB + ((lane % NB) ^ (4 * (row & (NB / 4 - 1))));
+                const int row = j * (64 / NB) + lane / NB, key = first_key(t) + ((lane % NB) ^ (4 * (row & (NB / 4 - 1))));
                 async_load_2B_addr(A.mask + (row0 + row) * (size_t)A.N + min(key, A.N - 1), lds_addr(L.mask[w]) + j * 256);    // (keys past the end fail the causal rule)
             }
         }
@@ -200,7 +210,7 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 #pragma unroll
             for (int u = 0; u < NU; ++u) sacc[NU == 2 ? u : s & 1] = Tag::mfma16(load_k(L.slot[w].k + 16 * u * ROWB, s), qf[s], sacc[NU == 2 ? u : s & 1]);
         if constexpr (NU == 1) sacc[0] += sacc[1];
-        const int key0 = t * NB, last_visible = Nb - kM + n;        // row n sees keys 0 .. Nb-16+n
+        const int key0 = first_key(t), last_visible = Nb - kM + n;        // row n sees keys 0 .. Nb-16+n
         float x[4 * NU], mloc = -INFINITY;
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
@@ -271,7 +281,7 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
         }
     };
     // Without a mask only the last tile can be hidden from a row, where it begins behind the first of the block's keys.
-    const int plain = !MASKED && (nt - 1) * NB > Nb - kM ? nt - 1 : nt;
+    const int plain = !MASKED && nt > 0 && first_key(nt - 1) > Nb - kM ? nt - 1 : nt;
     for (int t = w; t < plain; t += W) tile(t, std::bool_constant<MASKED>{});
     if (plain < nt && plain % W == w) tile(plain, std::true_type{});
 
@@ -296,9 +306,16 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 #pragma unroll
         for (int i = 0; i < DB; ++i) o[(4 * i + g) ^ n] = oacc[i] * f;
     }
-    if (w == 0 && g == 0 && A.lse) A.lse[row0 + n] = (M + log2f(l_tot)) * 0.6931471805599453f;
+    if (w == 0 && g == 0) {
+        if (S > 1) {
+            __hip_atomic_store(A.part_m + (row0 + n) * S + split, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(A.part_l + (row0 + n) * S + split, l_tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (A.lse) {
+            A.lse[row0 + n] = (M + log2f(l_tot)) * 0.6931471805599453f;
+        }
+    }
     // the block's own K/V rows into the cache: the group's first head does it
-    if (fused && A.k_cache && blockIdx.y == 0) {
+    if (fused && A.k_cache && blockIdx.y == 0 && split == 0) {
         for (int i = tid; i < kM * CPR; i += 64 * W) {
             const int key = cache_rows + i / CPR;
             size_t off = head_off + (size_t)(i % CPR) * 16;
@@ -311,13 +328,15 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
             *reinterpret_cast<u32x4_t*>(reinterpret_cast<unsigned char*>(A.v_cache) + off) = vx;
         }
     }
+    if (S > 1 && nt == 0) return;                                    // (its partial rows are not read)
     __syncthreads();
     constexpr int PER = D / 4;                                       // threads x 4 channels of a row
+    uint16_t* const out = A.part_o + ((size_t)split * A.B * A.Hq * kM + row0) * D;      // the split's rows [split][B * Hq * 16], or the output
     for (int i = tid; i < kM * PER; i += 64 * W) {
         const int r = i / PER, p = i % PER;
         f32x4_t o = {0.f, 0.f, 0.f, 0.f};
         for (int j = 0; j < waves; ++j) o += reinterpret_cast<const f32x4_t*>(L.o[j])[r * PER + (p ^ r)];
-        *reinterpret_cast<u32x2_t*>(A.part_o + (row0 + r) * D + 4 * p) = __builtin_bit_cast(u32x2_t, Tag::pack4(o));
+        *reinterpret_cast<u32x2_t*>(out + r * D + 4 * p) = __builtin_bit_cast(u32x2_t, Tag::pack4(o));
     }
 }
 
@@ -331,17 +350,42 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 //     128 (B=4)         6.1 4.8   10.2 7.0    11.0 8.1    11.0 9.3    11.5 10.5         8.2 6.2   11.3 9.1    12.5 10.7   12.2 11.9
 //     256 (B=8)         6.1 4.9   12.1 7.5    12.6 8.6    13.3 9.8    14.5 11.2         8.5 6.6   13.6 9.6    15.2 11.3   16.6 12.7
 //     512 (B=8)         6.4 7.0   14.2 12.9   15.5 15.1   16.5 17.4   17.9 20.2         9.0 11.6  16.5 17.3   18.5 20.3   19.6 23.0
-bool sdpa_short_applies(int B, int Hq, int N, int D) {
+//
+// Behind that line several workgroups share a head's keys, as many as fill the chip, and the combine kernel merges their rows: it
+// has S partial rows of each query row to read where the form with shared tiles has a multiple of that, and its own launch has
+// no pipeline to fill.  As long as one workgroup's share is small, as the group's heads read their KV head's rows G times through
+// the L2s (which share nothing: S is a multiple that keeps the heads of a group on one XCD; with S = 21 for 12 heads over 2 KV heads
+// 3,000 keys took 12.7 us, with 20 11.2), and all K/V rows come from memory at most 48 MB.  Few heads take no more than 16 splits,
+// or shares of 512 keys, at D = 128, as the combine then needs one round per lane.  All forms of a call take the same line, so that
+// they give the same bits.  us per call, shared tiles against this form:
+//     heads, keys        1500        2048        3000        4112        6000        8208        12000
+//     D=128  8 (Hk=1)  8.6  8.3    8.7  8.4    8.9  8.5    9.3  9.1    9.4  9.4    10.0 9.6    10.8 10.2
+//           16 (Hk=2)  9.0  8.3    9.2  8.3    9.5  8.6    10.1 9.1    11.0 9.7    11.5 10.2   12.5 11.5
+//           32 (Hk=8)  9.1  8.6    9.9  9.2    11.1 9.8    11.7 10.6   12.5 11.8   13.7 13.4   15.7 16.3
+//           64 (Hk=8)  10.6 9.9    11.4 10.4   12.5 11.5   12.6 12.8   13.3 15.6
+//     D=256  8 (Hk=1)  9.6  9.1    10.0 9.3    11.3 10.2   13.7 10.7   12.3 11.4   14.7 11.7   14.2 12.9
+//           16 (Hk=2)  11.0 10.2   11.9 10.7   11.9 11.5   13.0 11.9   13.6 12.8   14.7 14.4   15.1 16.9   (paged 5000 12.6 13.3)
+//           32 (Hk=8)  13.2 10.9   14.1 11.3   15.3 12.6   15.4 14.4   17.4 17.4
+//           64 (Hk=8)  15.5 12.8   16.4 14.0   17.4 16.8   19.2 20.1
+int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     const int64_t heads = (int64_t)B * Hq;
     const int cus = num_compute_units();
     const bool few = heads < cus / 4;
-    return heads <= cus && N <= (D == 128 ? (few ? 896 : 1152) : (few ? 416 : 576));
+    if (heads > cus) return 0;
+    if (N <= (D == 128 ? (few ? 896 : 1152) : (few ? 416 : 576))) return 1;
+    if (heads < (D == 128 ? 8 : 4) || (int64_t)B * Hk * N * D > 12000000) return 0;
+    int64_t S = cus / heads;
+    if (D == 128 && S > 16) S = S < N / 512 ? S : N / 512 > 16 ? N / 512 : 16;
+    if (S > most) S = most;
+    const int same_xcd = Hk % 8 == 0 ? 1 : Hk % 4 == 0 ? 2 : Hk % 2 == 0 ? 4 : 8;
+    if (S > same_xcd) S -= S % same_xcd;
+    return S >= (D == 128 ? 3 : 2) && N <= (D == 128 ? 900 : heads < 32 ? 288 : 512) * S ? (int)S : 0;
 }
 
 template <typename Tag, int D, bool MASKED, bool PAGED>
 static int launch_short(hipStream_t st, const SdpaArgs& A, int B) {
     LaunchBracket br(DFLASH_KERNEL_SDPA_PARTIAL, st);
-    DFLASH_HIP_TRY(br.launch(sdpa_short_kernel<Tag, D, MASKED, PAGED>, dim3(A.Hk, A.G, B), dim3(64 * SdpaShortLds<D>::WAVES), sizeof(SdpaShortLds<D>), A));
+    DFLASH_HIP_TRY(br.launch(sdpa_short_kernel<Tag, D, MASKED, PAGED>, dim3(A.Hk * A.S, A.G, B), dim3(64 * SdpaShortLds<D>::WAVES), sizeof(SdpaShortLds<D>), A));
     return DFLASH_OK;
 }
 template <typename Tag, int D> static int launch_short(hipStream_t st, const SdpaArgs& A, int B, bool paged) {

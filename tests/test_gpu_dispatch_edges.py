@@ -117,16 +117,18 @@ def test_attention_split_counts(gpu_lib, N, Hq, Hk, D):
     attend(*tensors(N + D, 1, Hq, Hk, N, D), [N], D)
 
 
-# Short contexts in one launch, up to a line of keys that depends on the query heads (B * Hq), and the split forms behind it; more
-# heads than compute units take the split forms at once.  Tiles of 32 (D = 128) and 16 keys, eight waves, one tile a wave and more.
+# Short contexts in one launch, up to a line of keys that depends on the query heads (B * Hq), then a few splits of the same form, then
+# the form with shared tiles, which more heads than compute units take at once.  Tiles of 32 (D = 128) and 16 keys, eight waves, one
+# tile a wave and more; the second sequence leaves splits without a tile; 12 heads whose splits are rounded to whole XCDs.
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("Hq,Hk,D,N", [(2, 1, 128, 31), (3, 1, 128, 256), (3, 1, 128, 257), (12, 2, 128, 600), (8, 1, 128, 896), (8, 1, 128, 897),
                                        (32, 8, 128, 1152), (32, 8, 128, 1153), (2, 1, 256, 17), (3, 1, 256, 128), (3, 1, 256, 129),
-                                       (8, 1, 256, 416), (8, 1, 256, 417), (32, 8, 256, 576), (32, 8, 256, 577), (130, 2, 128, 100), (130, 2, 256, 129)])
+                                       (8, 1, 256, 416), (8, 1, 256, 417), (32, 8, 256, 576), (32, 8, 256, 577), (130, 2, 128, 100), (130, 2, 256, 129),
+                                       (6, 1, 128, 1750), (4, 1, 128, 7200), (4, 1, 128, 7201), (6, 2, 256, 5760), (6, 2, 256, 5761), (16, 8, 256, 2048), (16, 8, 256, 2049)])
 def test_short_contexts(gpu_lib, Hq, Hk, D, N, dt):
     from swiftlm_amd import DFlashKernels as K
 
-    lens = [N, max(16, N // 2 + 1)]
+    lens = [N, max(16, N // 2 + 1) if N < 4000 else 17]
     q, k, v = tensors(N + D, 2, Hq, Hk, N, D, dt)
     kv_len = torch.tensor(lens, dtype=torch.int32, device="cuda")
     out, lse = attend(q, k, v, lens, D, kv_len=kv_len)
