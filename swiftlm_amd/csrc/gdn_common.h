@@ -83,9 +83,45 @@ template <int S> struct SolveStep {
     }
 };
 
+// A barrier that orders LDS only: loads and stores of global memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ f32x4v lds4(const float* p) { return *reinterpret_cast<const f32x4v*>(p); }
+
+// X = (I + A)^-1, A strictly lower: lane n of a 16-lane row holds A[n][.], negated, and four columns of X[n][.]; row S of X
+// is final when its turn comes and is taken off the rows below it.  One fused multiply-add per step and column, its first
+// factor broadcast from lane S of the row (DPP row_newbcast).  One block of assembly: a DPP operand may be read two wait
+// states after it was written, which the order of the columns gives; the s_nop is for what stands in front.
+#define DFLASH_INVERSE_STEP(S, A)                                              \
+    "v_fmac_f32_dpp %0, %0, " A " row_newbcast:" S " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %1, %1, " A " row_newbcast:" S " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %2, %2, " A " row_newbcast:" S " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %3, %3, " A " row_newbcast:" S " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ f32x4v unit_inverse(f32x4v x, const float (&na)[16]) {
+    float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+    asm volatile("s_nop 1\n\t" DFLASH_INVERSE_STEP("0", "%4") DFLASH_INVERSE_STEP("1", "%5") DFLASH_INVERSE_STEP("2", "%6")
+                 DFLASH_INVERSE_STEP("3", "%7") DFLASH_INVERSE_STEP("4", "%8") DFLASH_INVERSE_STEP("5", "%9")
+                 DFLASH_INVERSE_STEP("6", "%10") DFLASH_INVERSE_STEP("7", "%11") DFLASH_INVERSE_STEP("8", "%12")
+                 DFLASH_INVERSE_STEP("9", "%13") DFLASH_INVERSE_STEP("10", "%14") DFLASH_INVERSE_STEP("11", "%15")
+                 DFLASH_INVERSE_STEP("12", "%16") DFLASH_INVERSE_STEP("13", "%17") DFLASH_INVERSE_STEP("14", "%18")
+                 : "+&v"(x0), "+&v"(x1), "+&v"(x2), "+&v"(x3)
+                 : "v"(na[0]), "v"(na[1]), "v"(na[2]), "v"(na[3]), "v"(na[4]), "v"(na[5]), "v"(na[6]), "v"(na[7]), "v"(na[8]),
+                   "v"(na[9]), "v"(na[10]), "v"(na[11]), "v"(na[12]), "v"(na[13]), "v"(na[14]));
+    return f32x4v{x0, x1, x2, x3};
+}
+#undef DFLASH_INVERSE_STEP
+
 // The chunked form for longer calls (gdn_long.hip)
 bool gdn_long_applies(const GdnArgs& A, int Dk);
 int launch_gdn_long(hipStream_t st, const GdnArgs& A, int B, int Dk);
 int gdn_long_device_setup();
+
+// The chunked form for one decay per channel (gdn_channel.hip)
+bool gdn_channel_applies(const GdnArgs& A, int B, int Dk);
+int launch_gdn_channel(hipStream_t st, const GdnArgs& A, int B, int Dk);
+int gdn_channel_device_setup();
 
 }  // namespace dflash

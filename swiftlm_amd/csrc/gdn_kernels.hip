@@ -1593,6 +1593,7 @@ int gdn_device_setup() {
     if (rc == DFLASH_OK) rc = gdn_chunk_setup<128>();
     if (rc == DFLASH_OK) rc = gdn_chunk_setup<256>();
     if (rc == DFLASH_OK) rc = gdn_long_device_setup();
+    if (rc == DFLASH_OK) rc = gdn_channel_device_setup();
     return rc;
 }
 
@@ -1702,6 +1703,8 @@ extern "C" int dflash_gated_delta_tape(void* stream, const void* q, const void* 
     }
     DFLASH_SUPPORTED(state_out != nullptr, "gated delta: a call without state_out needs the chunked form (fp32 state, one decay "
                      "per head and step, Dk in {64, 128, 256}, Dv a multiple of 16, T >= 1)");
+    if (state_dtype == DFLASH_F32 && g_ndim == 4 && Dv % kChunkRows == 0 && T > 0 && chunk_index_setup(A, B, Dk) && gdn_channel_applies(A, B, Dk))
+        return launch_gdn_channel((hipStream_t)stream, A, B, Dk);
     switch (state_dtype) {
         case DFLASH_F32: return launch_gdn_state<float>((hipStream_t)stream, A, B, g_ndim, Dk);
         case DFLASH_BF16: return launch_gdn_state<bf16_t>((hipStream_t)stream, A, B, g_ndim, Dk);

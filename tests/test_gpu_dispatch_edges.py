@@ -343,3 +343,79 @@ def test_tile_with_only_a_nan_score_is_not_hidden(gpu_lib):
     k[:, :, 32] = float("nan")                                # seen by the last row alone
     nan = torch.isnan(K.batched_sdpa_2pass(q, k, v, 0.1))
     assert nan[:, :, 15].all() and not nan[:, :, :15].any()
+
+
+# GatedDelta forward with one decay per channel, chunk by chunk: 2 to 6 chunks, whole and ragged last ones, several row tiles; decays of
+# zero, of one and below zero among them.  The same steps in calls of 16, which the step kernel takes, are held to the same bounds.
+@pytest.mark.parametrize("Dk,Dv,dt", [(64, 16, "bf16"), (128, 48, "bf16"), (128, 16, "f16"), (64, 32, "f16")], ids=lambda v: str(v))
+@pytest.mark.parametrize("T", [24, 31, 32, 33, 49, 87])
+@pytest.mark.parametrize("masked", [False, True])
+def test_channel_gate_chunks(gpu_lib, Dk, Dv, dt, T, masked):
+    from swiftlm_amd import DFlashKernels as K
+
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16}[dt]
+    d = O.make_gdn_inputs(Dk + Dv + T, 2, T, 2, 4, Dk, Dv, in_dtype=dt, vec_gate=True)
+    d["g"][:, 5::7, :, ::3] = 0.0
+    d["g"][:, 3::5, :, 1::4] = 1.0
+    d["g"][:, 4::6, :, 2::5] = -0.5
+    mask = None
+    if masked:
+        mask = np.ones((2, T), np.float32)
+        mask[0, 2:5] = 0
+        mask[0, 15:18] = 0
+        mask[1, T - 5:] = 0
+    ins = [dev(d[n], tdt) for n in ("q", "k", "v", "g", "beta")]
+    dmask = None if mask is None else dev(mask)
+    yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], mask, dtype=np.float64)
+
+    def run(steps):
+        state, parts = dev(d["state"]), []
+        for t in range(0, T, steps):
+            y, state, tape = K.gated_delta_kernel_with_tape(*[x[:, t:t + steps].contiguous() for x in ins], state,
+                                                            None if mask is None else dmask[:, t:t + steps].contiguous())
+            parts.append((y, tape))
+        return torch.cat([p[0] for p in parts], 1), state, torch.cat([p[1] for p in parts], 1)
+
+    for steps in (T, 16):
+        y, s, tape = run(steps)
+        np.testing.assert_allclose(host(s), sw, rtol=1e-4, atol=1e-6)
+        np.testing.assert_allclose(host(tape), tw, rtol=1e-4, atol=1e-5)
+        np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
+        if masked:
+            off = mask < 0.5
+            assert np.all(host(y)[off] == 0) and np.all(host(tape)[off] == 0)
+
+
+# An infinity or NaN of one step stays out of the steps before it (products over all steps of a chunk would spread it), of the other state
+# rows and, where the step is masked, out of everything
+@pytest.mark.parametrize("what", ["v", "beta", "k_masked", "state"])
+def test_channel_gate_not_finite(gpu_lib, what):
+    from swiftlm_amd import DFlashKernels as K
+
+    T, t, Dk, Dv = 40, 21, 64, 16
+    d = O.make_gdn_inputs(5, 1, T, 1, 2, Dk, Dv, in_dtype="bf16", vec_gate=True)
+    mask = np.ones((1, T), np.float32)
+    clean = {n: a.copy() for n, a in d.items()}
+    if what == "v":
+        d["v"][0, t, 1, 3] = np.inf
+    elif what == "beta":
+        d["beta"][0, t, 1] = np.nan
+    elif what == "k_masked":
+        d["k"][0, t] = np.inf
+        mask[0, t] = 0
+    else:
+        d["state"][0, 1, 3, 7] = np.nan
+    run = lambda x: [host(a) for a in K.gated_delta_kernel_with_tape(*[dev(x[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")], dev(x["state"]),
+                                                                     dev(mask))]
+    y, s, tape = run(d)
+    yc, sc, tc = run(clean)
+    bad = np.zeros((1, T, 2, Dv), bool)
+    rows = slice(None) if what == "beta" else slice(3, 4)
+    if what != "k_masked":
+        bad[0, 0 if what == "state" else t:, 1, rows] = True
+    for got, want in ((y, yc), (tape, tc)):
+        np.testing.assert_allclose(got[~bad], want[~bad], rtol=1e-4 if got is tape else 2e-2, atol=1e-5 if got is tape else 2e-2)
+        assert not np.isfinite(got[bad]).any()
+    hit = bad[0, -1]                                   # [Hv, Dv]
+    np.testing.assert_allclose(s[0][~hit], sc[0][~hit], rtol=1e-4, atol=1e-6)
+    assert not np.isfinite(s[0][hit]).any()
