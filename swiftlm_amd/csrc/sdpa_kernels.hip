@@ -850,12 +850,12 @@ __device__ __forceinline__ RowParts row_parts(const CombineArgs& A, int row, int
     return {A.part_m + stat, A.part_l + stat, A.part_o + ((size_t)first * A.hqm + r) * D, __builtin_amdgcn_readfirstlane(share_s[1]), (size_t)A.hqm * D};
 }
 
-// One workgroup per row, for many splits: up to 16 partial rows per thread, all in flight at once.
-template <typename Tag, int D>
+// One workgroup per row, for many splits: UNROLL partial rows per thread, all in flight at once (one round trip for
+// S <= UNROLL * NG).
+template <typename Tag, int D, int UNROLL>
 __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineArgs A) {
     constexpr int TPG = D / 8;                     // threads spanning one row, 8 elements (16 B) each
     constexpr int NG = kCombineThreads / TPG;         // split groups walking the partials in parallel
-    constexpr int UNROLL = 16;                     // row loads in flight per thread: one round trip for S <= 16 * NG
     __shared__ float w_s[kMaxSplits];
     __shared__ float redm_s[kCombineThreads / 64], reds_s[kCombineThreads / 64];
     __shared__ float acc_s[NG][D];
@@ -1075,7 +1075,16 @@ static int launch_combine(hipStream_t st, const CombineArgs& C) {
     auto one_wave = [&]() { return D == 128 ? C.S <= (C.balance ? 32 : 64) : C.S <= 32 && C.rows > 4 * num_compute_units(); };
     if (C.S <= 4 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 4>, waves, threads, 0, C));
     else if (one_wave()) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
-    else DFLASH_HIP_TRY(br.launch(sdpa_combine_kernel<Tag, D>, dim3(C.rows), threads, 0, C));
+    else {
+        // As many partial rows in flight per thread as there are to take, as a row that is asked for and dropped costs its load
+        // (16 for any count, before: 64 query heads of D = 256, 4,112 keys, 26 splits 20.1 us, now 18.0; 16 heads, 6,000 keys, 64
+        // splits 16.0 and 14.7).  A dealt launch has sequences of more than S.
+        const int each = C.balance ? 16 : (C.S + 4 * groups - 1) / (4 * groups);
+        auto kern = each <= 8 ? sdpa_combine_kernel<Tag, D, 8> : each <= 12 ? sdpa_combine_kernel<Tag, D, 12> : sdpa_combine_kernel<Tag, D, 16>;
+        if constexpr (D == 256)                        // (D = 128 takes the wave form there)
+            if (each <= 4) kern = sdpa_combine_kernel<Tag, D, 4>;
+        DFLASH_HIP_TRY(br.launch(kern, dim3(C.rows), threads, 0, C));
+    }
     return DFLASH_OK;
 }
 

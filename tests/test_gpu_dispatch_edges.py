@@ -117,6 +117,14 @@ def test_attention_split_counts(gpu_lib, N, Hq, Hk, D):
     attend(*tensors(N + D, 1, Hq, Hk, N, D), [N], D)
 
 
+# a workgroup per row has as many partial rows in flight per thread as the splits ask for: 4, 8, 12, 16 (above up to 65 splits at D = 256)
+@pytest.mark.parametrize("D,N,S", [(256, 3072, 96), (256, 3104, 97), (256, 4096, 128), (256, 40000, 209), (128, 2080, 65), (128, 4096, 128), (128, 5000, 157),
+                                   (128, 33000, 172), (128, 65568, 256)])
+def test_combine_rows_in_flight(gpu_lib, D, N, S):
+    assert splits(1, 3, 1, N, D) == S
+    attend(*tensors(N + D, 1, 3, 1, N, D), [N], D)
+
+
 # Short contexts in one launch, up to a line of keys that depends on the query heads (B * Hq), then a few splits of the same form, then
 # the form with shared tiles, which more heads than compute units take at once.  Tiles of 32 (D = 128) and 16 keys, eight waves, one
 # tile a wave and more; the second sequence leaves splits without a tile; 12 heads whose splits are rounded to whole XCDs.
