@@ -609,6 +609,59 @@ PyObject* restore(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- the calls of a verify step on buffers that are there already, on a given stream ---------
+
+void* handle_of(PyObject* o) {
+    void* p = PyLong_AsVoidPtr(o);
+    if (!p && PyErr_Occurred()) throw python_error();
+    return p;
+}
+// (stream, q, k, v, g, beta, state_in, state_out or None, y, tape, Hk, Hv, Dk, Dv): one sequence, one decay per head and step
+PyObject* gated_delta_into(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 14, "gated_delta_into");
+    void* st = handle_of(a[0]);
+    const at::Tensor &q = tensor(a[1], "q"), &k = tensor(a[2], "k"), &v = tensor(a[3], "v"), &g = tensor(a[4], "g"), &beta = tensor(a[5], "beta"),
+                     &in = tensor(a[6], "state_in"), &out = tensor_or_none(a[7], "state_out"), &y = tensor(a[8], "y"), &tape = tensor(a[9], "tape");
+    need_rank(k, 4, "gated_delta_into", "k");
+    const int qc = code(q), sc = code(in), T = (int)k.size(1), Hk = (int)integer(a[10]), Hv = (int)integer(a[11]), Dk = (int)integer(a[12]),
+              Dv = (int)integer(a[13]);
+    check(enqueue([&] {
+              return dflash_gated_delta_tape(st, ptr(q), ptr(k), ptr(v), ptr(g), 3, ptr(beta), qc, ptr(in), ptr(out), sc, ptr(y), (float*)ptr(tape),
+                                             nullptr, 0, 1, T, Hk, Hv, Dk, Dv);
+          }),
+          "gated_delta_tape");
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+// (stream, q, k, v, k_new, v_new, out, lse, scale, n_keys, length, workspace, page_table or None, page_size): one sequence; k, v the caches
+// [1, Hk, rows, D] or, with a page table [1, pages], the pools [pages, Hk, page_size, D]
+PyObject* sdpa_append_into(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need_args(n, 14, "sdpa_append_into");
+    void* st = handle_of(a[0]);
+    const at::Tensor &q = tensor(a[1], "q"), &k = tensor(a[2], "k"), &v = tensor(a[3], "v"), &kn = tensor(a[4], "k_new"), &vn = tensor(a[5], "v_new"),
+                     &out = tensor(a[6], "out"), &lse = tensor(a[7], "lse"), &len = tensor(a[10], "length"), &ws = tensor(a[11], "workspace"),
+                     &table = tensor_or_none(a[12], "page_table");
+    need_rank(q, 4, "sdpa_append_into", "q");
+    need_rank(k, 4, "sdpa_append_into", "k");
+    const float scale = number(a[8]);
+    const int N = (int)integer(a[9]), page = (int)integer(a[13]), Hq = (int)q.size(1), M = (int)q.size(2), D = (int)q.size(3), Hk = (int)k.size(1);
+    const int dt = code(q);
+    if (table.defined()) need_rank(table, 2, "sdpa_append_into", "page_table");
+    check(enqueue([&] {
+              return table.defined()
+                         ? dflash_sdpa_block_causal_paged(st, ptr(q), ptr(k), ptr(v), (const int32_t*)ptr(table), (int)table.size(1), page, (int)k.size(0),
+                                                          k.stride(0), k.stride(1), ptr(kn), ptr(vn), ptr(out), (float*)ptr(lse), dt, scale, 1, Hq, Hk, M, N, D,
+                                                          (const int32_t*)ptr(len), ptr(ws), (size_t)ws.numel())
+                         : dflash_sdpa_block_causal_append(st, ptr(q), ptr(k), ptr(v), ptr(kn), ptr(vn), ptr(out), (float*)ptr(lse), dt, scale, 1, Hq, Hk, M, N,
+                                                           D, k.stride(0), k.stride(1), (const int32_t*)ptr(len), ptr(ws), (size_t)ws.numel());
+          }),
+          table.defined() ? "sdpa_block_causal_paged" : "sdpa_block_causal");
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
 // () -> the current stream's handle
 PyObject* current_stream(PyObject*, PyObject* const*, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -634,6 +687,7 @@ PyMethodDef methods[] = {
     FAST("set_errors", set_errors), FAST("tape_replay", tape_replay), FAST("gated_delta", gated_delta),
     FAST("gdn_layer", gdn_layer),   FAST("sdpa", sdpa),               FAST("sdpa_append", sdpa_append),
     FAST("sdpa_paged", sdpa_paged), FAST("current_stream", current_stream),
+    FAST("gated_delta_into", gated_delta_into), FAST("sdpa_append_into", sdpa_append_into),
     FAST("greedy_accept", greedy_accept), FAST("accept_commit", accept_commit), FAST("cache_set_slot", cache_set_slot),
     FAST("cache_get_slot", cache_get_slot), FAST("cache_record_tape", cache_record_tape), FAST("cache_is_armed", cache_is_armed), FAST("cache_arm", cache_arm), FAST("restore", restore),
     {nullptr, nullptr, 0, nullptr},

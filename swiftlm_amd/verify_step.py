@@ -29,6 +29,7 @@ from typing import List, Optional
 import torch
 
 from . import _lib
+from ._lib import native
 
 
 @dataclass
@@ -117,6 +118,7 @@ class HybridVerifyStack:
                         layer[name] = pool
                     del layer["k_cache"], layer["v_cache"]
                 self.attn.append(layer)
+        self._kinds = cfg.kinds()
         self.scale = 1.0 / (cfg.D ** 0.5)
         n_max = cfg.capacity
         ws = int(self.lib.dflash_sdpa_workspace_bytes(1, cfg.Hq, cfg.Hkv, T, n_max, cfg.D))
@@ -137,7 +139,7 @@ class HybridVerifyStack:
         # host pointer tables for the batched replay, one per phase
         self._tables = []
         for ph in (0, 1):
-            mk = lambda ts: (C.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+            mk = lambda ts: C.cast((C.c_void_p * len(ts))(*[t.data_ptr() for t in ts]), _lib.vpp)
             self._tables.append(dict(
                 tape=mk([l["tape"] for l in self.gdn]), k=mk([l["k"] for l in self.gdn]),
                 g=mk([l["g"] for l in self.gdn]), sin=mk([l["state"][ph] for l in self.gdn]),
@@ -150,38 +152,25 @@ class HybridVerifyStack:
         ``slot``: which row of ``accept_inputs`` holds this step's token ids (default: the phase)."""
         cfg, lib, T = self.cfg, self.lib, self.cfg.block
         note = before_launch or (lambda name: None)
-        st = C.c_void_p(torch.cuda.current_stream().cuda_stream if stream is None else stream)
+        st_int = native.current_stream() if stream is None else stream
+        st = C.c_void_p(st_int)
         ph = self.phase
         slot = ph if slot is None else slot
         gi = ai = 0
-        for kind in cfg.kinds():
+        for kind in self._kinds:
             if kind == "gdn":
                 l = self.gdn[gi]; gi += 1
                 note("gdn_forward")
-                rc = lib.dflash_gated_delta_tape(
-                    st, _p(l["q"]), _p(l["k"]), _p(l["v"]), _p(l["g"]), 3, _p(l["beta"]), _lib.BF16,
-                    _p(l["state"][ph]), _p(l["state"][1 - ph]) if self.post_block_state else None, _lib.F32, _p(l["y"]),
-                    _p(l["tape"]), None, 0, 1, T, cfg.Hk, cfg.Hv, cfg.Dk, cfg.Dv)
-                _lib.check(rc, "gated_delta_tape")
+                native.gated_delta_into(st_int, l["q"], l["k"], l["v"], l["g"], l["beta"], l["state"][ph],
+                                        l["state"][1 - ph] if self.post_block_state else None, l["y"], l["tape"],
+                                        cfg.Hk, cfg.Hv, cfg.Dk, cfg.Dv)
             else:
                 l = self.attn[ai]; ai += 1
-                hs = cfg.capacity * cfg.D
                 note("sdpa")
-                if cfg.page_size:
-                    kp = l["k_pool"]
-                    rc = lib.dflash_sdpa_block_causal_paged(
-                        st, _p(l["q"]), _p(kp), _p(l["v_pool"]), _p(l["page_table"]), l["page_table"].shape[1], cfg.page_size,
-                        kp.shape[0], kp.stride(0), kp.stride(1), _p(l["k_new"]), _p(l["v_new"]), _p(l["out"]), _p(l["lse"]),
-                        _lib.BF16, self.scale, 1, cfg.Hq, cfg.Hkv, T, self.n_max, cfg.D, _p(self.offset), _p(self.workspace),
-                        self.workspace.numel())
-                    _lib.check(rc, "sdpa_block_causal_paged")
-                    continue
-                rc = lib.dflash_sdpa_block_causal_append(
-                    st, _p(l["q"]), _p(l["k_cache"]), _p(l["v_cache"]), _p(l["k_new"]), _p(l["v_new"]), _p(l["out"]),
-                    _p(l["lse"]), _lib.BF16, self.scale, 1, cfg.Hq, cfg.Hkv, T, self.n_max, cfg.D, cfg.Hkv * hs, hs,
-                    _p(self.offset), _p(self.workspace), self.workspace.numel())
-                _lib.check(rc, "sdpa_block_causal")
-        cast = lambda a: C.cast(a, _lib.vpp)
+                paged = "page_table" in l
+                native.sdpa_append_into(st_int, l["q"], l["k_pool" if paged else "k_cache"], l["v_pool" if paged else "v_cache"],
+                                        l["k_new"], l["v_new"], l["out"], l["lse"], self.scale, self.n_max, self.offset,
+                                        self.workspace, l["page_table"] if paged else None, cfg.page_size)
         if self.gdn and self.fuse_accept:
             # acceptance + rollback of every GatedDelta layer in ONE launch: the replay kernel counts the
             # leading matches itself, writes accept[0..3] and advances the offset
@@ -189,8 +178,8 @@ class HybridVerifyStack:
             note("tape_replay")
             rc = lib.dflash_accept_commit_replay_batched(
                 st, _p(self.verify_ids[slot]), _p(self.posterior[slot]), T, _p(self.offset), _p(self.accept),
-                len(self.gdn), cast(tb["tape"]), _lib.F32, cast(tb["k"]), cast(tb["g"]), _lib.BF16, 3,
-                cast(tb["sin"]), cast(tb["sout"]), _lib.F32, 1 if self.post_block_state else 0, 1, T, cfg.Hk, cfg.Hv,
+                len(self.gdn), tb["tape"], _lib.F32, tb["k"], tb["g"], _lib.BF16, 3,
+                tb["sin"], tb["sout"], _lib.F32, 1 if self.post_block_state else 0, 1, T, cfg.Hk, cfg.Hv,
                 cfg.Dk, cfg.Dv)
             _lib.check(rc, "accept_commit_replay_batched")
             self.phase = 1 - ph
@@ -204,8 +193,8 @@ class HybridVerifyStack:
             tb = self._tables[ph]
             note("tape_replay")
             rc = lib.dflash_tape_replay_batched(
-                st, len(self.gdn), cast(tb["tape"]), _lib.F32, cast(tb["k"]), cast(tb["g"]), _lib.BF16, 3,
-                cast(tb["sin"]), cast(tb["sout"]), _lib.F32, 0, C.c_void_p(self.accept.data_ptr() + 4),
+                st, len(self.gdn), tb["tape"], _lib.F32, tb["k"], tb["g"], _lib.BF16, 3,
+                tb["sin"], tb["sout"], _lib.F32, 0, C.c_void_p(self.accept.data_ptr() + 4),
                 1 if self.post_block_state else 0, 1, T, cfg.Hk, cfg.Hv, cfg.Dk, cfg.Dv)
             _lib.check(rc, "tape_replay_batched")
         self.phase = 1 - ph
@@ -216,12 +205,14 @@ class HybridVerifyStack:
         the shapes the library's host code picks for this configuration (csrc: launch_gdn_chunk, launch_sdpa,
         launch_replay_nr), for pricing a step's launches with empty kernels of the same shapes.  Only the
         benchmark's kernel choices are covered (chunked GatedDelta forward, dense or paged attention with at
-        most 8 query heads per KV head, 4 state rows per replay thread)."""
+        most 8 query heads per KV head over a context too long for a workgroup per query head, 4 state rows per replay
+        thread)."""
         cfg, T = self.cfg, self.cfg.block
+        assert not self.attn or cfg.Hkv * self.n_max * cfg.D > 12_000_000
         assert cfg.Dk in (64, 128, 256) and cfg.Dv % 16 == 0 and cfg.Hq // cfg.Hkv <= 8 and cfg.D in (128, 256)
         ld = cfg.Dk + 4
-        gdn_lds = (4 * (2 * 32 * ld + 16 * 33 + 2 * 16 * 16 + 16 * 17 + 16 * 16 + 4 * 16 + 16)   # fp32 operands and tables
-                   + 2 * 5 * 16 * (cfg.Dk + 8))                                                    # bf16 operands
+        gdn_lds = (4 * (16 * ld + 4 + 16 * 33 + 2 * 16 * 16 + 16 * 17 + 16 * 16 + 4 * 16 + 16)   # fp32 operands and tables
+                   + 2 * 5 * 16 * (cfg.Dk + 8) + 8)                                               # bf16 operands
         gdn = (cfg.Dv // 16, cfg.Hv, 1, 256, gdn_lds)
         # splits: the S whose workspace layout gives the size the library reports
         rows = cfg.Hq * T
