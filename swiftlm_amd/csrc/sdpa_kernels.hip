@@ -1078,11 +1078,13 @@ static int launch_combine(hipStream_t st, const CombineArgs& C) {
     else {
         // As many partial rows in flight per thread as there are to take, as a row that is asked for and dropped costs its load
         // (16 for any count, before: 64 query heads of D = 256, 4,112 keys, 26 splits 20.1 us, now 18.0; 16 heads, 6,000 keys, 64
-        // splits 16.0 and 14.7).  A dealt launch has sequences of more than S.
-        const int each = C.balance ? 16 : (C.S + 4 * groups - 1) / (4 * groups);
+        // splits 16.0 and 14.7).  A dealt launch has sequences of more than S: eight at least, and theirs take another round (16, 8 and 4
+        // in flight, four sequences of up to 20,000 keys 33.4, 31.9, 31.8 us; eight paged ones, appended to, 45.9, 44.4, 44.0; two of up
+        // to 50,000 42.0, 41.4, 41.5).
+        const int each = (C.S + 4 * groups - 1) / (4 * groups);
         auto kern = each <= 8 ? sdpa_combine_kernel<Tag, D, 8> : each <= 12 ? sdpa_combine_kernel<Tag, D, 12> : sdpa_combine_kernel<Tag, D, 16>;
         if constexpr (D == 256)                        // (D = 128 takes the wave form there)
-            if (each <= 4) kern = sdpa_combine_kernel<Tag, D, 4>;
+            if (each <= 4 && !C.balance) kern = sdpa_combine_kernel<Tag, D, 4>;
         DFLASH_HIP_TRY(br.launch(kern, dim3(C.rows), threads, 0, C));
     }
     return DFLASH_OK;
