@@ -42,8 +42,7 @@ template <int DK> struct GdnLongLds {
     static constexpr int LB = DK + 8;      // row pitch: 16 bytes of pad spread 16-byte reads of a column of rows over the banks
     // Every array is read at most one barrier after the interval that follows its writing, so two sets (the chunk's parity) do.
     // k and q rows; inside each 32 channels position 8g + 4h + x holds channel 16h + 4g + x (what one lane of the product takes)
-    uint16_t k[2][16][LB], q[2][16][LB];
-    uint16_t kt[2][DK][16];                // k transposed: steps of a channel
+    uint16_t k[4][16][LB], q[2][16][LB];   // (k is read again by the update, two intervals after it is written)
     float na[2][16][16];                   // na[t][s] = -beta_t G[s][t] k_s.k_t for s < t, else 0
     float t2[2][64][4];                    // lane (g, n): T[t = n][s = 4g + i]
     float v[2][64][4];                     // lane (g, n): v_s of row n, s = 4g + i
@@ -147,10 +146,14 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             const Rows qrow = rows(L.q[par]);
             const f32x4v wv = lds4(&L.w[par][4 * g]);
             const float gam_end = L.gam[par][kChunkSteps - 1];
-            uint2 kt[NB];
+            uint2 kt[NB];                              // four steps of a channel: transposing reads of the rows
 #pragma unroll
-            for (int i = 0; i < NB; ++i) kt[i] = *reinterpret_cast<const uint2*>(&L.kt[par][cb + 16 * i + n][4 * g]);
-            const Rows krow = rows(L.k[par ^ 1]);      // of the next chunk (behind the last one: not used)
+            for (int i = 0; i < NB; ++i) {
+                const int ch = cb + 16 * i, pos = (ch & ~31) + 8 * (n % 4) + 4 * ((ch / 16) & 1);      // of channels ch + 4 (n % 4) .. + 3
+                kt[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                      (__attribute__((address_space(3))) s16x4v*)(&L.k[m & 3][4 * g + n / 4][pos])));
+            }
+            const Rows krow = rows(L.k[(m + 1) & 3]);    // of the next chunk (behind the last one: not used)
             // S_0 q_t, from the split state of before the update
             const f32x4v pq = product(qrow);
             // A product with T mixes all steps of a row: an infinity or NaN would reach the steps before it (0 * inf), and T may
@@ -244,32 +247,8 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
                 A.tape[o + v * step] = dl[v];
             }
     };
-    // k of chunk m transposed, two neighbouring channels per lane
-    auto transpose_k = [&](int par) {
-#pragma unroll
-        for (int c0 = 0; c0 < DK; c0 += 128) {
-            const int pos = c0 + 2 * lane;
-            if (DK >= 128 || lane < DK / 2) {
-                const int ch = (pos & ~31) + 16 * ((pos / 4) & 1) + 4 * ((pos % 32) / 8) + pos % 4;
-                uint32_t x[16], even[8], odd[8];
-#pragma unroll
-                for (int t = 0; t < 16; ++t) x[t] = *reinterpret_cast<const uint32_t*>(&L.k[par][t][pos]);
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    even[t] = __builtin_amdgcn_perm(x[2 * t + 1], x[2 * t], 0x05040100u);
-                    odd[t] = upper_halves(x[2 * t], x[2 * t + 1]);
-                }
-                uint4* d = reinterpret_cast<uint4*>(L.kt[par][ch]);
-                d[0] = make_uint4(even[0], even[1], even[2], even[3]);
-                d[1] = make_uint4(even[4], even[5], even[6], even[7]);
-                d[2] = make_uint4(odd[0], odd[1], odd[2], odd[3]);
-                d[3] = make_uint4(odd[4], odd[5], odd[6], odd[7]);
-            }
-        }
-    };
     if (p < chunks) request(p);
     for (int j = 0; j < p; ++j) {                      // intervals -2 .. p - 3
-        if (j == 1 && p == 3) transpose_k(0);
         lds_barrier();
     }
     for (int m = p; m < chunks; m += 4) {
@@ -287,7 +266,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             }
 #pragma unroll
             for (int j = 0; j < NK; ++j) {
-                park(L.k[par][n], j, kr[j]);
+                park(L.k[m & 3][n], j, kr[j]);
                 const bf16x8v k8 = __builtin_bit_cast(bf16x8v, kr[j]);
                 kk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, k8, kk, 0, 0, 0);
                 kq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, __builtin_bit_cast(bf16x8v, qr[j]), kq, 0, 0, 0);
@@ -354,7 +333,6 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
         // the wait for the loads would include stores behind them (where loops join, the count is not exact).
         if (m > p) store_rows(m - 4, kChunkSteps);
         if (m + 4 < chunks) request(m + 4);
-        if (m + 1 < chunks) transpose_k(par ^ 1);
         lds_barrier();
         {   // interval m + 1: read-out and tape, rows t = 4g + v, column = state row n
             const f32x4v pq = (lds4(L.pq[par][0][lane]) + lds4(L.pq[par][1][lane])) + (lds4(L.pq[par][2][lane]) + lds4(L.pq[par][3][lane]));
