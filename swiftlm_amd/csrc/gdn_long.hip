@@ -2,6 +2,8 @@
 //
 // Semantics follow Sources/DFlash/DFlashKernels.swift:122-199 (Metal kernel) and :409-466 (ops restatement).
 
+#include <type_traits>
+
 #include "gdn_common.h"
 
 namespace dflash {
@@ -19,20 +21,24 @@ namespace dflash {
 //                         registers.  Chunk m: add the four partial S_0 k_t, delta = T (v - gam S_0 k_t), update, split
 //                         the new state into three bf16 terms, partial S_0 k_t of chunk m+1 into LDS, barrier.
 //   waves 4-7 (producers) wave 4+p prepares chunks p, p+4, ...: interval m-2 k rows, k_s.k_t, k_s.q_t, decays; interval
-//                         m-1 T = (I + diag(beta) A)^-1 diag(beta) by substitution; interval m the loads of chunk m+4 and
-//                         k of chunk m+1 transposed; interval m+1 y and the tape of the chunk.
+//                         m-1 T = (I + diag(beta) A)^-1 diag(beta) by substitution; interval m the loads of chunk m+4;
+//                         interval m+1 y and the tape of the chunk.
 //
 // One barrier per chunk, no wave waits for memory inside a chunk (loads are asked for two chunks ahead of their use), and
 // no operand crosses lanes: with S^T as the accumulator a lane holds row l%16 and channels 4*(l/16)+v, which is also how
 // the next product's b operand may be laid out, as the order of a contraction's indices is free.
 //
-// Bound by the length of an interval: 1,400 / 1,600 / 2,200 cycles at Dk = 64 / 128 / 256, of which the chain works 1,200 /
-// 1,400 / 1,900 (the split of the state on the VALU, the exchange of the partial sums through LDS, three groups of
-// dependent MFMAs) and the busiest producer about as long.  us, chunk by chunk kernel against this one: 1,003 steps,
-// 32 heads of 128x128 152 -> 44; 730 steps, 8 heads, Dk = 256 147 -> 45; two sequences of 1,000 steps, 32 heads, Dk = 256
-// 419 -> 123; 40 steps 8.3 -> 5.7.
-// 106 / 122 / 160 registers: two workgroups share a compute unit at Dk = 64 and 128 (two sequences of 1,000 steps 75 where one takes
-// 44), at 256 a second sequence waits for the first (62 for one).
+// Loads and stores go by whole rows, four neighbouring lanes to 64 bytes: a wave is held until the memory pipeline takes a load,
+// and with a row per lane, or two bytes per lane, every lane is a request (22 instructions of up to 64 requests per chunk; now
+// 13).  So the products' operands, v and the tape change lanes through LDS, and k is transposed by the LDS as the update reads it.
+//
+// Bound by the length of an interval: 1,350 / 1,600 / 2,200 cycles at Dk = 64 / 128 / 256, of which the chain works 1,200 /
+// 1,350 / 1,800 (the split of the state on the VALU, the exchange of the partial sums through LDS, three groups of
+// dependent MFMAs) and the busiest producer as long.  us, chunk by chunk kernel against this one: 1,003 steps,
+// 32 heads of 128x128 152 -> 43; 730 steps, 8 heads, Dk = 256 147 -> 43; two sequences of 1,000 steps, 32 heads, Dk = 256
+// 419 -> 116; 40 steps 8.3 -> 5.4.
+// 89 / 106 / 145 registers: two workgroups share a compute unit at Dk = 64 and 128 (two sequences of 1,000 steps 71 where one takes
+// 43), at 256 a second sequence waits for the first (59 for one).
 // ---------------------------------------------------------------------------
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));
@@ -42,7 +48,8 @@ template <int DK> struct GdnLongLds {
     static constexpr int LB = DK + 8;      // row pitch: 16 bytes of pad spread 16-byte reads of a column of rows over the banks
     // Every array is read at most one barrier after the interval that follows its writing, so two sets (the chunk's parity) do.
     // k and q rows; inside each 32 channels position 8g + 4h + x holds channel 16h + 4g + x (what one lane of the product takes)
-    uint16_t k[4][16][LB], q[2][16][LB];   // (k is read again by the update, two intervals after it is written)
+    // (written two intervals before the chunk's own, where q and, by the update, k are read)
+    uint16_t k[4][16][LB], q[4][16][LB];
     float na[2][16][16];                   // na[t][s] = -beta_t G[s][t] k_s.k_t for s < t, else 0
     float t2[2][64][4];                    // lane (g, n): T[t = n][s = 4g + i]
     float v[2][64][4];                     // lane (g, n): v_s of row n, s = 4g + i
@@ -105,20 +112,28 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             }
             return r;
         };
-        auto product = [&](const Rows r) -> f32x4v {
+        auto product = [&](const Rows r, auto state_first) __attribute__((always_inline)) -> f32x4v {
             f32x4v acc = {0.f, 0.f, 0.f, 0.f};
+            auto mul32 = [&](bf16x8v x, bf16x8v st, f32x4v a) -> f32x4v {
+                if constexpr (state_first) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(st, x, a, 0, 0, 0);
+                else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, st, a, 0, 0, 0);
+            };
+            auto mul16 = [&](s16x4v x, s16x4v st, f32x4v a) -> f32x4v {
+                if constexpr (state_first) return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(st, x, a, 0, 0, 0);
+                else return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, st, a, 0, 0, 0);
+            };
             if constexpr (NB == 1) {
                 const s16x4v xv = __builtin_bit_cast(s16x4v, r);
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xv, as_s16x4(lo[0]), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xv, as_s16x4(mid[0]), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xv, as_s16x4(hi[0]), acc, 0, 0, 0);
+                acc = mul16(xv, as_s16x4(lo[0]), acc);
+                acc = mul16(xv, as_s16x4(mid[0]), acc);
+                acc = mul16(xv, as_s16x4(hi[0]), acc);
             } else {
 #pragma unroll
                 for (int j = 0; j < NB / 2; ++j) {
                     const bf16x8v xv = __builtin_bit_cast(bf16x8v, u32x4v{r[4 * j], r[4 * j + 1], r[4 * j + 2], r[4 * j + 3]});
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, as_bf16x8(lo[2 * j], lo[2 * j + 1]), acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, as_bf16x8(mid[2 * j], mid[2 * j + 1]), acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, as_bf16x8(hi[2 * j], hi[2 * j + 1]), acc, 0, 0, 0);
+                    acc = mul32(xv, as_bf16x8(lo[2 * j], lo[2 * j + 1]), acc);
+                    acc = mul32(xv, as_bf16x8(mid[2 * j], mid[2 * j + 1]), acc);
+                    acc = mul32(xv, as_bf16x8(hi[2 * j], hi[2 * j + 1]), acc);
                 }
             }
             return acc;
@@ -127,7 +142,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
         lds_barrier();                                 // interval -2
 #pragma unroll
         for (int i = 0; i < NB; ++i) split3_bf16(s[i], hi[i], mid[i], lo[i]);
-        f32x4v own = product(rows(L.k[0]));
+        f32x4v own = product(rows(L.k[0]), std::false_type{});
         *reinterpret_cast<f32x4v*>(L.pk[0][w][lane]) = own;
         lds_barrier();                                 // interval -1
 
@@ -143,7 +158,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
 #pragma unroll
             for (int i = 0; i < 4; ++i) dl = __builtin_amdgcn_mfma_f32_16x16x4f32(t2[i], rhs[i], dl, 0, 0, 0);
             // the other reads, while the matrix pipe is on T
-            const Rows qrow = rows(L.q[par]);
+            const Rows qrow = rows(L.q[m & 3]);
             const f32x4v wv = lds4(&L.w[par][4 * g]);
             const float gam_end = L.gam[par][kChunkSteps - 1];
             uint2 kt[NB];                              // four steps of a channel: transposing reads of the rows
@@ -155,7 +170,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             }
             const Rows krow = rows(L.k[(m + 1) & 3]);    // of the next chunk (behind the last one: not used)
             // S_0 q_t, from the split state of before the update
-            const f32x4v pq = product(qrow);
+            const f32x4v pq = product(qrow, std::true_type{});
             // A product with T mixes all steps of a row: an infinity or NaN would reach the steps before it (0 * inf), and T may
             // overflow where no delta does.  Then the deltas are substituted for one step after the other.
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(dl[0]) + fabsf(dl[1]) + fabsf(dl[2]) + fabsf(dl[3]) < __builtin_inff())) != 0, 0)) {
@@ -187,7 +202,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             if (m + 1 < chunks) {
 #pragma unroll
                 for (int i = 0; i < NB; ++i) split3_bf16(s[i], hi[i], mid[i], lo[i]);
-                own = product(krow);
+                own = product(krow, std::false_type{});
                 *reinterpret_cast<f32x4v*>(L.pk[par ^ 1][w][lane]) = own;
             }
             lds_barrier();
@@ -208,44 +223,50 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
     const bf16_t* gp = reinterpret_cast<const bf16_t*>(A.g);
     const bf16_t* bp = reinterpret_cast<const bf16_t*>(A.beta);
     const uint32_t k_step = (uint32_t)A.Hk * DK, step = (uint32_t)A.Hv * A.Dv;           // elements per step, below 2^24
-    u32x4v kr[NK], qr[NK];                              // rows n of k and q, channels 32j + 8g .. +7: both operands of the products
-    bf16_t vr[4], gr, br;
+    // A load takes whole rows, 64 bytes by four neighbouring lanes (with a row per lane, as the products want them, every lane is a
+    // request of its own: a quarter of the rate, and the wave is held for it); the products' operands are read back from LDS.
+    constexpr int CPR = DK / 8, RPI = 64 / CPR;         // 16-byte pieces of a row; rows of a load
+    static_assert(16 / RPI == NK, "as many loads as steps of the contraction");
+    const int rs = lane / CPR, pc = lane % CPR;
+    u32x4v kr[NK], qr[NK];                              // row j * RPI + rs, channels 8 pc .. +7
+    uint2 vr;                                           // v of step n, rows 4g .. +3
+    bf16_t gr, br;
     auto request = [&](int m) {
         const int t0 = m * kChunkSteps, tc = min(A.T - t0, kChunkSteps);
         const uint32_t bt0 = (uint32_t)b * A.T + t0;                                   // uniform, as are the products with it
         const int tl = min(n, tc - 1);                 // clamped: always a valid address, selected away where it is used
-        const uint32_t o = (bt0 * A.Hk + hk) * DK + __umul24(tl, k_step) + 8 * g;
+        const uint32_t o = (bt0 * A.Hk + hk) * DK + 8 * pc;
 #pragma unroll
         for (int j = 0; j < NK; ++j) {
-            kr[j] = *reinterpret_cast<const u32x4v*>(kp + o + 32 * j);
-            qr[j] = *reinterpret_cast<const u32x4v*>(qp + o + 32 * j);
+            const uint32_t oj = o + __umul24(min(j * RPI + rs, tc - 1), k_step);
+            kr[j] = *reinterpret_cast<const u32x4v*>(kp + oj);
+            qr[j] = *reinterpret_cast<const u32x4v*>(qp + oj);
         }
-        const uint32_t vo = (bt0 * A.Hv + hv) * A.Dv + row0 + n;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vr[i] = vp[vo + __umul24(min(4 * g + i, tc - 1), step)];
+        vr = *reinterpret_cast<const uint2*>(vp + ((bt0 * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(tl, step)));
         const uint32_t go = bt0 * A.Hv + hv + __umul24(tl, A.Hv);
         gr = gp[go];
         br = bp[go];
     };
-    // a row's 8 channels 32j + 8g .. +7 at their positions
-    auto park = [&](uint16_t* row, int j, u32x4v x) {
-        uint16_t* d = row + 32 * j + 4 * (g / 2) + 16 * (g & 1);
+    // a row's channels 8 pc .. +7 at their positions
+    auto park = [&](uint16_t* row, u32x4v x) {
+        uint16_t* d = row + 32 * (pc / 4) + 4 * (pc % 4 / 2) + 16 * (pc & 1);
         *reinterpret_cast<uint2*>(d) = make_uint2(x[0], x[1]);
         *reinterpret_cast<uint2*>(d + 8) = make_uint2(x[2], x[3]);
     };
     const u32x4v none = {0u, 0u, 0u, 0u};
-    f32x4v av, cv, gam4;                               // of the chunk in hand: a and c columns, gam of steps 4g .. +3
-    float G[4], gam = 0.f, beta = 0.f;
-    f32x4v vf, yv, dl;                                 // v of the chunk in hand; y and tape of the one before, not yet stored
-    uint64_t on_bits = 0;
-    auto store_rows = [&](int m, int tc) {             // rows t = 4g + v, column = state row n
-        const uint32_t o = (((uint32_t)b * A.T + m * kChunkSteps) * A.Hv + hv) * A.Dv + row0 + n + __umul24(4 * g, step);
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (4 * g + v < tc) {
-                reinterpret_cast<bf16_t*>(A.y)[o + v * step] = from_float<bf16_t>(yv[v]);
-                A.tape[o + v * step] = dl[v];
-            }
+    f32x4v av, cv;                                     // of the chunk in hand: a and c columns
+    float G[4], gam = 0.f, gam_n = 0.f, beta = 0.f;   // gam_n: that of step n in every lane
+    f32x4v vf, yv, dl;                                 // v of the chunk in hand; y and tape of the one before, not yet stored: step n, rows 4g .. +3
+    bool step_on = false;
+    auto store_rows = [&](int m, int tc) {             // one store each: row by row, two and four bytes per lane, they were eight
+        const uint32_t o = (((uint32_t)b * A.T + m * kChunkSteps) * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(n, step);
+        if (n < tc) {
+            uint2 y2;
+            y2.x = (uint32_t)from_float<bf16_t>(yv[0]).bits | ((uint32_t)from_float<bf16_t>(yv[1]).bits << 16);
+            y2.y = (uint32_t)from_float<bf16_t>(yv[2]).bits | ((uint32_t)from_float<bf16_t>(yv[3]).bits << 16);
+            *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(A.y) + o) = y2;
+            *reinterpret_cast<f32x4v*>(A.tape + o) = dl;
+        }
     };
     if (p < chunks) request(p);
     for (int j = 0; j < p; ++j) {                      // intervals -2 .. p - 3
@@ -258,27 +279,31 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             if (tc < kChunkSteps) {                    // the last chunk's missing steps are zeros
 #pragma unroll
                 for (int j = 0; j < NK; ++j) {
-                    kr[j] = n < tc ? kr[j] : none;
-                    qr[j] = n < tc ? qr[j] : none;
+                    kr[j] = j * RPI + rs < tc ? kr[j] : none;
+                    qr[j] = j * RPI + rs < tc ? qr[j] : none;
                 }
-#pragma unroll
-                for (int v = 0; v < 4; ++v) vr[v].bits = 4 * g + v < tc ? vr[v].bits : 0;
+                vr = n < tc ? vr : make_uint2(0u, 0u);
             }
 #pragma unroll
             for (int j = 0; j < NK; ++j) {
-                park(L.k[m & 3][n], j, kr[j]);
-                const bf16x8v k8 = __builtin_bit_cast(bf16x8v, kr[j]);
+                park(L.k[m & 3][j * RPI + rs], kr[j]);
+                park(L.q[m & 3][j * RPI + rs], qr[j]);
+            }
+            asm volatile("" ::: "memory");             // LDS serves a wave's accesses in order: read back without a wait
+#pragma unroll
+            for (int j = 0; j < NK; ++j) {             // (in their order in LDS: the same channels of k and q)
+                const bf16x8v k8 = __builtin_bit_cast(bf16x8v, *reinterpret_cast<const u32x4v*>(&L.k[m & 3][n][32 * j + 8 * g]));
+                const bf16x8v q8 = __builtin_bit_cast(bf16x8v, *reinterpret_cast<const u32x4v*>(&L.q[m & 3][n][32 * j + 8 * g]));
                 kk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, k8, kk, 0, 0, 0);
-                kq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, __builtin_bit_cast(bf16x8v, qr[j]), kq, 0, 0, 0);
+                kq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, q8, kq, 0, 0, 0);
             }
             // decay products G[v] = g_{s+1} ... g_t of the lane's pairs (s, t) = (4g + v, n), 1 where s >= t
             bool on = n < tc;
             if (A.mask != nullptr) on = on && mask_on(A.mask, A.mask_dtype, (int)((uint32_t)b * A.T + t0 + min(n, tc - 1)));
             const float gl = on ? to_float(gr) : 1.f;
             beta = on ? to_float(br) : 0.f;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) vf[v] = to_float(vr[v]);
-            on_bits = __builtin_amdgcn_ballot_w64(on);
+            vf = f32x4v{__uint_as_float(vr.x << 16), __uint_as_float(vr.x & 0xffff0000u), __uint_as_float(vr.y << 16), __uint_as_float(vr.y & 0xffff0000u)};
+            step_on = on;
             // steps in blocks of four: pre = the product from the block's first step up to the lane's, block products by broadcast
             // (lane exchanges outside the selects: a select may become a branch, with the lanes that are read switched off)
             const float left1 = quad_take<0, 0, 1, 2>(gl);
@@ -308,6 +333,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             // T = (I + A)^-1 diag(beta), in the layout of the chain's a operand: lane (g, n) forms T[n][4g .. +3].  What other lanes
             // of this wave wrote is read back without a wait: LDS serves a wave's accesses in order.
             if (g == 0) { L.beta[par][n] = beta; L.gam[par][n] = gam; }
+            asm volatile("" ::: "memory");             // written by the lanes g = 0, read by all
             *reinterpret_cast<f32x4v*>(&L.na[par][n][4 * g]) = av;
             float na[16];                              // row n of -A, the four lanes' pieces gathered
             f32x4v x;
@@ -319,11 +345,10 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
                 na[4 + v] = __uint_as_float(o[0]); na[12 + v] = __uint_as_float(o[1]);
             }
             const f32x4v b4 = lds4(&L.beta[par][4 * g]);
-            gam4 = lds4(&L.gam[par][4 * g]);
-            *reinterpret_cast<f32x4v*>(L.v[par][lane]) = vf;
-            if (n == kChunkSteps - 1) *reinterpret_cast<float4*>(&L.w[par][4 * g]) = make_float4(G[0], G[1], G[2], G[3]);
+            gam_n = L.gam[par][n];
 #pragma unroll
-            for (int j = 0; j < NK; ++j) park(L.q[par][n], j, qr[j]);
+            for (int i = 0; i < 4; ++i) L.v[par][16 * (n / 4) + 4 * g + i][n % 4] = vf[i];
+            if (n == kChunkSteps - 1) *reinterpret_cast<float4*>(&L.w[par][4 * g]) = make_float4(G[0], G[1], G[2], G[3]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) x[e] = 4 * g + e == n ? 1.f : 0.f;
             *reinterpret_cast<f32x4v*>(L.t2[par][lane]) = unit_inverse(x, na) * b4;
@@ -334,14 +359,16 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
         if (m > p) store_rows(m - 4, kChunkSteps);
         if (m + 4 < chunks) request(m + 4);
         lds_barrier();
-        {   // interval m + 1: read-out and tape, rows t = 4g + v, column = state row n
+        {   // interval m + 1: read-out and tape, rows = state rows 4g + v, column = step n
             const f32x4v pq = (lds4(L.pq[par][0][lane]) + lds4(L.pq[par][1][lane])) + (lds4(L.pq[par][2][lane]) + lds4(L.pq[par][3][lane]));
-            dl = lds4(L.dl[par][lane]);
-            yv = gam4 * pq;
+            const f32x4v ds = lds4(L.dl[par][lane]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) yv = __builtin_amdgcn_mfma_f32_16x16x4f32(cv[e], dl[e], yv, 0, 0, 0);
+            for (int i = 0; i < 4; ++i) dl[i] = L.dl[par][16 * (n / 4) + 4 * g + i][n % 4];
+            yv = gam_n * pq;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) yv[v] = (on_bits >> (4 * g + v)) & 1 ? yv[v] : 0.f;
+            for (int e = 0; e < 4; ++e) yv = __builtin_amdgcn_mfma_f32_16x16x4f32(ds[e], cv[e], yv, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) yv[v] = step_on ? yv[v] : 0.f;
             if (m + 4 >= chunks) store_rows(m, tc);
             if (m + 1 == chunks) return;               // behind the last barrier
         }
@@ -358,12 +385,13 @@ static int launch_long(hipStream_t st, const GdnArgs& A, int B) {
     return DFLASH_OK;
 }
 
-// More than one chunk, and k and q rows readable 16 bytes at a time.  The line lies at the second chunk as that is where
+// More than one chunk, k and q rows readable and tape rows writable 16 bytes at a time, v and y rows eight.  The line lies at the second chunk as that is where
 // there is something to prepare ahead; this kernel is the faster one from there on (us, 17 and 32 steps: 32 heads of 128x128
-// 6.1 -> 5.3 and 6.3 -> 5.2, two such sequences 7.5 -> 6.3 and 7.9 -> 7.4, Dk = 256 17.0 -> 11.6 and 17.5 -> 12.3).  f16 inputs
+// 6.1 -> 5.1 and 6.3 -> 5.1, two such sequences 7.5 -> 5.9 and 7.9 -> 6.8, Dk = 256 17.0 -> 11.6 and 17.5 -> 11.8).  f16 inputs
 // stay with the chunk by chunk kernel: three f16 terms do not hold an fp32 state.
 bool gdn_long_applies(const GdnArgs& A, int Dk) {
-    return A.in_dtype == DFLASH_BF16 && A.T > kChunkSteps && (((uintptr_t)A.k | (uintptr_t)A.q) & 15) == 0 && (Dk == 64 || Dk == 128 || Dk == 256);
+    return A.in_dtype == DFLASH_BF16 && A.T > kChunkSteps && (((uintptr_t)A.k | (uintptr_t)A.q | (uintptr_t)A.tape) & 15) == 0 &&
+           (((uintptr_t)A.v | (uintptr_t)A.y) & 7) == 0 && (Dk == 64 || Dk == 128 || Dk == 256);
 }
 
 int launch_gdn_long(hipStream_t st, const GdnArgs& A, int B, int Dk) {

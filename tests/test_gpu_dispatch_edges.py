@@ -69,6 +69,21 @@ def test_long_forward(gpu_lib, Dk, Dv, T, masked):
     np.testing.assert_allclose(host(y2), host(y), rtol=2e-2, atol=2e-2)
 
 
+# v rows that cannot be read eight bytes at a time take the chunk-by-chunk kernel as well
+@pytest.mark.parametrize("off", [2, 4])
+def test_long_forward_v_alignment(gpu_lib, off):
+    from swiftlm_amd import DFlashKernels as K
+
+    d = O.make_gdn_inputs(3, 1, 50, 2, 4, 128, 48, in_dtype="bf16")
+    q, k, v, g, beta = [dev(d[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")]
+    moved = torch.empty(v.numel() + off, dtype=v.dtype, device="cuda")[off:].view(v.shape).copy_(v)
+    y, s, tape = K.gated_delta_kernel_with_tape(q, k, moved, g, beta, dev(d["state"]))
+    yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], dtype=np.float64)
+    np.testing.assert_allclose(host(s), sw, rtol=1e-4, atol=1e-6)
+    np.testing.assert_allclose(host(tape), tw, rtol=1e-4, atol=1e-5)
+    np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
+
+
 # A value that is not finite stays in its row and in the steps from it on; a chunk whose solve matrix overflows (1e4^15) where no
 # delta does has the deltas that substitution gives.
 def test_long_forward_not_finite(gpu_lib):
