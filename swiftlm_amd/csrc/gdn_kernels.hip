@@ -643,10 +643,8 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
 #pragma unroll
                 for (int c = 0; c < CH; ++c) {
                     const float4 k4 = cur.k[c];
-                    s[c].x = requant<StateT>(fmaf(k4.x, delta, s[c].x));
-                    s[c].y = requant<StateT>(fmaf(k4.y, delta, s[c].y));
-                    s[c].z = requant<StateT>(fmaf(k4.z, delta, s[c].z));
-                    s[c].w = requant<StateT>(fmaf(k4.w, delta, s[c].w));
+                    s[c] = requant4<StateT>(make_float4(fmaf(k4.x, delta, s[c].x), fmaf(k4.y, delta, s[c].y), fmaf(k4.z, delta, s[c].z),
+                                                        fmaf(k4.w, delta, s[c].w)));
                 }
             }
             // Lane j of the row keeps step j's results until the chunk ends: two selects, where a store by one lane was a branch
