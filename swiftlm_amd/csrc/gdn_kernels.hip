@@ -444,15 +444,16 @@ constexpr int kGdnChunk = 16;  // steps staged in LDS at a time
 // Grid: x = Dv tiles of ROWS = 256/LPR rows, y = b*Hv + hv.
 __device__ __forceinline__ float dot4(float4 a, float4 b) { return fmaf(a.x, b.x, a.y * b.y) + fmaf(a.z, b.z, a.w * b.w); }
 
-template <int CH> struct GdnStepOps {
+template <int CH, int RPT> struct GdnStepOps {
     float4 k[CH], q[CH], g[CH];
-    float gs, v, beta, kq;
+    float v[RPT];
+    float gs, beta, kq;
     int on;
 };
 
-template <typename StateT, bool VEC_G, bool HAS_MASK, int DK, int LPR>
+template <typename StateT, bool VEC_G, bool HAS_MASK, int DK, int LPR, int RPT>
 __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
-    constexpr int ROWS = kThreads / LPR;
+    constexpr int GR = kThreads / LPR, ROWS = RPT * GR;           // row groups; thread (group, j) has rows group, group + GR, ..
     constexpr int CH = DK / (4 * LPR);
     constexpr int TC = kGdnChunk;
     constexpr int TPR = DK / 4;                                   // threads spanning one step's q (or k) row, 4 channels each
@@ -481,16 +482,19 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
     const int tid = threadIdx.x;
     const int j = tid % LPR;
     const int rloc = tid / LPR;
-    const int row = row0 + rloc;
-    const bool row_ok = row < A.Dv;
-
-    const StateT* s_in = reinterpret_cast<const StateT*>(A.state_in) + ((size_t)bh * A.Dv + (row_ok ? row : 0)) * DK;
-    StateT* s_out = reinterpret_cast<StateT*>(A.state_out) + ((size_t)bh * A.Dv + (row_ok ? row : 0)) * DK;
+    StateT* s_out[RPT];
 
     // The state rows are the largest operand: their loads go out first.
-    float4 s[CH];
+    float4 s[RPT][CH];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) s[c] = load4(s_in + c * 4 * LPR + 4 * j);
+    for (int u = 0; u < RPT; ++u) {
+        const int row = row0 + rloc + u * GR;
+        const size_t at = ((size_t)bh * A.Dv + (row < A.Dv ? row : 0)) * DK;
+        const StateT* s_in = reinterpret_cast<const StateT*>(A.state_in) + at;
+        s_out[u] = reinterpret_cast<StateT*>(A.state_out) + at;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) s[u][c] = load4(s_in + c * 4 * LPR + 4 * j);
+    }
 
     // ---- a chunk's operands: requested as raw bits, array by array, inside branches that hold nothing but loads, and
     // converted only after the last request has gone out -- one memory round trip per chunk.  (With a conversion or an
@@ -584,7 +588,7 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
         }
     };
 
-    auto fetch = [&](int t, GdnStepOps<CH>& o) {
+    auto fetch = [&](int t, GdnStepOps<CH, RPT>& o) {
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             const int d = c * 4 * LPR + 4 * j;
@@ -593,7 +597,8 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
             if (VEC_G) o.g[c] = *reinterpret_cast<const float4*>(&g_s[t][d]);
         }
         o.gs = VEC_G ? 1.f : g_s[0][t];
-        o.v = v_s[t][rloc];
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) o.v[u] = v_s[t][rloc + u * GR];
         o.beta = beta_s[t];
         o.on = HAS_MASK ? on_s[t] : 1;
         o.kq = kq_s[t];
@@ -609,7 +614,7 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
         park_chunk(tc);
         __syncthreads();
         if constexpr (!KQ_AT_STAGING) {
-            for (int t = rloc; t < tc; t += ROWS) {
+            for (int t = rloc; t < tc; t += GR) {
                 float kq = 0.f;
 #pragma unroll
                 for (int c = 0; c < CH; ++c)
@@ -621,38 +626,55 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
         }
 
         // ---- serial steps ----
-        float y_mine = 0.f, t_mine = 0.f;
-        auto step = [&](int t, const GdnStepOps<CH>& cur) {
-            float yv = 0.f, delta = 0.f;
+        float y_mine[RPT], t_mine[RPT];
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) y_mine[u] = t_mine[u] = 0.f;
+        auto step = [&](int t, const GdnStepOps<CH, RPT>& cur) {
+            float yv[RPT], delta[RPT];
+#pragma unroll
+            for (int u = 0; u < RPT; ++u) yv[u] = delta[u] = 0.f;
             if (!HAS_MASK || cur.on) {                // uniform across the workgroup
-                float sk0 = 0.f, sk1 = 0.f, sq0 = 0.f, sq1 = 0.f;
+                float sk[RPT], sq[RPT];
 #pragma unroll
-                for (int c = 0; c < CH; ++c) {
-                    const float4 k4 = cur.k[c], q4 = cur.q[c];
-                    const float4 g4 = VEC_G ? cur.g[c] : make_float4(cur.gs, cur.gs, cur.gs, cur.gs);
-                    s[c].x *= g4.x; s[c].y *= g4.y; s[c].z *= g4.z; s[c].w *= g4.w;
-                    sk0 = fmaf(s[c].x, k4.x, sk0); sk1 = fmaf(s[c].y, k4.y, sk1);
-                    sk0 = fmaf(s[c].z, k4.z, sk0); sk1 = fmaf(s[c].w, k4.w, sk1);
-                    sq0 = fmaf(s[c].x, q4.x, sq0); sq1 = fmaf(s[c].y, q4.y, sq1);
-                    sq0 = fmaf(s[c].z, q4.z, sq0); sq1 = fmaf(s[c].w, q4.w, sq1);
+                for (int u = 0; u < RPT; ++u) {
+                    float sk0 = 0.f, sk1 = 0.f, sq0 = 0.f, sq1 = 0.f;
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) {
+                        const float4 k4 = cur.k[c], q4 = cur.q[c];
+                        const float4 g4 = VEC_G ? cur.g[c] : make_float4(cur.gs, cur.gs, cur.gs, cur.gs);
+                        float4& x = s[u][c];
+                        x.x *= g4.x; x.y *= g4.y; x.z *= g4.z; x.w *= g4.w;
+                        sk0 = fmaf(x.x, k4.x, sk0); sk1 = fmaf(x.y, k4.y, sk1);
+                        sk0 = fmaf(x.z, k4.z, sk0); sk1 = fmaf(x.w, k4.w, sk1);
+                        sq0 = fmaf(x.x, q4.x, sq0); sq1 = fmaf(x.y, q4.y, sq1);
+                        sq0 = fmaf(x.z, q4.z, sq0); sq1 = fmaf(x.w, q4.w, sq1);
+                    }
+                    sk[u] = sk0 + sk1;
+                    sq[u] = sq0 + sq1;
                 }
-                const float sk = butterfly_sum<LPR>(sk0 + sk1);
-                const float sq = butterfly_sum<LPR>(sq0 + sq1);
-                delta = (cur.v - sk) * cur.beta;
-                yv = fmaf(delta, cur.kq, sq);
 #pragma unroll
-                for (int c = 0; c < CH; ++c) {
-                    const float4 k4 = cur.k[c];
-                    s[c] = requant4<StateT>(make_float4(fmaf(k4.x, delta, s[c].x), fmaf(k4.y, delta, s[c].y), fmaf(k4.z, delta, s[c].z),
-                                                        fmaf(k4.w, delta, s[c].w)));
+                for (int u = 0; u < RPT; ++u) { sk[u] = butterfly_sum<LPR>(sk[u]); sq[u] = butterfly_sum<LPR>(sq[u]); }
+#pragma unroll
+                for (int u = 0; u < RPT; ++u) {
+                    delta[u] = (cur.v[u] - sk[u]) * cur.beta;
+                    yv[u] = fmaf(delta[u], cur.kq, sq[u]);
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) {
+                        const float4 k4 = cur.k[c], x = s[u][c];
+                        s[u][c] = requant4<StateT>(make_float4(fmaf(k4.x, delta[u], x.x), fmaf(k4.y, delta[u], x.y), fmaf(k4.z, delta[u], x.z),
+                                                               fmaf(k4.w, delta[u], x.w)));
+                    }
                 }
             }
             // Lane j of the row keeps step j's results until the chunk ends: two selects, where a store by one lane was a branch
             // that stood between the steps and kept the two reductions of a step from filling each other's wait states.
-            if constexpr (LPR >= TC) {
-                y_mine = j == t ? yv : y_mine;
-                t_mine = j == t ? delta : t_mine;
-            } else if (j == 0) { y_s[t][rloc] = yv; t_s[t][rloc] = delta; }
+#pragma unroll
+            for (int u = 0; u < RPT; ++u) {
+                if constexpr (LPR >= TC) {
+                    y_mine[u] = j == t ? yv[u] : y_mine[u];
+                    t_mine[u] = j == t ? delta[u] : t_mine[u];
+                } else if (j == 0) { y_s[t][rloc + u * GR] = yv[u]; t_s[t][rloc + u * GR] = delta[u]; }
+            }
         };
         {
             // Operands are fetched ahead of their use, so no step waits for LDS, into sets of registers that the loop goes
@@ -660,7 +682,7 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
             // refilled ahead of the step, which is what still fits the registers.
             constexpr bool kWideSet = CH * (VEC_G ? 3 : 2) > 6;
             constexpr int kSets = kWideSet ? 3 : 4;
-            GdnStepOps<CH> ops[kSets];
+            GdnStepOps<CH, RPT> ops[kSets];
 #pragma unroll
             for (int u = 0; u < kSets - (kWideSet ? 1 : 0); ++u) fetch(u, ops[u]);
             int t0s = 0;
@@ -683,7 +705,10 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
             }
         }
         if constexpr (LPR >= TC)
-            if (j < tc) { y_s[j][rloc] = y_mine; t_s[j][rloc] = t_mine; }
+            if (j < tc) {
+#pragma unroll
+                for (int u = 0; u < RPT; ++u) { y_s[j][rloc + u * GR] = y_mine[u]; t_s[j][rloc + u * GR] = t_mine[u]; }
+            }
         __syncthreads();
         // ---- write this chunk's y and tape rows ----
         for (int i = tid; i < tc * ROWS; i += kThreads) {
@@ -696,10 +721,12 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
         }
     }
 
-    if (row_ok) {
 #pragma unroll
-        for (int c = 0; c < CH; ++c) store4(s_out + c * 4 * LPR + 4 * j, s[c]);
-    }
+    for (int u = 0; u < RPT; ++u)
+        if (row0 + rloc + u * GR < A.Dv) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) store4(s_out[u] + c * 4 * LPR + 4 * j, s[u][c]);
+        }
 }
 
 // ---------------------------------------------------------------------------
@@ -1595,12 +1622,13 @@ int gdn_device_setup() {
     return rc;
 }
 
-template <typename StateT, int DK, int LPR>
+template <typename StateT, int DK, int LPR, int RPT = 1>
 static int launch_gdn_steps(hipStream_t st, const GdnArgs& A, int B, bool vec) {
-    dim3 grid((A.Dv + (kThreads / LPR) - 1) / (kThreads / LPR), B * A.Hv);
+    constexpr int rows = RPT * (kThreads / LPR);
+    dim3 grid((A.Dv + rows - 1) / rows, B * A.Hv);
     LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);
-    auto kern = vec ? (A.mask ? gated_delta_tape_kernel<StateT, true, true, DK, LPR> : gated_delta_tape_kernel<StateT, true, false, DK, LPR>)
-                    : (A.mask ? gated_delta_tape_kernel<StateT, false, true, DK, LPR> : gated_delta_tape_kernel<StateT, false, false, DK, LPR>);
+    auto kern = vec ? (A.mask ? gated_delta_tape_kernel<StateT, true, true, DK, LPR, RPT> : gated_delta_tape_kernel<StateT, true, false, DK, LPR, RPT>)
+                    : (A.mask ? gated_delta_tape_kernel<StateT, false, true, DK, LPR, RPT> : gated_delta_tape_kernel<StateT, false, false, DK, LPR, RPT>);
     DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), 0, A));
     return DFLASH_OK;
 }
@@ -1613,16 +1641,27 @@ static int launch_gdn_state(hipStream_t st, const GdnArgs& A, int B, int g_ndim,
     // 146 us at T=300, 32 heads, Dk=256).
     const long rows = (long)B * A.Hv * A.Dv, lanes = (long)num_compute_units() * kThreads;
     const bool wide = rows * 32 <= lanes, widest = rows * 64 <= lanes;
+    // Two rows per thread, which share the step's operands, where the workgroups of the one-row form take more than one round: by
+    // their registers two fit a compute unit with a gate per channel (one at Dk = 256), three without.  us, one row and two (16 steps,
+    // 32 heads, Dv = 128; workgroups per compute unit in front):
+    //     Dk=128  gate per channel, fp32 state   2: 7.2 7.8   3: 11.3 11.1   4: 13.1 12.1   (40 steps 28.3 23.7)
+    //             gate per head, bf16 state      3: 9.3 10.8  4: 12.4 11.2
+    //     Dk=256  gate per channel, fp32 state   1.5: 14.7 10.9   2: 15.3 12.4   4: 28.6 23.0   (87 steps, 2: 67.1 49.1)
+    //             gate per head, bf16 state      2: 10.0 10.2     3: 14.8 16.1   4: 18.4 16.9
+    // At Dk = 64 four to five fit, and two rows gain nothing or lose (eight: bf16 13.2 13.1, fp32 12.7 13.5).
+    const bool two = rows * 16 > (vec ? (Dk == 256 ? 1 : 2) : 3) * lanes;
     switch (Dk) {
         case 32: return launch_gdn_steps<StateT, 32, 8>(st, A, B, vec);
         case 64: return launch_gdn_steps<StateT, 64, 16>(st, A, B, vec);
         case 96: return launch_gdn_steps<StateT, 96, 8>(st, A, B, vec);
-        case 128: return wide ? launch_gdn_steps<StateT, 128, 32>(st, A, B, vec) : launch_gdn_steps<StateT, 128, 16>(st, A, B, vec);
+        case 128: return wide ? launch_gdn_steps<StateT, 128, 32>(st, A, B, vec)
+                         : two ? launch_gdn_steps<StateT, 128, 16, 2>(st, A, B, vec) : launch_gdn_steps<StateT, 128, 16>(st, A, B, vec);
         case 160: return launch_gdn_steps<StateT, 160, 8>(st, A, B, vec);
         case 192: return launch_gdn_steps<StateT, 192, 16>(st, A, B, vec);
         case 224: return launch_gdn_steps<StateT, 224, 8>(st, A, B, vec);
         case 256: return widest ? launch_gdn_steps<StateT, 256, 64>(st, A, B, vec)
-                         : wide ? launch_gdn_steps<StateT, 256, 32>(st, A, B, vec) : launch_gdn_steps<StateT, 256, 16>(st, A, B, vec);
+                         : wide ? launch_gdn_steps<StateT, 256, 32>(st, A, B, vec)
+                         : two ? launch_gdn_steps<StateT, 256, 16, 2>(st, A, B, vec) : launch_gdn_steps<StateT, 256, 16>(st, A, B, vec);
         default: break;
     }
     set_error("gated delta: Dk=%d is not a multiple of 32 in [32, 256]", Dk);

@@ -40,6 +40,35 @@ def test_step_kernel_lanes_per_row(gpu_lib, Dk, Hv, Dv, T):
     np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
 
 
+# ... and rows per thread: two where the one-row form takes several rounds (Dv beyond a whole tile of either)
+@pytest.mark.parametrize("Dk,Hv,Dv,vec", [(128, 65, 128, True), (128, 98, 120, False), (256, 33, 128, True), (256, 98, 120, False)], ids=lambda v: str(v))
+@pytest.mark.parametrize("T", [1, 2, 5, 16, 18])
+@pytest.mark.parametrize("state", ["f32", "bf16"])
+def test_step_kernel_rows_per_thread(gpu_lib, Dk, Hv, Dv, vec, T, state):
+    from swiftlm_amd import DFlashKernels as K
+
+    if state == "f32" and not vec:
+        Dv -= 1                                        # (a whole number of tiles takes the chunked kernels)
+    d = O.make_gdn_inputs(Dk + Hv + T, 1, T, 1, Hv, Dk, Dv, in_dtype="bf16", vec_gate=vec)
+    d["state"] = O.quantize(d["state"], state)
+    mask = np.ones((1, T), np.float32)
+    mask[0, T // 2] = float(T == 1)
+    sdt = {"f32": torch.float32, "bf16": torch.bfloat16}[state]
+    # two copies of the batch: B * Hv * Dv beyond the line
+    run = lambda x: torch.cat([x, x])
+    y, s, tape = K.gated_delta_kernel_with_tape(*[run(dev(d[n], torch.bfloat16)) for n in ("q", "k", "v", "g", "beta")], run(dev(d["state"], sdt)), run(dev(mask)))
+    assert torch.equal(y[0], y[1]) and torch.equal(s[0], s[1]) and torch.equal(tape[0], tape[1])
+    if state == "f32":
+        yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], mask, dtype=np.float64)
+        np.testing.assert_allclose(host(s[:1]), sw, rtol=1e-4, atol=1e-6)
+        np.testing.assert_allclose(host(tape[:1]), tw, rtol=1e-4, atol=1e-5)
+    else:
+        yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], mask, requant="bf16")
+        np.testing.assert_allclose(host(s[:1]), sw, rtol=2e-2, atol=2e-2)
+        np.testing.assert_allclose(host(tape[:1]), tw, rtol=2e-2, atol=2e-2)
+    np.testing.assert_allclose(host(y[:1]), yw, rtol=2e-2, atol=2e-2)
+
+
 # GatedDelta forward over more than one chunk of 16 steps: 2 to 9 chunks (the producer waves take every fourth), whole and ragged
 # last chunks, one and several row tiles
 @pytest.mark.parametrize("Dk,Dv", [(64, 16), (128, 128), (256, 32)], ids=lambda v: str(v))
