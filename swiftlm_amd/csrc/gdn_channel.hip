@@ -504,14 +504,16 @@ static int launch_channel(hipStream_t st, const GdnArgs& A, int B) {
 // this one, 32 heads of 128x128: 17 steps 6.8 / 7.0, 24 steps 7.8 / 7.1, 48 steps 13.0 / 9.0; two heads of 64x64 5.3 / 5.7, 5.9 / 5.8,
 // 9.1 / 6.8).  Two workgroups of the step kernel share a unit and fill each other's waits: with more than one round the line is at 96
 // steps (two rounds of 128x128, 33 steps 14.3 / 17.3, 64 steps 21.9 / 21.9, 100 steps 33.5 / 31.9, 257 steps 78.9 / 65.6; of 64x128 64
-// steps 15.5 / 16.5, 128 steps 28.1 / 25.4), and from three rounds on Dk = 64 stays with the step kernel (four rounds, 257 steps
-// 82.2 / 87.7; of 128x128 152 / 129).  Wider rows (Dk = 256) do not fit LDS.
+// steps 15.5 / 16.5, 128 steps 28.1 / 25.4; three rounds of 128x128, 100 steps 51.3 / 46.8).  From three rounds on Dk = 64 stays with
+// the step kernel (four rounds, 257 steps 82.2 / 87.7); more than three rounds of Dk = 128, where that has two rows per thread, leave
+// it at 320 steps (four rounds, 100 steps 52.1 / 61.4, 257 steps 124.4 / 128.7, 500 steps 236.6 / 230.0; six, 500 steps 379 / 346).
+// Wider rows (Dk = 256) do not fit LDS.
 bool gdn_channel_applies(const GdnArgs& A, int B, int Dk) {
     if (A.in_dtype != DFLASH_BF16 && A.in_dtype != DFLASH_F16) return false;
     if ((Dk != 64 && Dk != 128) || (uint64_t)A.Hv * Dk >= (1u << 23)) return false;
     if ((((uintptr_t)A.k | (uintptr_t)A.q | (uintptr_t)A.g) & 3) != 0 || (((uintptr_t)A.state_in | (uintptr_t)A.state_out) & 15) != 0) return false;
     const long tiles = (long)B * A.Hv * (A.Dv / kChunkRows), units = num_compute_units();
-    return tiles <= units ? A.T >= 24 : A.T >= 96 && (Dk == 128 || tiles <= 2 * units);
+    return tiles <= units ? A.T >= 24 : tiles <= (Dk == 128 ? 3 : 2) * units ? A.T >= 96 : Dk == 128 && A.T >= 320;
 }
 
 int launch_gdn_channel(hipStream_t st, const GdnArgs& A, int B, int Dk) {
