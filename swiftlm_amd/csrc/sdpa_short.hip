@@ -359,14 +359,16 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 // or shares of 512 keys, at D = 128, as the combine then needs one round per lane.  All forms of a call take the same line, so that
 // they give the same bits.  us per call, shared tiles against this form:
 //     heads, keys        1500        2048        3000        4112        6000        8208        12000
-//     D=128  8 (Hk=1)  8.6  8.3    8.7  8.4    8.9  8.5    9.3  9.1    9.4  9.4    10.0 9.6    10.8 10.2
-//           16 (Hk=2)  9.0  8.3    9.2  8.3    9.5  8.6    10.1 9.1    11.0 9.7    11.5 10.2   12.5 11.5
-//           32 (Hk=8)  9.1  8.6    9.9  9.2    11.1 9.8    11.7 10.6   12.5 11.8   13.7 13.4   15.7 16.3
-//           64 (Hk=8)  10.6 9.9    11.4 10.4   12.5 11.5   12.6 12.8   13.3 15.6
-//     D=256  8 (Hk=1)  9.6  9.1    10.0 9.3    11.3 10.2   13.7 10.7   12.3 11.4   14.7 11.7   14.2 12.9
-//           16 (Hk=2)  11.0 10.2   11.9 10.7   11.9 11.5   13.0 11.9   13.6 12.8   14.7 14.4   15.1 16.9   (paged 5000 12.6 13.3)
-//           32 (Hk=8)  13.2 10.9   14.1 11.3   15.3 12.6   15.4 14.4   17.4 17.4
-//           64 (Hk=8)  15.5 12.8   16.4 14.0   17.4 16.8   19.2 20.1
+//     D=128  8 (Hk=1)  8.3  8.2    8.4  8.4    8.5  8.5    8.9  9.1    9.0  9.5    9.7  10.0   10.3 11.0
+//           16 (Hk=2)  9.1  8.2    9.3  8.5    9.5  8.6    9.5  9.2    10.9 9.7    11.0 10.2   11.9 11.4
+//           32 (Hk=8)  9.0  8.5    9.9  9.1    11.2 9.9    11.7 10.7   12.5 11.8   13.6 13.5   15.7 16.2
+//           64 (Hk=8)  10.7 9.8    11.5 10.3   12.5 11.5   12.7 12.9   13.0 15.5
+//     D=256  8 (Hk=1)  9.1  8.4    9.3  8.6    10.9 9.5    13.7 10.2   12.3 10.7   14.7 11.2   14.0 12.3
+//           16 (Hk=2)  10.6 9.6    11.3 10.1   11.3 10.8   12.5 11.3   13.1 12.3   14.3 13.6   14.6 16.3
+//                      (5000 12.2 11.7, paged 12.6 12.8; 7500 13.0 13.9, paged 13.7 14.8)
+//           24 (Hk=4)  (5000 13.8 14.2, paged 14.1 14.9)
+//           32 (Hk=8)  12.0 10.9   13.0 11.3   14.0 12.7   14.4 14.2   16.2 17.4
+//           64 (Hk=8)  13.4 12.5   14.4 13.9   15.7 16.7   17.0 19.4
 int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     const int64_t heads = (int64_t)B * Hq;
     const int cus = num_compute_units();
@@ -379,7 +381,8 @@ int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     if (S > most) S = most;
     const int same_xcd = Hk % 8 == 0 ? 1 : Hk % 4 == 0 ? 2 : Hk % 2 == 0 ? 4 : 8;
     if (S > same_xcd) S -= S % same_xcd;
-    return S >= (D == 128 ? 3 : 2) && N <= (D == 128 ? 900 : heads < 32 ? 288 : 512) * S ? (int)S : 0;
+    const int64_t most_keys = D == 256 ? (heads < 32 ? 320 : 512) * S : heads < 16 ? 3584 : 900 * S;
+    return S >= (D == 128 ? 3 : 2) && N <= most_keys ? (int)S : 0;
 }
 
 template <typename Tag, int D, bool MASKED, bool PAGED>

@@ -176,7 +176,7 @@ def test_combine_rows_in_flight(gpu_lib, D, N, S):
 @pytest.mark.parametrize("Hq,Hk,D,N", [(2, 1, 128, 31), (3, 1, 128, 256), (3, 1, 128, 257), (12, 2, 128, 600), (8, 1, 128, 896), (8, 1, 128, 897),
                                        (32, 8, 128, 1152), (32, 8, 128, 1153), (2, 1, 256, 17), (3, 1, 256, 128), (3, 1, 256, 129),
                                        (8, 1, 256, 416), (8, 1, 256, 417), (32, 8, 256, 576), (32, 8, 256, 577), (130, 2, 128, 100), (130, 2, 256, 129),
-                                       (6, 1, 128, 1750), (4, 1, 128, 7200), (4, 1, 128, 7201), (6, 2, 256, 5760), (6, 2, 256, 5761), (16, 8, 256, 2048), (16, 8, 256, 2049)])
+                                       (6, 1, 128, 1750), (4, 1, 128, 3584), (4, 1, 128, 3585), (6, 2, 256, 6400), (6, 2, 256, 6401), (4, 1, 128, 7200), (4, 1, 128, 7201), (6, 2, 256, 5760), (6, 2, 256, 5761), (16, 8, 256, 2048), (16, 8, 256, 2049)])
 def test_short_contexts(gpu_lib, Hq, Hk, D, N, dt):
     from swiftlm_amd import DFlashKernels as K
 
