@@ -356,7 +356,7 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 // no pipeline to fill.  As long as one workgroup's share is small, as the group's heads read their KV head's rows G times through
 // the L2s (which share nothing: S is a multiple that keeps the heads of a group on one XCD; with S = 21 for 12 heads over 2 KV heads
 // 3,000 keys took 12.7 us, with 20 11.2), and all K/V rows come from memory at most 48 MB.  Few heads take no more than 16 splits,
-// or shares of 512 keys, at D = 128, as the combine then needs one round per lane.  All forms of a call take the same line, so that
+// or shares of 512 keys, at D = 128, as the combine then needs one round per lane, and fewer than 16 heads no more than 3,584 keys.  All forms of a call take the same line, so that
 // they give the same bits.  us per call, shared tiles against this form:
 //     heads, keys        1500        2048        3000        4112        6000        8208        12000
 //     D=128  8 (Hk=1)  8.3  8.2    8.4  8.4    8.5  8.5    8.9  9.1    9.0  9.5    9.7  10.0   10.3 11.0
