@@ -87,6 +87,10 @@ struct SdpaArgs {
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+// What a part of a row's keys (maximum m, sum l of exp2) adds to the sum over all of them, whose maximum is mx.  A part without any
+// key has m = -inf and l = 0; one with nothing but NaN scores has m = -inf, too, as a maximum passes over NaN, but a sum of NaN,
+// which the row has to show.
+__device__ __forceinline__ float split_weight(float m, float l, float mx) { return m == -INFINITY ? l : fast_exp2(m - mx) * l; }
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((ext_vector_type(8))) short s16x8_t;

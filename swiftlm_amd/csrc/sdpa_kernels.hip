@@ -874,7 +874,7 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
     // for one after the other -- maxima, then sums, then rows -- they are three dependent trips to memory.
     const int sa = tid < S ? tid : S - 1, sb = tid + kCombineThreads < S ? tid + kCombineThreads : S - 1;
     float m0 = R.m[sa], m1 = R.m[sb];
-    const float l0 = R.l[sa], l1 = R.l[sb];
+    float l0 = R.l[sa], l1 = R.l[sb];
     u32x4_t raw[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
@@ -883,8 +883,8 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
         // empty splits hold no data, whatever was read from them is dropped below.
         raw[u] = *reinterpret_cast<const u32x4_t*>(po + (size_t)(sp < S ? sp : 0) * R.pitch);
     }
-    if (tid >= S) m0 = -INFINITY;
-    if (tid + kCombineThreads >= S) m1 = -INFINITY;
+    if (tid >= S) { m0 = -INFINITY; l0 = 0.f; }
+    if (tid + kCombineThreads >= S) { m1 = -INFINITY; l1 = 0.f; }
 
     // global max
     float mx = wave_max(fmaxf(m0, m1));
@@ -892,8 +892,7 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(CombineAr
     __syncthreads();
     mx = fmaxf(fmaxf(redm_s[0], redm_s[1]), fmaxf(redm_s[2], redm_s[3]));
     // weights and denominator (the partial rows are O / l: weight by l)
-    const float w0 = m0 == -INFINITY ? 0.f : fast_exp2(m0 - mx) * l0;
-    const float w1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - mx) * l1;
+    const float w0 = split_weight(m0, l0, mx), w1 = split_weight(m1, l1, mx);
     if (tid < S) w_s[tid] = w0;
     if (tid + kCombineThreads < S) w_s[tid + kCombineThreads] = w1;
     float lsum = butterfly_sum<64>(w0 + w1);
@@ -950,14 +949,14 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_wave_kernel(Comb
     const uint16_t* po = R.o + d8;
     // the statistics of split `lane` and the first U partial rows of the group in one round trip
     float m0 = R.m[lane < S ? lane : S - 1];
-    const float l0 = R.l[lane < S ? lane : S - 1];
+    float l0 = R.l[lane < S ? lane : S - 1];
     u32x4_t raw[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int sp = grp + u * SG;
         raw[u] = *reinterpret_cast<const u32x4_t*>(po + (size_t)(sp < S ? sp : 0) * R.pitch);
     }
-    if (lane >= S) m0 = -INFINITY;
+    if (lane >= S) { m0 = -INFINITY; l0 = 0.f; }
     float mx = m0;
     for (int s0 = 64; s0 < S; s0 += 64) mx = fmaxf(mx, s0 + lane < S ? R.m[s0 + lane] : -INFINITY);   // rare: more than 64 splits
     mx = wave_max(mx);
@@ -968,7 +967,7 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_wave_kernel(Comb
     for (int s0 = 0; s0 < S; s0 += 64) {
         if (s0) m0 = s0 + lane < S ? R.m[s0 + lane] : -INFINITY;
         const float l = s0 == 0 ? l0 : (s0 + lane < S ? R.l[s0 + lane] : 0.f);
-        const float w0 = m0 == -INFINITY ? 0.f : fast_exp2(m0 - mx) * l;
+        const float w0 = split_weight(m0, l, mx);
         lpart += w0;
         for (int i0 = 0; i0 < 64 && s0 + i0 < S; i0 += SG * U) {
             if (s0 + i0) {

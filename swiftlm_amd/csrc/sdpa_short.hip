@@ -298,7 +298,7 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 #pragma unroll
     for (int i = 0; i < W; ++i) M = fmaxf(M, L.m[i][n]);
 #pragma unroll
-    for (int i = 0; i < W; ++i) l_tot += L.m[i][n] == -INFINITY ? 0.f : fast_exp2(L.m[i][n] - M) * L.l[i][n];
+    for (int i = 0; i < W; ++i) l_tot += split_weight(L.m[i][n], L.l[i][n], M);
     const int waves = nt < W ? nt : W;                               // those that had a tile
     if (w < waves) {
         const float f = m_run == -INFINITY ? 0.f : fast_exp2(m_run - M) * (l_tot > 0.f ? 1.f / l_tot : 0.f);

@@ -388,13 +388,23 @@ def test_tiles_hidden_by_the_mask(gpu_lib, N, tiles, Hq, Hk, D, dt):
     assert torch.isnan(out[0, 2, 3]).all()
 
 
-def test_tile_with_only_a_nan_score_is_not_hidden(gpu_lib):
+# ... whoever holds it: a wave of the one workgroup per head or a split of its own, of either form, behind either combine kernel.
+# Row r of the block sees keys up to N - 16 + r.
+@pytest.mark.parametrize("Hq,Hk,D,N,key", [(4, 2, 128, 33, 32), (4, 2, 256, 33, 32), (3, 1, 128, 300, 299), (3, 1, 256, 300, 31), (16, 2, 256, 1025, 1024),
+                                           (16, 2, 256, 4100, 63), (8, 1, 128, 1025, 1024), (8, 1, 128, 8193, 8192), (8, 8, 128, 8193, 703), (64, 8, 256, 4097, 4096),
+                                           (520, 1, 128, 97, 96), (520, 1, 128, 300, 290)])
+def test_tile_with_only_a_nan_score_is_not_hidden(gpu_lib, Hq, Hk, D, N, key):
     from swiftlm_amd import DFlashKernels as K
 
-    q, k, v = tensors(1, 1, 4, 2, 33, 128)
-    k[:, :, 32] = float("nan")                                # seen by the last row alone
-    nan = torch.isnan(K.batched_sdpa_2pass(q, k, v, 0.1))
-    assert nan[:, :, 15].all() and not nan[:, :, :15].any()
+    q, k, v = tensors(1, 1, Hq, Hk, N, D)
+    k[:, :, key // 32 * 32:key + 1] = float("nan")
+    first = max(0, key // 32 * 32 - (N - 16))
+    out, lse = K.batched_sdpa_2pass(q, k, v, 0.1, return_lse=True)
+    for nan in (torch.isnan(out), torch.isnan(lse)):
+        assert nan[:, :, first:].all() and not nan[:, :, :first].any()
+    # nothing but NaN
+    out, lse = K.batched_sdpa_2pass(q, torch.full_like(k, float("nan")), v, 0.1, return_lse=True)
+    assert torch.isnan(out).all() and torch.isnan(lse).all()
 
 
 # GatedDelta forward with one decay per channel, chunk by chunk: 2 to 6 chunks, whole and ragged last ones, several row tiles; decays of
