@@ -3,8 +3,8 @@
  *
  * NOT part of the drop-in surface (include/dflash_hip.h, include/dflash_cache.h): nothing the reference's call
  * sites need is declared here, the module map does not export this header, and a host that only serves requests
- * never includes it.  The benchmark and the profiles use these two entries to time single kernels and to price a
- * launch that does no work.
+ * never includes it.  The benchmark and the profiles use these entries to time single kernels and to price
+ * launches that do no work.
  */
 #ifndef DFLASH_PROFILE_H
 #define DFLASH_PROFILE_H
@@ -39,6 +39,16 @@ int dflash_profile_next_launch(int kernel_id, void* start_event, void* stop_even
  * i.e. the floor under each kernel of a verify step.  No counterpart in the reference.  Kernel id
  * DFLASH_KERNEL_EMPTY for dflash_profile_next_launch. */
 int dflash_profile_empty_launch(void* stream, int grid_x, int grid_y, int grid_z, int threads, int lds_bytes);
+
+/* What dflash_sdpa_block_causal* launches for a batch whose sequences all have N keys (with lengths on the device the
+ * workgroups may be dealt, which changes the first grid): kernel names and launch shapes, in launch order, for pricing and
+ * labelling a step's launches.  Returns how many there are (1 or 2), or 0 for a call that those entries refuse.
+ * No counterpart in the reference. */
+typedef struct {
+    const char* kernel;
+    int grid_x, grid_y, grid_z, threads, lds_bytes;
+} dflash_launch_shape;
+int dflash_profile_sdpa_launches(int dtype, int B, int Hq, int Hk, int N, int D, dflash_launch_shape shapes[2]);
 
 #ifdef __cplusplus
 }

@@ -25,6 +25,12 @@ KERNEL_GREEDY_PARTIAL, KERNEL_GDN_PREPARE, KERNEL_EMPTY, KERNEL_GDN_LAYER, KERNE
 vp, i32, i64, f32, sz = C.c_void_p, C.c_int, C.c_int64, C.c_float, C.c_size_t
 vpp = C.POINTER(C.c_void_p)
 
+
+class LaunchShape(C.Structure):
+    """dflash_launch_shape of include/dflash_profile.h"""
+    _fields_ = [("kernel", C.c_char_p)] + [(n, i32) for n in ("grid_x", "grid_y", "grid_z", "threads", "lds_bytes")]
+
+
 # name -> (restype, argtypes); the single source of truth the symbol test walks.
 SIGNATURES = {
     "dflash_version": (i32, []),
@@ -55,6 +61,7 @@ SIGNATURES = {
     "dflash_set_status_word": (i32, [vp]),
     "dflash_profile_next_launch": (i32, [i32, vp, vp]),
     "dflash_profile_empty_launch": (i32, [vp, i32, i32, i32, i32, i32]),
+    "dflash_profile_sdpa_launches": (i32, [i32] * 6 + [C.POINTER(LaunchShape)]),
     "dflash_cache_create": (vp, [i32, i32]),
     "dflash_cache_destroy": (None, [vp]),
     "dflash_cache_kind": (i32, [vp]),

@@ -148,6 +148,7 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 // Attention by one workgroup per query head and split (sdpa_short.hip).  One split writes the output itself (A.part_o, A.lse).
 // How many splits, at most `most`: 0 where the form does not apply.
 int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most);
+dflash_launch_shape sdpa_short_shape(int B, int Hk, int G, int S, int D);
 int launch_sdpa_short(hipStream_t st, const SdpaArgs& A, int B, int D, int dtype, bool paged);
 int sdpa_short_device_setup();
 

@@ -1059,11 +1059,14 @@ static size_t ws_layout(int B, int Hq, int S, int D, size_t* off_m, size_t* off_
     return (o + 255) & ~(size_t)255;
 }
 
+struct CombineForm {
+    void (*kernel)(CombineArgs);
+    const char* name;
+    int workgroups;
+};
 template <typename Tag, int D>
-static int launch_combine(hipStream_t st, const CombineArgs& C) {
-    LaunchBracket br(DFLASH_KERNEL_SDPA_COMBINE, st);
-    const dim3 waves(C.rows / (kCombineThreads / 64)), threads(kCombineThreads);
-    const int groups = 64 / (D / 8);
+static CombineForm combine_form(const CombineArgs& C) {
+    const int waves = C.rows / (kCombineThreads / 64), groups = 64 / (D / 8);
     // More than four splits per lane group: one wave per row, 16 partial rows per lane in flight, up to 64 splits at D = 128 (a
     // dealt launch 32, as its long sequences take more than S), at D = 256 where a workgroup per row would be more than the
     // chip holds at once.  us per call, wave against workgroup, rows x splits:
@@ -1072,20 +1075,24 @@ static int launch_combine(hipStream_t st, const CombineArgs& C) {
     //   D=256  2,048 x 16 38.9 42.3  1,280 x 26 38.4 40.9  1,024 x 32 29.0 29.5  256 x 16 29.1 28.5  512 x 64 32.7 27.8
     //   dealt  2,048 x 16 43.4 48.2  1,280 x 26 34.2 35.0  1,024 x 32 32.1 30.1
     auto one_wave = [&]() { return D == 128 ? C.S <= (C.balance ? 32 : 64) : C.S <= 32 && C.rows > 4 * num_compute_units(); };
-    if (C.S <= 4 * groups) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 4>, waves, threads, 0, C));
-    else if (one_wave()) DFLASH_HIP_TRY(br.launch(sdpa_combine_wave_kernel<Tag, D, 16>, waves, threads, 0, C));
-    else {
-        // As many partial rows in flight per thread as there are to take, as a row that is asked for and dropped costs its load
-        // (16 for any count, before: 64 query heads of D = 256, 4,112 keys, 26 splits 20.1 us, now 18.0; 16 heads, 6,000 keys, 64
-        // splits 16.0 and 14.7).  A dealt launch has sequences of more than S: eight at least, and theirs take another round (16, 8 and 4
-        // in flight, four sequences of up to 20,000 keys 33.4, 31.9, 31.8 us; eight paged ones, appended to, 45.9, 44.4, 44.0; two of up
-        // to 50,000 42.0, 41.4, 41.5).
-        const int each = (C.S + 4 * groups - 1) / (4 * groups);
-        auto kern = each <= 8 ? sdpa_combine_kernel<Tag, D, 8> : each <= 12 ? sdpa_combine_kernel<Tag, D, 12> : sdpa_combine_kernel<Tag, D, 16>;
-        if constexpr (D == 256)                        // (D = 128 takes the wave form there)
-            if (each <= 4 && !C.balance) kern = sdpa_combine_kernel<Tag, D, 4>;
-        DFLASH_HIP_TRY(br.launch(kern, dim3(C.rows), threads, 0, C));
-    }
+    if (C.S <= 4 * groups) return {sdpa_combine_wave_kernel<Tag, D, 4>, "sdpa_combine_wave_kernel", waves};
+    if (one_wave()) return {sdpa_combine_wave_kernel<Tag, D, 16>, "sdpa_combine_wave_kernel", waves};
+    // As many partial rows in flight per thread as there are to take, as a row that is asked for and dropped costs its load
+    // (16 for any count, before: 64 query heads of D = 256, 4,112 keys, 26 splits 20.1 us, now 18.0; 16 heads, 6,000 keys, 64
+    // splits 16.0 and 14.7).  A dealt launch has sequences of more than S: eight at least, and theirs take another round (16, 8 and 4
+    // in flight, four sequences of up to 20,000 keys 33.4, 31.9, 31.8 us; eight paged ones, appended to, 45.9, 44.4, 44.0; two of up
+    // to 50,000 42.0, 41.4, 41.5).
+    const int each = (C.S + 4 * groups - 1) / (4 * groups);
+    auto kern = each <= 8 ? sdpa_combine_kernel<Tag, D, 8> : each <= 12 ? sdpa_combine_kernel<Tag, D, 12> : sdpa_combine_kernel<Tag, D, 16>;
+    if constexpr (D == 256)                        // (D = 128 takes the wave form there)
+        if (each <= 4 && !C.balance) kern = sdpa_combine_kernel<Tag, D, 4>;
+    return {kern, "sdpa_combine_kernel", C.rows};
+}
+template <typename Tag, int D>
+static int launch_combine(hipStream_t st, const CombineArgs& C) {
+    LaunchBracket br(DFLASH_KERNEL_SDPA_COMBINE, st);
+    const CombineForm f = combine_form<Tag, D>(C);
+    DFLASH_HIP_TRY(br.launch(f.kernel, dim3(f.workgroups), dim3(kCombineThreads), 0, C));
     return DFLASH_OK;
 }
 
@@ -1286,6 +1293,28 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
     if (paged) DFLASH_SDPA_CASE(false, true);
     DFLASH_SDPA_CASE(false, false);
 #undef DFLASH_SDPA_CASE
+}
+
+extern "C" int dflash_profile_sdpa_launches(int dtype, int B, int Hq, int Hk, int N, int D, dflash_launch_shape shapes[2]) {
+    if (!shapes || B <= 0 || Hq <= 0 || Hk <= 0 || N < kM || Hq % Hk != 0 || (D != 128 && D != 256)) return 0;
+    if ((dtype != DFLASH_BF16 && dtype != DFLASH_F16) || B > 65535 || (long)Hq * 2 > 65535 || ensure_init()) return 0;
+    const int G = Hq / Hk, groups = (G + kHeadsPerWG - 1) / kHeadsPerWG;
+    int S = choose_splits(B, Hk, groups, N);
+    if (const int few = sdpa_short_splits(B, Hq, Hk, N, D, S)) {
+        S = few;
+        shapes[0] = sdpa_short_shape(B, Hk, G, S, D);
+    } else {
+        shapes[0] = {"sdpa_partial_kernel", S, Hk * groups, B, kPartialThreads, D == 256 ? SdpaLds<256>::BYTES : SdpaLds<128>::BYTES};
+    }
+    if (S == 1) return 1;
+    CombineArgs C = {};
+    C.S = S; C.rows = B * Hq * kM;
+    const CombineForm f = dtype == DFLASH_BF16 ? (D == 256 ? combine_form<Bf16Tag, 256>(C) : combine_form<Bf16Tag, 128>(C))
+                                               : (D == 256 ? combine_form<F16Tag, 256>(C) : combine_form<F16Tag, 128>(C));
+    hipFuncAttributes attr = {};
+    if (hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(f.kernel)) != hipSuccess) return 0;
+    shapes[1] = {f.name, f.workgroups, 1, 1, kCombineThreads, (int)attr.sharedSizeBytes};
+    return 2;
 }
 
 extern "C" int dflash_sdpa_block_causal(void* stream, const void* q, const void* k, const void* v, void* out,

@@ -385,10 +385,17 @@ int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     return S >= (D == 128 ? 3 : 2) && N <= most_keys ? (int)S : 0;
 }
 
+dflash_launch_shape sdpa_short_shape(int B, int Hk, int G, int S, int D) {
+    const int lds = D == 256 ? (int)sizeof(SdpaShortLds<256>) : (int)sizeof(SdpaShortLds<128>);
+    return {"sdpa_short_kernel", Hk * S, G, B, 64 * SdpaShortLds<128>::WAVES, lds};
+}
+static_assert(SdpaShortLds<128>::WAVES == SdpaShortLds<256>::WAVES, "one workgroup size");
+
 template <typename Tag, int D, bool MASKED, bool PAGED>
 static int launch_short(hipStream_t st, const SdpaArgs& A, int B) {
     LaunchBracket br(DFLASH_KERNEL_SDPA_PARTIAL, st);
-    DFLASH_HIP_TRY(br.launch(sdpa_short_kernel<Tag, D, MASKED, PAGED>, dim3(A.Hk * A.S, A.G, B), dim3(64 * SdpaShortLds<D>::WAVES), sizeof(SdpaShortLds<D>), A));
+    const dflash_launch_shape g = sdpa_short_shape(B, A.Hk, A.G, A.S, D);
+    DFLASH_HIP_TRY(br.launch(sdpa_short_kernel<Tag, D, MASKED, PAGED>, dim3(g.grid_x, g.grid_y, g.grid_z), dim3(g.threads), g.lds_bytes, A));
     return DFLASH_OK;
 }
 template <typename Tag, int D> static int launch_short(hipStream_t st, const SdpaArgs& A, int B, bool paged) {

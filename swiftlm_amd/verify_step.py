@@ -200,37 +200,38 @@ class HybridVerifyStack:
         self.phase = 1 - ph
 
     # -- launch shapes --------------------------------------------------------------
+    def attention_launches(self):
+        """(kernel name, (grid_x, grid_y, grid_z, threads, lds_bytes)) of every launch of one attention layer, as the library
+        chooses them."""
+        cfg = self.cfg
+        shapes = (_lib.LaunchShape * 2)()
+        n = self.lib.dflash_profile_sdpa_launches(_lib.BF16, 1, cfg.Hq, cfg.Hkv, self.n_max, cfg.D, shapes)
+        if n == 0:
+            raise _lib.DFlashError("no attention launches for this configuration: " + _lib.last_error())
+        return [(s.kernel.decode(), (s.grid_x, s.grid_y, s.grid_z, s.threads, s.lds_bytes)) for s in shapes[:n]]
+
     def launch_shapes(self):
         """(grid_x, grid_y, grid_z, threads, lds_bytes) of every kernel one step launches, in launch order:
-        the shapes the library's host code picks for this configuration (csrc: launch_gdn_chunk, launch_sdpa,
-        launch_replay_nr), for pricing a step's launches with empty kernels of the same shapes.  Only the
-        benchmark's kernel choices are covered (chunked GatedDelta forward, dense or paged attention with at
-        most 8 query heads per KV head over a context too long for a workgroup per query head, 4 state rows per replay
+        the shapes the library's host code picks for this configuration (csrc: launch_gdn_chunk, launch_replay_nr; the
+        attention's by its own account), for pricing a step's launches with empty kernels of the same shapes.  Only the
+        benchmark's kernel choices are covered for the recurrences (chunked GatedDelta forward, 4 state rows per replay
         thread)."""
-        cfg, T = self.cfg, self.cfg.block
-        assert not self.attn or cfg.Hkv * self.n_max * cfg.D > 12_000_000
-        assert cfg.Dk in (64, 128, 256) and cfg.Dv % 16 == 0 and cfg.Hq // cfg.Hkv <= 8 and cfg.D in (128, 256)
-        ld = cfg.Dk + 4
-        gdn_lds = (4 * (16 * ld + 4 + 16 * 33 + 2 * 16 * 16 + 16 * 17 + 16 * 16 + 4 * 16 + 16)   # fp32 operands and tables
-                   + 2 * 5 * 16 * (cfg.Dk + 8) + 8)                                               # bf16 operands
-        gdn = (cfg.Dv // 16, cfg.Hv, 1, 256, gdn_lds)
-        # splits: the S whose workspace layout gives the size the library reports
-        rows = cfg.Hq * T
-        need = int(self.lib.dflash_sdpa_workspace_bytes(1, cfg.Hq, cfg.Hkv, T, self.n_max, cfg.D))
-        a256 = lambda x: (x + 255) & ~255
-        splits = [S for S in range(1, 513) if a256(a256(a256(rows * S * cfg.D * 2) + rows * S * 4) + rows * S * 4) == need]
-        assert len(splits) == 1, "cannot recover the split count from the workspace size"
-        row_bytes = cfg.D * 2
-        partial = (splits[0], cfg.Hkv, 1, 384, 4 * 32 * row_bytes + 2 * 3 * 32 * row_bytes)
-        combine = (rows, 1, 1, 256, 4 * 512 + 16 + 4 * (256 // (cfg.D // 8)) * cfg.D)
-        rpp = 256 // (cfg.Dk // 4)
-        n_gdn = len(self.gdn)
-        assert (cfg.Dv // rpp) * cfg.Hv * n_gdn >= 16 * 256 and cfg.Dv >= 4 * rpp
-        tc = 8 if cfg.Dk >= 256 else 16
-        replay = (cfg.Dv // (4 * rpp), cfg.Hv, n_gdn, 256, 4 * (tc * cfg.Dk + tc + tc * 4 * rpp + tc))
+        cfg = self.cfg
         out = []
+        n_gdn = len(self.gdn)
+        if n_gdn:
+            assert cfg.Dk in (64, 128, 256) and cfg.Dv % 16 == 0
+            ld = cfg.Dk + 4
+            gdn_lds = (4 * (16 * ld + 4 + 16 * 33 + 2 * 16 * 16 + 16 * 17 + 16 * 16 + 4 * 16 + 16)   # fp32 operands and tables
+                       + 2 * 5 * 16 * (cfg.Dk + 8) + 8)                                               # bf16 operands
+            gdn = (cfg.Dv // 16, cfg.Hv, 1, 256, gdn_lds)
+            rpp = 256 // (cfg.Dk // 4)
+            assert (cfg.Dv // rpp) * cfg.Hv * n_gdn >= 16 * 256 and cfg.Dv >= 4 * rpp
+            tc = 8 if cfg.Dk >= 256 else 16
+            replay = (cfg.Dv // (4 * rpp), cfg.Hv, n_gdn, 256, 4 * (tc * cfg.Dk + tc + tc * 4 * rpp + tc))
+        attn = [shape for _, shape in self.attention_launches()] if self.attn else []
         for kind in cfg.kinds():
-            out += [gdn] if kind == "gdn" else [partial, combine]
+            out += [gdn] if kind == "gdn" else attn
         if n_gdn:
             out.append(replay)
         return out

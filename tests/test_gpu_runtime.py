@@ -484,3 +484,33 @@ def test_device_status_word_reports_out_of_contract_device_lengths(gpu_lib):
         assert int(status) == _lib.STATUS_CONV_STEPS
     finally:
         lib.dflash_set_status_word(None)
+
+
+# The shapes and the number of a step's launches, on both sides of the lines between the attention's forms: one launch, a few splits
+# of the same form, shared tiles.  Armed events are read back, so the kernels named here are those that ran.
+@pytest.mark.parametrize("context,names", [(64, ["sdpa_short_kernel"]), (1000, ["sdpa_short_kernel", "sdpa_combine_kernel"]),
+                                           (16384, ["sdpa_partial_kernel", "sdpa_combine_kernel"])])
+@pytest.mark.parametrize("page", [0, 64])
+def test_launch_shapes_of_a_step(gpu_lib, context, names, page):
+    import bench
+    from swiftlm_amd import _lib
+    from swiftlm_amd.verify_step import HybridVerifyStack, StackConfig
+
+    st = HybridVerifyStack(StackConfig(n_layers=12, context=context, max_steps=1, page_size=page))
+    launches = st.attention_launches()
+    assert [n for n, _ in launches] == names
+    shapes = st.launch_shapes()
+    assert len(shapes) == 9 + 3 * len(names) + 1 and [s for _, s in launches] == shapes[3:3 + len(names)]
+    us, n = bench.launch_floor(gpu_lib, st, 2, 2)
+    assert us > 0 and n == len(shapes)
+    ev = bench.HipEvents()
+
+    def arm(name):
+        if name == "sdpa" and len(ev.pairs) < 2 * len(names):
+            for kid in (_lib.KERNEL_SDPA_PARTIAL, _lib.KERNEL_SDPA_COMBINE)[:len(names)]:
+                _lib.check(gpu_lib.dflash_profile_next_launch(kid, *ev.pair()), "profile_next_launch")
+
+    st.enqueue_step(before_launch=arm)
+    torch.cuda.synchronize()
+    assert len(ev.pairs) == 2 * len(names) and all(us > 0 for us in ev.durations_us())
+    ev.destroy()
