@@ -1399,6 +1399,15 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             float yv = L.gam[t] * L.p[r][16 + t];
 #pragma unroll
             for (int s = 0; s < kChunkSteps; ++s) yv = fmaf(L.c[s][t], L.dl[s][r], yv);
+            // c is 0 for the steps behind t, but 0 times an infinity or NaN of theirs is not: a sum that is not finite is formed again
+            // from the steps that it may see
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(yv) < __builtin_inff())) != 0, 0)) {
+                yv = L.gam[t] * L.p[r][16 + t];
+                for (int s = 0; s < kChunkSteps; ++s) {
+                    const float more = fmaf(L.c[s][t], L.dl[s][r], yv);
+                    yv = s <= t ? more : yv;
+                }
+            }
             yv = L.on[t] ? yv : 0.f;
             if (t < tc) {
                 const uint32_t o = (((uint32_t)b * A.T + t0) * A.Hv + hv) * A.Dv + row0 + __umul24(t, v_step) + r;

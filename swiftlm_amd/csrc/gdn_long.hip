@@ -367,6 +367,20 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             yv = gam_n * pq;
 #pragma unroll
             for (int e = 0; e < 4; ++e) yv = __builtin_amdgcn_mfma_f32_16x16x4f32(ds[e], cv[e], yv, 0, 0, 0);
+            // 0 times an infinity or NaN of a step behind n is not 0: sums that are not finite are formed again from the steps up to n
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(yv[0]) + fabsf(yv[1]) + fabsf(yv[2]) + fabsf(yv[3]) < __builtin_inff())) != 0, 0)) {
+                yv = gam_n * pq;
+                for (int sg = 0; sg < 4; ++sg)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float c = __shfl(cv[e], 16 * sg + n);
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            const float more = fmaf(L.dl[par][16 * sg + 4 * g + v][e], c, yv[v]);
+                            yv[v] = 4 * sg + e <= n ? more : yv[v];
+                        }
+                    }
+            }
 #pragma unroll
             for (int v = 0; v < 4; ++v) yv[v] = step_on ? yv[v] : 0.f;
             if (m + 4 >= chunks) store_rows(m, tc);

@@ -131,10 +131,38 @@ def test_long_forward_not_finite(gpu_lib):
         keep = torch.ones_like(tape, dtype=torch.bool)
         keep[0, :, 1, row] = False
         np.testing.assert_allclose(host(tb[keep]), host(tape[keep]), rtol=1e-4, atol=1e-5)
+        keep[0, :step, 1, row] = True
         np.testing.assert_allclose(host(yb[keep]), host(y[keep]), rtol=2e-2, atol=2e-2)
     big = torch.full_like(k, 10.0)                            # k.k = 12800
     y, s, tape = K.gated_delta_kernel_with_tape(q, big, torch.zeros_like(v), torch.ones_like(g), torch.ones_like(beta), torch.zeros_like(s))
     assert not y.any() and not s.any() and not tape.any()
+
+
+# ... and y of the steps in front of it is what it is without it, in every form of the forward: one chunk, chunk by chunk (f16, fp32),
+# several chunks, and with a decay per channel the steps one by one and 16 at a time.  Whatever holds it: v, which one state row
+# sees, or k, q, the gate or beta.
+@pytest.mark.parametrize("vec", [False, True], ids=["head", "channel"])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("T,step", [(16, 0), (16, 5), (13, 12), (50, 23), (50, 49)], ids=str)
+def test_forward_not_finite_is_causal(gpu_lib, T, step, dt, vec):
+    from swiftlm_amd import DFlashKernels as K
+
+    d = O.make_gdn_inputs(T + step, 1, T, 2, 4, 128, 32, in_dtype="bf16", vec_gate=vec)
+    ins = {n: dev(d[n], dt) for n in ("q", "k", "v", "g", "beta")}
+    state = dev(d["state"])
+    y, s, tape = K.gated_delta_kernel_with_tape(*ins.values(), state)
+    for name in ins:
+        for bad in (float("inf"), float("nan")):
+            with_bad = {n: x.clone() for n, x in ins.items()}
+            x = with_bad[name][0, step, 0]
+            x[...] = bad
+            yb, sb, tb = K.gated_delta_kernel_with_tape(*with_bad.values(), state)
+            np.testing.assert_allclose(host(yb[:, :step]), host(y[:, :step]), rtol=2e-2, atol=2e-2, err_msg=f"{bad} in {name}")
+            np.testing.assert_allclose(host(tb[:, :step]), host(tape[:, :step]), rtol=1e-4, atol=1e-5, err_msg=f"{bad} in {name}")
+            assert not torch.isfinite(yb[0, step, 0]).any()
+            for h in (2, 3):                                  # heads of the other key head
+                np.testing.assert_allclose(host(yb[:, :, h]), host(y[:, :, h]), rtol=2e-2, atol=2e-2, err_msg=f"{bad} in {name}")
+                np.testing.assert_allclose(host(sb[:, h]), host(s[:, h]), rtol=1e-4, atol=1e-6, err_msg=f"{bad} in {name}")
 
 
 def attend(q, k, v, lens, D, **kw):
