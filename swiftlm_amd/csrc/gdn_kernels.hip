@@ -1234,6 +1234,7 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             }
         }
 
+        bool spoilt = false;
         // ---- [S_0 ; k] x [k | q]^T: one 16x16 block per wave, over all DK channels ----
         //   wave 0: S_0 k_t -> p[r][t]     wave 1: S_0 q_t -> p[r][16+t]     wave 2: k_s.k_t -> a     wave 3: k_s.q_t -> c
         // A 16x16x4 fp32 MFMA takes lane l's a as row l%16, contraction index l/16 (b alike) and leaves lane l with
@@ -1359,7 +1360,20 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             }
             // row 4*kk + v of the block: a state row (waves 0, 1) or step s (waves 2, 3); column n
 #pragma unroll
-            for (int v = 0; v < 4; ++v) lds_f[tbl + v * pitch] = coef[v] * (acc0[v] + acc1[v]);
+            for (int v = 0; v < 4; ++v) {
+                acc0[v] += acc1[v];
+                lds_f[tbl + v * pitch] = coef[v] * acc0[v];
+            }
+            // A masked step's rows may hold anything, infinities and NaN among it.  Those of v and q reach only the step's own delta and y,
+            // which are dropped; that of k is in coefficients beside those of other steps and in the update, times a delta of zero: where
+            // a product with it is not finite, zeros take its place, here and (behind the next barrier) in the row.
+            if constexpr (HAS_MASK) {
+                spoilt = ws >= 2 && __builtin_amdgcn_ballot_w64(!(fabsf(acc0[0]) + fabsf(acc0[1]) + fabsf(acc0[2]) + fabsf(acc0[3]) < __builtin_inff())) != 0;
+                if (__builtin_expect(spoilt, 0))
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (!L.on[4 * kk + v] || !L.on[n]) lds_f[tbl + v * pitch] = 0.f;
+            }
             if (ws == 3) {
                 if (kk == 0) L.gam[n] = gj[0] * G[0];
                 if (n == kChunkSteps - 1) {
@@ -1384,13 +1398,24 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
             for (int e = 0; e < 4; ++e) { gm[e] = L.gam[4 * q + e]; pv[e] = L.p[r][4 * q + e]; vv[e] = L.v[4 * q + e][r]; bet[e] = L.beta[4 * q + e]; }
 #pragma unroll
             for (int s = 0; s < 16; ++s) arow[s] = *reinterpret_cast<const float4*>(&L.a[s][4 * q]);
+            bool on[4];                                // a masked step has no delta, whatever its v row and the state hold
+#pragma unroll
+            for (int e = 0; e < 4; ++e) on[e] = HAS_MASK ? L.on[4 * q + e] != 0 : true;
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = fmaf(-gm[e], pv[e], vv[e]);
+            for (int e = 0; e < 4; ++e) acc[e] = on[e] ? fmaf(-gm[e], pv[e], vv[e]) : 0.f;
             SolveStep<0>::run(acc, arow, bet, mine, q);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) L.dl[4 * q + e][r] = mine[e];
+            for (int e = 0; e < 4; ++e) L.dl[4 * q + e][r] = on[e] ? mine[e] : 0.f;
         }
+        if constexpr (HAS_MASK)
+            if (__builtin_expect(spoilt && w == 2, 0))
+                for (int s = 0; s < kChunkSteps; ++s)
+                    if (!L.on[s])
+                        for (int c = lane; c < DK; c += 64) {
+                            if constexpr (BF) L.kb[s][c] = 0;
+                            else L.y[s][c] = 0.f;
+                        }
         __syncthreads();
 
         // ---- read-out and tape: thread (t, r) ----

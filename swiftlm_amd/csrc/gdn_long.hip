@@ -56,6 +56,7 @@ template <int DK> struct GdnLongLds {
     float pk[2][4][64][4], pq[2][4][64][4];// partial S_0 k_t and S_0 q_t of the four chain waves, as accumulators
     float dl[2][64][4];                    // lane (g, n): delta_s of row n, s = 4g + i
     float gam[2][16], w[2][16], beta[2][16];
+    uint32_t on[2];                        // bit t: step t counts
 };
 
 __device__ __forceinline__ void split3_bf16(f32x4v v, uint2& hi, uint2& mid, uint2& lo) {
@@ -175,11 +176,13 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             // overflow where no delta does.  Then the deltas are substituted for one step after the other.
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(dl[0]) + fabsf(dl[1]) + fabsf(dl[2]) + fabsf(dl[3]) < __builtin_inff())) != 0, 0)) {
                 rhs *= lds4(&L.beta[par][4 * g]);
+                const uint32_t on = L.on[par];
                 for (int tg = 0; tg < 4; ++tg)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int t = 4 * tg + i;
-                        const float d = __shfl(rhs[i], 16 * tg + n);
+                        float d = __shfl(rhs[i], 16 * tg + n);
+                        d = (on >> t) & 1 ? d : 0.f;
                         if (g == tg) dl[i] = d;
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
@@ -258,6 +261,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
     float G[4], gam = 0.f, gam_n = 0.f, beta = 0.f;   // gam_n: that of step n in every lane
     f32x4v vf, yv, dl;                                 // v of the chunk in hand; y and tape of the one before, not yet stored: step n, rows 4g .. +3
     bool step_on = false;
+    uint32_t counted = 0xffffu;                        // bit t: step t counts (without a mask all: what is missing of the last chunk meets nothing)
     auto store_rows = [&](int m, int tc) {             // one store each: row by row, two and four bytes per lane, they were eight
         const uint32_t o = (((uint32_t)b * A.T + m * kChunkSteps) * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(n, step);
         if (n < tc) {
@@ -297,13 +301,33 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
                 kk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, k8, kk, 0, 0, 0);
                 kq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, q8, kq, 0, 0, 0);
             }
+            step_on = n < tc;
+            if (A.mask != nullptr) {
+                step_on = step_on && mask_on(A.mask, A.mask_dtype, (int)((uint32_t)b * A.T + t0 + min(n, tc - 1)));
+                counted = (uint32_t)__builtin_amdgcn_ballot_w64(step_on) & 0xffffu;
+                vr = step_on ? vr : make_uint2(0u, 0u);
+                // A masked step's rows may hold anything, infinities and NaN among it, and zero times these is not zero: where a product
+                // with them is not finite, zeros take the rows' place.
+                auto size = [](f32x4v x) { return fabsf(x[0]) + fabsf(x[1]) + fabsf(x[2]) + fabsf(x[3]); };
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(size(kk) + size(kq) < __builtin_inff())) != 0, 0)) {
+#pragma unroll
+                    for (int j = 0; j < NK; ++j)
+                        if (!((counted >> (j * RPI + rs)) & 1)) {
+                            park(L.k[m & 3][j * RPI + rs], none);
+                            park(L.q[m & 3][j * RPI + rs], none);
+                        }
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const bool both = step_on && ((counted >> (4 * g + v)) & 1);
+                        kk[v] = both ? kk[v] : 0.f;
+                        kq[v] = both ? kq[v] : 0.f;
+                    }
+                }
+            }
             // decay products G[v] = g_{s+1} ... g_t of the lane's pairs (s, t) = (4g + v, n), 1 where s >= t
-            bool on = n < tc;
-            if (A.mask != nullptr) on = on && mask_on(A.mask, A.mask_dtype, (int)((uint32_t)b * A.T + t0 + min(n, tc - 1)));
-            const float gl = on ? to_float(gr) : 1.f;
-            beta = on ? to_float(br) : 0.f;
+            const float gl = step_on ? to_float(gr) : 1.f;
+            beta = step_on ? to_float(br) : 0.f;
             vf = f32x4v{__uint_as_float(vr.x << 16), __uint_as_float(vr.x & 0xffff0000u), __uint_as_float(vr.y << 16), __uint_as_float(vr.y & 0xffff0000u)};
-            step_on = on;
             // steps in blocks of four: pre = the product from the block's first step up to the lane's, block products by broadcast
             // (lane exchanges outside the selects: a select may become a branch, with the lanes that are read switched off)
             const float left1 = quad_take<0, 0, 1, 2>(gl);
@@ -333,6 +357,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             // T = (I + A)^-1 diag(beta), in the layout of the chain's a operand: lane (g, n) forms T[n][4g .. +3].  What other lanes
             // of this wave wrote is read back without a wait: LDS serves a wave's accesses in order.
             if (g == 0) { L.beta[par][n] = beta; L.gam[par][n] = gam; }
+            if (lane == 0) L.on[par] = counted;
             asm volatile("" ::: "memory");             // written by the lanes g = 0, read by all
             *reinterpret_cast<f32x4v*>(&L.na[par][n][4 * g]) = av;
             float na[16];                              // row n of -A, the four lanes' pieces gathered

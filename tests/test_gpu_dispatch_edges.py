@@ -165,6 +165,45 @@ def test_forward_not_finite_is_causal(gpu_lib, T, step, dt, vec):
                 np.testing.assert_allclose(host(sb[:, h]), host(s[:, h]), rtol=1e-4, atol=1e-6, err_msg=f"{bad} in {name}")
 
 
+# A masked step keeps the state and writes zeros, whatever its rows hold (padding): every form of the forward, as above, and an fp16
+# state, gives the bits that it gives over zeros there; a state row that is not finite makes no delta either.
+@pytest.mark.parametrize("vec", [False, True], ids=["head", "channel"])
+@pytest.mark.parametrize("dt,state", [("bf16", "f32"), ("f16", "f32"), ("f32", "f32"), ("f16", "f16")], ids=str)
+@pytest.mark.parametrize("T,off", [(16, [0]), (16, [3, 4, 9]), (13, [12]), (50, [0, 15, 16]), (50, [23, 48, 49])], ids=str)
+def test_masked_steps_hold_anything(gpu_lib, T, off, dt, state, vec):
+    from swiftlm_amd import DFlashKernels as K
+
+    types = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}
+    d = O.make_gdn_inputs(T + len(off), 1, T, 2, 4, 128, 32, in_dtype="bf16", vec_gate=vec)
+    d["state"] = O.quantize(d["state"], state)
+    mask = np.ones((1, T), np.float32)
+    mask[0, off] = 0
+    ins = {n: dev(d[n], types[dt]) for n in ("q", "k", "v", "g", "beta")}
+    for x in ins.values():
+        x[0, off] = 0
+    s0 = dev(d["state"], types[state])
+    run = lambda x, s: K.gated_delta_kernel_with_tape(*x.values(), s, dev(mask))
+    y, s, tape = run(ins, s0)
+    if state == "f32":
+        yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], mask, dtype=np.float64)
+        np.testing.assert_allclose(host(s), sw, rtol=1e-4, atol=1e-6)
+        np.testing.assert_allclose(host(tape), tw, rtol=1e-4, atol=1e-5)
+        np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
+    for name in ins:
+        for bad in (float("inf"), float("nan")):
+            held = {n: x.clone() for n, x in ins.items()}
+            held[name][0, off] = bad
+            for got, want in zip(run(held, s0), (y, s, tape)):
+                assert torch.equal(got, want), f"{bad} in {name}"
+    for bad in (float("inf"), float("nan")):
+        sb = s0.clone()
+        sb[0, 1, 5, 7] = bad
+        yb, _, tb = run(ins, sb)
+        assert not tb[0, off].any() and not yb[0, off].any()
+        first = min(t for t in range(T) if t not in off)
+        assert not torch.isfinite(tb[0, first, 1, 5])
+
+
 def attend(q, k, v, lens, D, **kw):
     from swiftlm_amd import DFlashKernels as K
 
