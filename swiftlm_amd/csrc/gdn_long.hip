@@ -42,6 +42,9 @@ namespace dflash {
 // ---------------------------------------------------------------------------
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));
+// rows of v, y and the tape at any address that their elements may have: one load or store all the same
+struct __attribute__((packed, aligned(2))) Rows4x16 { uint2 x; };
+struct __attribute__((packed, aligned(4))) Rows4x32 { f32x4v x; };
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));   // (a select between two HIP uint4 is a select of addresses: the arrays end in scratch)
 
 template <int DK> struct GdnLongLds {
@@ -245,7 +248,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             kr[j] = *reinterpret_cast<const u32x4v*>(kp + oj);
             qr[j] = *reinterpret_cast<const u32x4v*>(qp + oj);
         }
-        vr = *reinterpret_cast<const uint2*>(vp + ((bt0 * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(tl, step)));
+        vr = reinterpret_cast<const Rows4x16*>(vp + ((bt0 * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(tl, step)))->x;
         const uint32_t go = bt0 * A.Hv + hv + __umul24(tl, A.Hv);
         gr = gp[go];
         br = bp[go];
@@ -268,8 +271,8 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             uint2 y2;
             y2.x = (uint32_t)from_float<bf16_t>(yv[0]).bits | ((uint32_t)from_float<bf16_t>(yv[1]).bits << 16);
             y2.y = (uint32_t)from_float<bf16_t>(yv[2]).bits | ((uint32_t)from_float<bf16_t>(yv[3]).bits << 16);
-            *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(A.y) + o) = y2;
-            *reinterpret_cast<f32x4v*>(A.tape + o) = dl;
+            reinterpret_cast<Rows4x16*>(reinterpret_cast<bf16_t*>(A.y) + o)->x = y2;
+            reinterpret_cast<Rows4x32*>(A.tape + o)->x = dl;
         }
     };
     if (p < chunks) request(p);
@@ -424,13 +427,12 @@ static int launch_long(hipStream_t st, const GdnArgs& A, int B) {
     return DFLASH_OK;
 }
 
-// More than one chunk, k and q rows readable and tape rows writable 16 bytes at a time, v and y rows eight.  The line lies at the second chunk as that is where
+// More than one chunk, and k and q rows readable 16 bytes at a time.  The line lies at the second chunk as that is where
 // there is something to prepare ahead; this kernel is the faster one from there on (us, 17 and 32 steps: 32 heads of 128x128
 // 6.1 -> 5.1 and 6.3 -> 5.1, two such sequences 7.5 -> 5.9 and 7.9 -> 6.8, Dk = 256 17.0 -> 11.6 and 17.5 -> 11.8).  f16 inputs
 // stay with the chunk by chunk kernel: three f16 terms do not hold an fp32 state.
 bool gdn_long_applies(const GdnArgs& A, int Dk) {
-    return A.in_dtype == DFLASH_BF16 && A.T > kChunkSteps && (((uintptr_t)A.k | (uintptr_t)A.q | (uintptr_t)A.tape) & 15) == 0 &&
-           (((uintptr_t)A.v | (uintptr_t)A.y) & 7) == 0 && (Dk == 64 || Dk == 128 || Dk == 256);
+    return A.in_dtype == DFLASH_BF16 && A.T > kChunkSteps && (((uintptr_t)A.k | (uintptr_t)A.q) & 15) == 0 && (Dk == 64 || Dk == 128 || Dk == 256);
 }
 
 int launch_gdn_long(hipStream_t st, const GdnArgs& A, int B, int Dk) {

@@ -98,15 +98,24 @@ def test_long_forward(gpu_lib, Dk, Dv, T, masked):
     np.testing.assert_allclose(host(y2), host(y), rtol=2e-2, atol=2e-2)
 
 
-# v rows that cannot be read eight bytes at a time take the chunk-by-chunk kernel as well
-@pytest.mark.parametrize("off", [2, 4])
+# v, y and the tape may lie at any address of their elements: the kernel of aligned ones, hence its bits, and nothing beside them
+@pytest.mark.parametrize("off", [1, 2, 4])
 def test_long_forward_v_alignment(gpu_lib, off):
     from swiftlm_amd import DFlashKernels as K
+    from swiftlm_amd._lib import native
 
     d = O.make_gdn_inputs(3, 1, 50, 2, 4, 128, 48, in_dtype="bf16")
     q, k, v, g, beta = [dev(d[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")]
     moved = torch.empty(v.numel() + off, dtype=v.dtype, device="cuda")[off:].view(v.shape).copy_(v)
     y, s, tape = K.gated_delta_kernel_with_tape(q, k, moved, g, beta, dev(d["state"]))
+    for got, want in zip((y, s, tape), K.gated_delta_kernel_with_tape(q, k, v, g, beta, dev(d["state"]))):
+        assert torch.equal(got, want)
+    ym, tm = (torch.full((t.numel() + 2 * off,), 7.0, dtype=t.dtype, device="cuda") for t in (y, tape))
+    inner = lambda t, like: t[off:-off].view(like.shape)
+    sm = torch.empty_like(s)
+    native.gated_delta_into(native.current_stream(), q, k, moved, g, beta, dev(d["state"]), sm, inner(ym, y), inner(tm, tape), 2, 4, 128, 48)
+    assert torch.equal(inner(ym, y), y) and torch.equal(inner(tm, tape), tape) and torch.equal(sm, s)
+    assert all(bool((t[:off] == 7).all() and (t[-off:] == 7).all()) for t in (ym, tm))
     yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], dtype=np.float64)
     np.testing.assert_allclose(host(s), sw, rtol=1e-4, atol=1e-6)
     np.testing.assert_allclose(host(tape), tw, rtol=1e-4, atol=1e-5)
