@@ -342,47 +342,55 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 
 // Where one workgroup per query head is the faster form: no more heads than compute units, as the workgroups of a second round
 // wait for the first, and few enough keys for the split form's second launch and its partial rows to cost more than the serial
-// tiles here; with many heads that form has longer splits to do, too.  us per call, split form against this one:
-//     heads, keys  D=128   128        600         800         1000        1200       D=256   128       350         500         600
-//     8 (Hk=1)          6.1 4.8   8.3 6.6     8.3 7.6     8.5 8.5     8.4 9.5           8.1 6.0   9.2 8.7     9.2 9.9     9.3 11.1
-//     16 (Hk=2)         6.1 4.8   8.2 6.6     8.3 7.7     8.5 8.6     8.7 9.6           8.2 6.0   9.3 8.7     9.4 10.0    9.4 11.1
-//     64 (B=2)          6.0 4.7   8.8 6.7     9.1 7.8     10.1 8.7    10.0 9.8          8.1 6.1   10.4 8.8    10.9 10.1   13.2 11.4
-//     128 (B=4)         6.1 4.8   10.2 7.0    11.0 8.1    11.0 9.3    11.5 10.5         8.2 6.2   11.3 9.1    12.5 10.7   12.2 11.9
-//     256 (B=8)         6.1 4.9   12.1 7.5    12.6 8.6    13.3 9.8    14.5 11.2         8.5 6.6   13.6 9.6    15.2 11.3   16.6 12.7
-//     512 (B=8)         6.4 7.0   14.2 12.9   15.5 15.1   16.5 17.4   17.9 20.2         9.0 11.6  16.5 17.3   18.5 20.3   19.6 23.0
+// tiles here; with many heads that form has longer splits to do, too.  Behind that line several workgroups share a head's keys, as
+// many as fill the chip, and the combine kernel merges their rows: it has S partial rows of each query row to read where the form
+// with shared tiles has a multiple of that, and its own launch has no pipeline to fill.  S is a multiple that keeps the heads of a
+// group, which read their KV head's rows G times, on one XCD (the L2s share nothing; with S = 21 for 12 heads over 2 KV heads 3,000
+// keys took 12.7 us, with 20 11.2); at D = 128 no more than 16, as the combine then needs one round per lane.
 //
-// Behind that line several workgroups share a head's keys, as many as fill the chip, and the combine kernel merges their rows: it
-// has S partial rows of each query row to read where the form with shared tiles has a multiple of that, and its own launch has
-// no pipeline to fill.  As long as one workgroup's share is small, as the group's heads read their KV head's rows G times through
-// the L2s (which share nothing: S is a multiple that keeps the heads of a group on one XCD; with S = 21 for 12 heads over 2 KV heads
-// 3,000 keys took 12.7 us, with 20 11.2), and all K/V rows come from memory at most 48 MB.  Few heads take no more than 16 splits,
-// or shares of 512 keys, at D = 128, as the combine then needs one round per lane, and fewer than 16 heads no more than 3,584 keys.  All forms of a call take the same line, so that
-// they give the same bits.  us per call, shared tiles against this form:
-//     heads, keys        1500        2048        3000        4112        6000        8208        12000
-//     D=128  8 (Hk=1)  8.3  8.2    8.4  8.4    8.5  8.5    8.9  9.1    9.0  9.5    9.7  10.0   10.3 11.0
-//           16 (Hk=2)  9.1  8.2    9.3  8.5    9.5  8.6    9.5  9.2    10.9 9.7    11.0 10.2   11.9 11.4
-//           32 (Hk=8)  9.0  8.5    9.9  9.1    11.2 9.9    11.7 10.7   12.5 11.8   13.6 13.5   15.7 16.2
-//           64 (Hk=8)  10.7 9.8    11.5 10.3   12.5 11.5   12.7 12.9   13.0 15.5
-//     D=256  8 (Hk=1)  9.1  8.4    9.3  8.6    10.9 9.5    13.7 10.2   12.3 10.7   14.7 11.2   14.0 12.3
-//           16 (Hk=2)  10.6 9.6    11.3 10.1   11.3 10.8   12.5 11.3   13.1 12.3   14.3 13.6   14.6 16.3
-//                      (5000 12.2 11.7, paged 12.6 12.8; 7500 13.0 13.9, paged 13.7 14.8)
-//           24 (Hk=4)  (5000 13.8 14.2, paged 14.1 14.9)
-//           32 (Hk=8)  12.0 10.9   13.0 11.3   14.0 12.7   14.4 14.2   16.2 17.4
-//           64 (Hk=8)  13.4 12.5   14.4 13.9   15.7 16.7   17.0 19.4
+// A wave has one tile under way where the form with shared tiles has several, so K and V from memory cost this form more than from a
+// cache, and a model that goes through its weights between two calls finds them in memory.  The lines lie where the sum of
+// both times is least: us per call, launches of a captured graph, K and V of 20 MB in turn (cache) and of 500 MB (memory).  All forms of a
+// call take the same line, so that they give the same bits.
+//     heads, keys            one workgroup   a few splits   shared tiles           heads, keys            one workgroup   a few splits   shared tiles
+//     D=128  8 (Hk=1)   512   6.7  6.6        7.1  7.7       7.5  7.8       D=256  8 (Hk=1)   160   7.0  6.9        7.2  7.1       8.3  8.2
+//                       700   8.0  8.2        7.2  7.7       8.2  8.5                         256   7.7  7.5        7.3  7.8       8.4  8.6
+//            32 (Hk=8)  400   6.2  7.6        7.4  7.7       7.9  7.8              32 (Hk=8)  200   7.6  8.8        8.3  8.2       8.9  9.0
+//                       600   7.0  9.1        7.5  7.8       8.5  8.4                         300   8.1 10.2        8.5  8.5       9.3  9.3
+//            64 (Hk=8)  600   7.1  9.0        8.2  8.7       9.1  9.4              64 (Hk=8)  300   8.1 10.0        9.4  9.8      10.8 11.0
+//                       800   8.0 10.3        8.4  9.2       9.2  9.3                         416   9.1 11.4        9.8 10.2      11.0 11.2
+//            128 (B=4)  896   9.1 12.0       10.3 12.2      11.3 11.4              128 (B=4)  416   9.8 12.3       11.4 12.8      11.8 12.4
+//                       1152 10.4 14.0       11.3 13.4      12.4 12.2                         576  11.5 15.1       12.1 14.5      12.8 13.3
+//            256 (B=8)  1152 11.6 16.9                      14.8 15.5              256 (B=8)  576  12.6 17.4                      16.7 16.8
+//     a few splits against shared tiles, and the same from pages (which cost this form a table look-up per tile):
+//     D=128  4 (Hk=1)   2048  7.6  8.2   8.2  8.3      3000   8.2  8.8   8.2  8.1
+//            8 (Hk=1)   2048  7.6  8.2   8.6  8.7      3000   8.3  8.8   8.6  8.5 (paged 8.7  9.4   8.8  8.6)   4112   8.8  9.8   8.8  9.0
+//            16 (Hk=2)  3000  8.4  9.1   9.6  9.7 (paged 8.8  9.6   9.8  9.8)     4112   9.3 10.1  10.1  9.5    8208   9.9 12.0  11.2 10.5
+//            32 (Hk=8)  3000 10.0 11.2  11.3 11.0 (paged 10.4 12.0  11.6 11.1)    4112  10.9 12.6  11.9 11.4    6000  12.2 14.9  12.9 12.7
+//            64 (Hk=8)  1500  9.6 10.7  10.9 10.1      2048  10.0 11.9  11.7 10.7      3000  11.8 14.0  12.8 11.9
+//     D=256  4 (Hk=1)   8208 10.3 11.2  12.8 12.3      12000 11.1 12.3  12.5 11.6
+//            8 (Hk=1)   6000 11.0 11.6  11.6 12.2 (paged 11.3 12.6  11.8 12.3)    8208  11.5 12.7  15.0 13.5    12000 12.8 14.7  14.3 13.5
+//            16 (Hk=2)  1000  8.5  8.7   9.4  9.8      2048  10.1 10.5   9.8 10.2      4112  11.3 12.8  13.2 11.9    5000  11.8 13.7  12.4 12.5
+//            24 (Hk=4)  2048 11.2 12.4  12.7 11.6      3000  12.3 14.0  13.5 12.7      4112  13.6 15.8  14.3 13.4
+//            32 (Hk=8)  2048 11.3 13.3  13.4 12.6 (paged 12.2 14.1  13.8 12.7)    3000  13.2 15.9  14.9 14.0
+//            64 (Hk=8)  1000 11.6 12.9  13.0 13.2      1500  12.9 15.1  14.0 14.3      2048  14.2 17.2  14.8 15.3
+// From 1,500 to 3,000 keys at 16 heads of D = 256 the two are within 0.7 us of each other.  Two splits do not pay (96 heads of D = 256, 448 keys:
+// 11.2 12.6, shared tiles 11.2 11.8), and more than 48 MB of K and V rows, which the form with shared tiles streams, were not looked for.
 int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     const int64_t heads = (int64_t)B * Hq;
     const int cus = num_compute_units();
-    const bool few = heads < cus / 4;
     if (heads > cus) return 0;
-    if (N <= (D == 128 ? (few ? 896 : 1152) : (few ? 416 : 576))) return 1;
-    if (heads < (D == 128 ? 8 : 4) || (int64_t)B * Hk * N * D > 12000000) return 0;
+    const int one = D == 128 ? (heads < cus / 4 ? 512 : heads == cus / 4 ? 640 : heads <= cus / 2 ? 896 : 1152)
+                             : (heads < cus / 8 ? 192 : heads < cus / 4 ? 256 : heads == cus / 4 ? 320 : heads <= cus / 2 ? 448 : 576);
+    if (N <= one) return 1;
+    if ((int64_t)B * Hk * N * D > 12000000) return 0;
     int64_t S = cus / heads;
-    if (D == 128 && S > 16) S = S < N / 512 ? S : N / 512 > 16 ? N / 512 : 16;
+    if (D == 128 && S > 16) S = 16;
     if (S > most) S = most;
     const int same_xcd = Hk % 8 == 0 ? 1 : Hk % 4 == 0 ? 2 : Hk % 2 == 0 ? 4 : 8;
     if (S > same_xcd) S -= S % same_xcd;
-    const int64_t most_keys = D == 256 ? (heads < 32 ? 320 : 512) * S : heads < 16 ? 3584 : 900 * S;
-    return S >= (D == 128 ? 3 : 2) && N <= most_keys ? (int)S : 0;
+    const int64_t most_keys = D == 256 ? 288 * S : heads < 8 ? 2048 : S > 8 ? 3584 : 400 * S;
+    return S >= 3 && N <= most_keys ? (int)S : 0;
 }
 
 dflash_launch_shape sdpa_short_shape(int B, int Hk, int G, int S, int D) {

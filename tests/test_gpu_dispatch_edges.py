@@ -245,17 +245,30 @@ def test_combine_rows_in_flight(gpu_lib, D, N, S):
     attend(*tensors(N + D, 1, 3, 1, N, D), [N], D)
 
 
+def short_splits(B, Hq, Hk, N, D):
+    """Splits of the form with a workgroup per query head, 0 where the form with shared tiles runs; by the library's own account."""
+    from swiftlm_amd import _lib
+
+    shapes = (_lib.LaunchShape * 2)()
+    assert _lib.load().dflash_profile_sdpa_launches(_lib.BF16, B, Hq, Hk, N, D, shapes) > 0
+    return shapes[0].grid_x // Hk if shapes[0].kernel == b"sdpa_short_kernel" else 0
+
+
 # Short contexts in one launch, up to a line of keys that depends on the query heads (B * Hq), then a few splits of the same form, then
 # the form with shared tiles, which more heads than compute units take at once.  Tiles of 32 (D = 128) and 16 keys, eight waves, one
-# tile a wave and more; the second sequence leaves splits without a tile; 12 heads whose splits are rounded to whole XCDs.
+# tile a wave and more; the second sequence leaves splits without a tile; 24 heads whose splits are rounded to whole XCDs.
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("Hq,Hk,D,N", [(2, 1, 128, 31), (3, 1, 128, 256), (3, 1, 128, 257), (12, 2, 128, 600), (8, 1, 128, 896), (8, 1, 128, 897),
-                                       (32, 8, 128, 1152), (32, 8, 128, 1153), (2, 1, 256, 17), (3, 1, 256, 128), (3, 1, 256, 129),
-                                       (8, 1, 256, 416), (8, 1, 256, 417), (32, 8, 256, 576), (32, 8, 256, 577), (130, 2, 128, 100), (130, 2, 256, 129),
-                                       (6, 1, 128, 1750), (4, 1, 128, 3584), (4, 1, 128, 3585), (6, 2, 256, 6400), (6, 2, 256, 6401), (4, 1, 128, 7200), (4, 1, 128, 7201), (6, 2, 256, 5760), (6, 2, 256, 5761), (16, 8, 256, 2048), (16, 8, 256, 2049)])
-def test_short_contexts(gpu_lib, Hq, Hk, D, N, dt):
+@pytest.mark.parametrize("Hq,Hk,D,N,S", [
+    (2, 1, 128, 31, 1), (3, 1, 128, 257, 1), (8, 1, 128, 512, 1), (8, 1, 128, 513, 16), (32, 8, 128, 640, 1), (32, 8, 128, 641, 4), (64, 8, 128, 896, 1),
+    (64, 8, 128, 897, 0), (66, 6, 128, 1152, 1), (66, 6, 128, 1153, 0), (130, 2, 128, 100, 0),
+    (2, 1, 256, 17, 1), (3, 1, 256, 129, 1), (8, 1, 256, 192, 1), (8, 1, 256, 193, 7), (16, 2, 256, 256, 1), (16, 2, 256, 257, 8), (32, 8, 256, 320, 1),
+    (32, 8, 256, 321, 4), (64, 8, 256, 448, 1), (64, 8, 256, 449, 0), (66, 6, 256, 576, 1), (66, 6, 256, 577, 0), (130, 2, 256, 129, 0),
+    (1, 1, 128, 2048, 16), (1, 1, 128, 2049, 0), (12, 2, 128, 3200, 8), (12, 2, 128, 3201, 0), (4, 1, 128, 3584, 16), (4, 1, 128, 3585, 0), (32, 8, 128, 1600, 4),
+    (32, 8, 128, 1601, 0), (6, 2, 256, 5760, 20), (6, 2, 256, 5761, 0), (16, 8, 256, 2304, 8), (16, 8, 256, 2305, 0), (1, 1, 256, 9000, 64)])
+def test_short_contexts(gpu_lib, Hq, Hk, D, N, S, dt):
     from swiftlm_amd import DFlashKernels as K
 
+    assert short_splits(2, Hq, Hk, N, D) == S
     lens = [N, max(16, N // 2 + 1) if N < 4000 else 17]
     q, k, v = tensors(N + D, 2, Hq, Hk, N, D, dt)
     kv_len = torch.tensor(lens, dtype=torch.int32, device="cuda")
@@ -273,12 +286,16 @@ def test_short_contexts(gpu_lib, Hq, Hk, D, N, dt):
     assert torch.equal(kc, k) and torch.equal(vc, v)
 
 
-# The split form's mask, four keys per load: rows of odd and even length, a last tile of one key and of all but one.
-@pytest.mark.parametrize("N", [1185, 1186, 1187, 1189, 1215, 1216])
-@pytest.mark.parametrize("Hq,Hk,D", [(3, 1, 256), (10, 2, 128)])
-def test_mask_row_ends(gpu_lib, N, Hq, Hk, D):
+# The mask's loads, four keys each in the form with shared tiles: rows of odd and even length, a last tile of one key and of all but
+# one; one split of either form and several.
+@pytest.mark.parametrize("N", [0, 1, 2, 3, 5, 31])
+@pytest.mark.parametrize("Hq,Hk,D,base,short", [(3, 1, 256, 1184, True), (10, 2, 128, 1184, True), (64, 8, 256, 1184, False), (64, 8, 128, 1184, False),
+                                                (130, 10, 128, 64, False), (130, 10, 256, 64, False)])
+def test_mask_row_ends(gpu_lib, N, Hq, Hk, D, base, short):
     from swiftlm_amd import DFlashKernels as K
 
+    N += base
+    assert (short_splits(2, Hq, Hk, N, D) > 0) == short
     q, k, v = tensors(N + D, 2, Hq, Hk, N, D)
     g = torch.Generator(device="cuda").manual_seed(N)
     mask = torch.randn(2, Hq, 16, N, generator=g, device="cuda").masked_fill(torch.rand(2, Hq, 16, N, generator=g, device="cuda") < 0.3, float("-inf"))
@@ -426,10 +443,11 @@ def same_rows(out, lse, ow, lw):
 
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 @pytest.mark.parametrize("N", [33, 47, 97, 110, 129, 2049, 2063])
-@pytest.mark.parametrize("Hq,Hk,D", [(3, 1, 256), (8, 8, 128)])
-def test_last_tile_hidden_by_the_causal_rule(gpu_lib, N, Hq, Hk, D, bad):
+@pytest.mark.parametrize("Hq,Hk,D,short", [(3, 1, 256, True), (8, 8, 128, True), (264, 8, 128, False), (264, 8, 256, False)])
+def test_last_tile_hidden_by_the_causal_rule(gpu_lib, N, Hq, Hk, D, short, bad):
     from swiftlm_amd import DFlashKernels as K
 
+    assert (short_splits(1, Hq, Hk, N, D) > 0) == short
     q, k, v = tensors(N + D, 1, Hq, Hk, N, D)
     keys = N % 32                                             # of the last tile; row r sees keys up to N - 16 + r
     want = O.sdpa_block_causal(host(q), host(k), host(v), 0.1)
@@ -442,10 +460,11 @@ def test_last_tile_hidden_by_the_causal_rule(gpu_lib, N, Hq, Hk, D, bad):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("N,tiles", [(64, [1]), (100, [0, 2]), (128, [0]), (128, [1, 3]), (2048, [0]), (2048, [16, 33]), (2048, [48]), (2048, [0, 16, 47])],
                          ids=str)
-@pytest.mark.parametrize("Hq,Hk,D", [(8, 8, 128), (32, 8, 256)])
-def test_tiles_hidden_by_the_mask(gpu_lib, N, tiles, Hq, Hk, D, dt):
+@pytest.mark.parametrize("Hq,Hk,D,short", [(8, 8, 128, True), (32, 8, 256, True), (264, 8, 128, False), (264, 8, 256, False)])
+def test_tiles_hidden_by_the_mask(gpu_lib, N, tiles, Hq, Hk, D, short, dt):
     from swiftlm_amd import DFlashKernels as K
 
+    assert (short_splits(1, Hq, Hk, N, D) > 0) == short
     q, k, v = tensors(N + D, 1, Hq, Hk, N, D, dt)
     mask = 0.1 * torch.randn(1, Hq, 16, N, generator=torch.Generator(device="cuda").manual_seed(N), device="cuda")
     for t in tiles:
@@ -468,7 +487,7 @@ def test_tiles_hidden_by_the_mask(gpu_lib, N, tiles, Hq, Hk, D, dt):
 # Row r of the block sees keys up to N - 16 + r.
 @pytest.mark.parametrize("Hq,Hk,D,N,key", [(4, 2, 128, 33, 32), (4, 2, 256, 33, 32), (3, 1, 128, 300, 299), (3, 1, 256, 300, 31), (16, 2, 256, 1025, 1024),
                                            (16, 2, 256, 4100, 63), (8, 1, 128, 1025, 1024), (8, 1, 128, 8193, 8192), (8, 8, 128, 8193, 703), (64, 8, 256, 4097, 4096),
-                                           (520, 1, 128, 97, 96), (520, 1, 128, 300, 290)])
+                                           (520, 8, 128, 97, 96), (520, 8, 128, 300, 290), (264, 8, 256, 97, 96), (264, 8, 256, 300, 290)])
 def test_tile_with_only_a_nan_score_is_not_hidden(gpu_lib, Hq, Hk, D, N, key):
     from swiftlm_amd import DFlashKernels as K
 
