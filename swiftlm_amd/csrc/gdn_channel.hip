@@ -32,8 +32,8 @@ namespace dflash {
 // Bound by the SIMDs' issue: an fp32 MFMA keeps the vector instructions of other waves on its SIMD from issuing (32 cycles each;
 // 28 of the chain and 16 of waves 4-11 per chunk at Dk = 128, beside 290 + 200 vector instructions), so an interval is 4,200
 // cycles at Dk = 128 and 2,700 at 64; with one set of pair waves, whose waits nothing filled, it was 4,700 and 3,100.
-// us, step kernel against this one: 1,003 steps, 32 heads of 128x128 228 -> 111; 8 heads of 64x64 168 -> 74; two sequences of
-// 300 steps 90 -> 72.
+// us, step kernel against this one: 1,003 steps, 32 heads of 128x128 228 -> 119; 8 heads of 64x64 170 -> 75; two sequences of
+// 300 steps 90 -> 75.
 // ---------------------------------------------------------------------------
 
 template <int DK> struct GdnChannelLds {
@@ -42,9 +42,10 @@ template <int DK> struct GdnChannelLds {
     static constexpr int LD = DK + 4;
     static constexpr int TP = 20;              // (and here the 16 steps of a channel)
     float kd[2][16][LD], qd[2][16][LD];        // D(-1, t) k_t and D(-1, t) q_t
-    float kt[2][DK][TP];                       // D(s, 15) k_s, steps of a channel
+    float kt[2][DK][TP];                       // D(s, 15) k_s of a channel, step s at 4 (s % 4) + s / 4
     float gend[2][DK];                         // D(-1, 15)
-    // waves 4-7, private: operands of the pairs across the boundaries 4 and 12 [0] and 8 [1]: eight rows k_s, then k_t, then q_t
+    // operands of the pairs across the boundaries 4 and 12 [0] and 8 [1]: eight rows k_s, then k_t, then q_t.  Waves 4 + p and 8 + p share
+    // x[p] without a barrier of their own: each writes it and reads it back within one interval, the two in alternate ones.
     float x[4][2][24][XP];
     float pt[2][4][2][16][20];                 // partial A and C of the four channel groups, [t][s]
     float na[2][16][16];                       // na[t][s] = -beta_t A[t][s] for s < t, else 0
@@ -93,6 +94,13 @@ __device__ __forceinline__ void of_rows(float x, float (&r)[4]) {
     const auto e = __builtin_amdgcn_permlane32_swap(h[0], h[0], false, false), o = __builtin_amdgcn_permlane32_swap(h[1], h[1], false, false);
     r[0] = __uint_as_float(e[0]); r[1] = __uint_as_float(o[0]);
     r[2] = __uint_as_float(e[1]); r[3] = __uint_as_float(o[1]);
+}
+// The 4 x 4 of registers and 16-lane rows transposed: element e of row g gets element g of row e.
+__device__ __forceinline__ f32x4v across_rows(f32x4v x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[0]), __float_as_uint(x[1]), false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[2]), __float_as_uint(x[3]), false, false);
+    const auto even = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false), odd = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+    return f32x4v{__uint_as_float(even[0]), __uint_as_float(odd[0]), __uint_as_float(even[1]), __uint_as_float(odd[1])};
 }
 __device__ __forceinline__ bool any_not_finite(f32x4v x) {
     return __builtin_amdgcn_ballot_w64(!(fabsf(x[0]) + fabsf(x[1]) + fabsf(x[2]) + fabsf(x[3]) < __builtin_inff())) != 0;
@@ -189,10 +197,13 @@ __global__ __launch_bounds__(kChannelThreads) void gated_delta_channel_kernel(Gd
             if (w == 0) *reinterpret_cast<f32x4v*>(L.dl[par][lane]) = dl;
 #pragma unroll
             for (int i = 0; i < NB; ++i) s[i] *= ge[i];
+            // Added in the order of the steps, four neighbours per product, so that the latest ones, which fast decays leave the largest, come
+            // last: with every fourth step in a product the state's error was up to 1.6 times that of the steps one by one.
+            const f32x4v ds = across_rows(dl);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int i = 0; i < NB; ++i) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[i][e], dl[e], s[i], 0, 0, 0);
+                for (int i = 0; i < NB; ++i) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[i][e], ds[e], s[i], 0, 0, 0);
             if (m + 1 < chunks) {
                 own = product(kx);
                 *reinterpret_cast<f32x4v*>(L.pk[par ^ 1][w][lane]) = own;
@@ -254,7 +265,8 @@ __global__ __launch_bounds__(kChannelThreads) void gated_delta_channel_kernel(Gd
         auto put_held = [&](int par) __attribute__((always_inline)) {      // read one interval later than the rest
 #pragma unroll
             for (int e = 0; e < NB; ++e) {
-                *reinterpret_cast<f32x4v*>(&L.kt[par][ch + e][4 * g]) = held[e];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) L.kt[par][ch + e][4 * r + g] = held[e][r];
                 if (g == 0) L.gend[par][ch + e] = gend[e];
             }
         };
@@ -501,12 +513,14 @@ static int launch_channel(hipStream_t st, const GdnArgs& A, int B) {
 
 // Where it is the faster one.  A workgroup (16 state rows of a head) has a compute unit to itself, and its first two chunks cost what
 // 22 steps of the step kernel do, so with a workgroup for every unit or fewer the line lies at 24 steps (us, step kernel against
-// this one, 32 heads of 128x128: 17 steps 6.8 / 7.0, 24 steps 7.8 / 7.1, 48 steps 13.0 / 9.0; two heads of 64x64 5.3 / 5.7, 5.9 / 5.8,
-// 9.1 / 6.8).  Two workgroups of the step kernel share a unit and fill each other's waits: with more than one round the line is at 96
-// steps (two rounds of 128x128, 33 steps 14.3 / 17.3, 64 steps 21.9 / 21.9, 100 steps 33.5 / 31.9, 257 steps 78.9 / 65.6; of 64x128 64
-// steps 15.5 / 16.5, 128 steps 28.1 / 25.4; three rounds of 128x128, 100 steps 51.3 / 46.8).  From three rounds on Dk = 64 stays with
-// the step kernel (four rounds, 257 steps 82.2 / 87.7); more than three rounds of Dk = 128, where that has two rows per thread, leave
-// it at 320 steps (four rounds, 100 steps 52.1 / 61.4, 257 steps 124.4 / 128.7, 500 steps 236.6 / 230.0; six, 500 steps 379 / 346).
+// this one, 32 heads of 128x128: 17 steps 7.4 / 7.7, 24 steps 8.7 / 7.9, 48 steps 14.5 / 10.8; two heads of 64x128 5.4 / 5.8, 6.1 / 6.0,
+// 9.5 / 7.1).  Two workgroups of the step kernel share a unit and fill each other's waits: with more than one round the line is at 96
+// steps (two rounds of 128x128, 33 steps 15.6 / 18.9, 64 steps 23.7 / 24.0, 100 steps 35.2 / 34.4, 257 steps 80.2 / 68.4; of 64x128 64
+// steps 15.9 / 17.3, 128 steps 28.7 / 26.7; three rounds of 128x128, 64 steps 34.2 / 32.8, 96 steps 49.0 / 43.1, 128 steps 63.4 / 53.9,
+// 192 steps 93 / 75, 257 steps 124 / 100).  From three rounds on Dk = 64 stays with the step kernel (three rounds, 128 steps 35.6 / 38.1,
+// 257 steps 67.9 / 68.1; four, 257 steps 86.4 / 91.0); more than three rounds of Dk = 128, where that has two rows per thread, leave
+// it at 320 steps (a little over three, 192 steps 93 / 97, 257 steps 124 / 131, 320 steps 151 / 152; four, 100 steps 53.9 / 62.8, 257 steps
+// 125.5 / 133.3, 320 steps 152.5 / 153.2, 500 steps 237.6 / 236.5; six, 320 steps 244 / 230, 500 steps 380 / 354).
 // Wider rows (Dk = 256) do not fit LDS.
 bool gdn_channel_applies(const GdnArgs& A, int B, int Dk) {
     if (A.in_dtype != DFLASH_BF16 && A.in_dtype != DFLASH_F16) return false;

@@ -543,6 +543,29 @@ def test_channel_gate_chunks(gpu_lib, Dk, Dv, dt, T, masked):
             assert np.all(host(y)[off] == 0) and np.all(host(tape)[off] == 0)
 
 
+# The state is as near to 64 bits as the step kernel leaves it, also where decays are fast and the last chunk is a ragged one: the latest
+# steps are the largest terms, and each rounding of the sum behind them counts in full.  65,536 values: the ratio of the two errors
+# spreads by half a percent.
+@pytest.mark.parametrize("T", [29, 36, 42, 64, 78])
+@pytest.mark.parametrize("Dk", [64, 128])
+def test_channel_gate_state_error(gpu_lib, Dk, T):
+    from swiftlm_amd import DFlashKernels as K
+
+    d = O.make_gdn_inputs(Dk + T, 1, T, 4, 8, Dk, 8192 // Dk, in_dtype="bf16", vec_gate=True)
+    g = torch.sigmoid(torch.randn(d["g"].shape, generator=torch.Generator().manual_seed(T))).bfloat16()
+    d["g"] = g.float().numpy()
+    ins = [dev(d[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")]
+    want = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], dtype=np.float64)[1]
+
+    def error(steps):
+        state = dev(d["state"])
+        for t in range(0, T, steps):
+            state = K.gated_delta_kernel_with_tape(*[x[:, t:t + steps].contiguous() for x in ins], state)[1]
+        return np.linalg.norm(host(state).astype(np.float64) - want)
+
+    assert error(T) <= 1.05 * error(16)
+
+
 # An infinity or NaN of one step stays out of the steps before it (products over all steps of a chunk would spread it), of the other state
 # rows and, where the step is masked, out of everything
 @pytest.mark.parametrize("what", ["v", "beta", "k_masked", "state"])
