@@ -59,7 +59,7 @@ template <int DK> struct GdnLongLds {
     float pk[2][4][64][4], pq[2][4][64][4];// partial S_0 k_t and S_0 q_t of the four chain waves, as accumulators
     float dl[2][64][4];                    // lane (g, n): delta_s of row n, s = 4g + i
     float gam[2][16], w[2][16], beta[2][16];
-    uint32_t on[2];                        // bit t: step t counts
+    uint32_t on[2];                        // MASKED: bit t: step t counts
 };
 
 __device__ __forceinline__ void split3_bf16(f32x4v v, uint2& hi, uint2& mid, uint2& lo) {
@@ -73,7 +73,7 @@ template <int L0, int L1, int L2, int L3> __device__ __forceinline__ float quad_
 }
 constexpr int kLongThreads = 512;
 
-template <int DK>
+template <int DK, bool MASKED>
 __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnArgs A) {
     using Lds = GdnLongLds<DK>;
     extern __shared__ __align__(16) unsigned char gdn_chunk_smem[];
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             // overflow where no delta does.  Then the deltas are substituted for one step after the other.
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(dl[0]) + fabsf(dl[1]) + fabsf(dl[2]) + fabsf(dl[3]) < __builtin_inff())) != 0, 0)) {
                 rhs *= lds4(&L.beta[par][4 * g]);
-                const uint32_t on = L.on[par];
+                const uint32_t on = MASKED ? L.on[par] : 0xffffu;
                 for (int tg = 0; tg < 4; ++tg)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
     float G[4], gam = 0.f, gam_n = 0.f, beta = 0.f;   // gam_n: that of step n in every lane
     f32x4v vf, yv, dl;                                 // v of the chunk in hand; y and tape of the one before, not yet stored: step n, rows 4g .. +3
     bool step_on = false;
-    uint32_t counted = 0xffffu;                        // bit t: step t counts (without a mask all: what is missing of the last chunk meets nothing)
+    uint32_t counted = 0;                              // MASKED: bit t: step t counts
     auto store_rows = [&](int m, int tc) {             // one store each: row by row, two and four bytes per lane, they were eight
         const uint32_t o = (((uint32_t)b * A.T + m * kChunkSteps) * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(n, step);
         if (n < tc) {
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
                 kq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, q8, kq, 0, 0, 0);
             }
             step_on = n < tc;
-            if (A.mask != nullptr) {
+            if constexpr (MASKED) {
                 step_on = step_on && mask_on(A.mask, A.mask_dtype, (int)((uint32_t)b * A.T + t0 + min(n, tc - 1)));
                 counted = (uint32_t)__builtin_amdgcn_ballot_w64(step_on) & 0xffffu;
                 vr = step_on ? vr : make_uint2(0u, 0u);
@@ -360,7 +360,8 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             // T = (I + A)^-1 diag(beta), in the layout of the chain's a operand: lane (g, n) forms T[n][4g .. +3].  What other lanes
             // of this wave wrote is read back without a wait: LDS serves a wave's accesses in order.
             if (g == 0) { L.beta[par][n] = beta; L.gam[par][n] = gam; }
-            if (lane == 0) L.on[par] = counted;
+            if constexpr (MASKED)
+                if (lane == 0) L.on[par] = counted;
             asm volatile("" ::: "memory");             // written by the lanes g = 0, read by all
             *reinterpret_cast<f32x4v*>(&L.na[par][n][4 * g]) = av;
             float na[16];                              // row n of -A, the four lanes' pieces gathered
@@ -423,7 +424,7 @@ template <int DK>
 static int launch_long(hipStream_t st, const GdnArgs& A, int B) {
     dim3 grid(A.Dv / kChunkRows, A.Hv, B);
     LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);
-    DFLASH_HIP_TRY(br.launch(gated_delta_long_kernel<DK>, grid, dim3(kLongThreads), sizeof(GdnLongLds<DK>), A));
+    DFLASH_HIP_TRY(br.launch(A.mask ? gated_delta_long_kernel<DK, true> : gated_delta_long_kernel<DK, false>, grid, dim3(kLongThreads), sizeof(GdnLongLds<DK>), A));
     return DFLASH_OK;
 }
 
@@ -443,7 +444,8 @@ int launch_gdn_long(hipStream_t st, const GdnArgs& A, int B, int Dk) {
 
 template <int DK>
 static int long_setup() {
-    DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gated_delta_long_kernel<DK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GdnLongLds<DK>)));
+    const void* kernels[] = {(const void*)gated_delta_long_kernel<DK, true>, (const void*)gated_delta_long_kernel<DK, false>};
+    for (const void* k : kernels) DFLASH_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GdnLongLds<DK>)));
     return DFLASH_OK;
 }
 
