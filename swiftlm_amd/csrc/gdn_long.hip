@@ -35,10 +35,10 @@ namespace dflash {
 // Bound by the length of an interval: 1,350 / 1,600 / 2,200 cycles at Dk = 64 / 128 / 256, of which the chain works 1,200 /
 // 1,350 / 1,800 (the split of the state on the VALU, the exchange of the partial sums through LDS, three groups of
 // dependent MFMAs) and the busiest producer as long.  us, chunk by chunk kernel against this one: 1,003 steps,
-// 32 heads of 128x128 152 -> 43; 730 steps, 8 heads, Dk = 256 147 -> 43; two sequences of 1,000 steps, 32 heads, Dk = 256
+// 32 heads of 128x128 152 -> 42; 730 steps, 8 heads, Dk = 256 147 -> 43; two sequences of 1,000 steps, 32 heads, Dk = 256
 // 419 -> 116; 40 steps 8.3 -> 5.4.
 // 89 / 106 / 145 registers: two workgroups share a compute unit at Dk = 64 and 128 (two sequences of 1,000 steps 71 where one takes
-// 43), at 256 a second sequence waits for the first (59 for one).
+// 42), at 256 a second sequence waits for the first (59 for one).
 // ---------------------------------------------------------------------------
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));

@@ -25,8 +25,9 @@ namespace dflash {
 // MFMA 16x16x32, n = lane % 16, g = lane / 16: operands hold row (column) n, k-elements 8g .. 8g+7; the accumulator column n, rows
 // 4g .. 4g+3.  S^T = K Q^T, then O^T += V^T P^T, with P^T taken from the accumulators of S^T as they are: lane (n, g) holds keys
 // 4g .. 4g+3 of each 16 keys, and V^T is gathered in that order by the transposing LDS read (16x16x16 for a tile of 16 keys).
-// 16-byte piece p of row r stands at p ^ (r % 16) (K, Q) or p ^ 4 (r % 4) (V), which keeps the reads free of conflicts.  A wave's K
-// slot is asked for again behind its scores, its V slot behind the product.
+// 16-byte piece p of row r stands at p ^ (r % 16) (K, Q) or p ^ 4 (r % 4) (V), which leaves
+// few conflicts (by the counters, with the merge's among them, 19 % of the LDS cycles over 512 keys of D = 128, 14 % over 4,112 of
+// D = 256).  A wave's K slot is asked for again behind its scores, its V slot behind the product.
 // ---------------------------------------------------------------------------
 template <int D> struct SdpaShortLds {
     static constexpr int WAVES = 8;
