@@ -37,7 +37,9 @@ namespace dflash {
 // dependent MFMAs) and the busiest producer as long.  us, chunk by chunk kernel against this one: 1,003 steps,
 // 32 heads of 128x128 152 -> 42; 730 steps, 8 heads, Dk = 256 147 -> 43; two sequences of 1,000 steps, 32 heads, Dk = 256
 // 419 -> 116; 40 steps 8.3 -> 5.4.
-// 89 / 106 / 145 registers: two workgroups share a compute unit at Dk = 64 and 128 (two sequences of 1,000 steps 71 where one takes
+// The care for what is not finite (y, the rows of masked steps) costs or gives 3 %: 1,000 steps of Dk = 256 64.8 -> 66.9, Dk = 64 36.7 ->
+// 37.1, 1,003 steps of Dk = 128 43.1 -> 42.1.
+// 95 / 121 / 189 registers: two workgroups share a compute unit at Dk = 64 and 128 (two sequences of 1,000 steps 71 where one takes
 // 42), at 256 a second sequence waits for the first (59 for one).
 // ---------------------------------------------------------------------------
 
@@ -397,6 +399,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
 #pragma unroll
             for (int e = 0; e < 4; ++e) yv = __builtin_amdgcn_mfma_f32_16x16x4f32(ds[e], cv[e], yv, 0, 0, 0);
             // 0 times an infinity or NaN of a step behind n is not 0: sums that are not finite are formed again from the steps up to n
+            // (a test of the deltas, ahead of the product, takes as long)
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(yv[0]) + fabsf(yv[1]) + fabsf(yv[2]) + fabsf(yv[3]) < __builtin_inff())) != 0, 0)) {
                 yv = gam_n * pq;
                 for (int sg = 0; sg < 4; ++sg)
