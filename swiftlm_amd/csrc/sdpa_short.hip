@@ -350,8 +350,10 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 // keys took 12.7 us, with 20 11.2); at D = 128 no more than 16, as the combine then needs one round per lane.
 //
 // A wave has one tile under way where the form with shared tiles has several, so K and V from memory cost this form more than from a
-// cache, and a model that goes through its weights between two calls finds them in memory.  The lines lie where the sum of
-// both times is least: us per call, launches of a captured graph, K and V of 20 MB in turn (cache) and of 500 MB (memory).  All forms of a
+// cache, and a model that goes through its weights between two calls finds them in memory.  The ends of the few splits lie where the sum
+// of both times is least.  By that sum they would begin earlier, too, at 512 to 1,152 keys (D = 128) and 192 to 576: but one workgroup
+// merges in fp32 where partial rows have 16 bits (700 keys of D = 128: error against 64 bits 2.08e-3, split 2.63e-3; 300 of D = 256
+// 2.00e-3, 2.56e-3), so it keeps what it takes from a cache in about the time of the others.  us per call, launches of a captured graph, K and V of 20 MB in turn (cache) and of 500 MB (memory).  All forms of a
 // call take the same line, so that they give the same bits.
 //     heads, keys            one workgroup   a few splits   shared tiles           heads, keys            one workgroup   a few splits   shared tiles
 //     D=128  8 (Hk=1)   512   6.7  6.6        7.1  7.7       7.5  7.8       D=256  8 (Hk=1)   160   7.0  6.9        7.2  7.1       8.3  8.2
@@ -381,9 +383,8 @@ int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     const int64_t heads = (int64_t)B * Hq;
     const int cus = num_compute_units();
     if (heads > cus) return 0;
-    const int one = D == 128 ? (heads < cus / 4 ? 512 : heads == cus / 4 ? 640 : heads <= cus / 2 ? 896 : 1152)
-                             : (heads < cus / 8 ? 192 : heads < cus / 4 ? 256 : heads == cus / 4 ? 320 : heads <= cus / 2 ? 448 : 576);
-    if (N <= one) return 1;
+    const bool few = heads < cus / 4;
+    if (N <= (D == 128 ? (few ? 896 : 1152) : (few ? 416 : 576))) return 1;
     if ((int64_t)B * Hk * N * D > 12000000) return 0;
     int64_t S = cus / heads;
     if (D == 128 && S > 16) S = 16;

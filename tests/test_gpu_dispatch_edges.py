@@ -259,10 +259,10 @@ def short_splits(B, Hq, Hk, N, D):
 # tile a wave and more; the second sequence leaves splits without a tile; 24 heads whose splits are rounded to whole XCDs.
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("Hq,Hk,D,N,S", [
-    (2, 1, 128, 31, 1), (3, 1, 128, 257, 1), (8, 1, 128, 512, 1), (8, 1, 128, 513, 16), (32, 8, 128, 640, 1), (32, 8, 128, 641, 4), (64, 8, 128, 896, 1),
-    (64, 8, 128, 897, 0), (66, 6, 128, 1152, 1), (66, 6, 128, 1153, 0), (130, 2, 128, 100, 0),
-    (2, 1, 256, 17, 1), (3, 1, 256, 129, 1), (8, 1, 256, 192, 1), (8, 1, 256, 193, 7), (16, 2, 256, 256, 1), (16, 2, 256, 257, 8), (32, 8, 256, 320, 1),
-    (32, 8, 256, 321, 4), (64, 8, 256, 448, 1), (64, 8, 256, 449, 0), (66, 6, 256, 576, 1), (66, 6, 256, 577, 0), (130, 2, 256, 129, 0),
+    (2, 1, 128, 31, 1), (3, 1, 128, 257, 1), (8, 1, 128, 896, 1), (8, 1, 128, 897, 16), (32, 8, 128, 1152, 1), (32, 8, 128, 1153, 4), (64, 8, 128, 1152, 1),
+    (64, 8, 128, 1153, 0), (66, 6, 128, 1152, 1), (66, 6, 128, 1153, 0), (130, 2, 128, 100, 0),
+    (2, 1, 256, 17, 1), (3, 1, 256, 129, 1), (8, 1, 256, 416, 1), (8, 1, 256, 417, 8), (16, 2, 256, 416, 1), (16, 2, 256, 417, 8), (32, 8, 256, 576, 1),
+    (32, 8, 256, 577, 4), (64, 8, 256, 576, 1), (64, 8, 256, 577, 0), (66, 6, 256, 576, 1), (66, 6, 256, 577, 0), (130, 2, 256, 129, 0),
     (1, 1, 128, 2048, 16), (1, 1, 128, 2049, 0), (12, 2, 128, 3200, 8), (12, 2, 128, 3201, 0), (4, 1, 128, 3584, 16), (4, 1, 128, 3585, 0), (32, 8, 128, 1600, 4),
     (32, 8, 128, 1601, 0), (6, 2, 256, 5760, 20), (6, 2, 256, 5761, 0), (16, 8, 256, 2304, 8), (16, 8, 256, 2305, 0), (1, 1, 256, 9000, 64)])
 def test_short_contexts(gpu_lib, Hq, Hk, D, N, S, dt):
