@@ -112,7 +112,7 @@ __global__ __launch_bounds__(64) void accept_commit_kernel(const uint32_t* verif
 constexpr int kArgmaxThreads = 256;
 constexpr int kArgmaxChunk = 8192;
 constexpr int kArgmaxMaxRows = 1024;
-constexpr int kArgmaxMaxPartials = 4096;   // T * chunks the last workgroup can hold in LDS
+constexpr int kArgmaxMaxPartials = 4096;   // T * chunks that the last workgroup goes through
 
 struct GreedyArgs {
     const void* logits;            // [T, V]
@@ -128,6 +128,10 @@ struct GreedyArgs {
 
 __device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
 
+// Bound by two launches and a trip to memory each.  A thread's loads of the chunk are all under way before the first value is
+// looked at, 16 bytes each at whatever address the row begins: a vocabulary that is no multiple of eight leaves most rows
+// unaligned.  us, both kernels, 16 rows of bf16 logits: 151,937 entries 18.7 (unaligned rows element by element) -> 6.9, 151,936
+// entries 7.9 (a round trip per load, a row of partials per lane) -> 6.6.
 template <typename Elem>
 __global__ __launch_bounds__(kArgmaxThreads) void greedy_partial_kernel(GreedyArgs A) {
     __shared__ float val_s[kArgmaxThreads / 64];
@@ -136,40 +140,41 @@ __global__ __launch_bounds__(kArgmaxThreads) void greedy_partial_kernel(GreedyAr
     const Elem* lrow = reinterpret_cast<const Elem*>(A.logits) + (size_t)row * A.V;
     const float floor_v = to_float(from_float<Elem>(-1e9f));      // MLXArray(-1e9, dtype: logits.dtype) (:124)
     const int v0 = chunk * kArgmaxChunk;
-    const int v1 = (v0 + kArgmaxChunk) < A.V ? (v0 + kArgmaxChunk) : A.V;
 
+    constexpr int VEC = 16 / sizeof(Elem), PIECES = kArgmaxChunk / (VEC * kArgmaxThreads);   // elements of a load, loads of a thread
+    typedef uint32_t Words __attribute__((ext_vector_type(4)));
+    struct __attribute__((packed, aligned(sizeof(Elem)))) Piece { Words x; };
+    typedef typename std::conditional<VEC == 8, uint64_t, uint32_t>::type MaskWord;          // VEC mask bytes at once
+    struct __attribute__((packed, aligned(1))) MaskPiece { MaskWord x; };
     float best = -INFINITY;
     int besti = 0x7fffffff;
-    constexpr int VEC = 16 / sizeof(Elem);                        // elements per 16-byte load
-    typedef typename std::conditional<VEC == 8, uint64_t, uint32_t>::type MaskWord;   // VEC mask bytes at once
-    const bool aligned = ((size_t)row * A.V * sizeof(Elem)) % 16 == 0 && (uintptr_t)A.logits % 16 == 0 &&
-                         (uintptr_t)A.suppress % sizeof(MaskWord) == 0;
-    if (aligned) {
-        for (int i = v0 + tid * VEC; i < v1; i += kArgmaxThreads * VEC) {
-            if (i + VEC <= v1) {
-                Elem e[VEC];
-                *reinterpret_cast<uint4*>(e) = *reinterpret_cast<const uint4*>(lrow + i);
-                const MaskWord mw = A.suppress ? *reinterpret_cast<const MaskWord*>(A.suppress + i) : (MaskWord)0;
+    if (A.V >= VEC) {                                             // uniform
+        // pieces past the row's end are its last one again: the same values at the same indices, and '>' keeps the first
+        auto first = [&](int p) { return min(v0 + (p * kArgmaxThreads + tid) * VEC, A.V - VEC); };
+        Piece e[PIECES];
+        MaskPiece mw[PIECES];
 #pragma unroll
-                for (int u = 0; u < VEC; ++u) {
-                    float x = to_float(e[u]);
-                    if ((mw >> (8 * u)) & 0xff) x = floor_v;
-                    if (x > best) { best = x; besti = i + u; }    // ascending indices: '>' keeps the first maximum
-                }
-            } else {
-                for (int j = i; j < v1; ++j) {
-                    float x = to_float(lrow[j]);
-                    if (A.suppress && A.suppress[j]) x = floor_v;
-                    if (x > best) { best = x; besti = j; }
-                }
+        for (int p = 0; p < PIECES; ++p) {
+            e[p] = *reinterpret_cast<const Piece*>(lrow + first(p));
+            mw[p].x = 0;
+        }
+        if (A.suppress)
+#pragma unroll
+            for (int p = 0; p < PIECES; ++p) mw[p] = *reinterpret_cast<const MaskPiece*>(A.suppress + first(p));
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            Elem x8[VEC];
+            __builtin_memcpy(x8, &e[p], 16);
+#pragma unroll
+            for (int u = 0; u < VEC; ++u) {
+                float x = to_float(x8[u]);
+                if ((mw[p].x >> (8 * u)) & 0xff) x = floor_v;
+                if (x > best) { best = x; besti = first(p) + u; } // ascending indices: '>' keeps the first maximum
             }
         }
-    } else {
-        for (int j = v0 + tid; j < v1; j += kArgmaxThreads) {
-            float x = to_float(lrow[j]);
-            if (A.suppress && A.suppress[j]) x = floor_v;
-            if (x > best) { best = x; besti = j; }
-        }
+    } else if (tid < A.V) {
+        const float x = A.suppress && A.suppress[tid] ? floor_v : to_float(lrow[tid]);
+        if (x > best) { best = x; besti = tid; }
     }
     for (int o = 32; o >= 1; o >>= 1) {
         const float ov = __shfl_xor(best, o);
@@ -186,36 +191,52 @@ __global__ __launch_bounds__(kArgmaxThreads) void greedy_partial_kernel(GreedyAr
     }
 }
 
+// Sixteen lanes to a row, four partials of each asked for at once; the tokens to compare with and the start offset come in on the
+// same trip.
 __global__ __launch_bounds__(kArgmaxThreads) void greedy_finish_kernel(GreedyArgs A) {
-    const int tid = threadIdx.x;
-    // every thread fetches partials at once (one memory round trip), then one wave reduces them per
-    // row out of LDS
-    __shared__ float pv_s[kArgmaxMaxPartials];
-    __shared__ int pi_s[kArgmaxMaxPartials];
-    const int total = A.T * A.chunks;
-    for (int p = tid; p < total; p += kArgmaxThreads) {
-        pv_s[p] = A.part_val[p];
-        pi_s[p] = A.part_idx[p];
-    }
-    __syncthreads();
-    if (tid >= 64) return;
+    const int tid = threadIdx.x, sub = tid & 15;
     __shared__ uint32_t post_s[kArgmaxMaxRows];
-    for (int r = tid; r < A.T; r += 64) {
+    const uint32_t next_id = A.verify_ids && tid + 1 < A.T ? A.verify_ids[tid + 1] : 0u;
+    for (int r = tid >> 4; r < A.T; r += kArgmaxThreads / 16) {
+        const float* pv = A.part_val + r * A.chunks;
+        const int* pi = A.part_idx + r * A.chunks;
         float bv = -INFINITY;
         int bi = 0x7fffffff;
-        for (int c = 0; c < A.chunks; ++c)
-            if (better(pv_s[r * A.chunks + c], pi_s[r * A.chunks + c], bv, bi)) { bv = pv_s[r * A.chunks + c]; bi = pi_s[r * A.chunks + c]; }
+        for (int c0 = sub; c0 < A.chunks; c0 += 64) {
+            float v[4];
+            int x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int c = c0 + 16 * u < A.chunks ? c0 + 16 * u : c0;
+                v[u] = pv[c];
+                x[u] = pi[c];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (better(v[u], x[u], bv, bi)) { bv = v[u]; bi = x[u]; }
+        }
+#pragma unroll
+        for (int o = 8; o >= 1; o >>= 1) {
+            const float ov = __shfl_xor(bv, o);
+            const int oi = __shfl_xor(bi, o);
+            if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
+        }
         // a row of NaNs never compares greater than anything: token 0, like a scan that starts at index 0
         const uint32_t tok = bi == 0x7fffffff ? 0u : (uint32_t)bi;
-        post_s[r] = tok;
-        A.posterior[r] = tok;
+        if (sub == 0) {
+            post_s[r] = tok;
+            A.posterior[r] = tok;
+        }
     }
-    if (A.verify_ids) {
-        __builtin_amdgcn_s_waitcnt(0xc07f);                       // lgkmcnt(0): this wave's LDS writes have landed
-        __builtin_amdgcn_wave_barrier();
-        const int acc = A.T > 1 ? leading_matches(A.verify_ids + 1, post_s, A.T - 1) : 0;
-        if (tid == 0) store_accept(acc, post_s[acc], A.start_inout, A.out4);
+    if (!A.verify_ids) return;                                    // uniform
+    __syncthreads();
+    if (tid >= 64) return;
+    int acc = 0;                                                  // leading matches of verify_ids[1:] with the tokens
+    if (A.T > 1) {
+        const unsigned long long bal = __builtin_amdgcn_ballot_w64(tid < A.T - 1 && next_id != post_s[tid]);
+        acc = bal ? __builtin_ctzll(bal) : A.T - 1 <= 64 ? A.T - 1 : 64 + leading_matches(A.verify_ids + 65, post_s + 64, A.T - 65);
     }
+    if (tid == 0) store_accept(acc, post_s[acc], A.start_inout, A.out4);
 }
 
 // ---- conv-state rebuild ----------------------------------------------------

@@ -270,6 +270,47 @@ def test_greedy_tokens_with_mask_matches_oracle(gpu_lib, dt, V):
         np.testing.assert_array_equal(got.cpu().numpy().astype(np.uint32), want)
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("T,V,off", [(1, 1, 0), (3, 3, 1), (5, 7, 3), (16, 8, 1), (16, 9, 5), (70, 8191, 0), (7, 8193, 1), (4, 8199, 7),
+                                     (130, 8201, 3), (16, 20483, 2)])
+def test_greedy_tokens_at_any_row_address(gpu_lib, dt, T, V, off):
+    """Rows, logits and suppress mask that begin at any address of their elements; vocabularies around the length of a load and of
+    a workgroup's chunk; the largest value at the row's first and last entries, tied, suppressed, NaN beside it; a row of NaNs.
+    Whole numbers: they have to be equal.  The acceptance over them for every first mismatch that a block of T may have."""
+    import torch
+    from swiftlm_amd import DFlashRuntime
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dt]
+    g = torch.Generator(device="cuda").manual_seed(V + T)
+    logits = torch.empty(T * V + off, dtype=tdt, device="cuda")[off:].view(T, V)
+    logits.copy_(torch.randn(T, V, generator=g, device="cuda"))
+    for t in range(T):
+        logits[t, (0, V - 1, V // 2, max(V - 8, 0), min(8191, V - 1), min(8192, V - 1))[t % 6]] = 50.0
+        if t % 7 == 3:
+            logits[t, V - 1] = logits[t, V // 3] = 50.0
+        if t % 5 == 4:
+            logits[t, V // 4] = float("nan")
+    if T > 2:
+        logits[2] = float("nan")
+    host = logits.float().cpu().numpy()
+    for ids in (None, [0], [V - 1, V // 2], list(range(0, V, 3))):
+        mask_o = O.build_suppress_token_mask(V, ids)
+        mask_d = DFlashRuntime.build_suppress_token_mask(V, ids)
+        if mask_d is not None:
+            mask_d = torch.cat([mask_d.new_zeros(off), mask_d])[off:]
+        floor = {"bf16": O.round_to_bf16(np.float32([-1e9]))[0], "f16": np.float32(-np.inf), "f32": np.float32(-1e9)}[dt]
+        seen = host if mask_o is None else np.where(np.asarray(mask_o).astype(bool), floor, host)
+        want = np.array([0 if np.isnan(r).all() or np.nanmax(r) == -np.inf else np.nanargmax(r) for r in seen])
+        np.testing.assert_array_equal(DFlashRuntime.greedy_tokens_with_mask(logits, mask_d).cpu().numpy(), want)
+    for acc in sorted({0, 1, T // 2, T - 2, T - 1, 63, 64, 65} & set(range(T))):
+        verify = np.empty(T, np.int32)
+        verify[0], verify[1:] = 1, want[:-1]
+        if acc < T - 1:
+            verify[1 + acc] = want[acc] + 1
+        res, post = DFlashRuntime.greedy_accept_commit(logits, mask_d, torch.from_numpy(verify).cuda(), 9)
+        np.testing.assert_array_equal(post.cpu().numpy(), want)
+        assert (res.acceptance_len, res.commit_count, res.staged_first_next, res.start) == (acc, acc + 1, want[acc], 10 + acc)
+
+
 def test_greedy_accept_commit_equals_two_steps(gpu_lib):
     """One call = greedyTokensWithMask + matchAcceptanceLength + the commit bookkeeping; repeated
     calls reuse the workspace."""
