@@ -59,6 +59,19 @@ int gdn_device_setup();
 int rebuild_conv_batched(void* stream, int n, const void* const* snapshot_conv, const void* const* tape_qkv, void* const* out,
                          int B, int keep, int T, int C, int elem_bytes, int accepted_steps, const int32_t* steps_dev);
 
+// dflash_tape_replay_batched over n caches and, in the same launch, the conv windows of those with an out pointer:
+// out[l][b] = concat(snap[l][b] (null: zeros), qkv[l][b])[steps : steps + keep], rows of row16 pieces of 16 bytes.  The caller has
+// checked the windows' pointers: aligned to 16 bytes, and no window shares memory with anything else the launch reads or writes.
+struct ConvWindows {
+    const void* const* snap;
+    const void* const* qkv;
+    void* const* out;
+    int keep, row16;
+};
+int tape_replay_windows(void* stream, int n_layers, const void* const* tape, int tape_dtype, const void* const* k, const void* const* g,
+                        int in_dtype, int g_ndim, const void* const* state_in, void* const* state_out, int state_dtype, int steps, int B,
+                        int T_tape, int Hk, int Hv, int Dk, int Dv, const ConvWindows& win);
+
 // Launches one kernel and returns the HIP status.  When the thread was armed by dflash_profile_next_launch() for this
 // kernel id, the caller's events are attached to the dispatch itself (hipExtLaunchKernel), so their elapsed
 // time is the kernel's own begin-to-end duration, as a profiler reports it, not a bracket around it.

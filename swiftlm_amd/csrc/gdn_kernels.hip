@@ -87,7 +87,19 @@ template <int LAYERS> struct ReplayBatch {
     const void* state_in[LAYERS];
     void* state_out[LAYERS];
 };
-typedef ReplayBatch<DFLASH_MAX_BATCHED_LAYERS> ReplayTable;
+// A rollback over several caches also rebuilds their conv windows (rebuild_conv_batched): the same launch copies them, 16 bytes per
+// thread of the layer's first workgroups, asked for with the state rows.  A launch of its own behind the replay cost the host 4 us and
+// the GPU a dependent trip to memory.
+template <int LAYERS> struct ReplayWindows : ReplayBatch<LAYERS> {
+    const uint4* win_snap[LAYERS];     // [B,keep,row], null: zeros
+    const uint4* win_qkv[LAYERS];      // [B,T_tape,row]
+    uint4* win_out[LAYERS];            // [B,keep,row], null: no window for this layer
+    int keep, row16;                   // rows of a window (0: none at all), 16-byte pieces of a row
+};
+typedef ReplayWindows<DFLASH_MAX_BATCHED_LAYERS> ReplayTable;
+constexpr int kFewLayers = 8;          // tables of 1, 8 and 64: 0.1, 0.6 and 4.2 KB of arguments
+template <int LAYERS> struct ReplayParam { typedef ReplayWindows<LAYERS> type; };
+template <> struct ReplayParam<1> { typedef ReplayBatch<1> type; };
 
 struct ReplayArgs {
     const void* mask;        // [B,T_tape] or null
@@ -110,7 +122,7 @@ constexpr int kReplayChunk = 16;  // steps staged in LDS at a time (8 for Dk = 2
 // and NR passes (when DK/4 does not divide 256 the last few threads only help
 // with staging).  Grid: x = Dv tiles, y = b*Hv + hv, z = layer.
 template <typename StateT, bool VEC_G, int DK, int NR, int LAYERS>
-__global__ __launch_bounds__(kThreads) void tape_replay_kernel(ReplayBatch<LAYERS> P, ReplayArgs A) {
+__global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayParam<LAYERS>::type P, ReplayArgs A) {
     constexpr int TPR = DK / 4;
     constexpr int RPP = kThreads / TPR;
     constexpr int ROWS = RPP * NR;
@@ -265,6 +277,26 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(ReplayBatch<LAYER
         r = r < A.Dv ? r : A.Dv - 1;                       // clamped: rows outside are never stored
         s[i] = load4(s_in + (size_t)r * DK + c4);
     }
+    // The conv window: concat(snapshot, qkv)[n : n + keep] of this sequence, a piece per thread of its workgroups in turn.
+    uint4 win = make_uint4(0u, 0u, 0u, 0u);
+    int win_at = -1;                                       // the thread's first piece (-1: none)
+    auto window_piece = [&](int i, uint4& x) -> bool {
+        if constexpr (LAYERS > 1) {
+            const int j = i / P.row16, p = i - j * P.row16, src = n + j;
+            if (src >= P.keep + A.T_tape) return false;    // clamped slice end (RecurrentRollbackCache.swift:156)
+            const uint4* from = src < P.keep ? P.win_snap[layer] : P.win_qkv[layer];
+            const size_t at = src < P.keep ? (size_t)b * P.keep + src : (size_t)b * A.T_tape + (src - P.keep);
+            if (from) x = from[at * P.row16 + p];
+            else x = make_uint4(0u, 0u, 0u, 0u);
+            return true;
+        }
+        return false;
+    };
+    const int win_of = (hv * gridDim.x + blockIdx.x) * kThreads + tid;
+    if constexpr (LAYERS > 1) {
+        if (P.keep > 0 && P.win_out[layer])                // uniform
+            if (win_of < P.keep * P.row16 && window_piece(win_of, win)) win_at = win_of;
+    }
 
     for (int t0 = 0; t0 < n; t0 += TC) {
         const int tc = (n - t0) < TC ? (n - t0) : TC;
@@ -297,13 +329,32 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(ReplayBatch<LAYER
         const int r = row0 + rsub + RPP * i;
         if (owner && r < A.Dv) store4(s_out + (size_t)r * DK + c4, s[i]);
     }
+    if constexpr (LAYERS > 1) {
+        if (P.keep > 0 && P.win_out[layer]) {
+            const int pieces = P.keep * P.row16, all = A.Hv * gridDim.x * kThreads;
+            uint4* out = P.win_out[layer] + (size_t)b * pieces;
+            if (win_at >= 0) out[win_at] = win;
+            for (int i = win_of + all; i < pieces; i += all)        // windows larger than the grid has threads
+                if (window_piece(i, win)) out[i] = win;
+        }
+    }
 }
 
 template <typename StateT, bool VEC_G, int DK, int NR>
 static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, const ReplayArgs& A, int B, int n_layers) {
     constexpr int ROWS = kThreads / (DK / 4) * NR;
     dim3 grid((A.Dv + ROWS - 1) / ROWS, B * A.Hv, n_layers);
-    if (n_layers > 1) return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, DFLASH_MAX_BATCHED_LAYERS>, grid, dim3(kThreads), 0, P, A);
+    if (n_layers > kFewLayers) return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, DFLASH_MAX_BATCHED_LAYERS>, grid, dim3(kThreads), 0, P, A);
+    if (n_layers > 1 || P.keep > 0) {
+        ReplayWindows<kFewLayers> few = {};
+        for (int l = 0; l < n_layers; ++l) {
+            few.tape[l] = P.tape[l]; few.k[l] = P.k[l]; few.g[l] = P.g[l];
+            few.state_in[l] = P.state_in[l]; few.state_out[l] = P.state_out[l];
+            if (P.keep > 0) { few.win_snap[l] = P.win_snap[l]; few.win_qkv[l] = P.win_qkv[l]; few.win_out[l] = P.win_out[l]; }
+        }
+        few.keep = P.keep; few.row16 = P.row16;
+        return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, kFewLayers>, grid, dim3(kThreads), 0, few, A);
+    }
     const ReplayBatch<1> one = {{P.tape[0]}, {P.k[0]}, {P.g[0]}, {P.state_in[0]}, {P.state_out[0]}};
     return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, 1>, grid, dim3(kThreads), 0, one, A);
 }
@@ -358,7 +409,7 @@ static int replay_common(hipStream_t st, int n_layers, const void* const* tape, 
                          const void* const* k, const void* const* g, int in_dtype, int g_ndim,
                          const void* const* state_in, void* const* state_out, int state_dtype,
                          const void* mask, int mask_dtype, int steps, const int32_t* steps_dev, int skip_if_full,
-                         int B, int T_tape, int Hk, int Hv, int Dk, int Dv, const FusedAccept& acc = FusedAccept()) {
+                         int B, int T_tape, int Hk, int Hv, int Dk, int Dv, const FusedAccept& acc = FusedAccept(), const ConvWindows* win = nullptr) {
     int rc = ensure_init();
     if (rc) return rc;
     DFLASH_REQUIRE(n_layers >= 1 && n_layers <= DFLASH_MAX_BATCHED_LAYERS, "tape replay: n_layers=%d out of range", n_layers);
@@ -379,7 +430,10 @@ static int replay_common(hipStream_t st, int n_layers, const void* const* tape, 
         DFLASH_REQUIRE(T_tape == 0 || (tape[l] && k[l] && g[l]), "tape replay: null input pointer (layer %d)", l);
         P.tape[l] = tape[l]; P.k[l] = k[l]; P.g[l] = g[l];
         P.state_in[l] = state_in[l]; P.state_out[l] = state_out[l];
+        if (win) { P.win_snap[l] = (const uint4*)win->snap[l]; P.win_qkv[l] = (const uint4*)win->qkv[l]; P.win_out[l] = (uint4*)win->out[l]; }
     }
+    P.keep = win ? win->keep : 0;
+    P.row16 = win ? win->row16 : 0;
     ReplayArgs A;
     A.mask = mask; A.steps_dev = steps_dev; A.mask_dtype = mask_dtype; A.tape_dtype = tape_dtype;
     A.verify_ids = acc.verify_ids; A.posterior = acc.posterior; A.start_inout = acc.start_inout; A.out4 = acc.out4; A.V = acc.V;
@@ -1718,6 +1772,12 @@ extern "C" int dflash_tape_replay(void* stream, const void* tape, int tape_dtype
                          mask, mask_dtype, T, nullptr, 0, B, T, Hk, Hv, Dk, Dv);
 }
 
+int dflash::tape_replay_windows(void* stream, int n_layers, const void* const* tape, int tape_dtype, const void* const* k, const void* const* g,
+                                int in_dtype, int g_ndim, const void* const* state_in, void* const* state_out, int state_dtype, int steps,
+                                int B, int T_tape, int Hk, int Hv, int Dk, int Dv, const ConvWindows& win) {
+    return replay_common((hipStream_t)stream, n_layers, tape, tape_dtype, k, g, in_dtype, g_ndim, state_in, state_out, state_dtype, nullptr, 0,
+                         steps, nullptr, 0, B, T_tape, Hk, Hv, Dk, Dv, FusedAccept(), &win);
+}
 extern "C" int dflash_tape_replay_batched(void* stream, int n_layers, const void* const* tape, int tape_dtype,
                                           const void* const* k, const void* const* g, int in_dtype, int g_ndim,
                                           const void* const* state_in, void* const* state_out, int state_dtype,

@@ -2,6 +2,7 @@
 // Mirrors Sources/DFlash/RecurrentRollbackCache.swift and
 // DFlashRuntime.restoreTargetCacheAfterAcceptance (DFlashRuntime.swift:188-223).
 
+#include <algorithm>
 #include <chrono>
 #include <new>
 #include <vector>
@@ -102,21 +103,20 @@ bool same_window(const ReplayJob& a, const ReplayJob& b) {
     return a.steps == b.steps && x->B == y->B && x->keep == y->keep && x->T == y->T && x->C == y->C && x->qkv_elem_bytes == y->qkv_elem_bytes;
 }
 
-// The conv windows of all jobs, one launch per group of equal shapes, and the slots as they are after the rollback.
-int finish_rollbacks(const std::vector<ReplayJob>& jobs, void* stream) {
-    std::vector<char> done(jobs.size(), 0);
+// The conv windows that no replay took along, one launch per group of equal shapes, and the slots as they are after the rollback.
+int finish_rollbacks(const std::vector<ReplayJob>& jobs, std::vector<char>& rebuilt, void* stream) {
     for (size_t i = 0; i < jobs.size(); ++i) {
         dflash_cache* c = jobs[i].c;
         c->slot[1] = jobs[i].post_state;                          // :126, the replayed state
         if (c->keep <= 0) c->slot[0] = nullptr;                   // :142
-        if (done[i] || !rebuilds_window(c)) continue;             // :140, without qkv the restored window stays
+        if (rebuilt[i] || !rebuilds_window(c)) continue;          // :140, without qkv the restored window stays
         const void *snap[DFLASH_MAX_BATCHED_LAYERS], *qkv[DFLASH_MAX_BATCHED_LAYERS];
         void* out[DFLASH_MAX_BATCHED_LAYERS];
         size_t member[DFLASH_MAX_BATCHED_LAYERS];
         int n = 0;
         for (size_t j = i; j < jobs.size() && n < DFLASH_MAX_BATCHED_LAYERS; ++j) {
-            if (done[j] || !rebuilds_window(jobs[j].c) || !same_window(jobs[i], jobs[j]) || (long)(n + 1) * c->B > 65535) continue;
-            done[j] = 1;
+            if (rebuilt[j] || !rebuilds_window(jobs[j].c) || !same_window(jobs[i], jobs[j]) || (long)(n + 1) * c->B > 65535) continue;
+            rebuilt[j] = 1;
             snap[n] = jobs[j].c->snap[0]; qkv[n] = jobs[j].c->qkv; out[n] = jobs[j].post_conv;
             member[n++] = j;
         }
@@ -127,25 +127,90 @@ int finish_rollbacks(const std::vector<ReplayJob>& jobs, void* stream) {
     return DFLASH_OK;
 }
 
+size_t bytes_of(int dtype) { return (size_t)dflash::dtype_size(dtype); }
+
+// Whether the windows of a group of replays (equal replay shapes and steps) may be rebuilt by the replay's own launch: one shape of
+// window, what rebuild_conv_batched asks of the pointers, and no window in memory that the launch reads or writes for something else.
+// In launches of their own the windows come behind the replay; what shares memory keeps that order.
+bool windows_ride_along(const std::vector<ReplayJob>& jobs, const std::vector<size_t>& group) {
+    struct Span { uintptr_t from, to; };
+    Span wins[DFLASH_MAX_BATCHED_LAYERS];
+    size_t n = 0;
+    const ReplayJob* first = nullptr;
+    for (size_t j : group) {
+        const dflash_cache* c = jobs[j].c;
+        if (!rebuilds_window(c)) continue;
+        if (!first) first = &jobs[j];
+        const size_t row = (size_t)c->C * c->qkv_elem_bytes;
+        if (!same_window(*first, jobs[j]) || row % 16 || (c->qkv_elem_bytes != 2 && c->qkv_elem_bytes != 4)) return false;
+        if ((size_t)c->keep * (row / 16) > 0x3fffffff || !jobs[j].post_conv) return false;
+        if (((uintptr_t)c->snap[0] | (uintptr_t)c->qkv | (uintptr_t)jobs[j].post_conv) % 16) return false;
+        const uintptr_t o = (uintptr_t)jobs[j].post_conv;
+        wins[n++] = {o, o + (size_t)c->B * c->keep * row};
+    }
+    if (n == 0) return false;
+    std::sort(wins, wins + n, [](const Span& x, const Span& y) { return x.from < y.from; });
+    for (size_t i = 1; i < n; ++i)
+        if (wins[i].from < wins[i - 1].to) return false;
+    auto apart = [&](const void* p, size_t bytes) {               // from every window
+        if (!p) return true;
+        const uintptr_t from = (uintptr_t)p, to = from + bytes;
+        const Span* behind = std::lower_bound(wins, wins + n, to, [](const Span& x, uintptr_t y) { return x.from < y; });   // begins at or past the end
+        return behind == wins || behind[-1].to <= from;
+    };
+    for (size_t j : group) {
+        const dflash_cache* c = jobs[j].c;
+        const size_t steps = (size_t)c->B * c->T, e = bytes_of(c->in_dtype);
+        const size_t state = (size_t)c->B * c->Hv * c->Dv * c->Dk * bytes_of(c->state_dtype);
+        if (!apart(c->tape, steps * c->Hv * c->Dv * bytes_of(c->tape_dtype)) || !apart(c->k, steps * c->Hk * c->Dk * e) ||
+            !apart(c->g, steps * c->Hv * (c->g_ndim == 4 ? c->Dk : 1) * e) || !apart(c->snap[1], state) || !apart(jobs[j].post_state, state))
+            return false;
+        if (!rebuilds_window(c)) continue;
+        const size_t row = (size_t)c->C * c->qkv_elem_bytes;
+        if (!apart(c->snap[0], (size_t)c->B * c->keep * row) || !apart(c->qkv, steps * row)) return false;
+    }
+    return true;
+}
+
 int replay_jobs(const std::vector<ReplayJob>& jobs, void* stream) {
-    std::vector<bool> done(jobs.size(), false);
+    std::vector<char> done(jobs.size(), 0), rebuilt(jobs.size(), 0);
     for (size_t i = 0; i < jobs.size(); ++i) {
         if (done[i]) continue;
         const dflash_cache* a = jobs[i].c;
         std::vector<const void*> tape, k, g, sin;
         std::vector<void*> sout;
+        std::vector<size_t> group;
         for (size_t j = i; j < jobs.size() && tape.size() < DFLASH_MAX_BATCHED_LAYERS; ++j) {
             if (done[j] || jobs[j].steps != jobs[i].steps || !same_shape(a, jobs[j].c)) continue;
-            done[j] = true;
+            done[j] = 1;
             tape.push_back(jobs[j].c->tape); k.push_back(jobs[j].c->k); g.push_back(jobs[j].c->g);
             sin.push_back(jobs[j].c->snap[1]); sout.push_back(jobs[j].post_state);
+            group.push_back(j);
         }
-        int rc = dflash_tape_replay_batched(stream, (int)tape.size(), tape.data(), a->tape_dtype, k.data(), g.data(),
+        int rc;
+        if (windows_ride_along(jobs, group)) {
+            const void *snap[DFLASH_MAX_BATCHED_LAYERS], *qkv[DFLASH_MAX_BATCHED_LAYERS];
+            void* out[DFLASH_MAX_BATCHED_LAYERS];
+            dflash::ConvWindows win = {snap, qkv, out, 0, 0};
+            for (size_t m = 0; m < group.size(); ++m) {
+                const ReplayJob& job = jobs[group[m]];
+                const bool own = rebuilds_window(job.c);
+                snap[m] = own ? job.c->snap[0] : nullptr; qkv[m] = own ? job.c->qkv : nullptr; out[m] = own ? job.post_conv : nullptr;
+                if (own) { win.keep = job.c->keep; win.row16 = (int)((size_t)job.c->C * job.c->qkv_elem_bytes / 16); }
+            }
+            rc = dflash::tape_replay_windows(stream, (int)tape.size(), tape.data(), a->tape_dtype, k.data(), g.data(), a->in_dtype, a->g_ndim,
+                                             sin.data(), sout.data(), a->state_dtype, jobs[i].steps, a->B, a->T, a->Hk, a->Hv, a->Dk, a->Dv, win);
+            if (rc) return rc;
+            for (size_t m = 0; m < group.size(); ++m)
+                if (out[m]) { rebuilt[group[m]] = 1; jobs[group[m]].c->slot[0] = out[m]; }      // :127
+        } else {
+            rc = dflash_tape_replay_batched(stream, (int)tape.size(), tape.data(), a->tape_dtype, k.data(), g.data(),
                                             a->in_dtype, a->g_ndim, sin.data(), sout.data(), a->state_dtype,
                                             jobs[i].steps, nullptr, 0, a->B, a->T, a->Hk, a->Hv, a->Dk, a->Dv);
-        if (rc) return rc;
+            if (rc) return rc;
+        }
     }
-    return finish_rollbacks(jobs, stream);
+    return finish_rollbacks(jobs, rebuilt, stream);
 }
 
 }  // namespace

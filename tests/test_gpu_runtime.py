@@ -229,6 +229,49 @@ def test_restore_target_cache_hybrid_stack(gpu_lib):
                 assert np.array_equal(host(c[0]), O.rebuild_conv_state(conv0, qkv, steps, 3))
 
 
+@pytest.mark.parametrize("n_accepted", [0, 2, 6])
+@pytest.mark.parametrize("B,Hv,Dk,Dv,C,keeps,odd", [
+    (1, 4, 64, 32, 512, (3, 3, 3), None),
+    (2, 2, 128, 16, 264, (3, 3), None),               # windows of several sequences
+    (1, 1, 256, 4, 32768, (9, 9), None),              # more pieces of a window than the replay's grid has threads
+    (1, 2, 64, 16, 64, (3,), None),                   # one cache
+    (1, 2, 64, 16, 64, (3, 0, 3), None),              # one without a window
+    (1, 2, 64, 16, 64, (3, 3, 3), "no qkv"),          # one whose window stays the restored one
+    (1, 2, 64, 16, 64, (3, 2), None),                 # two shapes of window: launches of their own
+    (1, 2, 64, 16, 64, (3, 3), "no snapshot"),        # zeros ahead of the block
+    (1, 4, 64, 32, 96, (3, 3), "shared"),             # a window over a tape that the replay reads: the window comes second
+])
+def test_rollback_of_conv_windows_of_every_shape(gpu_lib, B, Hv, Dk, Dv, C, keeps, odd, n_accepted):
+    """The windows are copies: bit for bit.  The states are those of the replay on its own, bit for bit."""
+    from swiftlm_amd import DFlashKernels as K, DFlashRuntime as R, RecurrentRollbackCache
+    T, n = 7, n_accepted + 1
+    g = torch.Generator(device="cuda").manual_seed(C + B)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    caches, want = [], []
+    for i, keep in enumerate(keeps):
+        c = RecurrentRollbackCache(conv_kernel_size=keep + 1)
+        snap, state = rnd(B, max(keep, 1), C).bfloat16(), rnd(B, Hv, Dv, Dk)
+        no_snap, no_qkv = odd == "no snapshot" and i == 0, odd == "no qkv" and i == 0
+        c[0], c[1] = None if no_snap else snap, state
+        c.arm_rollback(0)
+        tape, k, dec, qkv = rnd(B, T, Hv, Dv), rnd(B, T, Hv, Dk).bfloat16(), torch.sigmoid(rnd(B, T, Hv)).bfloat16(), rnd(B, T, C).bfloat16()
+        replayed = K.tape_replay_kernel(tape[:, :n].contiguous(), k[:, :n].contiguous(), dec[:, :n].contiguous(), state)
+        window = torch.cat([torch.zeros_like(snap) if no_snap else snap, qkv], dim=1)[:, n:n + keep]
+        out = torch.zeros(B, keep, C, device="cuda").bfloat16() if keep else snap
+        if odd == "shared" and i == 1:
+            out = caches[0]._tape_refs[0].view(torch.bfloat16).flatten()[:keep * C].view(B, keep, C)
+        c[1] = torch.zeros_like(state)
+        if keep:
+            c[0] = out
+        c.record_tape(tape, k, dec, None if no_qkv else qkv)
+        caches.append(c)
+        want.append((snap if no_qkv else window, replayed))
+    R.restore_target_cache_after_acceptance(caches, n, n_accepted, T)
+    for c, keep, (window, state) in zip(caches, keeps, want):
+        assert not c.is_armed and torch.equal(c[1], state)
+        assert torch.equal(c[0], window) if keep else c[0] is None
+
+
 def test_snapshot_cache_restores_pre_verify_state(gpu_lib):
     from swiftlm_amd import MambaSnapshotCache
 
