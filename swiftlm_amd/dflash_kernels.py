@@ -203,16 +203,6 @@ class DFlashKernels:
         per-sequence key counts for ragged batches.  The keys are split by the sizes of the call and
         all counts of the batch, and the splits' partial rows are rounded to the input type, so a
         sequence gives the same values in another batch but not the same bits."""
-        if mask is not None:
-            if queries.dim() != 4 or keys.dim() != 4 or values.dim() != 4:
-                return None
-            _dev(queries, keys, values, kv_len, workspace, mask)
-            # additive [B,Hq,16,N] (anything that broadcasts to it), cast to the input type (:783-787)
-            shape = (*queries.shape[:3], keys.shape[2])
-            try:
-                mask = mask.to(queries.dtype).expand(shape).contiguous()
-            except RuntimeError:
-                raise DFlashError(f"batched_sdpa_2pass: mask {tuple(mask.shape)} does not broadcast to {shape}")
         return _native.sdpa(queries, keys, values, scale, mask, return_lse, kv_len, workspace)
 
     @staticmethod

@@ -101,10 +101,7 @@ class DFlashRuntime:
         """``restoreTargetCacheAfterAcceptance`` (DFlashRuntime.swift:188-223); returns the
         nanoseconds spent enqueuing the rollbacks.  Every tape cache's replay goes out in one
         launch instead of one launch per cache."""
-        rc, ns = _native.restore([c._handle for c in cache_entries], int(target_len), int(acceptance_length), int(drafted_tokens))
-        for c in cache_entries:
-            if isinstance(c, _RollbackCache):
-                c._after_rollback()
+        rc, ns = _native.restore(list(cache_entries), int(target_len), int(acceptance_length), int(drafted_tokens))
         _lib.check(rc, "restore_target_cache_after_acceptance")
         return ns
 

@@ -598,3 +598,51 @@ def test_launch_shapes_of_a_step(gpu_lib, context, names, page):
     torch.cuda.synchronize()
     assert len(ev.pairs) == 2 * len(names) and all(us > 0 for us in ev.durations_us())
     ev.destroy()
+
+
+@pytest.mark.parametrize("T,Hv", [(1, 1), (16, 4), (600, 32)])
+def test_outputs_of_a_call_are_tensors_of_their_own(gpu_lib, T, Hv):
+    """Small outputs share an allocation, those of a long call do not: either way they cover separate memory, keep their values
+    when the others are gone and overwritten, and begin where a 16-byte load may."""
+    from swiftlm_amd import DFlashKernels as K
+    g = torch.Generator(device="cuda").manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    q, k, v = rnd(1, T, 1, 64).bfloat16(), rnd(1, T, 1, 64).bfloat16(), rnd(1, T, Hv, 128).bfloat16()
+    dec, beta, state = torch.sigmoid(rnd(1, T, Hv)).bfloat16(), torch.sigmoid(rnd(1, T, Hv)).bfloat16(), rnd(1, Hv, 128, 64)
+    first = K.gated_delta_kernel_with_tape(q, 0.1 * k, v, dec, beta, state)
+    kept = [t.clone() for t in first]
+    spans = sorted((t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in first)
+    assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])) and all(a[0] % 16 == 0 for a in spans)
+    assert all(t.is_contiguous() for t in first)
+    same = first[0].untyped_storage().data_ptr() == first[2].untyped_storage().data_ptr()
+    assert same == (first[0].numel() * 6 < 4 << 20)
+    y, new_state, tape = first
+    first = None
+    y.fill_(float("nan"))
+    new_state.zero_()
+    assert torch.equal(tape, kept[2])
+    y = new_state = None
+    junk = [torch.full((1, T, Hv, 128), 7.0, device="cuda") for _ in range(8)]           # what the freed memory may be used for
+    assert torch.equal(tape, kept[2]) and len(junk) == 8
+    out, lse = K.batched_sdpa_2pass(rnd(1, 2, 16, 128).bfloat16(), rnd(1, 1, 40, 128).bfloat16(), rnd(1, 1, 40, 128).bfloat16(), 0.1, return_lse=True)
+    want = lse.clone()
+    out.fill_(3.0)
+    assert torch.equal(lse, want) and lse.shape == (1, 2, 16)
+
+
+@pytest.mark.parametrize("shape", [(2, 4, 16, 50), (50,), (1, 1, 1, 50), (4, 16, 50), (2, 1, 16, 1), (2, 4, 1, 50)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_sdpa_mask_of_any_shape_that_broadcasts(gpu_lib, shape, dt):
+    """The same bits as with the mask written out in the queries' type; what does not broadcast is refused."""
+    from swiftlm_amd import DFlashError, DFlashKernels as K
+    g = torch.Generator(device="cuda").manual_seed(len(shape))
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    q, k, v = rnd(2, 4, 16, 128).bfloat16(), rnd(2, 2, 50, 128).bfloat16(), rnd(2, 2, 50, 128).bfloat16()
+    mask = rnd(*shape).to(dt)
+    want = K.batched_sdpa_2pass(q, k, v, 0.1, mask.to(q.dtype).expand(2, 4, 16, 50).contiguous())
+    assert torch.equal(K.batched_sdpa_2pass(q, k, v, 0.1, mask), want)
+    strided = torch.stack([mask, mask], dim=-1)[..., 0]
+    assert torch.equal(K.batched_sdpa_2pass(q, k, v, 0.1, strided), want)
+    for bad in ((49,), (3, 4, 16, 50), (1, 2, 4, 16, 50), (2, 16, 50)):
+        with pytest.raises(DFlashError):
+            K.batched_sdpa_2pass(q, k, v, 0.1, torch.zeros(bad, device="cuda"))
