@@ -79,7 +79,7 @@ __device__ __forceinline__ float requant_rt(int dtype, float v) {      // v afte
 // ===========================================================================
 
 // The layers' pointers travel in the kernel arguments.  A launch copies its whole argument block to device memory, so a
-// call for one layer (a rollback cache on its own) takes the table of one: 48 bytes instead of 2.5 KB.
+// call for one layer takes the table of one: 40 bytes instead of 2.5 KB.
 template <int LAYERS> struct ReplayBatch {
     const void* tape[LAYERS];
     const void* k[LAYERS];
@@ -95,21 +95,21 @@ template <int LAYERS> struct ReplayWindows : ReplayBatch<LAYERS> {
     const uint4* win_qkv[LAYERS];      // [B,T_tape,row]
     uint4* win_out[LAYERS];            // [B,keep,row], null: no window for this layer
     int keep, row16;                   // rows of a window (0: none at all), 16-byte pieces of a row
-};
-typedef ReplayWindows<DFLASH_MAX_BATCHED_LAYERS> ReplayTable;
-constexpr int kFewLayers = 8;          // tables of 1, 8 and 64: 0.1, 0.6 and 4.2 KB of arguments
-template <int LAYERS> struct ReplayParam { typedef ReplayWindows<LAYERS> type; };
-template <> struct ReplayParam<1> { typedef ReplayBatch<1> type; };
-
-struct ReplayArgs {
-    const void* mask;        // [B,T_tape] or null
-    const int32_t* steps_dev;
     // fused acceptance (null verify_ids = off): steps = 1 + leading matches of verify_ids[1:] vs posterior
     const uint32_t* verify_ids;
     const uint32_t* posterior;
     int32_t* start_inout;
     int32_t* out4;
     int V;
+};
+typedef ReplayWindows<DFLASH_MAX_BATCHED_LAYERS> ReplayTable;
+constexpr int kFewLayers = 8;          // tables of 1, 8 and 64: 92 bytes, 0.6 and 4.2 KB of arguments
+template <int LAYERS> struct ReplayParam { typedef ReplayWindows<LAYERS> type; };
+template <> struct ReplayParam<1> { typedef ReplayBatch<1> type; };
+
+struct ReplayArgs {
+    const void* mask;        // [B,T_tape] or null
+    const int32_t* steps_dev;
     int mask_dtype, tape_dtype, in_dtype;
     int steps, skip_if_full;
     int T_tape, Hk, Hv, Dv;
@@ -134,9 +134,9 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayPa
     __shared__ int on_s[TC];
 
     // the scalar arguments in one burst of loads (the per-layer pointer tables are indexed by the layer and stay lazy)
-    asm volatile("" ::"s"(A.mask), "s"(A.steps_dev), "s"(A.verify_ids), "s"(A.posterior), "s"(A.start_inout), "s"(A.out4),
-                 "s"(A.V), "s"(A.mask_dtype), "s"(A.tape_dtype), "s"(A.in_dtype), "s"(A.steps), "s"(A.skip_if_full),
+    asm volatile("" ::"s"(A.mask), "s"(A.steps_dev), "s"(A.mask_dtype), "s"(A.tape_dtype), "s"(A.in_dtype), "s"(A.steps), "s"(A.skip_if_full),
                  "s"(A.T_tape), "s"(A.Hk), "s"(A.Hv), "s"(A.Dv));
+    if constexpr (LAYERS > 1) asm volatile("" ::"s"(P.verify_ids), "s"(P.posterior), "s"(P.start_inout), "s"(P.out4), "s"(P.V), "s"(P.keep), "s"(P.row16));
     const int layer = LAYERS == 1 ? 0 : blockIdx.z;
     const int bh = blockIdx.y;
     const int b = bh / A.Hv, hv = bh % A.Hv;
@@ -147,32 +147,34 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayPa
     const bool owner = tid < RPP * TPR;            // false only for the spare threads of an odd TPR
     const int rsub = owner ? tid / TPR : 0;
 
-    int n;
-    if (A.verify_ids) {
-        // The cycle's acceptance (DFlashRuntime.swift:525-547) is decided here, by every workgroup for
-        // itself (two 64-byte reads), so the rollback needs no launch ahead of it; workgroup 0 also does
-        // the bookkeeping accept_commit_kernel would have done.
-        __shared__ int n_s;
-        if (tid < 64) {
-            const int acc = A.V > 1 ? leading_matches(A.verify_ids + 1, A.posterior, A.V - 1) : 0;
-            if (tid == 0) {
-                n_s = 1 + acc;
-                if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
-                    A.out4[0] = acc;
-                    A.out4[1] = 1 + acc;
-                    A.out4[2] = (int32_t)A.posterior[acc];
-                    int start = 1 + acc;
-                    if (A.start_inout) { start += *A.start_inout; *A.start_inout = start; }
-                    A.out4[3] = start;
+    int n = A.steps;
+    bool counted = false;
+    if constexpr (LAYERS > 1) {
+        if (P.verify_ids) {
+            counted = true;
+            // The cycle's acceptance (DFlashRuntime.swift:525-547) is decided here, by every workgroup for
+            // itself (two 64-byte reads), so the rollback needs no launch ahead of it; workgroup 0 also does
+            // the bookkeeping accept_commit_kernel would have done.
+            __shared__ int n_s;
+            if (tid < 64) {
+                const int acc = P.V > 1 ? leading_matches(P.verify_ids + 1, P.posterior, P.V - 1) : 0;
+                if (tid == 0) {
+                    n_s = 1 + acc;
+                    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
+                        P.out4[0] = acc;
+                        P.out4[1] = 1 + acc;
+                        P.out4[2] = (int32_t)P.posterior[acc];
+                        int start = 1 + acc;
+                        if (P.start_inout) { start += *P.start_inout; *P.start_inout = start; }
+                        P.out4[3] = start;
+                    }
                 }
             }
+            __syncthreads();
+            n = n_s;
         }
-        __syncthreads();
-        n = n_s;
-    } else {
-        n = A.steps;
-        if (A.steps_dev) n = __builtin_amdgcn_readfirstlane(*A.steps_dev);   // (kept a branch: as a select of two addresses the host-side count lands in scratch)
     }
+    if (!counted && A.steps_dev) n = __builtin_amdgcn_readfirstlane(*A.steps_dev);   // (kept a branch: as a select of two addresses the host-side count lands in scratch)
     n = n < 0 ? 0 : (n > A.T_tape ? A.T_tape : n);
     if (A.skip_if_full && n == A.T_tape) return;   // uniform over the grid
 
@@ -345,7 +347,7 @@ static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, 
     constexpr int ROWS = kThreads / (DK / 4) * NR;
     dim3 grid((A.Dv + ROWS - 1) / ROWS, B * A.Hv, n_layers);
     if (n_layers > kFewLayers) return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, DFLASH_MAX_BATCHED_LAYERS>, grid, dim3(kThreads), 0, P, A);
-    if (n_layers > 1 || P.keep > 0) {
+    if (n_layers > 1 || P.keep > 0 || P.verify_ids) {
         ReplayWindows<kFewLayers> few = {};
         for (int l = 0; l < n_layers; ++l) {
             few.tape[l] = P.tape[l]; few.k[l] = P.k[l]; few.g[l] = P.g[l];
@@ -353,6 +355,7 @@ static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, 
             if (P.keep > 0) { few.win_snap[l] = P.win_snap[l]; few.win_qkv[l] = P.win_qkv[l]; few.win_out[l] = P.win_out[l]; }
         }
         few.keep = P.keep; few.row16 = P.row16;
+        few.verify_ids = P.verify_ids; few.posterior = P.posterior; few.start_inout = P.start_inout; few.out4 = P.out4; few.V = P.V;
         return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, kFewLayers>, grid, dim3(kThreads), 0, few, A);
     }
     const ReplayBatch<1> one = {{P.tape[0]}, {P.k[0]}, {P.g[0]}, {P.state_in[0]}, {P.state_out[0]}};
@@ -436,7 +439,7 @@ static int replay_common(hipStream_t st, int n_layers, const void* const* tape, 
     P.row16 = win ? win->row16 : 0;
     ReplayArgs A;
     A.mask = mask; A.steps_dev = steps_dev; A.mask_dtype = mask_dtype; A.tape_dtype = tape_dtype;
-    A.verify_ids = acc.verify_ids; A.posterior = acc.posterior; A.start_inout = acc.start_inout; A.out4 = acc.out4; A.V = acc.V;
+    P.verify_ids = acc.verify_ids; P.posterior = acc.posterior; P.start_inout = acc.start_inout; P.out4 = acc.out4; P.V = acc.V;
     A.in_dtype = in_dtype; A.steps = steps; A.skip_if_full = skip_if_full;
     A.T_tape = T_tape; A.Hk = Hk; A.Hv = Hv; A.Dv = Dv;
 
@@ -1633,11 +1636,22 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
 // What stands between a wave's start and its loads -- the six input pointers and the sizes their addresses need --
 // is passed as leading scalar arguments: the command processor hands those over in SGPRs when the wave starts (kernarg
 // preload, 14 dwords at most, hence the sizes packed in pairs), so no load waits for a trip to the argument block.
-// The rest of the arguments (outputs, mask, types) follow in the struct and are fetched while the loads are in flight.
+// The rest of the arguments (outputs, mask, types) follow in a struct of just these and are fetched while the loads are in flight.  A launch
+// writes its whole argument block across the bus: 96 bytes, where all of GdnArgs behind the scalars made 184 (enqueue
+// on the host, two builds in turn: 4.0 us, now 3.5).
+struct GdnChunkRest {
+    const void* mask;
+    void* state_out;
+    void* y;
+    float* tape;
+    int in_dtype, mask_dtype;
+};
 template <bool HAS_MASK, int DK, bool BF, bool LOOP>
 __global__ __launch_bounds__(kThreads, DK == 256 || LOOP ? 2 : 4) void gated_delta_chunk_kernel(const void* state_in, const void* k, const void* q, const void* v,
                                                                      const void* g, const void* beta, uint32_t hv_dv, uint32_t hk_t,
-                                                                     GdnArgs A) {
+                                                                     GdnChunkRest R) {
+    GdnArgs A;
+    A.mask = R.mask; A.state_out = R.state_out; A.y = R.y; A.tape = R.tape; A.in_dtype = R.in_dtype; A.mask_dtype = R.mask_dtype;
     A.state_in = state_in; A.k = k; A.q = q; A.v = v; A.g = g; A.beta = beta;
     A.Hv = (int)(hv_dv >> 16); A.Dv = (int)(hv_dv & 0xffffu); A.Hk = (int)(hk_t >> 16); A.T = (int)(hk_t & 0xffffu);
     A.group = (uint32_t)A.Hv / (uint32_t)A.Hk;
@@ -1684,7 +1698,8 @@ static int launch_gdn_chunk(hipStream_t st, const GdnArgs& A, int B) {
                                              : (bf ? gated_delta_chunk_kernel<false, DK, true, false> : gated_delta_chunk_kernel<false, DK, false, false>))
                                    : (A.mask ? (bf ? gated_delta_chunk_kernel<true, DK, true, true> : gated_delta_chunk_kernel<true, DK, false, true>)
                                              : (bf ? gated_delta_chunk_kernel<false, DK, true, true> : gated_delta_chunk_kernel<false, DK, false, true>));
-    DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), lds, A.state_in, A.k, A.q, A.v, A.g, A.beta, hv_dv, hk_t, A));
+    DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), lds, A.state_in, A.k, A.q, A.v, A.g, A.beta, hv_dv, hk_t,
+                             GdnChunkRest{A.mask, A.state_out, A.y, A.tape, A.in_dtype, A.mask_dtype}));
     return DFLASH_OK;
 }
 
