@@ -20,9 +20,9 @@ namespace dflash {
 //   waves 0-3 (chain)     own Dk/4 channels of the 16 state rows each, as MFMA accumulators that never leave the
 //                         registers.  Chunk m: add the four partial S_0 k_t, delta = T (v - gam S_0 k_t), update, split
 //                         the new state into three bf16 terms, partial S_0 k_t of chunk m+1 into LDS, barrier.
-//   waves 4-7 (producers) wave 4+p prepares chunks p, p+4, ...: interval m-2 k rows, k_s.k_t, k_s.q_t, decays; interval
+//   waves 4-7 (producers) wave 4+p prepares chunks p, p+4, ...: interval m-3 decays; m-2 k rows, k_s.k_t, k_s.q_t;
 //                         m-1 T = (I + diag(beta) A)^-1 diag(beta) by substitution; interval m the loads of chunk m+4;
-//                         interval m+1 y and the tape of the chunk.
+//                         interval m+1 y and the tape of the chunk, and the decays of chunk m+4.
 //
 // One barrier per chunk, no wave waits for memory inside a chunk (loads are asked for two chunks ahead of their use), and
 // no operand crosses lanes: with S^T as the accumulator a lane holds row l%16 and channels 4*(l/16)+v, which is also how
@@ -32,11 +32,12 @@ namespace dflash {
 // and with a row per lane, or two bytes per lane, every lane is a request (22 instructions of up to 64 requests per chunk; now
 // 13).  So the products' operands, v and the tape change lanes through LDS, and k is transposed by the LDS as the update reads it.
 //
-// Bound by the length of an interval: 1,350 / 1,600 / 2,200 cycles at Dk = 64 / 128 / 256, of which the chain works 1,200 /
-// 1,350 / 1,800 (the split of the state on the VALU, the exchange of the partial sums through LDS, three groups of
-// dependent MFMAs) and the busiest producer as long.  us, chunk by chunk kernel against this one: 1,003 steps,
-// 32 heads of 128x128 152 -> 42; 730 steps, 8 heads, Dk = 256 147 -> 43; two sequences of 1,000 steps, 32 heads, Dk = 256
-// 419 -> 116; 40 steps 8.3 -> 5.4.
+// Bound by the length of an interval, of which the chain works 1,190 / 1,390 / 1,880 cycles at Dk = 64 / 128 / 256 (the split of the
+// state on the VALU, the exchange of the partial sums through LDS, three groups of dependent MFMAs), the producers 340 to 1,330 (1,940 at
+// Dk = 256: k rows).  With the decays formed beside the k rows that interval was as long as the chain's (1,320, 2,150 at 256), and all
+// wait for the longest: 1,003 steps, 32 heads of 128x128 45.4 -> 44.6 us, 730 of Dk = 256 45.4 -> 42.3, 257 of 8 heads 13.6 -> 13.2.
+// us, chunk by chunk kernel against this one: 1,003 steps, 32 heads of 128x128 152 -> 41; 730 steps, 8 heads, Dk = 256 147 -> 42;
+// two sequences of 1,000 steps, 32 heads, Dk = 256 419 -> 116; 40 steps 8.3 -> 5.4.
 // The care for what is not finite (y, the rows of masked steps) costs or gives 3 %: 1,000 steps of Dk = 256 64.8 -> 66.9, Dk = 64 36.7 ->
 // 37.1, 1,003 steps of Dk = 128 43.1 -> 42.1.
 // 95 / 121 / 189 registers: two workgroups share a compute unit at Dk = 64 and 128 (two sequences of 1,000 steps 71 where one takes
@@ -243,6 +244,10 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
         const int t0 = m * kChunkSteps, tc = min(A.T - t0, kChunkSteps);
         const uint32_t bt0 = (uint32_t)b * A.T + t0;                                   // uniform, as are the products with it
         const int tl = min(n, tc - 1);                 // clamped: always a valid address, selected away where it is used
+        const uint32_t go = bt0 * A.Hv + hv + __umul24(tl, A.Hv);
+        gr = gp[go];                                   // needed first
+        br = bp[go];
+        vr = reinterpret_cast<const Rows4x16*>(vp + ((bt0 * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(tl, step)))->x;
         const uint32_t o = (bt0 * A.Hk + hk) * DK + 8 * pc;
 #pragma unroll
         for (int j = 0; j < NK; ++j) {
@@ -250,10 +255,6 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             kr[j] = *reinterpret_cast<const u32x4v*>(kp + oj);
             qr[j] = *reinterpret_cast<const u32x4v*>(qp + oj);
         }
-        vr = reinterpret_cast<const Rows4x16*>(vp + ((bt0 * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(tl, step)))->x;
-        const uint32_t go = bt0 * A.Hv + hv + __umul24(tl, A.Hv);
-        gr = gp[go];
-        br = bp[go];
     };
     // a row's channels 8 pc .. +7 at their positions
     auto park = [&](uint16_t* row, u32x4v x) {
@@ -267,6 +268,38 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
     f32x4v vf, yv, dl;                                 // v of the chunk in hand; y and tape of the one before, not yet stored: step n, rows 4g .. +3
     bool step_on = false;
     uint32_t counted = 0;                              // MASKED: bit t: step t counts
+    // What of chunk m does not wait for its k and q: which steps count, decays, beta, v.  Formed behind the read-out of chunk m - 4, whose
+    // interval is short.
+    auto gates = [&](int m) __attribute__((always_inline)) {
+        const int t0 = m * kChunkSteps, tc = min(A.T - t0, kChunkSteps);
+        step_on = n < tc;
+        if constexpr (MASKED) {
+            step_on = step_on && mask_on(A.mask, A.mask_dtype, (int)((uint32_t)b * A.T + t0 + min(n, tc - 1)));
+            counted = (uint32_t)__builtin_amdgcn_ballot_w64(step_on) & 0xffffu;
+        }
+        vr = step_on ? vr : make_uint2(0u, 0u);
+        // decay products G[v] = g_{s+1} ... g_t of the lane's pairs (s, t) = (4g + v, n), 1 where s >= t
+        const float gl = step_on ? to_float(gr) : 1.f;
+        beta = step_on ? to_float(br) : 0.f;
+        vf = f32x4v{__uint_as_float(vr.x << 16), __uint_as_float(vr.x & 0xffff0000u), __uint_as_float(vr.y << 16), __uint_as_float(vr.y & 0xffff0000u)};
+        // steps in blocks of four: pre = the product from the block's first step up to the lane's, block products by broadcast
+        // (lane exchanges outside the selects: a select may become a branch, with the lanes that are read switched off)
+        const float left1 = quad_take<0, 0, 1, 2>(gl);
+        float pre = gl * (n % 4 >= 1 ? left1 : 1.f);
+        const float left2 = quad_take<0, 0, 0, 1>(pre);
+        pre *= n % 4 >= 2 ? left2 : 1.f;
+        const float b1 = row_broadcast<7>(pre), b2 = row_broadcast<11>(pre);
+        G[3] = n / 4 > g ? pre : 1.f;
+        G[3] *= g < 1 && n / 4 > 1 ? b1 : 1.f;
+        G[3] *= g < 2 && n / 4 > 2 ? b2 : 1.f;
+#pragma unroll
+        for (int v = 2; v >= 0; --v) {
+            const float gs = __shfl(gl, 4 * g + v + 1);
+            G[v] = G[v + 1] * (4 * g + v + 1 <= n ? gs : 1.f);
+        }
+        gam = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(gl), 0)) * G[0];      // of step n, in lanes g = 0
+        asm volatile("" : "+v"(gam), "+v"(beta), "+v"(vf), "+v"(G[0]), "+v"(G[1]), "+v"(G[2]), "+v"(G[3]));   // not sunk into the next interval
+    };
     auto store_rows = [&](int m, int tc) {             // one store each: row by row, two and four bytes per lane, they were eight
         const uint32_t o = (((uint32_t)b * A.T + m * kChunkSteps) * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(n, step);
         if (n < tc) {
@@ -277,7 +310,10 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             reinterpret_cast<Rows4x32*>(A.tape + o)->x = dl;
         }
     };
-    if (p < chunks) request(p);
+    if (p < chunks) {
+        request(p);
+        gates(p);
+    }
     for (int j = 0; j < p; ++j) {                      // intervals -2 .. p - 3
         lds_barrier();
     }
@@ -291,7 +327,6 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
                     kr[j] = j * RPI + rs < tc ? kr[j] : none;
                     qr[j] = j * RPI + rs < tc ? qr[j] : none;
                 }
-                vr = n < tc ? vr : make_uint2(0u, 0u);
             }
 #pragma unroll
             for (int j = 0; j < NK; ++j) {
@@ -306,11 +341,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
                 kk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, k8, kk, 0, 0, 0);
                 kq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k8, q8, kq, 0, 0, 0);
             }
-            step_on = n < tc;
             if constexpr (MASKED) {
-                step_on = step_on && mask_on(A.mask, A.mask_dtype, (int)((uint32_t)b * A.T + t0 + min(n, tc - 1)));
-                counted = (uint32_t)__builtin_amdgcn_ballot_w64(step_on) & 0xffffu;
-                vr = step_on ? vr : make_uint2(0u, 0u);
                 // A masked step's rows may hold anything, infinities and NaN among it, and zero times these is not zero: where a product
                 // with them is not finite, zeros take the rows' place.
                 auto size = [](f32x4v x) { return fabsf(x[0]) + fabsf(x[1]) + fabsf(x[2]) + fabsf(x[3]); };
@@ -329,33 +360,13 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
                     }
                 }
             }
-            // decay products G[v] = g_{s+1} ... g_t of the lane's pairs (s, t) = (4g + v, n), 1 where s >= t
-            const float gl = step_on ? to_float(gr) : 1.f;
-            beta = step_on ? to_float(br) : 0.f;
-            vf = f32x4v{__uint_as_float(vr.x << 16), __uint_as_float(vr.x & 0xffff0000u), __uint_as_float(vr.y << 16), __uint_as_float(vr.y & 0xffff0000u)};
-            // steps in blocks of four: pre = the product from the block's first step up to the lane's, block products by broadcast
-            // (lane exchanges outside the selects: a select may become a branch, with the lanes that are read switched off)
-            const float left1 = quad_take<0, 0, 1, 2>(gl);
-            float pre = gl * (n % 4 >= 1 ? left1 : 1.f);
-            const float left2 = quad_take<0, 0, 0, 1>(pre);
-            pre *= n % 4 >= 2 ? left2 : 1.f;
-            const float b1 = row_broadcast<7>(pre), b2 = row_broadcast<11>(pre);
-            G[3] = n / 4 > g ? pre : 1.f;
-            G[3] *= g < 1 && n / 4 > 1 ? b1 : 1.f;
-            G[3] *= g < 2 && n / 4 > 2 ? b2 : 1.f;
-#pragma unroll
-            for (int v = 2; v >= 0; --v) {
-                const float gs = __shfl(gl, 4 * g + v + 1);
-                G[v] = G[v + 1] * (4 * g + v + 1 <= n ? gs : 1.f);
-            }
-            gam = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(gl), 0)) * G[0];      // of step n, in lanes g = 0
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int s = 4 * g + v;
                 av[v] = s < n ? -beta * (G[v] * kk[v]) : 0.f;
                 cv[v] = s <= n ? G[v] * kq[v] : 0.f;
             }
-            asm volatile("" : "+v"(av), "+v"(cv), "+v"(gam), "+v"(G[0]), "+v"(G[1]), "+v"(G[2]), "+v"(G[3]));   // not sunk into the next interval
+            asm volatile("" : "+v"(av), "+v"(cv));     // not sunk into the next interval
         }
         lds_barrier();
         {   // interval m - 1
@@ -417,6 +428,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
             for (int v = 0; v < 4; ++v) yv[v] = step_on ? yv[v] : 0.f;
             if (m + 4 >= chunks) store_rows(m, tc);
             if (m + 1 == chunks) return;               // behind the last barrier
+            if (m + 4 < chunks) gates(m + 4);
         }
         lds_barrier();
     }
