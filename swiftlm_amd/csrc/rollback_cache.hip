@@ -130,8 +130,9 @@ int finish_rollbacks(const std::vector<ReplayJob>& jobs, std::vector<char>& rebu
 size_t bytes_of(int dtype) { return (size_t)dflash::dtype_size(dtype); }
 
 // Whether the windows of a group of replays (equal replay shapes and steps) may be rebuilt by the replay's own launch: one shape of
-// window, what rebuild_conv_batched asks of the pointers, and no window in memory that the launch reads or writes for something else.
-// In launches of their own the windows come behind the replay; what shares memory keeps that order.
+// window, what rebuild_conv_batched asks of the pointers, and no window in memory that any replay or other window of the rollback
+// reads or writes, the other groups' too.  In launches of their own the windows come behind all replays; what shares memory keeps
+// that order.
 bool windows_ride_along(const std::vector<ReplayJob>& jobs, const std::vector<size_t>& group) {
     struct Span { uintptr_t from, to; };
     Span wins[DFLASH_MAX_BATCHED_LAYERS];
@@ -158,8 +159,11 @@ bool windows_ride_along(const std::vector<ReplayJob>& jobs, const std::vector<si
         const Span* behind = std::lower_bound(wins, wins + n, to, [](const Span& x, uintptr_t y) { return x.from < y; });   // begins at or past the end
         return behind == wins || behind[-1].to <= from;
     };
-    for (size_t j : group) {
+    size_t at = 0;                                                // in the group, whose indices ascend
+    for (size_t j = 0; j < jobs.size(); ++j) {
         const dflash_cache* c = jobs[j].c;
+        const bool member = at < group.size() && group[at] == j;
+        at += member;
         const size_t steps = (size_t)c->B * c->T, e = bytes_of(c->in_dtype);
         const size_t state = (size_t)c->B * c->Hv * c->Dv * c->Dk * bytes_of(c->state_dtype);
         if (!apart(c->tape, steps * c->Hv * c->Dv * bytes_of(c->tape_dtype)) || !apart(c->k, steps * c->Hk * c->Dk * e) ||
@@ -168,6 +172,7 @@ bool windows_ride_along(const std::vector<ReplayJob>& jobs, const std::vector<si
         if (!rebuilds_window(c)) continue;
         const size_t row = (size_t)c->C * c->qkv_elem_bytes;
         if (!apart(c->snap[0], (size_t)c->B * c->keep * row) || !apart(c->qkv, steps * row)) return false;
+        if (!member && !apart(jobs[j].post_conv, (size_t)c->B * c->keep * row)) return false;
     }
     return true;
 }

@@ -272,6 +272,30 @@ def test_rollback_of_conv_windows_of_every_shape(gpu_lib, B, Hv, Dk, Dv, C, keep
         assert torch.equal(c[0], window) if keep else c[0] is None
 
 
+def test_rollback_of_a_window_over_another_shapes_tape(gpu_lib):
+    """Caches of two replay shapes are two launches; the first one's window lies over the tape of the second, which the replays
+    read before any window is written, as they do cache by cache of one shape."""
+    from swiftlm_amd import DFlashKernels as K, DFlashRuntime as R, RecurrentRollbackCache
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    T, n, C = 7, 3, 64
+    tapes = [rnd(1, T, 2, 16), rnd(1, T, 2, 16)]
+    over = tapes[1].view(torch.bfloat16).flatten()[:3 * C].view(1, 3, C)
+    caches, want = [], []
+    for Dk, tape, out in zip((64, 128), tapes, (over, torch.zeros(1, 3, C, device="cuda").bfloat16())):
+        c, snap, state = RecurrentRollbackCache(), rnd(1, 3, C).bfloat16(), rnd(1, 2, 16, Dk)
+        c[0], c[1] = snap, state
+        c.arm_rollback(0)
+        k, dec, qkv = rnd(1, T, 2, Dk).bfloat16(), torch.sigmoid(rnd(1, T, 2)).bfloat16(), rnd(1, T, C).bfloat16()
+        want.append((torch.cat([snap, qkv], dim=1)[:, n:n + 3], K.tape_replay_kernel(tape[:, :n].contiguous(), k[:, :n].contiguous(), dec[:, :n].contiguous(), state)))
+        c[0], c[1] = out, torch.zeros_like(state)
+        c.record_tape(tape, k, dec, qkv)
+        caches.append(c)
+    R.restore_target_cache_after_acceptance(caches, n, n - 1, T)
+    for c, (window, state) in zip(caches, want):
+        assert torch.equal(c[0], window) and torch.equal(c[1], state)
+
+
 def test_snapshot_cache_restores_pre_verify_state(gpu_lib):
     from swiftlm_amd import MambaSnapshotCache
 
