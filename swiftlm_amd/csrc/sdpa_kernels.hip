@@ -1047,6 +1047,19 @@ static int choose_splits(int B, int Hk, int groups_per_kv, int N) {
     return S;
 }
 
+// What a launch takes of these splits where they are not dealt to lengths of their own (the workspace asked for is that of
+// choose_splits either way).  A workgroup has a compute unit to itself and all take the same time, so splits that come to more
+// workgroups than there are compute units are a second round, nearly empty: those that fit at once are launched.
+// us, rounded up and what fits at once, Hk = 8:
+//     D=128   5 sequences, 8,208 keys, 7 and 6 splits 53.5 33.6    7 sequences, 4,112 keys, 5 and 4 41.4 27.6
+//            13 sequences, 2,000 keys, 3 and 2 36.6 27.7          17 sequences, 4,112 keys, 2 and 1 87.7 79.3 (24: 89.1 79.4)
+//     D=256  17 sequences, 2,064 keys, 2 and 1 92.7 70.2          24 sequences 94.1 78.8;  6 of Hk = 2, 16,400 keys, 22 and 21 71.9 45.0
+// Counts per sequence keep the splits rounded up: where they are not dealt, the sequences may end at different times.
+static int splits_at_once(int S, int workgroups_per_split) {
+    const int cus = num_compute_units();
+    return workgroups_per_split <= cus && S * workgroups_per_split > cus ? cus / workgroups_per_split : S;
+}
+
 static size_t ws_layout(int B, int Hq, int S, int D, size_t* off_m, size_t* off_l) {
     const size_t rows = (size_t)B * Hq * kM;
     size_t o = rows * S * D * sizeof(uint16_t);
@@ -1267,6 +1280,11 @@ static int sdpa_common(void* stream, const void* q, const void* k, const void* v
         A.balance = W > B && (B - 1) * tiles >= (int64_t)line * W && tiles < (1 << 20) && B * tiles < (1 << 24);
         if (A.balance) A.deal = {W, fast_div_magic((uint32_t)W), fast_div_magic((uint32_t)(W - B))};
     }
+    if (!kv_len_dev || B == 1) {
+        A.S = C.S = splits_at_once(S, B * Hk * groups);
+        A.S_magic = fast_div_magic((uint32_t)A.S);
+        if (A.S == 1) A.part_o = (uint16_t*)out;
+    }
     C.balance = A.balance; C.deal = A.deal; C.kv_len_dev = kv_len_dev; C.len_bias = A.len_bias; C.N = N;
 
     hipStream_t st = (hipStream_t)stream;
@@ -1304,6 +1322,7 @@ extern "C" int dflash_profile_sdpa_launches(int dtype, int B, int Hq, int Hk, in
         S = few;
         shapes[0] = sdpa_short_shape(B, Hk, G, S, D);
     } else {
+        S = splits_at_once(S, B * Hk * groups);
         shapes[0] = {"sdpa_partial_kernel", S, Hk * groups, B, kPartialThreads, D == 256 ? SdpaLds<256>::BYTES : SdpaLds<128>::BYTES};
     }
     if (S == 1) return 1;

@@ -115,6 +115,35 @@ def test_sdpa_single_kv_head_uses_every_split(gpu_lib, cfg):
     np.testing.assert_allclose(host(lse), host(lw), **LSE_TOL)
 
 
+@pytest.mark.parametrize("cfg", [(5, 32, 8, 1500, 128), (17, 16, 8, 200, 128), (32, 16, 8, 200, 128), (33, 16, 8, 200, 128), (6, 16, 2, 2000, 256),
+                                 (3, 48, 4, 1300, 256), (13, 24, 8, 333, 256)],
+                         ids=lambda c: f"B{c[0]}_Hq{c[1]}_Hk{c[2]}_L{c[3]}_D{c[4]}")
+def test_sdpa_splits_that_do_not_divide_the_chip(gpu_lib, cfg):
+    """Batches whose splits, rounded up, are more workgroups than compute units, one split that fits and just not, two head groups:
+    all forms of the call take the same splits and give the same bits, in the workspace that the sizes ask for and no byte more."""
+    from swiftlm_amd import DFlashKernels as K
+    from swiftlm_amd import _lib
+
+    B, Hq, Hk, L, D = cfg
+    N, scale = L + 16, 1.0 / math.sqrt(D)
+    q, k, v = gpu_inputs(L + B, B, Hq, Hk, L, D)
+    ow, lw = torch_reference(q, k, v, scale)
+    need = _lib.load().dflash_sdpa_workspace_bytes(B, Hq, Hk, 16, N, D)
+    room = torch.full((need + 256,), 77, dtype=torch.uint8, device="cuda")
+    out, lse = K.batched_sdpa_2pass(q, k, v, scale, return_lse=True, workspace=room[:need])
+    assert bool((room[need:] == 77).all())
+    np.testing.assert_allclose(host(out), host(ow), **OUT_TOL)
+    np.testing.assert_allclose(host(lse), host(lw), **LSE_TOL)
+    kc, vc = k.clone(), v.clone()
+    kc[:, :, L:] = vc[:, :, L:] = 0
+    got, got_lse = K.batched_sdpa_2pass_append(q, kc, vc, k[:, :, L:].contiguous(), v[:, :, L:].contiguous(), scale, N, return_lse=True)
+    assert torch.equal(got, out) and torch.equal(got_lse, lse) and torch.equal(kc, k) and torch.equal(vc, v)
+    zero = torch.zeros(1, device="cuda", dtype=q.dtype).expand(B, Hq, 16, N)
+    assert torch.equal(K.batched_sdpa_2pass(q, k, v, scale, zero), out)
+    lens = torch.full((B,), N, dtype=torch.int32, device="cuda")              # with counts per sequence: dealt, or the splits rounded up
+    np.testing.assert_allclose(host(K.batched_sdpa_2pass(q, k, v, scale, kv_len=lens)), host(ow), **OUT_TOL)
+
+
 @pytest.mark.parametrize("L", [32768, 40960, 102400])
 def test_sdpa_long_context_properties(gpu_lib, L):
     """Benchmark configuration 3 sizes.  Properties that do not need a CPU pass: constant V gives
