@@ -81,31 +81,36 @@ __device__ __forceinline__ float requant_rt(int dtype, float v) {      // v afte
 // The layers' pointers travel in the kernel arguments.  A launch copies its whole argument block to device memory, so a
 // call for one layer takes the table of one: 40 bytes instead of 2.5 KB.
 template <int LAYERS> struct ReplayBatch {
+    static constexpr int kLayers = LAYERS;
+    static constexpr bool kAccept = false, kWindows = false;
     const void* tape[LAYERS];
     const void* k[LAYERS];
     const void* g[LAYERS];
     const void* state_in[LAYERS];
     void* state_out[LAYERS];
 };
-// A rollback over several caches also rebuilds their conv windows (rebuild_conv_batched): the same launch copies them, 16 bytes per
-// thread of the layer's first workgroups, asked for with the state rows.  A launch of its own behind the replay cost the host 4 us and
-// the GPU a dependent trip to memory.
-template <int LAYERS> struct ReplayWindows : ReplayBatch<LAYERS> {
-    const uint4* win_snap[LAYERS];     // [B,keep,row], null: zeros
-    const uint4* win_qkv[LAYERS];      // [B,T_tape,row]
-    uint4* win_out[LAYERS];            // [B,keep,row], null: no window for this layer
-    int keep, row16;                   // rows of a window (0: none at all), 16-byte pieces of a row
-    // fused acceptance (null verify_ids = off): steps = 1 + leading matches of verify_ids[1:] vs posterior
+// fused acceptance (null verify_ids = off): steps = 1 + leading matches of verify_ids[1:] vs posterior
+template <int LAYERS> struct ReplayAccept : ReplayBatch<LAYERS> {
+    static constexpr bool kAccept = true;
     const uint32_t* verify_ids;
     const uint32_t* posterior;
     int32_t* start_inout;
     int32_t* out4;
     int V;
 };
+// A rollback over several caches also rebuilds their conv windows (rebuild_conv_batched): the same launch copies them, 16 bytes per
+// thread of the layer's first workgroups, asked for with the state rows.  A launch of its own behind the replay cost the host 4 us and
+// the GPU a dependent trip to memory.
+template <int LAYERS> struct ReplayWindows : ReplayAccept<LAYERS> {
+    static constexpr bool kWindows = true;
+    int keep, row16;                   // rows of a window (0: none at all), 16-byte pieces of a row
+    const uint4* win_snap[LAYERS];     // [B,keep,row], null: zeros
+    const uint4* win_qkv[LAYERS];      // [B,T_tape,row]
+    uint4* win_out[LAYERS];            // [B,keep,row], null: no window for this layer
+};
 typedef ReplayWindows<DFLASH_MAX_BATCHED_LAYERS> ReplayTable;
-constexpr int kFewLayers = 8;          // tables of 1, 8 and 64: 92 bytes, 0.6 and 4.2 KB of arguments
-template <int LAYERS> struct ReplayParam { typedef ReplayWindows<LAYERS> type; };
-template <> struct ReplayParam<1> { typedef ReplayBatch<1> type; };
+constexpr int kFewLayers = 8;          // tables of 1, 8 and 64: 92 bytes, 0.6 and 4.2 KB of arguments; 64 without windows 2.6
+// (more than eight layers without windows: four captured steps of 12 layers took 630 us, with the table that has room for windows 634 to 638)
 
 struct ReplayArgs {
     const void* mask;        // [B,T_tape] or null
@@ -121,8 +126,8 @@ constexpr int kReplayChunk = 16;  // steps staged in LDS at a time (8 for Dk = 2
 // span a row, so a 256-thread workgroup covers RPP = floor(1024/DK) rows per pass
 // and NR passes (when DK/4 does not divide 256 the last few threads only help
 // with staging).  Grid: x = Dv tiles, y = b*Hv + hv, z = layer.
-template <typename StateT, bool VEC_G, int DK, int NR, int LAYERS>
-__global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayParam<LAYERS>::type P, ReplayArgs A) {
+template <typename StateT, bool VEC_G, int DK, int NR, typename Table>
+__global__ __launch_bounds__(kThreads) void tape_replay_kernel(Table P, ReplayArgs A) {
     constexpr int TPR = DK / 4;
     constexpr int RPP = kThreads / TPR;
     constexpr int ROWS = RPP * NR;
@@ -136,8 +141,9 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayPa
     // the scalar arguments in one burst of loads (the per-layer pointer tables are indexed by the layer and stay lazy)
     asm volatile("" ::"s"(A.mask), "s"(A.steps_dev), "s"(A.mask_dtype), "s"(A.tape_dtype), "s"(A.in_dtype), "s"(A.steps), "s"(A.skip_if_full),
                  "s"(A.T_tape), "s"(A.Hk), "s"(A.Hv), "s"(A.Dv));
-    if constexpr (LAYERS > 1) asm volatile("" ::"s"(P.verify_ids), "s"(P.posterior), "s"(P.start_inout), "s"(P.out4), "s"(P.V), "s"(P.keep), "s"(P.row16));
-    const int layer = LAYERS == 1 ? 0 : blockIdx.z;
+    if constexpr (Table::kAccept) asm volatile("" ::"s"(P.verify_ids), "s"(P.posterior), "s"(P.start_inout), "s"(P.out4), "s"(P.V));
+    if constexpr (Table::kWindows) asm volatile("" ::"s"(P.keep), "s"(P.row16));
+    const int layer = Table::kLayers == 1 ? 0 : blockIdx.z;
     const int bh = blockIdx.y;
     const int b = bh / A.Hv, hv = bh % A.Hv;
     const int hk = hv / (A.Hv / A.Hk);
@@ -149,7 +155,7 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayPa
 
     int n = A.steps;
     bool counted = false;
-    if constexpr (LAYERS > 1) {
+    if constexpr (Table::kAccept) {
         if (P.verify_ids) {
             counted = true;
             // The cycle's acceptance (DFlashRuntime.swift:525-547) is decided here, by every workgroup for
@@ -283,7 +289,7 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayPa
     uint4 win = make_uint4(0u, 0u, 0u, 0u);
     int win_at = -1;                                       // the thread's first piece (-1: none)
     auto window_piece = [&](int i, uint4& x) -> bool {
-        if constexpr (LAYERS > 1) {
+        if constexpr (Table::kWindows) {
             const int j = i / P.row16, p = i - j * P.row16, src = n + j;
             if (src >= P.keep + A.T_tape) return false;    // clamped slice end (RecurrentRollbackCache.swift:156)
             const uint4* from = src < P.keep ? P.win_snap[layer] : P.win_qkv[layer];
@@ -295,7 +301,7 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayPa
         return false;
     };
     const int win_of = (hv * gridDim.x + blockIdx.x) * kThreads + tid;
-    if constexpr (LAYERS > 1) {
+    if constexpr (Table::kWindows) {
         if (P.keep > 0 && P.win_out[layer])                // uniform
             if (win_of < P.keep * P.row16 && window_piece(win_of, win)) win_at = win_of;
     }
@@ -331,7 +337,7 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(typename ReplayPa
         const int r = row0 + rsub + RPP * i;
         if (owner && r < A.Dv) store4(s_out + (size_t)r * DK + c4, s[i]);
     }
-    if constexpr (LAYERS > 1) {
+    if constexpr (Table::kWindows) {
         if (P.keep > 0 && P.win_out[layer]) {
             const int pieces = P.keep * P.row16, all = A.Hv * gridDim.x * kThreads;
             uint4* out = P.win_out[layer] + (size_t)b * pieces;
@@ -346,7 +352,11 @@ template <typename StateT, bool VEC_G, int DK, int NR>
 static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, const ReplayArgs& A, int B, int n_layers) {
     constexpr int ROWS = kThreads / (DK / 4) * NR;
     dim3 grid((A.Dv + ROWS - 1) / ROWS, B * A.Hv, n_layers);
-    if (n_layers > kFewLayers) return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, DFLASH_MAX_BATCHED_LAYERS>, grid, dim3(kThreads), 0, P, A);
+    if (n_layers > kFewLayers) {
+        typedef ReplayAccept<DFLASH_MAX_BATCHED_LAYERS> Plain;
+        if (P.keep > 0) return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, ReplayTable>, grid, dim3(kThreads), 0, P, A);
+        return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, Plain>, grid, dim3(kThreads), 0, static_cast<const Plain&>(P), A);
+    }
     if (n_layers > 1 || P.keep > 0 || P.verify_ids) {
         ReplayWindows<kFewLayers> few = {};
         for (int l = 0; l < n_layers; ++l) {
@@ -356,10 +366,10 @@ static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, 
         }
         few.keep = P.keep; few.row16 = P.row16;
         few.verify_ids = P.verify_ids; few.posterior = P.posterior; few.start_inout = P.start_inout; few.out4 = P.out4; few.V = P.V;
-        return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, kFewLayers>, grid, dim3(kThreads), 0, few, A);
+        return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, ReplayWindows<kFewLayers>>, grid, dim3(kThreads), 0, few, A);
     }
     const ReplayBatch<1> one = {{P.tape[0]}, {P.k[0]}, {P.g[0]}, {P.state_in[0]}, {P.state_out[0]}};
-    return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, 1>, grid, dim3(kThreads), 0, one, A);
+    return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, ReplayBatch<1>>, grid, dim3(kThreads), 0, one, A);
 }
 
 template <typename StateT, bool VEC_G, int DK>
