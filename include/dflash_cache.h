@@ -66,7 +66,9 @@ int dflash_cache_record_tape(dflash_cache_t* c, const void* tape, int tape_dtype
                              int B, int T, int Hk, int Hv, int Dk, int Dv, int C);
 /* rollback(nAccepted:) (:95-131, :208-214): restores the snapshot, replays
  * acceptedSteps = nAccepted + 1 tape steps (:115) and rebuilds the conv window
- * (:139-158), enqueued on `stream`; then clears the transients. */
+ * (:139-158), enqueued on `stream`; then clears the transients.  A call whose arguments or slots do not
+ * pass the check ahead of it changes nothing (the cache stays armed); where a launch is refused behind that
+ * (a head dim the replay does not take), the cache is disarmed with both slots as they were when it was armed. */
 int dflash_cache_rollback(dflash_cache_t* c, void* stream, int n_accepted);
 /* clearTransients() (:163-170, :216-220). */
 int dflash_cache_clear_transients(dflash_cache_t* c);

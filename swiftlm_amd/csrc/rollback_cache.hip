@@ -103,26 +103,30 @@ bool same_window(const ReplayJob& a, const ReplayJob& b) {
     return a.steps == b.steps && x->B == y->B && x->keep == y->keep && x->T == y->T && x->C == y->C && x->qkv_elem_bytes == y->qkv_elem_bytes;
 }
 
-// The conv windows that no replay took along, one launch per group of equal shapes, and the slots as they are after the rollback.
+// The conv windows that no replay took along, one launch per group of equal shapes, and then, with everything enqueued, the slots as they
+// are after the rollback.  A launch that is refused leaves every cache at its snapshot, window and state alike: what the launches before it
+// wrote is in the post-verify buffers, which no slot holds.
 int finish_rollbacks(const std::vector<ReplayJob>& jobs, std::vector<char>& rebuilt, void* stream) {
     for (size_t i = 0; i < jobs.size(); ++i) {
-        dflash_cache* c = jobs[i].c;
-        c->slot[1] = jobs[i].post_state;                          // :126, the replayed state
-        if (c->keep <= 0) c->slot[0] = nullptr;                   // :142
-        if (rebuilt[i] || !rebuilds_window(c)) continue;          // :140, without qkv the restored window stays
+        const dflash_cache* c = jobs[i].c;
+        if (rebuilt[i] || !rebuilds_window(c)) continue;
         const void *snap[DFLASH_MAX_BATCHED_LAYERS], *qkv[DFLASH_MAX_BATCHED_LAYERS];
         void* out[DFLASH_MAX_BATCHED_LAYERS];
-        size_t member[DFLASH_MAX_BATCHED_LAYERS];
         int n = 0;
         for (size_t j = i; j < jobs.size() && n < DFLASH_MAX_BATCHED_LAYERS; ++j) {
             if (rebuilt[j] || !rebuilds_window(jobs[j].c) || !same_window(jobs[i], jobs[j]) || (long)(n + 1) * c->B > 65535) continue;
             rebuilt[j] = 1;
             snap[n] = jobs[j].c->snap[0]; qkv[n] = jobs[j].c->qkv; out[n] = jobs[j].post_conv;
-            member[n++] = j;
+            ++n;
         }
         int rc = dflash::rebuild_conv_batched(stream, n, snap, qkv, out, c->B, c->keep, c->T, c->C, c->qkv_elem_bytes, jobs[i].steps, nullptr);
         if (rc) return rc;
-        for (int m = 0; m < n; ++m) jobs[member[m]].c->slot[0] = out[m];   // :127
+    }
+    for (const ReplayJob& job : jobs) {
+        dflash_cache* c = job.c;
+        c->slot[1] = job.post_state;                              // :126, the replayed state
+        if (c->keep <= 0) c->slot[0] = nullptr;                   // :142
+        else if (rebuilds_window(c)) c->slot[0] = job.post_conv;  // :127; without qkv (:140) the restored window stays
     }
     return DFLASH_OK;
 }
@@ -207,7 +211,7 @@ int replay_jobs(const std::vector<ReplayJob>& jobs, void* stream) {
                                              sin.data(), sout.data(), a->state_dtype, jobs[i].steps, a->B, a->T, a->Hk, a->Hv, a->Dk, a->Dv, win);
             if (rc) return rc;
             for (size_t m = 0; m < group.size(); ++m)
-                if (out[m]) { rebuilt[group[m]] = 1; jobs[group[m]].c->slot[0] = out[m]; }      // :127
+                if (out[m]) rebuilt[group[m]] = 1;
         } else {
             rc = dflash_tape_replay_batched(stream, (int)tape.size(), tape.data(), a->tape_dtype, k.data(), g.data(),
                                             a->in_dtype, a->g_ndim, sin.data(), sout.data(), a->state_dtype,

@@ -187,6 +187,44 @@ def test_restore_matches_oracle_actions(acc, drafted):
         lib.dflash_cache_destroy(h)
 
 
+@pytest.fixture(scope="module")
+def rollback_check(tmp_path_factory):
+    """Runs tests/rollback/rollback_check.cpp: (launches, status, [(armed, window, state)] per cache)."""
+    import subprocess
+
+    exe, lib = tmp_path_factory.mktemp("rollback") / "rollback_check", os.path.dirname(_lib.LIB_PATH)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-rdynamic", os.path.join(ROOT, "tests", "rollback", "rollback_check.cpp"),
+                           "-o", str(exe), "-L" + lib, "-ldflash_hip", "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath," + lib,
+                           "-Wl,-rpath,/opt/rocm/lib"])
+
+    def run(refuse, keep, channels, *dks):
+        lines = subprocess.run([str(exe)] + [str(x) for x in (refuse, keep, channels, *dks)], capture_output=True, text=True,
+                               check=True).stdout.splitlines()
+        at = next(i for i, line in enumerate(lines) if line.startswith("status"))
+        return lines[:at], int(lines[at].split()[1]), [(int(a), int(w, 16), int(s, 16)) for a, w, s in (line.split() for line in lines[at + 1:])]
+
+    return run
+
+
+BEFORE, AFTER = (0, 0x1000, 0x2000), (0, 0x3000, 0x4000)      # disarmed, window and state of before and after the verify step
+
+
+@pytest.mark.parametrize("keep,channels,dks,launches,after", [
+    (3, 64, (64, 128), ["replay+windows 1", "replay+windows 1"], AFTER),
+    (3, 64, (64, 64, 128), ["replay+windows 2", "replay+windows 1"], AFTER),
+    (3, 12, (64, 128), ["replay 1", "replay 1", "windows 2"], AFTER),           # rows of 24 bytes: windows in a launch of their own
+    (3, 0, (64, 128), ["replay 1", "replay 1"], (0, 0x1000, 0x4000)),           # no qkv: the restored window stays
+])
+def test_rollback_refused_at_any_launch_keeps_both_halves_of_a_cache(rollback_check, keep, channels, dks, launches, after):
+    """A rollback takes a launch per replay shape, and any of them may be refused (a head dim that the replay does not take, rows that
+    the windows' kernel does not): whichever it is, every cache has the window and the state of the same moment afterwards, those of
+    before the verify step, and nothing behind it is launched.  With all of them enqueued both are what the launches write."""
+    assert rollback_check(-1, keep, channels, *dks) == (launches, 0, [after] * len(dks))
+    for i in range(len(launches)):
+        want = launches[:i] + [launches[i] + " refused"]
+        assert rollback_check(i, keep, channels, *dks) == (want, _lib.UNSUPPORTED, [BEFORE] * len(dks))
+
+
 def test_argument_validation_needs_no_gpu_for_null_checks():
     # Null handles are rejected before anything touches a device.
     lib = _lib.load()
