@@ -686,7 +686,8 @@ PyObject* restore(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int rc = enqueue([&] { return dflash_restore_target_cache_after_acceptance(h.data(), (int)h.size(), st, target, acc, drafted, &ns); });
     for (size_t i = 0; i < h.size() && (Py_ssize_t)i < PyList_GET_SIZE(a[0]); ++i) {
         const int kind = dflash_cache_kind(h[i]);
-        if (kind == DFLASH_CACHE_TAPE || kind == DFLASH_CACHE_SNAPSHOT) forget_dead(PyList_GET_ITEM(a[0], (Py_ssize_t)i), h[i]);
+        // armed: the call was refused ahead of any change, and the handle still points at the snapshot, whose tensors no slot may hold
+        if ((kind == DFLASH_CACHE_TAPE || kind == DFLASH_CACHE_SNAPSHOT) && !dflash_cache_is_armed(h[i])) forget_dead(PyList_GET_ITEM(a[0], (Py_ssize_t)i), h[i]);
     }
     return Py_BuildValue("(iL)", rc, (long long)ns);
     END_HANDLE_TH_ERRORS

@@ -118,8 +118,10 @@ class _RollbackCache(_NativeCache):
 
     def _after_rollback(self) -> None:
         # tape tensors stay referenced until the next cycle records new ones: the replay
-        # that reads them may still be queued on the stream.
-        self._forget_dead()
+        # that reads them may still be queued on the stream.  A rollback that was refused leaves the cache
+        # armed: the handle still points at the snapshot, whose tensors no slot holds any more.
+        if not self._holds_snapshot():
+            self._forget_dead()
 
 
 class RecurrentRollbackCache(_RollbackCache):

@@ -96,6 +96,27 @@ def test_cache_rollback_requires_functional_update():
     lib.dflash_cache_destroy(c)
 
 
+def test_refused_rollback_keeps_the_snapshots_tensors(monkeypatch):
+    """A refused rollback leaves the handle armed and pointing at the snapshot, also where a slot holds another tensor by then: the
+    cache object still holds the snapshot's until a rollback or clear_transients has let go of them."""
+    from swiftlm_amd import RecurrentRollbackCache, rollback_cache
+
+    monkeypatch.setattr(rollback_cache, "_stream", lambda: None)
+    lib, c = _lib.load(), RecurrentRollbackCache()
+    for slot, p in enumerate((0x1000, 0x2000)):
+        lib.dflash_cache_set_slot(c._h, slot, p)
+        c._by_ptr[p] = f"snapshot {slot}"
+    c.arm_rollback(0)
+    lib.dflash_cache_set_slot(c._h, 0, 0x3000)                 # a new window, but the state is still the pre-verify one
+    c._by_ptr[0x3000] = "window"
+    assert lib.dflash_cache_record_tape(c._h, 0x10, _lib.F32, 0x20, 0x30, _lib.BF16, 3, None, 2, _lib.F32, 1, 16, 16, 32, 128, 128, 0) == 0
+    with pytest.raises(_lib.DFlashError, match="pre-verify"):
+        c.rollback(3)
+    assert c.is_armed and c._by_ptr == {0x1000: "snapshot 0", 0x2000: "snapshot 1", 0x3000: "window"}
+    c.clear_transients()
+    assert not c.is_armed and c._by_ptr == {0x2000: "snapshot 1", 0x3000: "window"}
+
+
 def test_restore_validates_every_cache_before_touching_any():
     """A list whose LAST cache cannot be rolled back (slot 1 still holds the pre-verify buffer), or that holds a
     null handle, is refused as a whole: the caches before it keep their snapshot, tape, armed flag and offsets."""

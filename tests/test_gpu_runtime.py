@@ -296,6 +296,32 @@ def test_rollback_of_a_window_over_another_shapes_tape(gpu_lib):
         assert torch.equal(c[0], window) and torch.equal(c[1], state)
 
 
+@pytest.mark.parametrize("whole_list", [True, False])
+def test_refused_rollback_can_be_corrected_and_called_again(gpu_lib, whole_list):
+    """The pre-verify window, which no slot holds any more when the first call is refused, is still the snapshot that the second reads."""
+    from swiftlm_amd import DFlashError, DFlashKernels as K, DFlashRuntime as R, RecurrentRollbackCache
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    T, n, C = 7, 2, 64
+    c, state, snap = RecurrentRollbackCache(), rnd(1, 2, 16, 64), rnd(1, 3, C).bfloat16()
+    tape, k, dec, qkv = rnd(1, T, 2, 16), rnd(1, T, 2, 64).bfloat16(), torch.sigmoid(rnd(1, T, 2)).bfloat16(), rnd(1, T, C).bfloat16()
+    want = K.tape_replay_kernel(tape[:, :n].contiguous(), k[:, :n].contiguous(), dec[:, :n].contiguous(), state)
+    window = torch.cat([snap, qkv], dim=1)[:, n:n + 3].clone()
+    c[0], c[1] = snap, state
+    c.arm_rollback(0)
+    c[0] = torch.zeros_like(snap)
+    c.record_tape(tape, k, dec, qkv)
+    at = snap.data_ptr()
+    snap = None
+    roll = (lambda: R.restore_target_cache_after_acceptance([c], n, n - 1, T)) if whole_list else (lambda: c.rollback(n - 1))
+    with pytest.raises(DFlashError):                           # slot 1 still holds the pre-verify state
+        roll()
+    assert c.is_armed and at in c._by_ptr
+    c[1] = torch.zeros_like(state)
+    roll()
+    assert not c.is_armed and torch.equal(c[0], window) and torch.equal(c[1], want) and at not in c._by_ptr
+
+
 def test_snapshot_cache_restores_pre_verify_state(gpu_lib):
     from swiftlm_amd import MambaSnapshotCache
 
