@@ -208,6 +208,19 @@ __device__ __forceinline__ float gdn_gated_out(float y, float inv, float w, floa
     return y * inv * w * act;
 }
 
+// mask element of run-time type, as it lies in memory, and what it says: for a load that is asked for ahead of its use
+__device__ __forceinline__ uint32_t mask_bits(const void* mask, int mask_dtype, int idx) {
+    if (mask_dtype == DFLASH_F32) return reinterpret_cast<const uint32_t*>(mask)[idx];
+    if (mask_dtype == DFLASH_U8) return reinterpret_cast<const uint8_t*>(mask)[idx];
+    return reinterpret_cast<const uint16_t*>(mask)[idx];
+}
+__device__ __forceinline__ bool mask_bits_on(uint32_t bits, int mask_dtype) {
+    const float m = mask_dtype == DFLASH_F32    ? __uint_as_float(bits)
+                    : mask_dtype == DFLASH_BF16 ? __uint_as_float(bits << 16)
+                    : mask_dtype == DFLASH_F16  ? (float)__builtin_bit_cast(_Float16, (uint16_t)bits)
+                                                : (float)bits;
+    return m > 0.5f;
+}
 // mask element of run-time type -> "this step runs"
 __device__ __forceinline__ bool mask_on(const void* mask, int mask_dtype, int idx) {
     float m;

@@ -24,7 +24,8 @@ namespace dflash {
 //                         m-1 T = (I + diag(beta) A)^-1 diag(beta) by substitution; interval m the loads of chunk m+4;
 //                         interval m+1 y and the tape of the chunk, and the decays of chunk m+4.
 //
-// One barrier per chunk, no wave waits for memory inside a chunk (loads are asked for two chunks ahead of their use), and
+// One barrier per chunk, loads asked for one interval ahead of their use (decays, beta, the mask, v) or two (k and q), all of them
+// before any is waited for: a load that is asked for and used in one place stands behind k and q, for which all waves wait then.  And
 // no operand crosses lanes: with S^T as the accumulator a lane holds row l%16 and channels 4*(l/16)+v, which is also how
 // the next product's b operand may be laid out, as the order of a contraction's indices is free.
 //
@@ -35,13 +36,15 @@ namespace dflash {
 // Bound by the length of an interval, of which the chain works 1,190 / 1,390 / 1,880 cycles at Dk = 64 / 128 / 256 (the split of the
 // state on the VALU, the exchange of the partial sums through LDS, three groups of dependent MFMAs), the producers 340 to 1,330 (1,940 at
 // Dk = 256: k rows).  With the decays formed beside the k rows that interval was as long as the chain's (1,320, 2,150 at 256), and all
-// wait for the longest: 1,003 steps, 32 heads of 128x128 45.4 -> 44.6 us, 730 of Dk = 256 45.4 -> 42.3, 257 of 8 heads 13.6 -> 13.2.
+// wait for the longest: 1,003 steps, 32 heads of 128x128 42.0 -> 41.3 us, 730 of 8 heads, Dk = 256 44.1 -> 40.9; with a mask 53.4 -> 43.8
+// and 49.6 -> 41.9 (52.1 and 43.7 with the mask's elements asked for where they are used).
 // us, chunk by chunk kernel against this one: 1,003 steps, 32 heads of 128x128 152 -> 41; 730 steps, 8 heads, Dk = 256 147 -> 42;
 // two sequences of 1,000 steps, 32 heads, Dk = 256 419 -> 116; 40 steps 8.3 -> 5.4.
 // The care for what is not finite (y, the rows of masked steps) costs or gives 3 %: 1,000 steps of Dk = 256 64.8 -> 66.9, Dk = 64 36.7 ->
 // 37.1, 1,003 steps of Dk = 128 43.1 -> 42.1.
-// 95 / 121 / 189 registers: two workgroups share a compute unit at Dk = 64 and 128 (two sequences of 1,000 steps 71 where one takes
-// 42), at 256 a second sequence waits for the first (59 for one).
+// 104 / 121 / 160 registers without a mask, 114 / 128 / 177 with one: two workgroups share a compute unit at Dk = 64 and 128 (two sequences
+// of 1,000 steps 68 where one takes 41), which the launch bounds ask for: at 133 registers one of them waits for the other (with a mask
+// 102, now 69).  At 256 a second sequence waits for the first (57 for one).
 // ---------------------------------------------------------------------------
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));
@@ -77,7 +80,7 @@ template <int L0, int L1, int L2, int L3> __device__ __forceinline__ float quad_
 constexpr int kLongThreads = 512;
 
 template <int DK, bool MASKED>
-__global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnArgs A) {
+__global__ __launch_bounds__(kLongThreads, DK == 256 ? 2 : 4) void gated_delta_long_kernel(GdnArgs A) {
     using Lds = GdnLongLds<DK>;
     extern __shared__ __align__(16) unsigned char gdn_chunk_smem[];
     Lds& L = *reinterpret_cast<Lds*>(gdn_chunk_smem);
@@ -240,6 +243,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
     u32x4v kr[NK], qr[NK];                              // row j * RPI + rs, channels 8 pc .. +7
     uint2 vr;                                           // v of step n, rows 4g .. +3
     bf16_t gr, br;
+    uint32_t mr = 0;                                    // MASKED: the bits of step n's mask element
     auto request = [&](int m) {
         const int t0 = m * kChunkSteps, tc = min(A.T - t0, kChunkSteps);
         const uint32_t bt0 = (uint32_t)b * A.T + t0;                                   // uniform, as are the products with it
@@ -247,6 +251,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
         const uint32_t go = bt0 * A.Hv + hv + __umul24(tl, A.Hv);
         gr = gp[go];                                   // needed first
         br = bp[go];
+        if constexpr (MASKED) mr = mask_bits(A.mask, A.mask_dtype, (int)(bt0 + tl));
         vr = reinterpret_cast<const Rows4x16*>(vp + ((bt0 * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(tl, step)))->x;
         const uint32_t o = (bt0 * A.Hk + hk) * DK + 8 * pc;
 #pragma unroll
@@ -274,7 +279,7 @@ __global__ __launch_bounds__(kLongThreads, 2) void gated_delta_long_kernel(GdnAr
         const int t0 = m * kChunkSteps, tc = min(A.T - t0, kChunkSteps);
         step_on = n < tc;
         if constexpr (MASKED) {
-            step_on = step_on && mask_on(A.mask, A.mask_dtype, (int)((uint32_t)b * A.T + t0 + min(n, tc - 1)));
+            step_on = step_on && mask_bits_on(mr, A.mask_dtype);
             counted = (uint32_t)__builtin_amdgcn_ballot_w64(step_on) & 0xffffu;
         }
         vr = step_on ? vr : make_uint2(0u, 0u);

@@ -290,6 +290,30 @@ def test_ragged_shares_are_found_in_few_sums(tmp_path):
     assert slowest > 200
 
 
+def _kernel_registers(tmp_path):
+    """{kernel name: (vector registers, bytes of scratch)} of the built library's device code."""
+    import glob
+    import subprocess
+
+    os.symlink(_lib.LIB_PATH, tmp_path / "lib.so")
+    subprocess.run(["/opt/rocm/llvm/bin/llvm-objdump", "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
+    found = {}
+    for f in glob.glob(str(tmp_path / "lib.so.*gfx950")):
+        notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", f], capture_output=True, text=True, check=True).stdout
+        for entry in notes.split("  - .agpr_count:")[1:]:
+            field = lambda name: re.search(r"\.%s:\s+(\S+)" % name, entry).group(1)
+            found[field("name")] = int(field("vgpr_count")), int(field("private_segment_fixed_size"))
+    return found
+
+
+@pytest.mark.parametrize("Dk", [64, 128])
+@pytest.mark.parametrize("masked", [0, 1])
+def test_two_workgroups_of_a_prompt_share_a_compute_unit(tmp_path, Dk, masked):
+    """Eight waves each: four waves on a SIMD, which share its 512 registers, and no state in scratch."""
+    registers, scratch = next(v for n, v in _kernel_registers(tmp_path).items() if f"gated_delta_long_kernelILi{Dk}ELb{masked}E" in n)
+    assert registers <= 128 and scratch == 0
+
+
 def test_library_builds_without_python():
     """The library and its plain-C clients are what `make` builds by default, on a machine without Python or PyTorch too; the
     Python package's binding is a target of its own."""

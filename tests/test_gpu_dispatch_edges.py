@@ -98,6 +98,30 @@ def test_long_forward(gpu_lib, Dk, Dv, T, masked):
     np.testing.assert_allclose(host(y2), host(y), rtol=2e-2, atol=2e-2)
 
 
+# A mask of any type, its elements around the line (0.5 does not run, the next value above does, NaN does not): the bits of zeros and ones.
+# Chunks whose mask is asked for ahead of the loop (the first four), in it, and in a ragged last one; two sequences; any address.
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16, torch.uint8], ids=str)
+@pytest.mark.parametrize("Dk,T", [(64, 17), (128, 70), (128, 131), (256, 97)])
+def test_long_forward_mask_types(gpu_lib, Dk, T, dt):
+    from swiftlm_amd import DFlashKernels as K
+
+    d = O.make_gdn_inputs(Dk + T, 2, T, 2, 4, Dk, 32, in_dtype="bf16")
+    ins = [dev(d[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")]
+    if dt == torch.uint8:
+        values, on = [0, 1, 2, 255], [0, 1, 1, 1]
+    else:
+        above = float(torch.tensor(0.5, dtype=dt).float()) * (1 + torch.finfo(dt).eps)
+        values, on = [0.0, 0.5, above, 1.0, float("nan"), float("inf"), -1.0, torch.finfo(dt).tiny], [0, 0, 1, 1, 0, 1, 0, 0]
+    pick = np.random.default_rng(T).integers(0, len(values), (2, T))
+    mask = torch.empty(2 * T + 1, dtype=dt, device="cuda")[1:].view(2, T).copy_(torch.tensor(values, dtype=torch.float64).to(dt)[torch.from_numpy(pick)])
+    plain = np.array(on, np.float32)[pick]
+    want = K.gated_delta_kernel_with_tape(*ins, dev(d["state"]), dev(plain))
+    for got, w in zip(K.gated_delta_kernel_with_tape(*ins, dev(d["state"]), mask), want):
+        assert torch.equal(got, w)
+    sw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], plain, dtype=np.float64)[1]
+    np.testing.assert_allclose(host(want[1]), sw, rtol=1e-4, atol=1e-6)
+
+
 # v, y and the tape may lie at any address of their elements: the kernel of aligned ones, hence its bits, and nothing beside them
 @pytest.mark.parametrize("off", [1, 2, 4])
 def test_long_forward_v_alignment(gpu_lib, off):
