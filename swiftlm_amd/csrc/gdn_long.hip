@@ -36,22 +36,25 @@ namespace dflash {
 // Bound by the length of an interval, of which the chain works 1,190 / 1,390 / 1,880 cycles at Dk = 64 / 128 / 256 (the split of the
 // state on the VALU, the exchange of the partial sums through LDS, three groups of dependent MFMAs), the producers 340 to 1,330 (1,940 at
 // Dk = 256: k rows).  With the decays formed beside the k rows that interval was as long as the chain's (1,320, 2,150 at 256), and all
-// wait for the longest: 1,003 steps, 32 heads of 128x128 42.0 -> 41.3 us, 730 of 8 heads, Dk = 256 44.1 -> 40.9; with a mask 53.4 -> 43.8
-// and 49.6 -> 41.9 (52.1 and 43.7 with the mask's elements asked for where they are used).
+// wait for the longest: 1,003 steps, 32 heads of 128x128 42.0 -> 41.3 us, 730 of 8 heads, Dk = 256 44.1 -> 41.3; with a mask 53.4 -> 42.5
+// and 49.6 -> 42.3 (52.1 and 43.7 with the mask's elements asked for where they are used).
 // us, chunk by chunk kernel against this one: 1,003 steps, 32 heads of 128x128 152 -> 41; 730 steps, 8 heads, Dk = 256 147 -> 42;
 // two sequences of 1,000 steps, 32 heads, Dk = 256 419 -> 116; 40 steps 8.3 -> 5.4.
 // The care for what is not finite (y, the rows of masked steps) costs or gives 3 %: 1,000 steps of Dk = 256 64.8 -> 66.9, Dk = 64 36.7 ->
 // 37.1, 1,003 steps of Dk = 128 43.1 -> 42.1.
-// 104 / 121 / 160 registers without a mask, 114 / 128 / 177 with one: two workgroups share a compute unit at Dk = 64 and 128 (two sequences
+// 102 / 119 / 158 registers without a mask, 109 / 128 / 171 with one: two workgroups share a compute unit at Dk = 64 and 128 (two sequences
 // of 1,000 steps 68 where one takes 41), which the launch bounds ask for: at 133 registers one of them waits for the other (with a mask
 // 102, now 69).  At 256 a second sequence waits for the first (57 for one).
 // ---------------------------------------------------------------------------
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));
-// rows of v, y and the tape at any address that their elements may have: one load or store all the same
-struct __attribute__((packed, aligned(2))) Rows4x16 { uint2 x; };
-struct __attribute__((packed, aligned(4))) Rows4x32 { f32x4v x; };
+typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));   // (a select between two HIP uint4 is a select of addresses: the arrays end in scratch)
+// rows of v, y and the tape at any address that their elements may have: one load or store all the same (a HIP uint2 is a class, which
+// is not packed: it would claim 8 bytes)
+struct __attribute__((packed, aligned(2))) Rows4x16 { u32x2v x; };
+struct __attribute__((packed, aligned(4))) Rows4x32 { f32x4v x; };
+static_assert(alignof(Rows4x16) == 2 && alignof(Rows4x32) == 4, "no more than the elements have");
 
 template <int DK> struct GdnLongLds {
     static constexpr int LB = DK + 8;      // row pitch: 16 bytes of pad spread 16-byte reads of a column of rows over the banks
@@ -241,7 +244,7 @@ __global__ __launch_bounds__(kLongThreads, DK == 256 ? 2 : 4) void gated_delta_l
     static_assert(16 / RPI == NK, "as many loads as steps of the contraction");
     const int rs = lane / CPR, pc = lane % CPR;
     u32x4v kr[NK], qr[NK];                              // row j * RPI + rs, channels 8 pc .. +7
-    uint2 vr;                                           // v of step n, rows 4g .. +3
+    u32x2v vr;                                          // v of step n, rows 4g .. +3
     bf16_t gr, br;
     uint32_t mr = 0;                                    // MASKED: the bits of step n's mask element
     auto request = [&](int m) {
@@ -282,7 +285,7 @@ __global__ __launch_bounds__(kLongThreads, DK == 256 ? 2 : 4) void gated_delta_l
             step_on = step_on && mask_bits_on(mr, A.mask_dtype);
             counted = (uint32_t)__builtin_amdgcn_ballot_w64(step_on) & 0xffffu;
         }
-        vr = step_on ? vr : make_uint2(0u, 0u);
+        vr = step_on ? vr : u32x2v{0u, 0u};
         // decay products G[v] = g_{s+1} ... g_t of the lane's pairs (s, t) = (4g + v, n), 1 where s >= t
         const float gl = step_on ? to_float(gr) : 1.f;
         beta = step_on ? to_float(br) : 0.f;
@@ -308,7 +311,7 @@ __global__ __launch_bounds__(kLongThreads, DK == 256 ? 2 : 4) void gated_delta_l
     auto store_rows = [&](int m, int tc) {             // one store each: row by row, two and four bytes per lane, they were eight
         const uint32_t o = (((uint32_t)b * A.T + m * kChunkSteps) * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(n, step);
         if (n < tc) {
-            uint2 y2;
+            u32x2v y2;
             y2.x = (uint32_t)from_float<bf16_t>(yv[0]).bits | ((uint32_t)from_float<bf16_t>(yv[1]).bits << 16);
             y2.y = (uint32_t)from_float<bf16_t>(yv[2]).bits | ((uint32_t)from_float<bf16_t>(yv[3]).bits << 16);
             reinterpret_cast<Rows4x16*>(reinterpret_cast<bf16_t*>(A.y) + o)->x = y2;
