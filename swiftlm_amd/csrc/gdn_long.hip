@@ -44,7 +44,7 @@ namespace dflash {
 // 37.1, 1,003 steps of Dk = 128 43.1 -> 42.1.
 // 102 / 119 / 158 registers without a mask, 109 / 128 / 171 with one: two workgroups share a compute unit at Dk = 64 and 128 (two sequences
 // of 1,000 steps 68 where one takes 41), which the launch bounds ask for: at 133 registers one of them waits for the other (with a mask
-// 102, now 69).  At 256 a second sequence waits for the first (57 for one).
+// 102, now 69).  At 256 a second sequence waits for the first (59 for one).
 // ---------------------------------------------------------------------------
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));

@@ -116,10 +116,11 @@ at::Tensor fresh(at::IntArrayRef size, at::ScalarType st, const at::Tensor& like
     return at::Tensor(at::detail::empty_cuda(size, st, like.device(), std::nullopt));
 }
 
-// The outputs of one call, small ones out of one allocation: a tensor costs the host 0.6 us from the allocator and back, of a call
-// that enqueues in 3 (a layer of seven outputs 9.6 us, now 7.7; a forward 6.0, now 5.5; attention with its logsumexp 8.8, now 8.4).  They are ordinary tensors over one storage, so
-// that record_stream and the like act on the memory that all of them are in; it is free when the last of them is.  Larger ones
-// (kSharedBytes together), of prompts say, have their own, as one of them would keep the others' memory.
+// The outputs of one call that a program lets go of together, small ones out of one allocation: a tensor costs the host 0.6 us from the
+// allocator and back, of a call that enqueues in 3 (a layer of nine outputs 9.4 us, now 8.0; a forward 5.7, now 5.2; attention with its
+// logsumexp 8.8, now 8.4).  They are ordinary tensors over one storage, so that record_stream and the like act on the memory that all of
+// them are in; it is free when the last of them is.  Hence what a cache keeps from block to block (the new state and conv window) is not
+// among them, and larger ones (kSharedBytes together), of prompts say, have their own, as one would keep the others' memory.
 class Outputs {
     static constexpr size_t kSharedBytes = 4 << 20, kAlign = 256;
     const at::Tensor& like;
@@ -282,13 +283,14 @@ PyObject* gdn_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::ScalarType dt = x_.scalar_type();
     const Held x = held(x_), w = held_as(w_, dt), cs = held_as(cs_, dt), al = held_as(al_, dt), bl = held_as(bl_, dt),
                alog = held_as(alog_, at::kFloat), dtb = held_as(dtb_, at::kFloat), state = held(state_);
-    const int64_t qk_size[4] = {B, T, Hk, Dk}, g_size[3] = {B, T, Hv}, y_size[4] = {B, T, Hv, Dv}, conv_size[3] = {B, K - 1, C}, none[1] = {0};
+    const int64_t qk_size[4] = {B, T, Hk, Dk}, g_size[3] = {B, T, Hv}, y_size[4] = {B, T, Hv, Dv}, none[1] = {0};
     const bool own_out = gate_.defined() && a[22] == Py_None;
     const auto only = [&](bool given, at::IntArrayRef size) { return given ? size : at::IntArrayRef(none); };
-    Outputs outs(*x, {{qk_size, dt}, {g_size, dt}, {y_size, dt}, {y_size, at::kFloat}, {conv_size, dt}, {only(want, qk_size), dt},
-                      {only(want, y_size), dt}, {only(want, g_size), dt}, {only(own_out, y_size), dt}});
+    Outputs outs(*x, {{qk_size, dt}, {g_size, dt}, {y_size, dt}, {y_size, at::kFloat}, {only(want, qk_size), dt}, {only(want, y_size), dt},
+                      {only(want, g_size), dt}, {only(own_out, y_size), dt}});
     at::Tensor k = outs.next(qk_size, dt), g = outs.next(g_size, dt), y = outs.next(y_size, dt), tape = outs.next(y_size, at::kFloat);
-    at::Tensor new_conv = outs.next(conv_size, dt), new_state = fresh(state->sizes(), at::kFloat, *state), q, v, beta, out, arrivals;
+    // on their own: a cache keeps them when the others are gone
+    at::Tensor new_conv = fresh({B, K - 1, C}, dt, *x), new_state = fresh(state->sizes(), at::kFloat, *state), q, v, beta, out, arrivals;
     if (want) {
         q = outs.next(qk_size, dt);
         v = outs.next(y_size, dt);

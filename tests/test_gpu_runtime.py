@@ -680,6 +680,23 @@ def test_outputs_of_a_call_are_tensors_of_their_own(gpu_lib, T, Hv):
     assert torch.equal(lse, want) and lse.shape == (1, 2, 16)
 
 
+@pytest.mark.parametrize("gate", [False, True])
+def test_what_a_cache_keeps_holds_no_other_output(gpu_lib, gate):
+    """A rollback cache keeps a layer's conv window and state from block to block: neither holds memory of another output."""
+    from swiftlm_amd import DFlashKernels as K
+    B, T, Hk, Hv, D = 1, 16, 2, 4, 64
+    C = 2 * Hk * D + Hv * D
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    kw = dict(gate=rnd(B, T, Hv, D), norm_weight=rnd(D)) if gate else {}
+    r = K.gdn_layer(rnd(B, T, C), rnd(B, 3, C), rnd(C, 4), rnd(B, T, Hv), rnd(B, T, Hv), rnd(Hv).float(), rnd(Hv).float(),
+                    torch.zeros(B, Hv, D, D, device="cuda"), Hk, Hv, D, D, q_scale=1.0, k_scale=1.0, want_intermediates=True, **kw)
+    for kept in ("conv_state", "state"):
+        assert r[kept].untyped_storage().nbytes() == r[kept].numel() * r[kept].element_size()
+        assert all(r[kept].untyped_storage().data_ptr() != t.untyped_storage().data_ptr() for n, t in r.items() if t is not None and n != kept)
+    assert r["y"].untyped_storage().data_ptr() == r["k"].untyped_storage().data_ptr()          # a block's own: one allocation
+
+
 @pytest.mark.parametrize("shape", [(2, 4, 16, 50), (50,), (1, 1, 1, 50), (4, 16, 50), (2, 1, 16, 1), (2, 4, 1, 50)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 def test_sdpa_mask_of_any_shape_that_broadcasts(gpu_lib, shape, dt):
