@@ -223,6 +223,39 @@ def test_batched_replay_equals_per_layer_replay(gpu_lib):
     assert all(bool((m == 7.0).all()) for m in marker)
 
 
+@pytest.mark.parametrize("layers", [1, 2, 8, 9, 64])
+@pytest.mark.parametrize("rows", [1, 4], ids=["one_row", "four_rows"])
+def test_batched_replay_of_any_number_of_layers(gpu_lib, layers, rows):
+    """The argument tables (1, up to 8 and up to 64 layers) with one row per thread and, from 4,096 workgroups on, four; the steps given,
+    and counted by the launch from the tokens.  Every layer's state is that of the replay on its own, bit for bit."""
+    from swiftlm_amd import DFlashKernels as K, _lib
+    from swiftlm_amd.dflash_kernels import _ptr, _ptr_array, _stream
+
+    T, Dk, Dv, n = 7, 128, 128, 3
+    Hv = 2 if rows == 1 else 4096 // (16 * layers) + 1
+    g = torch.Generator(device="cuda").manual_seed(layers)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    tapes = [rnd(1, T, Hv, Dv) for _ in range(layers)]
+    ks, gs = [rnd(1, T, 1, Dk).bfloat16() for _ in range(layers)], [torch.sigmoid(rnd(1, T, Hv)).bfloat16() for _ in range(layers)]
+    sin = [rnd(1, Hv, Dv, Dk) for _ in range(layers)]
+    want = [K.tape_replay_kernel(t[:, :n], k[:, :n], d[:, :n], s) for t, k, d, s in zip(tapes, ks, gs, sin)]
+    sout = [torch.full_like(s, float("nan")) for s in sin]
+    K.tape_replay_batched(tapes, ks, gs, sin, sout, steps=n)
+    assert all(torch.equal(a, b) for a, b in zip(sout, want))
+    sout = [torch.full_like(s, float("nan")) for s in sin]
+    ids = torch.arange(T, dtype=torch.int32, device="cuda")
+    post = ids + 1
+    post[n - 1] += 100                                         # ids[1:n] are the tokens, the next is not
+    out4, start = torch.zeros(4, dtype=torch.int32, device="cuda"), torch.full((1,), 50, dtype=torch.int32, device="cuda")
+    held = [_ptr_array(x) for x in (tapes, ks, gs, sin, sout)]
+    rc = _lib.load().dflash_accept_commit_replay_batched(
+        _stream(), _ptr(ids), _ptr(post), T, _ptr(start), _ptr(out4), layers, held[0][0], _lib.F32, held[1][0], held[2][0], _lib.BF16, 3,
+        held[3][0], held[4][0], _lib.F32, 0, 1, T, 1, Hv, Dk, Dv)
+    _lib.check(rc, "accept_commit_replay_batched")
+    assert all(torch.equal(a, b) for a, b in zip(sout, want))
+    assert out4.tolist() == [n - 1, n, n + 100, 50 + n] and start.item() == 50 + n
+
+
 @pytest.mark.parametrize("shape", [("cfg1", 1, 16, 16, 32, 128, 128), ("cfg0", 1, 8, 4, 8, 64, 64), ("dk256", 1, 6, 1, 2, 256, 64),
                                    ("long_T", 1, 40, 2, 4, 64, 32)], ids=lambda s: s[0])
 @pytest.mark.parametrize("in_dt", ["f32", "bf16"])
