@@ -272,6 +272,32 @@ def test_rollback_of_conv_windows_of_every_shape(gpu_lib, B, Hv, Dk, Dv, C, keep
         assert torch.equal(c[0], window) if keep else c[0] is None
 
 
+@pytest.mark.parametrize("layers,Hv", [(8, 2), (9, 2), (36, 2), (64, 2), (65, 2), (8, 33), (36, 32)])
+def test_rollback_of_many_caches_and_their_windows(gpu_lib, layers, Hv):
+    """The tables with room for the windows of 8 and of 64 caches, one cache more than a launch takes, and (33 heads of 8 caches, 32 of
+    36) the form with four rows per thread.  One cache has no window and one keeps the restored one.  Windows and states bit for bit."""
+    from swiftlm_amd import DFlashKernels as K, DFlashRuntime as R, RecurrentRollbackCache
+    T, n, D, C = 7, 3, 128, 264
+    g = torch.Generator(device="cuda").manual_seed(layers)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    caches, want = [], []
+    for i in range(layers):
+        c = RecurrentRollbackCache(conv_kernel_size=1 if i == 1 else 4)
+        snap, state, tape, k = rnd(1, 3, C).bfloat16(), rnd(1, Hv, D, D), rnd(1, T, Hv, D), rnd(1, T, 1, D).bfloat16()
+        dec, qkv = torch.sigmoid(rnd(1, T, Hv)).bfloat16(), rnd(1, T, C).bfloat16()
+        c[0], c[1] = snap, state
+        c.arm_rollback(0)
+        c[0], c[1] = torch.zeros_like(snap), torch.full_like(state, float("nan"))
+        c.record_tape(tape, k, dec, None if i == 2 else qkv)
+        caches.append(c)
+        window = None if i == 1 else snap if i == 2 else torch.cat([snap, qkv], dim=1)[:, n:n + 3]
+        want.append((window, K.tape_replay_kernel(tape[:, :n], k[:, :n], dec[:, :n], state)))
+    R.restore_target_cache_after_acceptance(caches, n, n - 1, T)
+    for c, (window, state) in zip(caches, want):
+        assert torch.equal(c[1], state)
+        assert c[0] is None if window is None else torch.equal(c[0], window)
+
+
 def test_rollback_of_a_window_over_another_shapes_tape(gpu_lib):
     """Caches of two replay shapes are two launches; the first one's window lies over the tape of the second, which the replays
     read before any window is written, as they do cache by cache of one shape."""
@@ -402,6 +428,21 @@ def test_greedy_tokens_at_any_row_address(gpu_lib, dt, T, V, off):
         res, post = DFlashRuntime.greedy_accept_commit(logits, mask_d, torch.from_numpy(verify).cuda(), 9)
         np.testing.assert_array_equal(post.cpu().numpy(), want)
         assert (res.acceptance_len, res.commit_count, res.staged_first_next, res.start) == (acc, acc + 1, want[acc], 10 + acc)
+
+
+@pytest.mark.parametrize("V", [64 * 8192, 64 * 8192 + 3, 130 * 8192 + 1])
+def test_greedy_tokens_of_rows_of_many_chunks(gpu_lib, V):
+    """More partials of a row than the finish's lanes ask for at once: the maximum in each of its rounds, tied, in the last chunk."""
+    from swiftlm_amd import DFlashRuntime
+    logits = torch.randn(4, V, generator=torch.Generator(device="cuda").manual_seed(V), device="cuda").bfloat16()
+    at = [V - 1, min(64 * 8192, V - 1), 63 * 8192 + 5, 17]
+    for t, i in enumerate(at):
+        logits[t, i] = 50.0
+    logits[3, V - 1] = logits[3, 40 * 8192] = 50.0             # tied: the first
+    assert DFlashRuntime.greedy_tokens_with_mask(logits).tolist() == at
+    ids = torch.tensor([1] + at[:3], dtype=torch.int32, device="cuda")
+    res, post = DFlashRuntime.greedy_accept_commit(logits, None, ids, 9)
+    assert post.tolist() == at and (res.acceptance_len, res.staged_first_next) == (3, at[3])
 
 
 def test_greedy_accept_commit_equals_two_steps(gpu_lib):
