@@ -109,7 +109,7 @@ template <int LAYERS> struct ReplayWindows : ReplayAccept<LAYERS> {
     uint4* win_out[LAYERS];            // [B,keep,row], null: no window for this layer
 };
 typedef ReplayWindows<DFLASH_MAX_BATCHED_LAYERS> ReplayTable;
-constexpr int kFewLayers = 8;          // tables of 1, 8 and 64: 92 bytes, 0.6 and 4.2 KB of arguments; without windows 0.4 and 2.6
+constexpr int kFewLayers = 8;          // tables of 1, 8 and 64: 92 bytes, 0.6 and 4.2 KB of arguments; 64 without windows 2.6
 // (more than eight layers without windows: four captured steps of 12 layers took 630 us, with the table that has room for windows 634 to 638)
 
 struct ReplayArgs {
@@ -348,23 +348,22 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(Table P, ReplayAr
     }
 }
 
-// The smallest table that holds the layers, and the windows' code and pointers only where there are windows.  us per launch with the
-// windows' table and without, no window to copy (a graph of launches, states from memory, 32 heads of 128x128, means of five runs that
-// differ by 0.1): 2 layers 5.27 5.25, 3 6.40 6.33, 4 7.61 7.55, 6 10.34 10.23, 8 (four rows per thread) 11.18 11.20; 3 of 8 heads of
-// 64x64 3.57 3.54.
-template <typename StateT, bool VEC_G, int DK, int NR, int LAYERS>
-static hipError_t launch_replay_table(LaunchBracket& br, dim3 grid, const ReplayWindows<LAYERS>& P, const ReplayArgs& A) {
-    typedef ReplayAccept<LAYERS> Plain;
-    if (P.keep > 0) return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, ReplayWindows<LAYERS>>, grid, dim3(kThreads), 0, P, A);
-    return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, Plain>, grid, dim3(kThreads), 0, static_cast<const Plain&>(P), A);
-}
-
+// Rollbacks of a few caches with their windows take the small table: 0.6 KB of arguments instead of 4.2 (the host's enqueue: 3.0 us with
+// 64 bytes, 4.3 with 2.5 KB).  Without windows more than one layer takes the table without them, whose kernel has 72 registers instead of
+// 76 to 82.  us per launch in a graph with the small windows' table and with this one (states from memory, 32 heads of 128x128, means of
+// five runs that differ by 0.1): 3 layers 6.40 6.34, 4 7.61 7.54, 6 10.34 10.21, 8 (four rows per thread) 11.20 11.25; 3 of 8 heads of
+// 64x64 3.57 3.55.  A small table without windows is as fast (6.33 7.55 10.23 11.20 3.54), but 96 kernels more to load: the first call of
+// a process 26 -> 30 ms.
 template <typename StateT, bool VEC_G, int DK, int NR>
 static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, const ReplayArgs& A, int B, int n_layers) {
     constexpr int ROWS = kThreads / (DK / 4) * NR;
     dim3 grid((A.Dv + ROWS - 1) / ROWS, B * A.Hv, n_layers);
-    if (n_layers > kFewLayers) return launch_replay_table<StateT, VEC_G, DK, NR>(br, grid, P, A);
-    if (n_layers > 1 || P.keep > 0 || P.verify_ids) {
+    if (P.keep == 0 && n_layers > 1) {
+        typedef ReplayAccept<DFLASH_MAX_BATCHED_LAYERS> Plain;
+        return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, Plain>, grid, dim3(kThreads), 0, static_cast<const Plain&>(P), A);
+    }
+    if (n_layers > kFewLayers) return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, ReplayTable>, grid, dim3(kThreads), 0, P, A);
+    if (P.keep > 0 || P.verify_ids) {
         ReplayWindows<kFewLayers> few = {};
         for (int l = 0; l < n_layers; ++l) {
             few.tape[l] = P.tape[l]; few.k[l] = P.k[l]; few.g[l] = P.g[l];
@@ -373,7 +372,7 @@ static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, 
         }
         few.keep = P.keep; few.row16 = P.row16;
         few.verify_ids = P.verify_ids; few.posterior = P.posterior; few.start_inout = P.start_inout; few.out4 = P.out4; few.V = P.V;
-        return launch_replay_table<StateT, VEC_G, DK, NR>(br, grid, few, A);
+        return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, ReplayWindows<kFewLayers>>, grid, dim3(kThreads), 0, few, A);
     }
     const ReplayBatch<1> one = {{P.tape[0]}, {P.k[0]}, {P.g[0]}, {P.state_in[0]}, {P.state_out[0]}};
     return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, ReplayBatch<1>>, grid, dim3(kThreads), 0, one, A);

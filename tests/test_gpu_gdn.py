@@ -226,7 +226,7 @@ def test_batched_replay_equals_per_layer_replay(gpu_lib):
 @pytest.mark.parametrize("layers", [1, 2, 8, 9, 64])
 @pytest.mark.parametrize("rows", [1, 4], ids=["one_row", "four_rows"])
 def test_batched_replay_of_any_number_of_layers(gpu_lib, layers, rows):
-    """The argument tables (1, up to 8 and up to 64 layers) with one row per thread and, from 4,096 workgroups on, four; the steps given,
+    """The argument tables (one layer, and more) with one row per thread and, from 4,096 workgroups on, four; the steps given,
     and counted by the launch from the tokens.  Every layer's state is that of the replay on its own, bit for bit."""
     from swiftlm_amd import DFlashKernels as K, _lib
     from swiftlm_amd.dflash_kernels import _ptr, _ptr_array, _stream
