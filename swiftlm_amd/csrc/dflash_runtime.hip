@@ -112,7 +112,8 @@ __global__ __launch_bounds__(64) void accept_commit_kernel(const uint32_t* verif
 constexpr int kArgmaxThreads = 256;
 constexpr int kArgmaxChunk = 8192;
 constexpr int kArgmaxMaxRows = 1024;
-constexpr int kArgmaxMaxPartials = 4096;   // T * chunks that the last workgroup goes through
+constexpr int kArgmaxMaxPartials = 4096;   // T * chunks of a call: larger ones are refused, though the finish, which reads them from the
+                                           // workspace, has no array that would end there (1,024 rows have post_s)
 
 struct GreedyArgs {
     const void* logits;            // [T, V]
@@ -191,8 +192,8 @@ __global__ __launch_bounds__(kArgmaxThreads) void greedy_partial_kernel(GreedyAr
     }
 }
 
-// Sixteen lanes to a row, four partials of each asked for at once; the tokens to compare with and the start offset come in on the
-// same trip.
+// Sixteen lanes to a row, four partials of each asked for at once; the tokens to compare with come in on the same trip (the start
+// offset, where there is one, is one lane's read at the end).
 __global__ __launch_bounds__(kArgmaxThreads) void greedy_finish_kernel(GreedyArgs A) {
     const int tid = threadIdx.x, sub = tid & 15;
     __shared__ uint32_t post_s[kArgmaxMaxRows];
