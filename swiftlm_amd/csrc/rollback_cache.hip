@@ -147,7 +147,7 @@ bool windows_ride_along(const std::vector<ReplayJob>& jobs, const std::vector<si
         if (!rebuilds_window(c)) continue;
         if (!first) first = &jobs[j];
         const size_t row = (size_t)c->C * c->qkv_elem_bytes;
-        if (!same_window(*first, jobs[j]) || row % 16 || (c->qkv_elem_bytes != 2 && c->qkv_elem_bytes != 4)) return false;
+        if (!same_window(*first, jobs[j]) || c->keep > 65535 || row % 16 || (c->qkv_elem_bytes != 2 && c->qkv_elem_bytes != 4)) return false;
         if ((size_t)c->keep * (row / 16) > 0x3fffffff || !jobs[j].post_conv) return false;
         if (((uintptr_t)c->snap[0] | (uintptr_t)c->qkv | (uintptr_t)jobs[j].post_conv) % 16) return false;
         const uintptr_t o = (uintptr_t)jobs[j].post_conv;

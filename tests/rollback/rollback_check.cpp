@@ -1,7 +1,7 @@
 // The rollback's host code, as libdflash_hip.so has it, on the CPU: its three launches are the functions below, which the dynamic
 // linker finds before the library's own.  They print what they are asked for and refuse the one that the command line names.
 //   rollback_check <launch to refuse, counted from 0, or -1> <rows of a window> <channels of a window, 0: no qkv> <Dk> [<Dk> ...]
-// One tape cache per Dk; its window and state are 0x1000 and 0x2000 before the verify step, 0x3000 and 0x4000 after it, plus
+// One tape cache per Dk; its window and state are 0x100000 and 0x300000 before the verify step, 0x500000 and 0x700000 after it, plus
 // 0x1000000 per cache.  Prints a line per launch, the status, and "armed window state" of every cache.
 #include <cstdio>
 #include <cstdlib>
@@ -43,12 +43,12 @@ int main(int argc, char** argv) {
         const uintptr_t base = (uintptr_t)(i - 4) * 0x1000000;
         auto at = [&](uintptr_t x) { return reinterpret_cast<void*>(base + x); };
         dflash_cache_t* c = dflash_cache_create(DFLASH_CACHE_TAPE, keep + 1);
-        dflash_cache_set_slot(c, 0, at(0x1000));
-        dflash_cache_set_slot(c, 1, at(0x2000));
+        dflash_cache_set_slot(c, 0, at(0x100000));
+        dflash_cache_set_slot(c, 1, at(0x300000));
         dflash_cache_arm_rollback(c, 0);
-        dflash_cache_set_slot(c, 0, at(0x3000));
-        dflash_cache_set_slot(c, 1, at(0x4000));
-        if (dflash_cache_record_tape(c, at(0x100000), DFLASH_F32, at(0x200000), at(0x300000), DFLASH_BF16, 3, C ? at(0x400000) : nullptr, 2,
+        dflash_cache_set_slot(c, 0, at(0x500000));
+        dflash_cache_set_slot(c, 1, at(0x700000));
+        if (dflash_cache_record_tape(c, at(0x900000), DFLASH_F32, at(0xa00000), at(0xb00000), DFLASH_BF16, 3, C ? at(0xc00000) : nullptr, 2,
                                      DFLASH_F32, 1, 7, 1, 1, std::atoi(argv[i]), 1, C))
             return 3;
         caches.push_back(c);

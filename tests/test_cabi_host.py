@@ -227,14 +227,16 @@ def rollback_check(tmp_path_factory):
     return run
 
 
-BEFORE, AFTER = (0, 0x1000, 0x2000), (0, 0x3000, 0x4000)      # disarmed, window and state of before and after the verify step
+BEFORE, AFTER = (0, 0x100000, 0x300000), (0, 0x500000, 0x700000)      # disarmed, window and state of before and after the verify step
 
 
 @pytest.mark.parametrize("keep,channels,dks,launches,after", [
     (3, 64, (64, 128), ["replay+windows 1", "replay+windows 1"], AFTER),
     (3, 64, (64, 64, 128), ["replay+windows 2", "replay+windows 1"], AFTER),
     (3, 12, (64, 128), ["replay 1", "replay 1", "windows 2"], AFTER),           # rows of 24 bytes: windows in a launch of their own
-    (3, 0, (64, 128), ["replay 1", "replay 1"], (0, 0x1000, 0x4000)),           # no qkv: the restored window stays
+    (65535, 8, (64,), ["replay+windows 1"], AFTER),
+    (65536, 8, (64,), ["replay 1", "windows 1"], AFTER),                        # more rows than the windows' kernel takes: its refusal
+    (3, 0, (64, 128), ["replay 1", "replay 1"], (0, 0x100000, 0x700000)),       # no qkv: the restored window stays
 ])
 def test_rollback_refused_at_any_launch_keeps_both_halves_of_a_cache(rollback_check, keep, channels, dks, launches, after):
     """A rollback takes a launch per replay shape, and any of them may be refused (a head dim that the replay does not take, rows that
