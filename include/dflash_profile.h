@@ -41,9 +41,9 @@ int dflash_profile_next_launch(int kernel_id, void* start_event, void* stop_even
 int dflash_profile_empty_launch(void* stream, int grid_x, int grid_y, int grid_z, int threads, int lds_bytes);
 
 /* What dflash_sdpa_block_causal* launches for a batch whose sequences all have N keys (with lengths on the device the
- * workgroups may be dealt, which changes the first grid): kernel names and launch shapes, in launch order, for pricing and
- * labelling a step's launches.  Returns how many there are (1 or 2), or 0 for a call that those entries refuse.
- * No counterpart in the reference. */
+ * workgroups may be dealt, or the splits more than fit at once, which changes the first grid): kernel names and launch
+ * shapes, in launch order, for pricing and labelling a step's launches.  Returns how many there are (1 or 2), or 0 for a
+ * call that those entries refuse.  No counterpart in the reference. */
 typedef struct {
     const char* kernel;
     int grid_x, grid_y, grid_z, threads, lds_bytes;
