@@ -10,35 +10,44 @@
 namespace dflash {
 
 // ---------------------------------------------------------------------------
-// One workgroup per (query head, sequence) and split of the keys; its eight waves take tiles of keys in turn, each with the running
-// maximum, the sum and O^T of its own tiles, and merge them through LDS at the end in fp32.  One split, for short contexts: no
-// partial rows in memory and no second launch.  Inside the loop no barrier, as a wave brings its own tiles.  The price is that the
-// query heads of a group each read their KV head's rows (from the L2), so it is for contexts whose rows one compute unit, or a
+// One workgroup per (query head, sequence), split of the keys and part of V's channels; its eight waves take tiles of keys in turn, each
+// with the running maximum, the sum and O^T of its own tiles, and merge them through LDS at the end in fp32.  One split, for short
+// contexts: no partial rows in memory and no second launch.  Inside the loop no barrier, as a wave brings its own tiles.  The price is
+// that the query heads of a group each read their KV head's rows (from the L2), so it is for contexts whose rows one compute unit, or a
 // few, can take in: see sdpa_short_splits().
 //
 // Bound by one launch and its first trip to memory (4.1 us) and, from some 200 keys on, by what a compute unit takes in, 64 bytes
 // per clock at best: that is reached by loads HBM -> LDS of 1 KB of whole rows.  K rows straight into the operand registers, where
-// neighbouring lanes hold different rows, come in at a quarter of it (16 query heads, D = 128, 512 keys: 8.5 us, and 6.1 as it
-// is; split over workgroups with a combine kernel behind them 8.1).  At D = 256 tiles of 16 keys, so that eight waves find room:
-// with four waves of 32 keys 700 keys took 14.1 us, now 11.2.
+// neighbouring lanes hold different rows, come in at a quarter of it (16 query heads, D = 128, 512 keys: 8.5 us, and 6.1 by way of
+// LDS).  At D = 256 tiles of 16 keys, so that eight waves find room: with four waves of 32 keys 700 keys took 14.1 us, then 11.2.
+// Where heads and splits leave compute units idle, 2^PS workgroups share a head's V by its channels (short_parts): each takes in all of K
+// and scores it, but only its part of V, and has as much less of O^T to sum and to merge.  us per call, one workgroup a head and parts:
+// 32 heads, D = 128, 512 keys 6.0 and 5.3, 8 heads, 896 keys 8.5 and 6.9; 16 heads, D = 256, 400 keys 8.8 and 6.4, 100 keys 5.9 and 4.5;
+// 64 heads, D = 128, 1,152 keys in two parts 8.3 and 7.2.
+// Beside the bytes it is bound by the length of a wave's instructions: a load's offsets formed once instead of per load, the causal rule
+// asked of the tiles alone that reach the block, the merge's reads all in flight (a loop over the waves, whose every read waited for the one before,
+// took 1 us of the 7 that a workgroup of D = 256 worked): 16 heads, D = 256, 4,112 keys 11.4 -> 10.8, 128 heads, D = 128, 896 keys 8.5 -> 7.8.
+// Not taken: the eight tiles of a round scored by their waves and the second product split over the channels, so that no O^T is merged.  Its
+// waves meet three times a round: at one round or with V in four parts as fast or faster (16 heads, D = 256, 256 keys 5.8, 400 8.1), but 256 heads, D = 128, 1,152 keys 12.8 (10.8
+// as it is); with rounds of half the size and two of them in flight 15.7.
 //
 // MFMA 16x16x32, n = lane % 16, g = lane / 16: operands hold row (column) n, k-elements 8g .. 8g+7; the accumulator column n, rows
 // 4g .. 4g+3.  S^T = K Q^T, then O^T += V^T P^T, with P^T taken from the accumulators of S^T as they are: lane (n, g) holds keys
 // 4g .. 4g+3 of each 16 keys, and V^T is gathered in that order by the transposing LDS read (16x16x16 for a tile of 16 keys).
-// 16-byte piece p of row r stands at p ^ (r % 16) (K, Q) or p ^ 4 (r % 4) (V), which leaves
+// 16-byte piece p of row r stands at p ^ (r % 16) (K, Q) or p ^ f(r) (V: four rows of 32 bytes each, read together, in different banks), which leaves
 // few conflicts (by the counters, with the merge's among them, 19 % of the LDS cycles over 512 keys of D = 128, 14 % over 4,112 of
-// D = 256).  A wave's K slot is asked for again behind its scores, its V slot behind the product.
+// D = 256, with V whole).  A wave's K slot is asked for again behind its scores, its V slot behind the product.
 // ---------------------------------------------------------------------------
-template <int D> struct SdpaShortLds {
-    static constexpr int WAVES = 8;
+constexpr int kShortWaves = 8;
+template <int D, int PS> struct SdpaShortLds {
+    static constexpr int WAVES = kShortWaves;
     static constexpr int NB = D == 128 ? 32 : 16;                   // keys of a tile
     static constexpr int ROWB = D * 2;
-    struct Slot { unsigned char k[NB * ROWB], v[NB * ROWB]; };
+    struct Slot { unsigned char k[NB * ROWB], v[NB * ROWB >> PS]; };
     unsigned char q[kM * ROWB];
-    union { Slot slot[WAVES]; float o[WAVES][kM * D]; };            // at the end the wave's O^T
+    union { Slot slot[WAVES]; float o[WAVES][kM * D >> PS]; };      // at the end the wave's O^T
     uint32_t mask[WAVES][kM][NB];                                   // 16 bits each; 4 keys p of row r at p ^ (r % (NB / 4))
-    float m[WAVES][kM], l[WAVES][kM];
-    static_assert(sizeof(Slot) >= kM * D * 4, "the wave's O fits its slot");
+    float m[kM][WAVES], l[kM][WAVES];
 };
 
 // One 16-bit element per lane, zero-extended, HBM -> LDS at lds_base + 4 * lane.
@@ -51,14 +60,15 @@ __device__ __forceinline__ void async_load_2B_addr(const uint16_t* gptr, uint32_
 // At most N of the wave's loads still under way.
 template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-template <typename Tag, int D, bool MASKED, bool PAGED>
-__global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_kernel(SdpaArgs A) {
+template <typename Tag, int D, int PS, bool MASKED, bool PAGED>
+__global__ __launch_bounds__(64 * kShortWaves, 2) void sdpa_short_kernel(SdpaArgs A) {
     typedef typename Tag::vec8 vec8;
-    typedef SdpaShortLds<D> Lds;
+    typedef SdpaShortLds<D, PS> Lds;
     constexpr int W = Lds::WAVES, NB = Lds::NB, NU = NB / 16, ROWB = D * 2, CPR = D / 8, RPI = 64 / CPR;       // bytes and 16-byte pieces of a row, rows per 1 KB load
-    constexpr int KSTEPS = D / 32, DB = D / 16;
-    constexpr int TILE_LOADS = NB / RPI, MASK_LOADS = MASKED ? kM * NB / 64 : 0, KM_LOADS = TILE_LOADS + MASK_LOADS;
-    static_assert(2 * TILE_LOADS + MASK_LOADS <= 63, "vmcnt is a 6-bit counter");
+    constexpr int KSTEPS = D / 32, DP = D >> PS, DB = DP / 16;       // channels and blocks of 16 of the workgroup's part of V
+    constexpr int PARTB = DP * 2, CPP = DP / 8, RPV = 64 / CPP;      // bytes and 16-byte pieces of a row of it, rows per 1 KB load
+    constexpr int TILE_LOADS = NB / RPI, V_LOADS = NB / RPV, MASK_LOADS = MASKED ? kM * NB / 64 : 0, KM_LOADS = TILE_LOADS + MASK_LOADS;
+    static_assert(V_LOADS >= 1 && 2 * TILE_LOADS + MASK_LOADS <= 63, "vmcnt is a 6-bit counter");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     Lds& L = *reinterpret_cast<Lds*>(smem);
 
@@ -69,9 +79,10 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
-    // x = KV head + Hk * split, y = head of the group: the heads that share rows are Hk * S apart, on one XCD where that is a multiple of 8
+    // x = KV head + Hk * split, y = part + parts * head of the group: the heads that share rows are multiples of Hk * S apart, on one XCD where
+    // that is a multiple of 8
     const int S = A.S, split = (int)fast_div(blockIdx.x, (uint32_t)A.Hk, A.gpk_magic);
-    const int hk = (int)blockIdx.x - split * A.Hk, b = blockIdx.z, hq = hk * A.G + (int)blockIdx.y;
+    const int hk = (int)blockIdx.x - split * A.Hk, b = blockIdx.z, hq = hk * A.G + ((int)blockIdx.y >> PS), part = (int)blockIdx.y & ((1 << PS) - 1);
     const size_t row0 = ((size_t)b * A.Hq + hq) * kM;               // first row of the head in q, out and lse
     auto lds_addr = [](const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; };
 
@@ -120,33 +131,39 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
         else
             return (size_t)first_key(t) * ROWB;
     };
-    auto request_rows = [&](int t, const unsigned char* base, const unsigned char* nw, uint32_t lds, bool is_k) __attribute__((always_inline)) {
+    // What a lane fetches into its place of a slot follows from the place alone: the offsets in a tile are formed once, and a load of a whole
+    // tile takes scalar instructions only (formed per load they were a third of a tile's vector instructions).
+    constexpr int K_OFFS = 16 / RPI, V_OFFS = RPV >= 4 ? 1 : 4 / RPV;       // loads until the pieces' order repeats
+    auto v_swizzle = [](int row) { return PARTB >= 256 ? 4 * (row & 3) : PARTB == 128 ? 4 * (row >> 1 & 1) : 0; };
+    uint32_t k_from[K_OFFS], v_from[V_OFFS];
+#pragma unroll
+    for (int j = 0; j < K_OFFS; ++j) k_from[j] = (uint32_t)((lane / CPR) * ROWB + ((lane % CPR) ^ (j * RPI + lane / CPR)) * 16);
+#pragma unroll
+    for (int j = 0; j < V_OFFS; ++j) v_from[j] = (uint32_t)((lane / CPP) * ROWB + ((lane % CPP) ^ v_swizzle(j * RPV + lane / CPP)) * 16);
+    auto request_rows = [&](int t, const unsigned char* base, const unsigned char* nw, uint32_t lds, auto is_k) __attribute__((always_inline)) {
+        constexpr bool K = decltype(is_k)::value;
+        constexpr int PIECES = K ? CPR : CPP, RPL = 64 / PIECES;
         const unsigned char* tile = uniform_ptr(base + tile_off(t));
         const int key0 = first_key(t);
-        uint32_t l = lane;
-        asm volatile("" : "+v"(l));                                 // offsets are formed anew: kept across the loop they are dozens of registers
-        const int last = Nb - 1 - key0, cut = fused ? cache_rows - key0 : NB;      // past `last` the last key once more (dropped later)
-        if (cut <= 0 || cut >= NB) {                                // uniform: all rows from one place
-            const unsigned char* from = cut > 0 ? tile : uniform_ptr(nw - (ptrdiff_t)cut * ROWB);
+        if (key0 + NB <= cache_rows) {                              // uniform: a whole tile from the cache
 #pragma unroll
-            for (int j = 0; j < TILE_LOADS; ++j) {
-                const int row = (int)(j * RPI + l / CPR);
-                const int piece = (int)(l % CPR) ^ (is_k ? row & 15 : 4 * (row & 3));
-                async_load_16B_plain(from, (uint32_t)(min(row, last) * ROWB + piece * 16), lds + j * 1024);
-            }
-        } else {                                                    // from row `cut` on the block's own rows, in k_new / v_new
+            for (int j = 0; j < NB / RPL; ++j)
+                async_load_16B_plain(tile + j * RPL * ROWB, K ? k_from[j % K_OFFS] : v_from[j % V_OFFS], lds + j * 1024);
+        } else {                                                    // past the last key that one once more (dropped later), from row `cut` on the block's own rows
+            const int last = Nb - 1 - key0, cut = fused ? cache_rows - key0 : NB;
             const uint64_t here = (uint64_t)tile, there = (uint64_t)(nw - (ptrdiff_t)cut * ROWB);
+            int l = lane;
+            asm volatile("" : "+v"(l));                             // formed here: kept for it they are dozens of registers
 #pragma unroll
-            for (int j = 0; j < TILE_LOADS; ++j) {
-                const int row = (int)(j * RPI + l / CPR), r = min(row, last);
-                const int piece = (int)(l % CPR) ^ (is_k ? row & 15 : 4 * (row & 3));
+            for (int j = 0; j < NB / RPL; ++j) {
+                const int row = j * RPL + l / PIECES, r = min(row, last), piece = (l % PIECES) ^ (K ? row & 15 : v_swizzle(row));
                 async_load_16B_addr<false>((const unsigned char*)((r < cut ? here : there) + (uint32_t)(r * ROWB + piece * 16)), lds + j * 1024);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
     auto request_k = [&](int t) __attribute__((always_inline)) {
-        request_rows(t, kbase, knew, lds_addr(L.slot[w].k), true);
+        request_rows(t, kbase, knew, lds_addr(L.slot[w].k), std::true_type{});
         if constexpr (MASKED) {
 #pragma unroll
             for (int j = 0; j < MASK_LOADS; ++j) {                   // whole rows of the tile
@@ -155,28 +172,28 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
             }
         }
     };
-    auto request_v = [&](int t) __attribute__((always_inline)) { request_rows(t, vbase, vnew, lds_addr(L.slot[w].v), false); };
+    auto request_v = [&](int t) __attribute__((always_inline)) { request_rows(t, vbase + part * PARTB, vnew + part * PARTB, lds_addr(L.slot[w].v), std::false_type{}); };
 
     f32x4_t oacc[DB];
 #pragma unroll
     for (int i = 0; i < DB; ++i) oacc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
     const int tj = n >> 2, tq = n & 3;                               // transposing read: this lane points at row 4g + tj, channels 4 tq .. +3
-    uint32_t koff[4], voff[4];
+    constexpr int V_BLOCKS = DB < 8 ? DB : 8;                        // blocks of 16 channels until the offsets repeat, 256 bytes on
+    uint32_t koff[4], voff[V_BLOCKS];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        koff[m] = (uint32_t)(n * ROWB + (((4 * m + g) ^ n) * 16));
-        voff[m] = (uint32_t)((4 * g + tj) * ROWB + (tq & 1) * 8 + (tq >> 1) * 16 + ((m ^ tj) * 64));
-    }
+    for (int m = 0; m < 4; ++m) koff[m] = (uint32_t)(n * ROWB + (((4 * m + g) ^ n) * 16));
+#pragma unroll
+    for (int i = 0; i < V_BLOCKS; ++i) voff[i] = (uint32_t)((4 * g + tj) * PARTB + ((2 * i + (tq >> 1)) ^ v_swizzle(4 * g + tj)) * 16 + (tq & 1) * 8);
     auto load_k = [&](const unsigned char* rows, int s) -> vec8 {    // row n, channels 32 s + 8 g .. +7
         return *reinterpret_cast<const vec8*>(rows + koff[s & 3] + 256 * (s >> 2));
     };
     auto load_v = [&](int i) {                               // channel 16 i + n, keys 4g .. +3 and 16 + 4g .. +3
-        const unsigned char* p = L.slot[w].v + voff[(i >> 1) & 3] + 32 * (i & 1) + 256 * (i >> 3);
+        const unsigned char* p = L.slot[w].v + voff[i % V_BLOCKS] + 256 * (i / V_BLOCKS);
         const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)p);
         if constexpr (NU == 1) return lo;
         else {
-            const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + 16 * ROWB));
+            const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + 16 * PARTB));
             return __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         }
     };
@@ -190,7 +207,7 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
     if (w < nt) {
         request_k(w);
         request_v(w);
-        wait_loads<KM_LOADS + TILE_LOADS>();
+        wait_loads<KM_LOADS + V_LOADS>();
     } else {
         wait_loads<0>();
     }
@@ -204,7 +221,7 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
     auto tile = [&](int t, auto hide) __attribute__((always_inline)) {
         constexpr bool HIDE = decltype(hide)::value;
         const bool more = t + W < nt;                                // uniform
-        wait_loads<TILE_LOADS>();                                    // all but V
+        wait_loads<V_LOADS>();                                       // all but V
         f32x4_t sacc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};      // NU == 1: two chains
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s)
@@ -225,11 +242,15 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
                     const float mv = Tag::to_f32((uint16_t)mk[e]);
                     s = mv >= -3.4028234663852886e38f ? fmaxf(fmaf(mv, 1.4426950408889634f, s), -3.4028234663852886e38f) : -INFINITY;
                 }
-                s = key0 + 16 * u + 4 * g + e <= last_visible ? s : -INFINITY;
                 x[4 * u + e] = s;
-                mloc = fmaxf(mloc, s);
             }
         }
+        if (key0 + NB > Nb - kM + 1) {                               // uniform: the causal rule hides some of it
+#pragma unroll
+            for (int e = 0; e < 4 * NU; ++e) x[e] = key0 + 16 * (e / 4) + 4 * g + e % 4 <= last_visible ? x[e] : -INFINITY;
+        }
+#pragma unroll
+        for (int e = 0; e < 4 * NU; ++e) mloc = fmaxf(mloc, x[e]);
         if (more) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // K and mask have been read
             request_k(t + W);
@@ -256,7 +277,7 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
         if (more) wait_loads<KM_LOADS>();                            // V
         else wait_loads<0>();
         decltype(pack_weights(pf)) pb = pack_weights(pf);
-        constexpr int kAhead = 4;
+        constexpr int kAhead = DB < 4 ? DB : 4;
         decltype(load_v(0)) va[DB];
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) va[i] = load_v(i);
@@ -293,21 +314,28 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
         r = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
         l_run = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
-    if (g == 0) { L.m[w][n] = m_run; L.l[w][n] = l_run; }
+    if (g == 0) { L.m[n][w] = m_run; L.l[n][w] = l_run; }
     __syncthreads();
     float M = -INFINITY, l_tot = 0.f;
+    f32x4_t ms[W / 4], ls[W / 4];
 #pragma unroll
-    for (int i = 0; i < W; ++i) M = fmaxf(M, L.m[i][n]);
-#pragma unroll
-    for (int i = 0; i < W; ++i) l_tot += split_weight(L.m[i][n], L.l[i][n], M);
-    const int waves = nt < W ? nt : W;                               // those that had a tile
-    if (w < waves) {
-        const float f = m_run == -INFINITY ? 0.f : fast_exp2(m_run - M) * (l_tot > 0.f ? 1.f / l_tot : 0.f);
-        f32x4_t* o = reinterpret_cast<f32x4_t*>(L.o[w]) + n * (D / 4);     // 16-byte piece p of row n at p ^ n
-#pragma unroll
-        for (int i = 0; i < DB; ++i) o[(4 * i + g) ^ n] = oacc[i] * f;
+    for (int i = 0; i < W / 4; ++i) {
+        ms[i] = *reinterpret_cast<const f32x4_t*>(&L.m[n][4 * i]);
+        ls[i] = *reinterpret_cast<const f32x4_t*>(&L.l[n][4 * i]);
     }
-    if (w == 0 && g == 0) {
+#pragma unroll
+    for (int i = 0; i < W; ++i) M = fmaxf(M, ms[i / 4][i % 4]);
+#pragma unroll
+    for (int i = 0; i < W; ++i) l_tot += split_weight(ms[i / 4][i % 4], ls[i / 4][i % 4], M);
+    constexpr int PER = DP / 4;                                      // threads x 4 channels of a row
+    const int merged = nt <= 2 ? 2 : nt <= 4 ? 4 : W;                 // waves whose sums are added
+    if (w < merged) {
+        const float f = m_run == -INFINITY ? 0.f : fast_exp2(m_run - M) * (l_tot > 0.f ? 1.f / l_tot : 0.f);
+        f32x4_t* o = reinterpret_cast<f32x4_t*>(L.o[w]) + n * PER;   // 16-byte piece p of row n at p ^ (n % pieces)
+#pragma unroll
+        for (int i = 0; i < DB; ++i) o[(4 * i + g) ^ (n & (PER - 1))] = oacc[i] * f;
+    }
+    if (part == 0 && w == 0 && g == 0) {
         if (S > 1) {
             __hip_atomic_store(A.part_m + (row0 + n) * S + split, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(A.part_l + (row0 + n) * S + split, l_tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -331,14 +359,27 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
     }
     if (S > 1 && nt == 0) return;                                    // (its partial rows are not read)
     __syncthreads();
-    constexpr int PER = D / 4;                                       // threads x 4 channels of a row
-    uint16_t* const out = A.part_o + ((size_t)split * A.B * A.Hq * kM + row0) * D;      // the split's rows [split][B * Hq * 16], or the output
-    for (int i = tid; i < kM * PER; i += 64 * W) {
-        const int r = i / PER, p = i % PER;
-        f32x4_t o = {0.f, 0.f, 0.f, 0.f};
-        for (int j = 0; j < waves; ++j) o += reinterpret_cast<const f32x4_t*>(L.o[j])[r * PER + (p ^ r)];
-        *reinterpret_cast<u32x2_t*>(out + r * D + 4 * p) = __builtin_bit_cast(u32x2_t, Tag::pack4(o));
-    }
+    uint16_t* const out = A.part_o + ((size_t)split * A.B * A.Hq * kM + row0) * D + part * DP;      // the split's rows [split][B * Hq * 16], or the output
+    // as many waves' sums as there are, rounded up to a power of two
+    auto merge = [&](auto count) __attribute__((always_inline)) {
+        constexpr int C = decltype(count)::value;
+#pragma unroll
+        for (int i0 = 0; i0 < kM * PER; i0 += 64 * W) {
+            const int i = i0 + tid, r = i / PER, p = i % PER;
+            if (kM * PER < 64 * W && i >= kM * PER) break;
+            f32x4_t o[C];
+#pragma unroll
+            for (int j = 0; j < C; ++j) o[j] = reinterpret_cast<const f32x4_t*>(L.o[j])[r * PER + (p ^ (r & (PER - 1)))];
+#pragma unroll
+            for (int h = C / 2; h > 0; h /= 2)
+#pragma unroll
+                for (int j = 0; j < h; ++j) o[j] += o[j + h];
+            *reinterpret_cast<u32x2_t*>(out + r * D + 4 * p) = __builtin_bit_cast(u32x2_t, Tag::pack4(o[0]));
+        }
+    };
+    if (merged == 2) merge(std::integral_constant<int, 2>{});
+    else if (merged == 4) merge(std::integral_constant<int, 4>{});
+    else merge(std::integral_constant<int, W>{});
 }
 
 // Where one workgroup per query head is the faster form: no more heads than compute units, as the workgroups of a second round
@@ -351,39 +392,42 @@ __global__ __launch_bounds__(64 * SdpaShortLds<D>::WAVES, 2) void sdpa_short_ker
 //
 // A wave has one tile under way where the form with shared tiles has several, so K and V from memory cost this form more than from a
 // cache, and a model that goes through its weights between two calls finds them in memory.  The ends of the few splits lie where the sum
-// of both times is least.  By that sum they would begin earlier, too, at 512 to 1,152 keys (D = 128) and 192 to 576: but one workgroup
-// merges in fp32 where partial rows have 16 bits (700 keys of D = 128: error against 64 bits 2.08e-3, split 2.63e-3; 300 of D = 256
-// 2.00e-3, 2.56e-3), so it keeps what it takes from a cache in about the time of the others.  us per call, launches of a captured graph, K and V of 20 MB in turn (cache) and of 500 MB (memory).  All forms of a
-// call take the same line, so that they give the same bits.
+// of both times is least: where many heads share a KV head they are further, as the form with shared tiles writes and reads 128 partial rows
+// per workgroup there.  One workgroup a head merges in fp32 where partial rows have 16 bits (700 keys of D = 128: error against 64 bits
+// 2.08e-3, split 2.63e-3; 300 of D = 256 2.00e-3, 2.56e-3), and has the lead up to its lines and, with 32 heads and more, somewhat beyond.
+// us per call, launches of a captured graph, K and V of 20 MB in turn (cache) and of 600 MB (memory).  All forms of a call take the same
+// line, so that they give the same bits.
 //     heads, keys            one workgroup   a few splits   shared tiles           heads, keys            one workgroup   a few splits   shared tiles
-//     D=128  8 (Hk=1)   512   6.7  6.6        7.1  7.7       7.5  7.8       D=256  8 (Hk=1)   160   7.0  6.9        7.2  7.1       8.3  8.2
-//                       700   8.0  8.2        7.2  7.7       8.2  8.5                         256   7.7  7.5        7.3  7.8       8.4  8.6
-//            32 (Hk=8)  400   6.2  7.6        7.4  7.7       7.9  7.8              32 (Hk=8)  200   7.6  8.8        8.3  8.2       8.9  9.0
-//                       600   7.0  9.1        7.5  7.8       8.5  8.4                         300   8.1 10.2        8.5  8.5       9.3  9.3
-//            64 (Hk=8)  600   7.1  9.0        8.2  8.7       9.1  9.4              64 (Hk=8)  300   8.1 10.0        9.4  9.8      10.8 11.0
-//                       800   8.0 10.3        8.4  9.2       9.2  9.3                         416   9.1 11.4        9.8 10.2      11.0 11.2
-//            128 (B=4)  896   9.1 12.0       10.3 12.2      11.3 11.4              128 (B=4)  416   9.8 12.3       11.4 12.8      11.8 12.4
-//                       1152 10.4 14.0       11.3 13.4      12.4 12.2                         576  11.5 15.1       12.1 14.5      12.8 13.3
-//            256 (B=8)  1152 11.6 16.9                      14.8 15.5              256 (B=8)  576  12.6 17.4                      16.7 16.8
+//     D=128  8 (Hk=1)   512   5.7  5.7        7.2  7.2       7.6  7.6       D=256  8 (Hk=1)   160   5.0  4.6        6.8  6.8       8.3  8.3
+//                       896   7.0  6.9        7.1  7.0       8.3  8.4                         256   5.6  5.5        7.0  6.9       8.6  8.6
+//                      1500   9.2  9.2        7.3  7.3       8.6  8.5                         416   6.5  6.6        6.9  6.9       9.0  8.8
+//            32 (Hk=8)  400   5.1  5.6        7.6  7.5       7.9  7.9              16 (Hk=2)  600   8.1  7.9        8.5  8.4       9.3  9.1
+//                       896   6.2  6.9        7.4  7.7       8.6  8.7                        1000  10.2 10.0        8.6  8.5       9.5  9.4
+//                      1152   6.8  7.6        8.1  8.2       9.1  9.1              32 (Hk=8)  200   5.3  5.7        8.4  8.2       8.9  8.8
+//                      1400   7.5  8.5        8.2  8.5       9.0  9.3                         416   6.1  6.6        8.4  8.1       9.7  9.1
+//            64 (Hk=8)  600   5.7  6.3        8.3  8.4       9.0  9.1              64 (Hk=8)  300   5.8  6.3        9.6  9.5      10.7 10.8
+//                      1152   7.1  7.9        8.9  9.2      10.5  9.8                         576   6.8  7.5       10.1 10.1      11.5 11.6
+//            128 (B=4)  896   6.9  9.6        9.9 11.5      11.2 11.2              128 (B=4)  416   7.4  9.5       10.7 12.0      12.2 12.2
+//                      1152   8.6 11.4       10.7 12.9      12.2 11.7                         576   8.8 11.7       11.5 13.7      12.8 12.9
+//            256 (B=8) 1152  10.7 14.8                      15.1 14.6              256 (B=8)  576  11.5 15.9                      15.7 16.4
 //     a few splits against shared tiles, and the same from pages (which cost this form a table look-up per tile):
-//     D=128  4 (Hk=1)   2048  7.6  8.2   8.2  8.3      3000   8.2  8.8   8.2  8.1
-//            8 (Hk=1)   2048  7.6  8.2   8.6  8.7      3000   8.3  8.8   8.6  8.5 (paged 8.7  9.4   8.8  8.6)   4112   8.8  9.8   8.8  9.0
-//            16 (Hk=2)  3000  8.4  9.1   9.6  9.7 (paged 8.8  9.6   9.8  9.8)     4112   9.3 10.1  10.1  9.5    8208   9.9 12.0  11.2 10.5
-//            32 (Hk=8)  3000 10.0 11.2  11.3 11.0 (paged 10.4 12.0  11.6 11.1)    4112  10.9 12.6  11.9 11.4    6000  12.2 14.9  12.9 12.7
-//            64 (Hk=8)  1500  9.6 10.7  10.9 10.1      2048  10.0 11.9  11.7 10.7      3000  11.8 14.0  12.8 11.9
-//     D=256  4 (Hk=1)   8208 10.3 11.2  12.8 12.3      12000 11.1 12.3  12.5 11.6
-//            8 (Hk=1)   6000 11.0 11.6  11.6 12.2 (paged 11.3 12.6  11.8 12.3)    8208  11.5 12.7  15.0 13.5    12000 12.8 14.7  14.3 13.5
-//            16 (Hk=2)  1000  8.5  8.7   9.4  9.8      2048  10.1 10.5   9.8 10.2      4112  11.3 12.8  13.2 11.9    5000  11.8 13.7  12.4 12.5
-//            24 (Hk=4)  2048 11.2 12.4  12.7 11.6      3000  12.3 14.0  13.5 12.7      4112  13.6 15.8  14.3 13.4
-//            32 (Hk=8)  2048 11.3 13.3  13.4 12.6 (paged 12.2 14.1  13.8 12.7)    3000  13.2 15.9  14.9 14.0
-//            64 (Hk=8)  1000 11.6 12.9  13.0 13.2      1500  12.9 15.1  14.0 14.3      2048  14.2 17.2  14.8 15.3
-// From 1,500 to 3,000 keys at 16 heads of D = 256 the two are within 0.7 us of each other.  Two splits do not pay (96 heads of D = 256, 448 keys:
-// 11.2 12.6, shared tiles 11.2 11.8), and more than 48 MB of K and V rows, which the form with shared tiles streams, were not looked for.
+//     D=128  4 (Hk=1)   2048  7.1  7.0   8.2  8.2      3000   7.7  7.5   8.1  7.9
+//            8 (Hk=1)   3000  8.0  7.9   8.7  8.3 (paged 8.1  8.0   8.8  8.4)   5000   8.2  8.5   9.1  8.9      12000   9.3 10.4  10.4 10.0
+//            16 (Hk=2)  4112  8.7  9.2  10.1  9.3      8208   9.6 10.4  10.9 10.6     10000   9.9 11.4  11.5 10.8      13000  11.2 13.5  12.4 11.5
+//            32 (Hk=8)  3000  9.1 10.5  10.9 11.0      4112  10.4 12.0  11.5 11.2      64 (Hk=8)  1500   8.4  8.4   9.4  9.4      2048   9.6  9.5   9.9  9.9
+//     D=256  4 (Hk=1)  16400 10.9 12.8  14.8 14.1      8 (Hk=1)  12000  11.8 13.9  14.5 12.7     16400  13.4 15.9  17.4 15.1
+//            8 (Hk=4)  12000 14.8 17.4  15.2 15.9      16 (Hk=2)  4112  10.7 11.6  13.5 11.6      6000  11.8 14.3  14.2 12.4      7000  12.6 15.2  15.2 13.4
+//            16 (Hk=4)  6000 12.6 15.0  14.2 13.2      24 (Hk=4)  3000  11.7 13.4  13.6 12.2      3500  12.4 14.9  14.1 12.6
+//            32 (Hk=8)  2048 10.9 12.9  13.4 12.6 (paged 10.9 13.1  13.8 12.8)    3000  12.6 15.3  14.7 13.7      3500  13.1 16.3  15.3 14.3
+//            64 (Hk=8)  1000 10.7 11.9  13.9 13.0      1500  12.2 14.5  14.9 14.1      2048  13.4 16.4  15.1 14.9
+// Two splits do not pay (96 heads of D = 256, 448 keys: 11.2 12.6, shared tiles 11.2 11.8), and more than 48 MB of K and V rows, which the
+// form with shared tiles streams, were not looked for.
 int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     const int64_t heads = (int64_t)B * Hq;
     const int cus = num_compute_units();
     if (heads > cus) return 0;
-    const bool few = heads < cus / 4;
+    const int G = Hq / Hk;
+    const bool few = heads < (D == 128 ? cus / 8 : cus / 4);
     if (N <= (D == 128 ? (few ? 896 : 1152) : (few ? 416 : 576))) return 1;
     if ((int64_t)B * Hk * N * D > 12000000) return 0;
     int64_t S = cus / heads;
@@ -391,38 +435,47 @@ int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     if (S > most) S = most;
     const int same_xcd = Hk % 8 == 0 ? 1 : Hk % 4 == 0 ? 2 : Hk % 2 == 0 ? 4 : 8;
     if (S > same_xcd) S -= S % same_xcd;
-    const int64_t most_keys = D == 256 ? 288 * S : heads < 8 ? 2048 : S > 8 ? 3584 : 400 * S;
+    const int64_t most_keys = D == 256 ? (G >= 4 ? 400 : 288) * S : heads < 8 ? 2048 : S <= 8 ? 400 * S : G >= 6 ? 10240 : 3584;
     return S >= 3 && N <= most_keys ? (int)S : 0;
 }
 
-dflash_launch_shape sdpa_short_shape(int B, int Hk, int G, int S, int D) {
-    const int lds = D == 256 ? (int)sizeof(SdpaShortLds<256>) : (int)sizeof(SdpaShortLds<128>);
-    return {"sdpa_short_kernel", Hk * S, G, B, 64 * SdpaShortLds<128>::WAVES, lds};
+// Parts of V's channels as a shift: as many as find a compute unit each, up to four (K, which every part takes in, is four fifths of the
+// bytes then).  Parts beyond that are a second round: 32 heads of four splits, 1,152 keys of D = 128, 8.2 us, in two parts 10.5.
+static int short_parts(int64_t workgroups) {
+    const int cus = num_compute_units();
+    return workgroups * 4 <= cus ? 2 : workgroups * 2 <= cus ? 1 : 0;
 }
-static_assert(SdpaShortLds<128>::WAVES == SdpaShortLds<256>::WAVES, "one workgroup size");
 
-template <typename Tag, int D, bool MASKED, bool PAGED>
-static int launch_short(hipStream_t st, const SdpaArgs& A, int B) {
-    LaunchBracket br(DFLASH_KERNEL_SDPA_PARTIAL, st);
-    const dflash_launch_shape g = sdpa_short_shape(B, A.Hk, A.G, A.S, D);
-    DFLASH_HIP_TRY(br.launch(sdpa_short_kernel<Tag, D, MASKED, PAGED>, dim3(g.grid_x, g.grid_y, g.grid_z), dim3(g.threads), g.lds_bytes, A));
-    return DFLASH_OK;
+template <int D> static int short_lds(int ps) {
+    return ps == 2 ? (int)sizeof(SdpaShortLds<D, 2>) : ps == 1 ? (int)sizeof(SdpaShortLds<D, 1>) : (int)sizeof(SdpaShortLds<D, 0>);
 }
-template <typename Tag, int D> static int launch_short(hipStream_t st, const SdpaArgs& A, int B, bool paged) {
-    if (A.mask) return launch_short<Tag, D, true, false>(st, A, B);
-    return paged ? launch_short<Tag, D, false, true>(st, A, B) : launch_short<Tag, D, false, false>(st, A, B);
+dflash_launch_shape sdpa_short_shape(int B, int Hk, int G, int S, int D) {
+    const int ps = short_parts((int64_t)B * Hk * G * S);
+    return {"sdpa_short_kernel", Hk * S, G << ps, B, 64 * kShortWaves, D == 256 ? short_lds<256>(ps) : short_lds<128>(ps)};
+}
+
+template <typename Tag, int D, int PS> static auto short_kernel(bool masked, bool paged) {
+    return masked ? sdpa_short_kernel<Tag, D, PS, true, false> : paged ? sdpa_short_kernel<Tag, D, PS, false, true> : sdpa_short_kernel<Tag, D, PS, false, false>;
+}
+template <typename Tag, int D> static auto short_kernel(int ps, bool masked, bool paged) {
+    return ps == 2 ? short_kernel<Tag, D, 2>(masked, paged) : ps == 1 ? short_kernel<Tag, D, 1>(masked, paged) : short_kernel<Tag, D, 0>(masked, paged);
 }
 int launch_sdpa_short(hipStream_t st, const SdpaArgs& A, int B, int D, int dtype, bool paged) {
-    if (dtype == DFLASH_BF16) return D == 256 ? launch_short<Bf16Tag, 256>(st, A, B, paged) : launch_short<Bf16Tag, 128>(st, A, B, paged);
-    return D == 256 ? launch_short<F16Tag, 256>(st, A, B, paged) : launch_short<F16Tag, 128>(st, A, B, paged);
+    const int ps = short_parts((int64_t)B * A.Hq * A.S);
+    const bool masked = A.mask != nullptr;
+    auto kern = dtype == DFLASH_BF16 ? (D == 256 ? short_kernel<Bf16Tag, 256>(ps, masked, paged) : short_kernel<Bf16Tag, 128>(ps, masked, paged))
+                                     : (D == 256 ? short_kernel<F16Tag, 256>(ps, masked, paged) : short_kernel<F16Tag, 128>(ps, masked, paged));
+    LaunchBracket br(DFLASH_KERNEL_SDPA_PARTIAL, st);
+    const dflash_launch_shape g = sdpa_short_shape(B, A.Hk, A.G, A.S, D);
+    DFLASH_HIP_TRY(br.launch(kern, dim3(g.grid_x, g.grid_y, g.grid_z), dim3(g.threads), g.lds_bytes, A));
+    return DFLASH_OK;
 }
 
 template <typename Tag, int D>
 static int short_setup() {
-    const int lds = sizeof(SdpaShortLds<D>);
-    DFLASH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(sdpa_short_kernel<Tag, D, false, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    DFLASH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(sdpa_short_kernel<Tag, D, true, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    DFLASH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(sdpa_short_kernel<Tag, D, false, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    for (int ps = 0; ps < 3; ++ps)
+        for (int form = 0; form < 3; ++form)
+            DFLASH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(short_kernel<Tag, D>(ps, form == 1, form == 2)), hipFuncAttributeMaxDynamicSharedMemorySize, short_lds<D>(ps)));
     return DFLASH_OK;
 }
 int sdpa_short_device_setup() {

@@ -310,6 +310,24 @@ def test_short_contexts(gpu_lib, Hq, Hk, D, N, S, dt):
     assert torch.equal(kc, k) and torch.equal(vc, v)
 
 
+# One split, with V's channels in four parts, two or one by how many heads the call has: a head's bits are the same, at contexts of one
+# key, a tile, a tile and one more, a wave's second tile, and a mask that hides a tile from some rows.
+@pytest.mark.parametrize("D,N", [(128, 17), (128, 64), (128, 257), (128, 300), (256, 16), (256, 65), (256, 129), (256, 400)])
+def test_short_parts_same_bits(gpu_lib, D, N):
+    from swiftlm_amd import DFlashKernels as K
+
+    q, k, v = tensors(N + D, 5, 32, 4, N, D)
+    mask = torch.zeros(5, 32, 16, N, dtype=q.dtype, device="cuda")
+    mask[:, :, 3:5, :min(N - 16, 40)] = float("-inf")
+    run = lambda n, m: K.batched_sdpa_2pass(q[:n], k[:n], v[:n], 1.0 / math.sqrt(D), None if m is None else m[:n], return_lse=True)
+    assert [short_splits(n, 32, 4, N, D) for n in (2, 3, 5)] == [1, 1, 1]
+    for m in (None, mask):
+        few, some, many = run(2, m), run(3, m), run(5, m)
+        for x, y, z in zip(few, some, many):
+            assert torch.equal(x, z[:2]) and torch.equal(y, z[:3])
+    attend(q[:2], k[:2], v[:2], [N, N], D)
+
+
 # The mask's loads, four keys each in the form with shared tiles: rows of odd and even length, a last tile of one key and of all but
 # one; one split of either form and several.
 @pytest.mark.parametrize("N", [0, 1, 2, 3, 5, 31])
