@@ -174,6 +174,7 @@ int dflash_gdn_finish(void* stream, const void* y, const void* gate, const void*
  * q, k, v, g and beta never travel through memory, and the gated norm -- which normalises over
  * the Dv rows of a head, spread by the forward over Dv/16 workgroups -- is done by whichever of
  * those workgroups finishes last (each counts itself in `arrivals`; none waits for another).
+ * Many heads, and small ones, take a workgroup each, whose norm needs no counter.
  *   inputs    mixed_qkv, conv_state_in (or NULL), conv_weight, a_logits [B,T,Hv], b_logits,
  *             A_log, dt_bias [Hv], q_scale, k_scale, norm_eps as for dflash_gdn_prepare;
  *             state_in [B,Hv,Dv,Dk] float32

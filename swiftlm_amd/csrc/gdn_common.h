@@ -19,6 +19,36 @@ struct GdnArgs {
     uint32_t group, group_magic;
 };
 
+// Inputs of the layer's pre-ops when they run inside the forward kernel (gdn_layer_kernel): the short
+// conv + SiLU over q|k|v, the q/k normalisation and the gate formulas of dflash_gdn_prepare.
+struct GdnPrep {
+    const void* x;            // mixed_qkv [B,T,C]
+    const void* conv_in;      // [B,K-1,C] or null (zeros)
+    const void* weight;       // [C,K]
+    const void* a;            // [B,T,Hv]
+    const void* b;            // [B,T,Hv]
+    const float* a_log;       // [Hv]
+    const float* dt_bias;     // [Hv]
+    void *q_out, *k_out, *v_out, *g_out, *beta_out;   // each may be null
+    void* conv_out;           // [B,K-1,C]
+    float q_scale, k_scale, eps;
+    int C;
+    // The layer's post-op inside the same launch (all null / 0 when it is not asked for): the workgroup of a head
+    // that finishes last -- counted in arrivals[b*Hv + hv], which is zero before the launch and zero again after
+    // it -- normalises and gates the head's y rows.
+    const void* fin_gate;     // [B,T,Hv,Dv]
+    const void* fin_weight;   // [Dv]
+    void* fin_out;            // [B,T,Hv,Dv]; until the last workgroup writes a row, its first Dv/16 floats hold
+                              // the row tiles' sums of squares
+    int32_t* arrivals;        // [B*Hv]
+    int32_t* status;          // device status word (dflash_set_status_word), or null
+    float fin_eps;
+    int fin_silu;
+    int fin_wide;             // bf16, and y, fin_gate, fin_weight and fin_out 16-byte aligned
+};
+constexpr int kLayerTaps = 4;            // conv kernel size the one-launch layer kernel is built for
+constexpr int kLayerFinishMaxDv = 256;   // head dim up to which the post-op runs inside the layer kernel
+
 constexpr int kChunkRows = 16;
 constexpr int kChunkSteps = 16;
 
@@ -118,6 +148,11 @@ __device__ __forceinline__ f32x4v unit_inverse(f32x4v x, const float (&na)[16]) 
 bool gdn_long_applies(const GdnArgs& A, int Dk);
 int launch_gdn_long(hipStream_t st, const GdnArgs& A, int B, int Dk);
 int gdn_long_device_setup();
+
+// The layer in one launch with a workgroup per head (gdn_head.hip)
+bool gdn_head_applies(const GdnArgs& A, const GdnPrep& P, int B, int Dk);
+int launch_gdn_head(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B, int Dk);
+int gdn_head_device_setup();
 
 // The chunked form for one decay per channel (gdn_channel.hip)
 bool gdn_channel_applies(const GdnArgs& A, int B, int Dk);

@@ -470,36 +470,6 @@ static int replay_common(hipStream_t st, int n_layers, const void* const* tape, 
 // Gated delta forward with tape
 // ===========================================================================
 
-// Inputs of the layer's pre-ops when they run inside the forward kernel (gdn_layer_kernel): the short
-// conv + SiLU over q|k|v, the q/k normalisation and the gate formulas of dflash_gdn_prepare.
-struct GdnPrep {
-    const void* x;            // mixed_qkv [B,T,C]
-    const void* conv_in;      // [B,K-1,C] or null (zeros)
-    const void* weight;       // [C,K]
-    const void* a;            // [B,T,Hv]
-    const void* b;            // [B,T,Hv]
-    const float* a_log;       // [Hv]
-    const float* dt_bias;     // [Hv]
-    void *q_out, *k_out, *v_out, *g_out, *beta_out;   // each may be null
-    void* conv_out;           // [B,K-1,C]
-    float q_scale, k_scale, eps;
-    int C;
-    // The layer's post-op inside the same launch (all null / 0 when it is not asked for): the workgroup of a head
-    // that finishes last -- counted in arrivals[b*Hv + hv], which is zero before the launch and zero again after
-    // it -- normalises and gates the head's y rows.
-    const void* fin_gate;     // [B,T,Hv,Dv]
-    const void* fin_weight;   // [Dv]
-    void* fin_out;            // [B,T,Hv,Dv]; until the last workgroup writes a row, its first Dv/16 floats hold
-                              // the row tiles' sums of squares
-    int32_t* arrivals;        // [B*Hv]
-    int32_t* status;          // device status word (dflash_set_status_word), or null
-    float fin_eps;
-    int fin_silu;
-    int fin_wide;             // bf16, and y, fin_gate, fin_weight and fin_out 16-byte aligned
-};
-constexpr int kLayerTaps = 4;            // conv kernel size the one-launch layer kernel is built for
-constexpr int kLayerFinishMaxDv = 256;   // head dim up to which the post-op runs inside the layer kernel
-
 constexpr int kGdnChunk = 16;  // steps staged in LDS at a time
 
 // LPR lanes share one state row; each keeps DK/LPR channels as float4 pieces
@@ -1737,6 +1707,7 @@ int gdn_device_setup() {
     if (rc == DFLASH_OK) rc = gdn_chunk_setup<128>();
     if (rc == DFLASH_OK) rc = gdn_chunk_setup<256>();
     if (rc == DFLASH_OK) rc = gdn_long_device_setup();
+    if (rc == DFLASH_OK) rc = gdn_head_device_setup();
     if (rc == DFLASH_OK) rc = gdn_channel_device_setup();
     return rc;
 }
@@ -1931,6 +1902,7 @@ extern "C" int dflash_gdn_layer(void* stream, const void* mixed_qkv, const void*
     P.fin_silu = gate_kind;
     P.fin_wide = in_dtype == DFLASH_BF16 && (((uintptr_t)y_out | (uintptr_t)gate | (uintptr_t)out_norm_weight | (uintptr_t)out) & 15) == 0;
     hipStream_t st = (hipStream_t)stream;
+    if (gdn_head_applies(A, P, B, Dk)) return launch_gdn_head(st, A, P, B, Dk);
     if (Dk == 64) rc = launch_gdn_layer<64>(st, A, P, B);
     else if (Dk == 128) rc = launch_gdn_layer<128>(st, A, P, B);
     else rc = launch_gdn_layer<256>(st, A, P, B);

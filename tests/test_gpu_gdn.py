@@ -454,6 +454,70 @@ def test_gdn_layer_equals_prepare_forward_finish_bitwise(gpu_lib, cfg, in_dt, ca
     np.testing.assert_allclose(host(r["out"]), O.gdn_finish(host(y), host(z), host(nw), 1e-6, "silu"), **tol)
 
 
+# A workgroup per head: each size of head that has the form, at the smallest head count that takes it and one below (the form with a
+# workgroup per row tile); one step, fewer steps than taps, a ragged and a whole block; several value heads per key head, two sequences; rows
+# of y, tape and the state that only the other form stores.
+@pytest.mark.parametrize("B,Hk,Hv,Dk,Dv", [(1, 1, 1, 64, 64), (1, 5, 15, 64, 128), (2, 4, 8, 64, 128), (1, 15, 15, 128, 64), (1, 4, 16, 128, 64),
+                                           (1, 47, 47, 128, 128), (2, 8, 24, 128, 128)], ids=str)
+@pytest.mark.parametrize("T,carry", [(1, True), (2, False), (9, True), (16, False)], ids=str)
+def test_gdn_layer_with_a_workgroup_per_head_bitwise(gpu_lib, B, Hk, Hv, Dk, Dv, T, carry):
+    from swiftlm_amd import DFlashKernels as K, _lib
+    from swiftlm_amd.dflash_kernels import _ptr
+
+    args, kw, _ = _layer_case(B + T + Dk + Dv, B, T, Hk, Hv, Dk, Dv)
+    if not carry:
+        args = (args[0], None) + args[2:]
+    sc = dict(q_scale=1.0 / Dk, k_scale=Dk ** -0.5)
+    q, k, v, g, beta, conv1 = K.gdn_prepare(*args[:7], Hk, Hv, Dk, Dv, **sc)
+    y, s1, tape = K.gated_delta_kernel_with_tape(q, k, v, g, beta, args[7])
+    want = dict(q=q, k=k, v=v, g=g, beta=beta, conv_state=conv1, y=y, state=s1, tape=tape, out=K.gdn_finish(y, kw["gate"], kw["norm_weight"], 1e-6, "silu"))
+    arrivals = torch.zeros(B * Hv, dtype=torch.int32, device="cuda")
+    for intermediates in (True, False):
+        r = K.gdn_layer(*args, **kw, arrivals=arrivals, want_intermediates=intermediates)
+        _assert_layer_equals(r, want if intermediates else {n: w for n, w in want.items() if n not in ("q", "v", "beta")})
+    assert not arrivals.any()
+    sig = K.gdn_layer(*args, **dict(kw, gate_kind="sigmoid"), arrivals=arrivals)
+    assert torch.equal(sig["out"], K.gdn_finish(y, kw["gate"], kw["norm_weight"], 1e-6, "sigmoid"))
+    # a tape 4 bytes off a 16-byte line, nothing written beside it
+    moved = torch.full((tape.numel() + 2,), 7.0, device="cuda")
+    outs = [torch.empty_like(t) for t in (s1, conv1, y, want["out"])]
+    rc = _lib.load().dflash_gdn_layer(
+        torch.cuda.current_stream().cuda_stream, *(_ptr(t) for t in args[:7]), _lib.BF16, 1.0 / Dk, Dk ** -0.5, 1e-6, _ptr(args[7]), _ptr(outs[0]), None, None,
+        moved[1:].data_ptr(), _ptr(outs[1]), _ptr(outs[2]), _ptr(kw["gate"]), _ptr(kw["norm_weight"]), 1e-6, 1, _ptr(outs[3]), _ptr(arrivals), None, None, None,
+        B, T, Hk, Hv, Dk, Dv, 4)
+    assert rc == 0
+    for got, name in zip(outs + [moved[1:-1].view(tape.shape)], ("state", "conv_state", "y", "out", "tape")):
+        assert torch.equal(got, want[name]), name
+    assert float(moved[0]) == 7.0 and float(moved[-1]) == 7.0
+    # counters that were not zero are reported
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    lib = _lib.load()
+    assert lib.dflash_set_status_word(_ptr(status)) == 0
+    try:
+        K.gdn_layer(*args, **kw, arrivals=torch.full_like(arrivals, 1000))
+        torch.cuda.synchronize()
+        assert int(status) == _lib.STATUS_LAYER_ARRIVALS
+    finally:
+        lib.dflash_set_status_word(None)
+
+
+# A value that is not finite stays in its head and in the steps from its own on, as in the three calls
+def test_gdn_layer_with_a_workgroup_per_head_not_finite(gpu_lib):
+    from swiftlm_amd import DFlashKernels as K
+
+    B, T, Hk, Hv, Dk, Dv = 1, 16, 4, 8, 64, 64
+    args, kw, want = _layer_case(31, B, T, Hk, Hv, Dk, Dv)
+    arrivals = torch.zeros(B * Hv, dtype=torch.int32, device="cuda")
+    for bad in (float("inf"), float("nan")):
+        x = args[0].clone()
+        x[0, 5, 2 * Hk * Dk + 3 * Dv + 17] = bad             # one channel of v of head 3
+        y, s = (K.gdn_layer(x, *args[1:], **kw, arrivals=arrivals)[n] for n in ("y", "state"))
+        keep = torch.ones_like(y, dtype=torch.bool)
+        keep[0, 5:, 3, 17] = False
+        assert torch.equal(y[keep], want["y"][keep]) and not torch.isfinite(y[0, 5, 3, 17])
+        assert torch.equal(s[0, :3], want["state"][0, :3]) and torch.equal(s[0, 3, 18:], want["state"][0, 3, 18:])
+
+
 def test_gdn_layer_reports_unsupported_outside_the_verify_block(gpu_lib):
     from swiftlm_amd import DFlashKernels as K
     from swiftlm_amd.dflash_kernels import DFlashUnsupported
