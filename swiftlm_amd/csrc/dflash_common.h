@@ -99,6 +99,12 @@ struct LaunchBracket {
     LaunchBracket& operator=(const LaunchBracket&) = delete;
 };
 
+// A pointer as a kernel argument of its own.  The runtime looks up the allocation behind every argument that is a pointer, 0.15 us each on the
+// host (six of them beside the rest: 3.7 us per launch, as integers or inside a struct 2.9), hence an integer.
+typedef uint64_t Address;
+inline Address address_of(const void* p) { return (Address)(uintptr_t)p; }
+__device__ __forceinline__ const void* device_pointer(Address a) { return (const void*)(const __attribute__((address_space(1))) void*)a; }
+
 inline int dtype_size(int dt) {
     switch (dt) {
         case DFLASH_F32: return 4;
