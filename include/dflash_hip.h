@@ -240,6 +240,10 @@ int dflash_gdn_layer(void* stream,
  *        bytes, 256-byte aligned; contents are undefined afterwards.
  * ---------------------------------------------------------------------- */
 size_t dflash_sdpa_workspace_bytes(int B, int Hq, int Hk, int M, int N, int D);
+/* 0 where a call of these sizes leaves its workspace alone, as one split writes the output itself, whatever
+ * the form of its keys and counts; otherwise dflash_sdpa_workspace_bytes().  The entries ask for
+ * the workspace either way; those that overlap may share one, or dflash_sdpa_block_causal_static()'s array, where this is 0. */
+size_t dflash_sdpa_scratch_bytes(int B, int Hq, int Hk, int M, int N, int D);
 
 int dflash_sdpa_block_causal(void* stream,
                              const void* q, const void* k, const void* v,

@@ -353,13 +353,16 @@ PyObject* gdn_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
 struct AttentionCall {
     at::Tensor workspace, out, lse;
     int dtype = 0;
-    // false: the shape or type is not covered (the caller returns None)
-    bool prepare(const at::Tensor& q, int64_t Hk, int64_t N, const at::Tensor& given, bool want_lse) {
-        const size_t need = dflash_sdpa_workspace_bytes((int)q.size(0), (int)q.size(1), (int)Hk, (int)q.size(2), (int)N, (int)q.size(3));
+    bool unused = false;                   // no workspace given, and none allocated: the call would not touch it
+    // false: the shape or type is not covered (the caller returns None).  may_skip: the caller has an entry that takes no workspace.
+    bool prepare(const at::Tensor& q, int64_t Hk, int64_t N, const at::Tensor& given, bool want_lse, bool may_skip = false) {
+        const int B = (int)q.size(0), Hq = (int)q.size(1), M = (int)q.size(2), D = (int)q.size(3);
+        const size_t need = dflash_sdpa_workspace_bytes(B, Hq, (int)Hk, M, (int)N, D);
         if (need == 0) return false;
         dtype = code_or(q.scalar_type(), -1);
         if (dtype < 0) return false;
-        workspace = given.defined() ? given : fresh({(int64_t)need}, at::kByte, q);
+        unused = may_skip && !given.defined() && need <= DFLASH_SDPA_STATIC_SCRATCH_BYTES && dflash_sdpa_scratch_bytes(B, Hq, (int)Hk, M, (int)N, D) == 0;
+        if (!unused) workspace = given.defined() ? given : fresh({(int64_t)need}, at::kByte, q);
         if (!want_lse) {
             out = fresh(q.sizes(), q.scalar_type(), q);
             return true;
@@ -422,10 +425,15 @@ PyObject* sdpa(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const bool as_is = rows_apart(k_, v_, D);
     const Held k = as_is ? Held::borrowed(k_) : held(k_), v = as_is ? Held::borrowed(v_) : held(v_);
     AttentionCall c;
-    if (!c.prepare(*q, Hk, N, ws, truth(a[5]))) Py_RETURN_NONE;
+    if (!c.prepare(*q, Hk, N, ws, truth(a[5]), !mask->defined())) Py_RETURN_NONE;
     void* st = stream();
     const int64_t bs = k->stride(0), hs = k->stride(1);
     const int rc = enqueue([&] {
+        // one split writes the output itself: no workspace is allocated for it (0.4 us of a call that enqueues in 5), the library's array, which
+        // is as little touched, stands in
+        if (c.unused)
+            return dflash_sdpa_block_causal_static(st, ptr(*q), ptr(*k), ptr(*v), ptr(c.out), (float*)ptr(c.lse), c.dtype, scale, (int)B, (int)Hq,
+                                                   (int)Hk, (int)M, (int)N, (int)D, bs, hs, (const int32_t*)ptr(len));
         return mask->defined() ? dflash_sdpa_block_causal_masked(st, ptr(*q), ptr(*k), ptr(*v), ptr(*mask), ptr(c.out), (float*)ptr(c.lse), c.dtype,
                                                                 scale, (int)B, (int)Hq, (int)Hk, (int)M, (int)N, (int)D, bs, hs,
                                                                 (const int32_t*)ptr(len), ptr(c.workspace), c.workspace_bytes())

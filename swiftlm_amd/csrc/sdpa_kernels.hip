@@ -1168,6 +1168,13 @@ extern "C" size_t dflash_sdpa_workspace_bytes(int B, int Hq, int Hk, int M, int 
     return ws_layout(B, Hq, choose_splits(B, Hk, groups, N), D, &om, &ol);
 }
 
+extern "C" size_t dflash_sdpa_scratch_bytes(int B, int Hq, int Hk, int M, int N, int D) {
+    const size_t need = dflash_sdpa_workspace_bytes(B, Hq, Hk, M, N, D);
+    if (need == 0) return 0;
+    const int G = Hq / Hk, S = choose_splits(B, Hk, (G + kHeadsPerWG - 1) / kHeadsPerWG, N);
+    return S == 1 || sdpa_short_splits(B, Hq, Hk, N, D, S) == 1 ? 0 : need;
+}
+
 // Page table of a paged K/V pool (null for the dense layout): kv_batch_stride is then the page pitch.
 struct PagedKv {
     const int32_t* table;

@@ -641,3 +641,29 @@ def test_channel_gate_not_finite(gpu_lib, what):
     hit = bad[0, -1]                                   # [Hv, Dv]
     np.testing.assert_allclose(s[0][~hit], sc[0][~hit], rtol=1e-4, atol=1e-6)
     assert not np.isfinite(s[0][hit]).any()
+
+
+# A call that one split answers leaves its workspace alone, so that one without a workspace allocates none; both sides of the lines (one split
+# for few keys, for many heads and few tiles, and for 4 tiles of keys), counts on the device too
+@pytest.mark.parametrize("B,Hq,Hk,D,N,one", [(1, 8, 2, 128, 896, True), (1, 8, 2, 128, 897, False), (1, 32, 8, 128, 1152, True), (1, 32, 8, 128, 1153, False),
+                                             (1, 8, 8, 256, 416, True), (1, 8, 8, 256, 417, False), (9, 32, 8, 128, 128, True), (9, 32, 8, 128, 1153, False),
+                                             (1, 1, 1, 256, 16, True)], ids=str)
+@pytest.mark.parametrize("ragged", [False, True])
+def test_attention_scratch(gpu_lib, B, Hq, Hk, D, N, one, ragged):
+    from swiftlm_amd import DFlashKernels as K, _lib
+
+    lib = _lib.load()
+    need, used = (f(B, Hq, Hk, 16, N, D) for f in (lib.dflash_sdpa_workspace_bytes, lib.dflash_sdpa_scratch_bytes))
+    assert used == (0 if one else need) and need > 0
+    rng = torch.Generator(device="cuda").manual_seed(N)
+    q, k, v = (torch.randn(B, h, n, D, generator=rng, device="cuda").bfloat16() for h, n in ((Hq, 16), (Hk, N), (Hk, N)))
+    lens = torch.randint(16, N + 1, (B,), generator=rng, device="cuda", dtype=torch.int32) if ragged else None
+    ws = torch.full((need,), 0xA5, dtype=torch.uint8, device="cuda")
+    want = K.batched_sdpa_2pass(q, k, v, D ** -0.5, kv_len=lens, return_lse=True, workspace=ws)
+    assert bool((ws == 0xA5).all()) == one
+    for got, w in zip(K.batched_sdpa_2pass(q, k, v, D ** -0.5, kv_len=lens, return_lse=True), want):
+        assert torch.equal(got, w)
+    ref = torch.softmax((q.double() @ k.double().repeat_interleave(Hq // Hk, 1).transpose(2, 3).contiguous() * D ** -0.5).masked_fill(
+        torch.arange(N, device="cuda") > ((lens if ragged else torch.full((B,), N, device="cuda")).view(B, 1, 1, 1) - 16
+                                          + torch.arange(16, device="cuda").view(1, 1, 16, 1)), float("-inf")), -1) @ v.double().repeat_interleave(Hq // Hk, 1)
+    np.testing.assert_allclose(host(want[0]), host(ref), rtol=2e-2, atol=2e-2)
