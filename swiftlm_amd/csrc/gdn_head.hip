@@ -13,21 +13,23 @@ namespace dflash {
 // for y's way to memory, a counter and the way back (some 3 us); here a conv is done once per value head and the norm is a barrier
 // away, but a head has one compute unit for all its work.
 //
-// Bound by the instructions of that unit's SIMDs (32 heads of 128x128: of 19,000 cycles 3,900 until the window rows are there, 4,700 conv and split
-// of the state, 2,400 the products, 1,900 the solve, 5,400 read-out and update, whose fp32 MFMAs, 2,048 cycles, keep other waves' vector
-// instructions from issuing).  us per call in a captured graph, a workgroup per tile and per head, T = 16:
+// Bound by the instructions of that unit's SIMDs (64 heads of 128x128: of 19,500 cycles 4,900 until the window rows are there, 4,600 conv and
+// split of the state, 2,300 the products, 2,000 the solve, 5,700 read-out, norm and update, whose fp32 MFMAs, 2,048 cycles, keep other waves'
+// vector instructions from issuing).  us per call in a captured graph, a workgroup per tile and per head, T = 16:
 //     heads     128x128        128x64         64x128 (Dk x Dv)   64x64
-//       2      7.4   8.9     7.4   7.6       6.8   7.3         6.6   6.2
-//      16                    7.9   7.7       7.9   7.5
-//      32      9.2   9.9     8.3   8.1       8.4   7.8         7.4   6.4
-//      48     10.5  10.2
-//      64     11.4  10.7     9.0   8.6       9.9   8.6         8.3   6.8
-//     128     15.2  11.9    11.5   9.5      12.9   9.8
-//     288     30.0  24.7    20.0  18.5      22.7  19.1        13.8  10.9
+//       2      7.4   8.7     7.4   7.4       6.8   6.8         6.6   6.0
+//      16                                    7.9   7.4
+//      32      9.2   9.7     8.2   7.9       8.4   7.8         7.4   6.3
+//      40     10.0  10.0
+//      48     10.5  10.0
+//      64     11.4  10.6     9.0   8.4       9.9   8.5         8.3   6.7
+//     128     15.2  11.9                    12.9   9.7
+//     288     30.0  24.7    20.0  18.4      22.7  18.9        13.8  10.8
 // Dk = 256 (one workgroup fits a compute unit, 32 heads 256x64 10.2 and 11.8) stays with a workgroup per tile.  Steps towards it (2 heads of
 // 128x128): a tile's waves neighbours, so that the solve had two of the four SIMDs, and k_s.k_t behind two waves' own products 10.2 -> 9.4;
-// S_0 k and S_0 q by one wave, which reads the split state once, window rows addressed by the wave -> 8.9.  Not taken: the state read a
-// second time as the product's operand instead of by way of LDS (10.8).
+// S_0 k and S_0 q by one wave, which reads the split state once, window rows addressed by the wave -> 8.9; the read-out by the second half
+// alone, four steps a lane, beside the first half's update (64 heads 10.8 -> 10.6, 32 heads of 64x128 8.1 -> 7.8).  Not taken: the state
+// read a second time as the product's operand instead of by way of LDS (10.8); c in registers ahead of the solve at 128x128, where it spills (12.5).
 // ---------------------------------------------------------------------------
 template <int DK, int TILES> struct GdnHeadLds {
     static constexpr int DV = 16 * TILES, CH = 2 * DK + DV, LB = DK + 8, WIN_ROWS = kChunkSteps + kLayerTaps - 1;
@@ -314,7 +316,9 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
     }
     lds_barrier();
 
-    // ---- unit-triangular solve for delta: one quad per state row, lane q owns steps 4q..4q+3 ----
+    // ---- unit-triangular solve for delta, by the first half: one quad per state row, lane q owns steps 4q..4q+3 ----
+    constexpr bool kAhead = DK * TILES < 1024;  // c does not fit the registers of sixteen waves beside the widest state
+    f32x4v c[16], sq;
     if (half == 0) {
         const int r = lane / 4, q = lane % 4;
         float acc[4], bet[4], mine[4] = {0.f, 0.f, 0.f, 0.f}, gm[4], pv[4], vv[4];
@@ -329,11 +333,19 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
         SolveStep<0>::run(acc, arow, bet, mine, q);
 #pragma unroll
         for (int e = 0; e < 4; ++e) L.dl[tile][4 * q + e][r] = mine[e];
+    } else {                                   // what the read-out has beside the deltas: lane (r, kk), steps 4 kk .. +3 of state row r
+        if constexpr (kAhead) {
+#pragma unroll
+            for (int t = 0; t < 16; ++t) c[t] = lds4(&L.c[t][4 * kk]);
+        }
+        const f32x4v gm = lds4(&L.gam[4 * kk]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sq[u] = gm[u] * L.p[tile][n][16 + 4 * kk + u];
     }
     lds_barrier();
 
-    // ---- state: S <- gam_15 S_0 + sum_s w_s delta_s (x) k_s, as 16x16x4 fp32 MFMAs; column n of MFMA e stands for channel base + e.  One
-    // half does it ahead of its part of the read-out, the other behind: the matrix pipe and the rest are busy at the same time. ----
+    // ---- state: S <- gam_15 S_0 + sum_s w_s delta_s (x) k_s, as 16x16x4 fp32 MFMAs; column n of MFMA e stands for channel base + e.  The first
+    // half does it beside the other's read-out, the second beside the other's norm. ----
     auto update = [&]() __attribute__((always_inline)) {
         const float gam_end = L.gam[kChunkSteps - 1];
         f32x4v acc[E];
@@ -361,49 +373,52 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
     };
     if (half == 0) update();
 
-    // ---- read-out: lane (r, kk) of half h has steps 8h + 2kk and the next of state row r ----
-    {
-        const int t0 = 8 * half + 2 * kk, r = n;
-        float y[2], d[16], gp[2];
-        float2 c[16];
+    // ---- read-out, by the second half ----
+    if (half == 1) {
+        float d[16];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            d[t] = L.dl[tile][t][r];
-            c[t] = *reinterpret_cast<const float2*>(&L.c[t][t0]);
-        }
+        for (int t = 0; t < 16; ++t) d[t] = L.dl[tile][t][n];
+        f32x4v y = sq;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) y[u] = gp[u] = L.gam[t0 + u] * L.p[tile][r][16 + t0 + u];
+        for (int t0 = 0; t0 < 16; t0 += 8) {
+            if constexpr (!kAhead) {
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            y[0] = fmaf(c[t].x, d[t], y[0]);
-            y[1] = fmaf(c[t].y, d[t], y[1]);
+                for (int t = t0; t < t0 + 8; ++t) c[t - t0] = lds4(&L.c[t][4 * kk]);
+            }
+#pragma unroll
+            for (int t = t0; t < t0 + 8; ++t)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) y[u] = fmaf(c[kAhead ? t : t - t0][u], d[t], y[u]);
+            if constexpr (!kAhead) __builtin_amdgcn_sched_barrier(0);
         }
         // c is 0 for the steps behind t, but 0 times an infinity or NaN of theirs is not: a sum that is not finite is formed again from the
         // steps that it may see
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(y[0]) + fabsf(y[1]) < __builtin_inff())) != 0, 0)) {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(y[0]) + fabsf(y[1]) + fabsf(y[2]) + fabsf(y[3]) < __builtin_inff())) != 0, 0)) {
+            y = sq;
+            for (int t = 0; t < 16; ++t) {
+                const f32x4v ct = lds4(&L.c[t][4 * kk]);
+                const float dt = L.dl[tile][t][n];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                y[u] = gp[u];
-#pragma unroll
-                for (int t = 0; t < 16; ++t) {
-                    const float more = fmaf(u ? c[t].y : c[t].x, d[t], y[u]);
-                    y[u] = t <= t0 + u ? more : y[u];
+                for (int u = 0; u < 4; ++u) {
+                    const float more = fmaf(ct[u], dt, y[u]);
+                    y[u] = t <= 4 * kk + u ? more : y[u];
                 }
             }
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < 4; ++u) {
             const bf16_t yb = from_float<bf16_t>(y[u]);
-            const float yq = to_float(yb), sq = group_sum<16>(__fmul_rn(yq, yq));
-            L.y[t0 + u][16 * tile + r] = yb.bits;
-            if (r == 0) L.part[t0 + u][tile] = sq;
+            const float yq = to_float(yb), sum = group_sum<16>(__fmul_rn(yq, yq));
+            L.y[4 * kk + u][16 * tile + n] = yb.bits;
+            if (n == 0) L.part[4 * kk + u][tile] = sum;
         }
     }
-    if (half == 1) update();
     lds_barrier();
 
-    // ---- out = rmsNorm(y; weight, eps) * act(gate), y and the tape, in whole lines ----
-    if (finishes) {
+    // ---- out = rmsNorm(y; weight, eps) * act(gate), y and the tape, in whole lines, by the first half ----
+    if (half == 1) {
+        update();
+    } else if (finishes) {
         if (ft < tc) {
             Eight y8, o8;
             y8.v = *reinterpret_cast<const uint4*>(&L.y[ft][fd]);
@@ -417,14 +432,16 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
             *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(A.y) + frow) = y8.v;
             *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(P.fin_out) + frow) = o8.v;
         }
-    } else if (tid < 6 * DV) {
-        const int i = tid - 2 * DV, t = i / (DV / 4), d = 4 * (i % (DV / 4));
-        if (t < tc) {
-            const float* from = &L.dl[d / 16][t][d % 16];
-            *reinterpret_cast<float4*>(A.tape + (((size_t)b * A.T + t) * A.Hv + hv) * DV + d) = make_float4(from[0], from[1], from[2], from[3]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int i = tid - 2 * DV + j * 2 * DV, t = i / (DV / 4), d = 4 * (i % (DV / 4));
+            if (t < tc) {
+                const float* from = &L.dl[d / 16][t][d % 16];
+                *reinterpret_cast<float4*>(A.tape + (((size_t)b * A.T + t) * A.Hv + hv) * DV + d) = make_float4(from[0], from[1], from[2], from[3]);
+            }
         }
     }
-
     // The counters of the form with a workgroup per row tile are not needed; one that no launch on a zeroed array can have left is reported as
     // it would be there.
     if (tid == 0 && P.status && __hip_atomic_load(P.arrivals + bh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > 0)
@@ -438,7 +455,7 @@ bool gdn_head_applies(const GdnArgs& A, const GdnPrep& P, int B, int Dk) {
     if ((((uintptr_t)A.tape | (uintptr_t)A.state_out) & 15) != 0 || ((uintptr_t)P.v_out & 7) != 0) return false;       // stored in wider pieces than by the other form
     if ((Dk != 64 && Dk != 128) || (A.Dv != 64 && A.Dv != 128)) return false;
     const int elems = Dk * A.Dv;
-    return B * A.Hv >= (elems == 64 * 64 ? 1 : elems == 64 * 128 ? 16 : 48);
+    return B * A.Hv >= (elems == 64 * 64 ? 1 : elems == 64 * 128 ? 4 : 40);
 }
 
 template <int DK, int TILES>
