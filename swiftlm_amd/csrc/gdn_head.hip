@@ -22,9 +22,9 @@ namespace dflash {
 //      32      9.2   9.7     8.2   7.9       8.4   7.8         7.4   6.3
 //      40     10.0  10.0
 //      48     10.5  10.0
-//      64     11.4  10.6     9.0   8.4       9.9   8.5         8.3   6.7
-//     128     15.2  11.9                    12.9   9.7
-//     288     30.0  24.7    20.0  18.4      22.7  18.9        13.8  10.8
+//      64     11.4  10.2     9.0   8.4       9.9   8.5         8.3   6.7
+//     128     15.2  11.8                    12.9   9.7
+//     288     30.0  24.1    20.0  17.4      22.7  18.9        13.8  10.8
 // Dk = 256 (one workgroup fits a compute unit, 32 heads 256x64 10.2 and 11.8) stays with a workgroup per tile.  Steps towards it (2 heads of
 // 128x128): a tile's waves neighbours, so that the solve had two of the four SIMDs, and k_s.k_t behind two waves' own products 10.2 -> 9.4;
 // S_0 k and S_0 q by one wave, which reads the split state once, window rows addressed by the wave -> 8.9; the read-out by the second half
@@ -48,6 +48,11 @@ template <int DK, int TILES> struct GdnHeadLds {
     float g[16], beta[16], gam[16], w[16];
 };
 
+// Written through (system scope): what a head has to store then drains while the launch runs instead of in a flush at its end (64 heads of
+// 128x128 10.4 -> 10.1 us, 288 of 128x64 18.5 -> 17.3).  At Dk = 64, in pieces of 8 bytes, a few heads lose what many gain (2 of 64x64
+// 6.0 -> 6.2, 288 10.8 -> 10.5): plain stores there.
+__device__ __forceinline__ void store_through(void* p, f32x4v x) { asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"((uint64_t)p), "v"(x) : "memory"); }
+
 template <int DK, int TILES>
 __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPrep P) {
     using Lds = GdnHeadLds<DK, TILES>;
@@ -61,6 +66,7 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
                  "s"(P.status), "s"(P.fin_eps), "s"(P.fin_silu));
     constexpr int DV = Lds::DV, CH = Lds::CH, THREADS = 128 * TILES, KT = kLayerTaps, keep = KT - 1, LPT = DK / 4, E = DK / 32, NK = DK / 32;
     typedef float Vec __attribute__((ext_vector_type(E)));
+    constexpr bool kThrough = DK == 128;
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int tile = wave % TILES, half = wave / TILES, n = lane % 16, kk = lane / 16;         // (a phase of one half has all SIMDs)
     const int htid = tid - 64 * TILES * half;  // of the half
@@ -368,7 +374,8 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
             Vec o;
 #pragma unroll
             for (int e = 0; e < E; ++e) o[e] = acc[e][v];
-            *reinterpret_cast<Vec*>(s_out + v * DK) = o;
+            if constexpr (kThrough) store_through(s_out + v * DK, __builtin_bit_cast(f32x4v, o));
+            else *reinterpret_cast<Vec*>(s_out + v * DK) = o;
         }
     };
     if (half == 0) update();
@@ -429,8 +436,13 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
 #pragma unroll
             for (int e = 0; e < 8; ++e)
                 o8.e[e] = from_float<bf16_t>(gdn_gated_out(to_float(y8.e[e]), inv, to_float(w8.e[e]), to_float(z8.e[e]), P.fin_silu != 0));
-            *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(A.y) + frow) = y8.v;
-            *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(P.fin_out) + frow) = o8.v;
+            if constexpr (kThrough) {
+                store_through(reinterpret_cast<bf16_t*>(A.y) + frow, __builtin_bit_cast(f32x4v, y8.v));
+                store_through(reinterpret_cast<bf16_t*>(P.fin_out) + frow, __builtin_bit_cast(f32x4v, o8.v));
+            } else {
+                *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(A.y) + frow) = y8.v;
+                *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(P.fin_out) + frow) = o8.v;
+            }
         }
     } else {
 #pragma unroll
