@@ -182,6 +182,24 @@ __device__ __forceinline__ void store4(f16_t* p, float4 v) {
     p[0].v = (_Float16)v.x; p[1].v = (_Float16)v.y; p[2].v = (_Float16)v.z; p[3].v = (_Float16)v.w;
 }
 
+// Written through (system scope): a launch's outputs then leave the L2s while it runs, instead of lying there until its end writes back
+// what is dirty.  The address may be any that the elements may have.
+typedef float store_f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t store_u32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void store_through(void* p, store_f32x4_t x) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"((uint64_t)p), "v"(x) : "memory");       // (the data registers stay as they are a wait state longer)
+}
+__device__ __forceinline__ void store_through(void* p, store_u32x2_t x) { asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" ::"v"((uint64_t)p), "v"(x) : "memory"); }
+__device__ __forceinline__ void store4_through(float* p, float4 v) { store_through(p, store_f32x4_t{v.x, v.y, v.z, v.w}); }
+__device__ __forceinline__ void store4_through(bf16_t* p, float4 v) {
+    store_through(p, store_u32x2_t{(uint32_t)f32_to_bf16_bits(v.x) | ((uint32_t)f32_to_bf16_bits(v.y) << 16),
+                                   (uint32_t)f32_to_bf16_bits(v.z) | ((uint32_t)f32_to_bf16_bits(v.w) << 16)});
+}
+__device__ __forceinline__ void store4_through(f16_t* p, float4 v) {
+    auto bits = [](float x) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x); };
+    store_through(p, store_u32x2_t{bits(v.x) | (bits(v.y) << 16), bits(v.z) | (bits(v.w) << 16)});
+}
+
 // ---- GatedDelta layer formulas shared by the pre-op kernel and the one-launch layer kernel ----
 // Both kernels must round identically, so the expressions live here once.
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.f ? z : log1pf(__expf(z)); }

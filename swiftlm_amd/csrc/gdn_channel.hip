@@ -213,7 +213,7 @@ __global__ __launch_bounds__(kChannelThreads) void gated_delta_channel_kernel(Gd
         }
         float* s_out = reinterpret_cast<float*>(A.state_out) + so;
 #pragma unroll
-        for (int i = 0; i < NB; ++i) *reinterpret_cast<f32x4v*>(s_out + 16 * i) = s[i];
+        for (int i = 0; i < NB; ++i) store_through(s_out + 16 * i, s[i]);
         return;
     }
 
@@ -494,8 +494,9 @@ __global__ __launch_bounds__(kChannelThreads) void gated_delta_channel_kernel(Gd
 #pragma unroll
         for (int v = 0; v < 4; ++v)
             if (4 * g + v < tc) {
-                reinterpret_cast<InT*>(A.y)[o + v * step] = from_float<InT>((on >> (4 * g + v)) & 1 ? yv[v] : 0.f);
-                A.tape[o + v * step] = dl[v];
+                __hip_atomic_store(reinterpret_cast<uint16_t*>(A.y) + o + v * step, __builtin_bit_cast(uint16_t, from_float<InT>((on >> (4 * g + v)) & 1 ? yv[v] : 0.f)),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(A.tape + o + v * step, dl[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         if (c + 1 < chunks) lds_barrier();
     }

@@ -51,8 +51,6 @@ template <int DK, int TILES> struct GdnHeadLds {
 // Written through (system scope): what a head has to store then drains while the launch runs instead of in a flush at its end (64 heads of
 // 128x128 10.4 -> 10.1 us, 288 of 128x64 18.5 -> 17.3).  At Dk = 64, in pieces of 8 bytes, a few heads lose what many gain (2 of 64x64
 // 6.0 -> 6.2, 288 10.8 -> 10.5): plain stores there.
-__device__ __forceinline__ void store_through(void* p, f32x4v x) { asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"((uint64_t)p), "v"(x) : "memory"); }
-
 template <int DK, int TILES>
 __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPrep P) {
     using Lds = GdnHeadLds<DK, TILES>;

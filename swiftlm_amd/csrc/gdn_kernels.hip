@@ -335,7 +335,7 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(Table P, ReplayAr
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
         const int r = row0 + rsub + RPP * i;
-        if (owner && r < A.Dv) store4(s_out + (size_t)r * DK + c4, s[i]);
+        if (owner && r < A.Dv) store4_through(s_out + (size_t)r * DK + c4, s[i]);      // (four sequences of 32 heads of 128x128 7.7 -> 6.8 us, one 3.60 -> 3.55)
     }
     if constexpr (Table::kWindows) {
         if (P.keep > 0 && P.win_out[layer]) {
@@ -526,6 +526,10 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
     const int j = tid % LPR;
     const int rloc = tid / LPR;
     StateT* s_out[RPT];
+    // Outputs are written through, but with an fp32 state where no compute unit has a second workgroup, which loses by it (us in a graph, plain and
+    // through, T = 16, gate per channel, 32 heads of 128x128: one sequence 6.45 6.64, two 8.71 8.55, four 13.4 12.4, four at Dk = 256 26.1 25.3;
+    // bf16 state, one 6.48 6.26, four 13.2 12.5, two heads of three steps 3.39 3.34).  Either half of it, y and the tape or the state, is slower.
+    const bool through = sizeof(StateT) == 2 || gridDim.x * gridDim.y > 256;
 
     // The state rows are the largest operand: their loads go out first.
     float4 s[RPT][CH];
@@ -758,8 +762,13 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
             const int t = i / ROWS, r = i % ROWS;
             if (row0 + r < A.Dv) {
                 const size_t o = (((size_t)b * A.T + t0 + t) * A.Hv + hv) * A.Dv + row0 + r;
-                store1_rt(A.y, A.in_dtype, o, y_s[t][r]);
-                A.tape[o] = t_s[t][r];
+                if (through) {
+                    store1_rt_agent(A.y, A.in_dtype, o, y_s[t][r]);
+                    __hip_atomic_store(A.tape + o, t_s[t][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } else {
+                    store1_rt(A.y, A.in_dtype, o, y_s[t][r]);
+                    A.tape[o] = t_s[t][r];
+                }
             }
         }
     }
@@ -768,7 +777,11 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
     for (int u = 0; u < RPT; ++u)
         if (row0 + rloc + u * GR < A.Dv) {
 #pragma unroll
-            for (int c = 0; c < CH; ++c) store4(s_out[u] + c * 4 * LPR + 4 * j, s[u][c]);
+            for (int c = 0; c < CH; ++c) {
+                StateT* const at = s_out[u] + c * 4 * LPR + 4 * j;
+                if (through) store4_through(at, s[u][c]);
+                else store4(at, s[u][c]);
+            }
         }
 }
 
