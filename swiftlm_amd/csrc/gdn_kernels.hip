@@ -335,7 +335,12 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(Table P, ReplayAr
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
         const int r = row0 + rsub + RPP * i;
-        if (owner && r < A.Dv) store4_through(s_out + (size_t)r * DK + c4, s[i]);      // (four sequences of 32 heads of 128x128 7.7 -> 6.8 us, one 3.60 -> 3.55)
+        // Written through by the replay of one layer (four sequences of 32 heads of 128x128 7.7 -> 6.8 us, one 3.60 -> 3.55).  A stack's states fit the
+        // L2s, where the next step's forwards look for them: four steps of 16 layers take 605.9 to 607.0 us with plain stores, 609.3 to 612.2 through.
+        if (owner && r < A.Dv) {
+            if constexpr (Table::kLayers == 1) store4_through(s_out + (size_t)r * DK + c4, s[i]);
+            else store4(s_out + (size_t)r * DK + c4, s[i]);
+        }
     }
     if constexpr (Table::kWindows) {
         if (P.keep > 0 && P.win_out[layer]) {
