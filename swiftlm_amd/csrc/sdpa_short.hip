@@ -391,12 +391,13 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void sdpa_short_kernel(SdpaArg
 // keys took 12.7 us, with 20 11.2); at D = 128 no more than 16, as the combine then needs one round per lane.
 //
 // A wave has one tile under way where the form with shared tiles has several, so K and V from memory cost this form more than from a
-// cache, and a model that goes through its weights between two calls finds them in memory.  The ends of the few splits lie where the sum
-// of both times is least: where many heads share a KV head they are further, as the form with shared tiles writes and reads 128 partial rows
-// per workgroup there.  One workgroup a head merges in fp32 where partial rows have 16 bits (700 keys of D = 128: error against 64 bits
-// 2.08e-3, split 2.63e-3; 300 of D = 256 2.00e-3, 2.56e-3), and has the lead up to its lines and, with 32 heads and more, somewhat beyond.
-// us per call, launches of a captured graph, K and V of 20 MB in turn (cache) and of 600 MB (memory).  All forms of a call take the same
-// line, so that they give the same bits.
+// cache, and a model that goes through its weights between two calls finds them in memory.  The few splits therefore end, as keys to a
+// split, where they have lost nothing from memory yet, or less than they gain from a cache.  Where many heads share a KV head they would
+// be the faster form from a cache further on, but from memory they lose up to as much there (16 heads of D = 256, 6,000 keys 14.2 -> 11.8
+// from a cache, 12.4 -> 14.3 from memory).  One workgroup a head merges in fp32 where partial rows have 16 bits (700 keys of D = 128: error
+// against 64 bits 2.08e-3, split 2.63e-3; 300 of D = 256 2.00e-3, 2.56e-3), and has the lead up to its lines and, with 32 heads and more,
+// somewhat beyond.  us per call, launches of a captured graph, K and V of 20 MB in turn (cache) and of 600 MB (memory).  All forms of a
+// call take the same line, so that they give the same bits.
 //     heads, keys            one workgroup   a few splits   shared tiles           heads, keys            one workgroup   a few splits   shared tiles
 //     D=128  8 (Hk=1)   512   5.7  5.7        7.2  7.2       7.6  7.6       D=256  8 (Hk=1)   160   5.0  4.6        6.8  6.8       8.3  8.3
 //                       896   7.0  6.9        7.1  7.0       8.3  8.4                         256   5.6  5.5        7.0  6.9       8.6  8.6
@@ -426,7 +427,6 @@ int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     const int64_t heads = (int64_t)B * Hq;
     const int cus = num_compute_units();
     if (heads > cus) return 0;
-    const int G = Hq / Hk;
     const bool few = heads < (D == 128 ? cus / 8 : cus / 4);
     if (N <= (D == 128 ? (few ? 896 : 1152) : (few ? 416 : 576))) return 1;
     if ((int64_t)B * Hk * N * D > 12000000) return 0;
@@ -435,7 +435,7 @@ int sdpa_short_splits(int B, int Hq, int Hk, int N, int D, int most) {
     if (S > most) S = most;
     const int same_xcd = Hk % 8 == 0 ? 1 : Hk % 4 == 0 ? 2 : Hk % 2 == 0 ? 4 : 8;
     if (S > same_xcd) S -= S % same_xcd;
-    const int64_t most_keys = D == 256 ? (G >= 4 ? 400 : 288) * S : heads < 8 ? 2048 : S <= 8 ? 400 * S : G >= 6 ? 10240 : 3584;
+    const int64_t most_keys = D == 256 ? 288 * S : heads < 8 ? 2048 : S <= 8 ? 400 * S : 3584;
     return S >= 3 && N <= most_keys ? (int)S : 0;
 }
 

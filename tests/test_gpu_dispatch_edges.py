@@ -310,6 +310,15 @@ def test_short_contexts(gpu_lib, Hq, Hk, D, N, S, dt):
     assert torch.equal(kc, k) and torch.equal(vc, v)
 
 
+# The few splits end at as many keys to a split where four and more query heads share a KV head: both sides of the line
+@pytest.mark.parametrize("Hq,Hk,D,last,S", [(8, 2, 256, 4608, 16), (16, 2, 256, 2304, 8), (4, 1, 256, 9216, 32), (12, 2, 256, 2304, 8), (8, 1, 128, 3584, 16),
+                                            (6, 1, 128, 3584, 16)], ids=str)
+def test_few_splits_end_with_shared_kv_heads(gpu_lib, Hq, Hk, D, last, S):
+    for N, want in ((last, S), (last + 1, 0)):
+        assert short_splits(2, Hq, Hk, N, D) == want
+        attend(*tensors(N + D, 2, Hq, Hk, N, D), [N, N], D)
+
+
 # One split, with V's channels in four parts, two or one by how many heads the call has: a head's bits are the same, at contexts of one
 # key, a tile, a tile and one more, a wave's second tile, and a mask that hides a tile from some rows.
 @pytest.mark.parametrize("D,N", [(128, 17), (128, 64), (128, 257), (128, 300), (256, 16), (256, 65), (256, 129), (256, 400)])
