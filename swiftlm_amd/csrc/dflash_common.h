@@ -182,9 +182,19 @@ __device__ __forceinline__ void store4(f16_t* p, float4 v) {
     p[0].v = (_Float16)v.x; p[1].v = (_Float16)v.y; p[2].v = (_Float16)v.z; p[3].v = (_Float16)v.w;
 }
 
+// Products of the matrix cores on their way into assembly.  Nothing holds back an instruction that reads an MFMA's result too early; the compiler
+// keeps the distance in front of its own (8 wait states behind 16x16x16 and 16x16x32, 10 behind 16x16x4, 12 behind 32x32x16), but does not see what assembly
+// reads.  So every store by assembly below takes a product behind this: 12 wait states behind the last of them, once per kernel and wave.
+// (Volatile assembly keeps its order, hence no product behind the wait; a copy that the compiler makes of one keeps its own distance.)
+typedef float store_f32x4_t __attribute__((ext_vector_type(4)));
+template <int N> __device__ __forceinline__ void settle(store_f32x4_t (&products)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(products[i]));
+    asm volatile("s_nop 11");
+}
+
 // Written through (system scope): a launch's outputs then leave the L2s while it runs, instead of lying there until its end writes back
 // what is dirty.  The address may be any that the elements may have.
-typedef float store_f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t store_u32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void store_through(void* p, store_f32x4_t x) {
     asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"((uint64_t)p), "v"(x) : "memory");       // (the data registers stay as they are a wait state longer)

@@ -212,6 +212,7 @@ __global__ __launch_bounds__(kChannelThreads) void gated_delta_channel_kernel(Gd
             lds_barrier();
         }
         float* s_out = reinterpret_cast<float*>(A.state_out) + so;
+        settle(s);
 #pragma unroll
         for (int i = 0; i < NB; ++i) store_through(s_out + 16 * i, s[i]);
         return;

@@ -367,6 +367,7 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
             for (int e = 0; e < E; ++e) acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, __uint_as_float((uint32_t)kx[e] << 16), acc[e], 0, 0, 0);
         }
         float* s_out = reinterpret_cast<float*>(A.state_out) + so;
+        if constexpr (kThrough) settle(acc);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             Vec o;

@@ -1557,19 +1557,21 @@ __device__ __forceinline__ void gdn_chunk_body(const GdnArgs& A, const GdnPrep& 
                 // Written through (system scope) like y and the tape: the 2 MB of new state then drain while the launch
                 // still runs instead of waiting dirty in the L2s for the end-of-launch flush (-0.7 % of a verify step).
                 // A caller that rolls back from the tape whatever is accepted passes no state_out: nothing is stored.
-                if (s_out != nullptr)
+                if (s_out != nullptr) {
+                    settle(cacc);
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    float* const ptr = s_out + (uint32_t)((4 * kk + v) * DK + base);
-                    if constexpr (E == 1) {
-                        asm volatile("global_store_dword %0, %1, off sc0 sc1" ::"v"((uint64_t)ptr), "v"(cacc[0][v]) : "memory");
-                    } else if constexpr (E == 2) {
-                        const f32x2v val = {cacc[0][v], cacc[1][v]};
-                        asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" ::"v"((uint64_t)ptr), "v"(val) : "memory");
-                    } else {
-                        static_assert(E == 1 || E == 2 || E == 4, "one store per row and lane");
-                        const f32x4v val = {cacc[0][v], cacc[1][v], cacc[2][v], cacc[3][v]};
-                        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"((uint64_t)ptr), "v"(val) : "memory");
+                    for (int v = 0; v < 4; ++v) {
+                        float* const ptr = s_out + (uint32_t)((4 * kk + v) * DK + base);
+                        if constexpr (E == 1) {
+                            asm volatile("global_store_dword %0, %1, off sc0 sc1" ::"v"((uint64_t)ptr), "v"(cacc[0][v]) : "memory");
+                        } else if constexpr (E == 2) {
+                            const f32x2v val = {cacc[0][v], cacc[1][v]};
+                            asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" ::"v"((uint64_t)ptr), "v"(val) : "memory");
+                        } else {
+                            static_assert(E == 1 || E == 2 || E == 4, "one store per row and lane");
+                            const f32x4v val = {cacc[0][v], cacc[1][v], cacc[2][v], cacc[3][v]};
+                            asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"((uint64_t)ptr), "v"(val) : "memory");
+                        }
                     }
                 }
             } else {

@@ -224,6 +224,7 @@ __global__ __launch_bounds__(kLongThreads, DK == 256 ? 2 : 4) void gated_delta_l
         }
         if (A.state_out != nullptr) {
             float* s_out = reinterpret_cast<float*>(A.state_out) + so;
+            settle(s);
 #pragma unroll
             for (int i = 0; i < NB; ++i) store_through(s_out + 16 * i, s[i]);
         }
