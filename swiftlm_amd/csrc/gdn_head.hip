@@ -453,9 +453,8 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
             }
         }
     }
-    // The counters of the form with a workgroup per row tile are not needed; one that no launch on a zeroed array can have left is reported as
-    // it would be there.
-    if (tid == 0 && P.status && __hip_atomic_load(P.arrivals + bh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > 0)
+    // The counters of the form with a workgroup per row tile are not needed; one that it would report, at or above its Dv/16 workgroups, is reported.
+    if (tid == 0 && P.status && __hip_atomic_load(P.arrivals + bh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= TILES)
         atomicOr(P.status, DFLASH_STATUS_LAYER_ARRIVALS);
 }
 

@@ -501,6 +501,27 @@ def test_gdn_layer_with_a_workgroup_per_head_bitwise(gpu_lib, B, Hk, Hv, Dk, Dv,
         lib.dflash_set_status_word(None)
 
 
+# The counters' bound is that of the form with a workgroup per row tile, Dv/16, and no output depends on them
+@pytest.mark.parametrize("Hk,Hv,Dk,Dv", [(2, 4, 64, 64), (2, 4, 64, 128), (8, 16, 128, 64), (20, 40, 128, 128)], ids=str)
+def test_gdn_layer_with_a_workgroup_per_head_arrivals(gpu_lib, Hk, Hv, Dk, Dv):
+    from swiftlm_amd import DFlashKernels as K, _lib
+    from swiftlm_amd.dflash_kernels import _ptr
+
+    args, kw, want = _layer_case(Hv + Dk, 1, 7, Hk, Hv, Dk, Dv)
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    lib = _lib.load()
+    assert lib.dflash_set_status_word(_ptr(status)) == 0
+    try:
+        for count, flag in ((Dv // 16 - 1, 0), (Dv // 16, _lib.STATUS_LAYER_ARRIVALS)):
+            arrivals = torch.zeros(Hv, dtype=torch.int32, device="cuda")
+            arrivals[Hv // 2] = count
+            _assert_layer_equals(K.gdn_layer(*args, **kw, arrivals=arrivals), want)
+            torch.cuda.synchronize()
+            assert int(status) == flag
+    finally:
+        lib.dflash_set_status_word(None)
+
+
 # A value that is not finite stays in its head and in the steps from its own on, as in the three calls
 def test_gdn_layer_with_a_workgroup_per_head_not_finite(gpu_lib):
     from swiftlm_amd import DFlashKernels as K
