@@ -48,10 +48,18 @@ template <int DK, int TILES> struct GdnHeadLds {
     float g[16], beta[16], gam[16], w[16];
 };
 
-// Written through (system scope): what a head has to store then drains while the launch runs instead of in a flush at its end (64 heads of
-// 128x128 10.4 -> 10.1 us, 288 of 128x64 18.5 -> 17.3).  At Dk = 64, in pieces of 8 bytes, a few heads lose what many gain (2 of 64x64
-// 6.0 -> 6.2, 288 10.8 -> 10.5): plain stores there.
-template <int DK, int TILES>
+// THROUGH: stores written through (system scope).  What a head has to store then drains while the launch runs instead of in a flush at its end,
+// which is the more work the more heads there are; a head that shares the chip with few waits for its own stores instead.  us per layer in a
+// graph, plain and through, T = 16, of 4 layers in turn, of 24, and with a product that reads `out` behind each (Hv Dv x 2048):
+//     heads     128x64                                     128x128
+//       16     7.65 8.00   7.68 7.95   14.00 14.06
+//       32     7.99 8.10   8.25 8.32   16.94 17.04
+//       48     8.37 8.35   8.38 8.42   17.95 17.93        10.15 10.15   10.15 10.16   25.84 25.86
+//       64     8.51 8.48   8.47 8.44   19.99 19.71        10.37 10.22   10.66 10.52   29.77 29.75
+//       96     8.73 8.58   8.76 8.61   24.32 23.91        10.88 10.44   12.00 11.46   43.49 42.78
+// (y and out alone make no difference, it is the state.)  At Dk = 64, in pieces of 8 bytes, a few heads lose what many gain (2 of 64x64 6.0 -> 6.2, 288
+// 10.8 -> 10.5): plain stores there.
+template <int DK, int TILES, bool THROUGH>
 __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPrep P) {
     using Lds = GdnHeadLds<DK, TILES>;
     extern __shared__ __align__(16) unsigned char gdn_head_smem[];
@@ -64,7 +72,6 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
                  "s"(P.status), "s"(P.fin_eps), "s"(P.fin_silu));
     constexpr int DV = Lds::DV, CH = Lds::CH, THREADS = 128 * TILES, KT = kLayerTaps, keep = KT - 1, LPT = DK / 4, E = DK / 32, NK = DK / 32;
     typedef float Vec __attribute__((ext_vector_type(E)));
-    constexpr bool kThrough = DK == 128;
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int tile = wave % TILES, half = wave / TILES, n = lane % 16, kk = lane / 16;         // (a phase of one half has all SIMDs)
     const int htid = tid - 64 * TILES * half;  // of the half
@@ -367,13 +374,13 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
             for (int e = 0; e < E; ++e) acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, __uint_as_float((uint32_t)kx[e] << 16), acc[e], 0, 0, 0);
         }
         float* s_out = reinterpret_cast<float*>(A.state_out) + so;
-        if constexpr (kThrough) settle(acc);
+        if constexpr (THROUGH) settle(acc);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             Vec o;
 #pragma unroll
             for (int e = 0; e < E; ++e) o[e] = acc[e][v];
-            if constexpr (kThrough) store_through(s_out + v * DK, __builtin_bit_cast(f32x4v, o));
+            if constexpr (THROUGH) store_through(s_out + v * DK, __builtin_bit_cast(f32x4v, o));
             else *reinterpret_cast<Vec*>(s_out + v * DK) = o;
         }
     };
@@ -435,7 +442,7 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
 #pragma unroll
             for (int e = 0; e < 8; ++e)
                 o8.e[e] = from_float<bf16_t>(gdn_gated_out(to_float(y8.e[e]), inv, to_float(w8.e[e]), to_float(z8.e[e]), P.fin_silu != 0));
-            if constexpr (kThrough) {
+            if constexpr (THROUGH) {
                 store_through(reinterpret_cast<bf16_t*>(A.y) + frow, __builtin_bit_cast(f32x4v, y8.v));
                 store_through(reinterpret_cast<bf16_t*>(P.fin_out) + frow, __builtin_bit_cast(f32x4v, o8.v));
             } else {
@@ -469,10 +476,15 @@ bool gdn_head_applies(const GdnArgs& A, const GdnPrep& P, int B, int Dk) {
     return B * A.Hv >= (elems == 64 * 64 ? 1 : elems == 128 * 128 ? 40 : Dk == 64 ? 4 : 16);
 }
 
+template <int DK, int TILES> static auto head_kernel(int heads) {
+    if constexpr (DK == 128)
+        if (heads >= 48) return gdn_head_kernel<DK, TILES, true>;
+    return gdn_head_kernel<DK, TILES, false>;
+}
 template <int DK, int TILES>
 static int launch_head(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B) {
     LaunchBracket br(DFLASH_KERNEL_GDN_LAYER, st);
-    DFLASH_HIP_TRY(br.launch(gdn_head_kernel<DK, TILES>, dim3(A.Hv, B), dim3(128 * TILES), sizeof(GdnHeadLds<DK, TILES>), A, P));
+    DFLASH_HIP_TRY(br.launch(head_kernel<DK, TILES>(B * A.Hv), dim3(A.Hv, B), dim3(128 * TILES), sizeof(GdnHeadLds<DK, TILES>), A, P));
     return DFLASH_OK;
 }
 int launch_gdn_head(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B, int Dk) {
@@ -483,7 +495,8 @@ int launch_gdn_head(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B, i
 template <int DK, int TILES>
 static int head_setup() {
     static_assert(sizeof(GdnHeadLds<DK, TILES>) <= 160 * 1024, "LDS of a compute unit");
-    DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)gdn_head_kernel<DK, TILES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GdnHeadLds<DK, TILES>)));
+    for (int heads : {0, 65535})
+        DFLASH_HIP_TRY(hipFuncSetAttribute((const void*)head_kernel<DK, TILES>(heads), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GdnHeadLds<DK, TILES>)));
     return DFLASH_OK;
 }
 int gdn_head_device_setup() {

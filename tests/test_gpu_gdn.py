@@ -455,10 +455,10 @@ def test_gdn_layer_equals_prepare_forward_finish_bitwise(gpu_lib, cfg, in_dt, ca
 
 
 # A workgroup per head: each size of head that has the form, at the smallest head count that takes it and one below (the form with a
-# workgroup per row tile); one step, fewer steps than taps, a ragged and a whole block; several value heads per key head, two sequences; rows
-# of y, tape and the state that only the other form stores.
+# workgroup per row tile), and where its stores begin to be written through; one step, fewer steps than taps, a ragged and a whole block;
+# several value heads per key head, two sequences; rows of y, tape and the state that only the other form stores.
 @pytest.mark.parametrize("B,Hk,Hv,Dk,Dv", [(1, 1, 1, 64, 64), (1, 1, 3, 64, 128), (2, 1, 2, 64, 128), (1, 5, 15, 128, 64), (2, 4, 8, 128, 64),
-                                           (1, 39, 39, 128, 128), (2, 10, 20, 128, 128)], ids=str)
+                                           (1, 39, 39, 128, 128), (2, 10, 20, 128, 128), (1, 47, 47, 128, 64), (2, 12, 24, 128, 64)], ids=str)
 @pytest.mark.parametrize("T,carry", [(1, True), (2, False), (9, True), (16, False)], ids=str)
 def test_gdn_layer_with_a_workgroup_per_head_bitwise(gpu_lib, B, Hk, Hv, Dk, Dv, T, carry):
     from swiftlm_amd import DFlashKernels as K, _lib
