@@ -50,6 +50,10 @@ typedef struct {
 } dflash_launch_shape;
 int dflash_profile_sdpa_launches(int dtype, int B, int Hq, int Hk, int N, int D, dflash_launch_shape shapes[2]);
 
+/* What dflash_gdn_layer launches first for rows aligned to 16 bytes and the gated norm in the same launch.  Returns 1, or 0 for
+ * sizes that it refuses.  No counterpart in the reference. */
+int dflash_profile_gdn_layer_launch(int in_dtype, int B, int Hv, int Dk, int Dv, dflash_launch_shape* shape);
+
 #ifdef __cplusplus
 }
 #endif

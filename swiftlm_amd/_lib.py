@@ -63,6 +63,7 @@ SIGNATURES = {
     "dflash_profile_next_launch": (i32, [i32, vp, vp]),
     "dflash_profile_empty_launch": (i32, [vp, i32, i32, i32, i32, i32]),
     "dflash_profile_sdpa_launches": (i32, [i32] * 6 + [C.POINTER(LaunchShape)]),
+    "dflash_profile_gdn_layer_launch": (i32, [i32] * 5 + [C.POINTER(LaunchShape)]),
     "dflash_cache_create": (vp, [i32, i32]),
     "dflash_cache_destroy": (None, [vp]),
     "dflash_cache_kind": (i32, [vp]),

@@ -151,6 +151,8 @@ int gdn_long_device_setup();
 
 // The layer in one launch with a workgroup per head (gdn_head.hip)
 bool gdn_head_applies(const GdnArgs& A, const GdnPrep& P, int B, int Dk);
+int gdn_head_from(int Dk, int Dv);
+dflash_launch_shape gdn_head_shape(int B, int Hv, int Dk, int Dv);
 int launch_gdn_head(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B, int Dk);
 int gdn_head_device_setup();
 

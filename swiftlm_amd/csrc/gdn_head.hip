@@ -15,16 +15,16 @@ namespace dflash {
 //
 // Bound by the instructions of that unit's SIMDs (64 heads of 128x128: of 19,500 cycles 4,900 until the window rows are there, 4,600 conv and
 // split of the state, 2,300 the products, 2,000 the solve, 5,700 read-out, norm and update, whose fp32 MFMAs, 2,048 cycles, keep other waves'
-// vector instructions from issuing).  us per call in a captured graph, a workgroup per tile and per head, T = 16:
+// vector instructions from issuing).  us per call, four layers in turn in a captured graph, a workgroup per tile and per head, T = 16:
 //     heads     128x128        128x64         64x128 (Dk x Dv)   64x64
-//       2      7.4   8.7     7.4   7.4       6.8   6.8         6.6   6.0
-//      16                                    7.9   7.4
-//      32      9.2   9.7     8.2   7.9       8.4   7.8         7.4   6.3
-//      40     10.0  10.0
-//      48     10.5  10.0
-//      64     11.4  10.2     9.0   8.4       9.9   8.5         8.3   6.7
-//     128     15.2  11.8                    12.9   9.7
-//     288     30.0  24.1    20.0  17.4      22.7  18.9        13.8  10.8
+//       2      7.5   8.8     7.4   7.4       6.8   7.2         6.6   6.1
+//       8      7.9   8.9     7.5   7.6       7.3   7.3         6.9   6.2
+//      16      8.7   9.1     8.1   7.6       8.1   7.4         7.3   6.3
+//      32      9.0   9.9     8.1   8.0       8.3   7.7         7.4   6.4
+//      48     10.3  10.2     8.5   8.4       9.2   8.3         7.7   6.4
+//      64     10.9  10.2     8.9   8.5       9.7   8.5         8.0   6.7
+//     128     14.1  10.8    10.8   8.6      12.0   9.0         9.0   7.2
+//     288     28.2  21.8    18.5  16.9      21.6  17.5        12.7   9.9
 // Dk = 256 (one workgroup fits a compute unit, 32 heads 256x64 10.2 and 11.8) stays with a workgroup per tile.  Steps towards it (2 heads of
 // 128x128): a tile's waves neighbours, so that the solve had two of the four SIMDs, and k_s.k_t behind two waves' own products 10.2 -> 9.4;
 // S_0 k and S_0 q by one wave, which reads the split state once, window rows addressed by the wave -> 8.9; the read-out by the second half
@@ -465,15 +465,29 @@ __global__ __launch_bounds__(128 * TILES) void gdn_head_kernel(GdnArgs A, GdnPre
         atomicOr(P.status, DFLASH_STATUS_LAYER_ARRIVALS);
 }
 
-// The gated norm inside the launch, bf16 at aligned rows, and as many heads as the table above asks for: the more work a head has, the more of
-// the compute units its tiles would have had must be taken anyway.
+// Heads (B * Hv) from which this form is taken, 0 where it is not built: the more work a head has, the more of the compute units its tiles would
+// have had must be taken anyway.  Fewer steps move the line by little, so that it holds for all.  us in a graph, a workgroup per tile and per head, at
+// T = 2 and 16 of 4 layers in turn and at T = 16 with a product that reads `out` behind:
+//     64x128   6  7.13 7.18   7.08 7.30   12.34 12.51     8  7.31 7.20   7.30 7.35   13.14 13.10    12  7.71 7.24   7.74 7.39   14.80 15.03
+//     128x64   8  7.69 7.52   7.57 7.57   12.25 12.22    16  7.95 7.58   7.94 7.65   14.01 14.00    24  7.99 7.61   8.03 7.67   15.44 15.45
+//     128x128 40  9.59 9.67   9.85 10.0   23.53 23.83    48  10.1 9.85   10.3 10.2   25.95 25.86    56  10.3 9.92   10.5 10.2   28.42 27.94
+//     64x64    1  6.74 5.98   6.59 5.97   10.37  9.75     8  6.97 6.22   6.86 6.24   11.53 10.87
+int gdn_head_from(int Dk, int Dv) {
+    if ((Dk != 64 && Dk != 128) || (Dv != 64 && Dv != 128)) return 0;
+    return Dk == Dv ? (Dk == 64 ? 1 : 48) : Dk == 64 ? 8 : 16;
+}
+dflash_launch_shape gdn_head_shape(int B, int Hv, int Dk, int Dv) {
+    const size_t lds = Dv == 64 ? (Dk == 64 ? sizeof(GdnHeadLds<64, 4>) : sizeof(GdnHeadLds<128, 4>))
+                                : (Dk == 64 ? sizeof(GdnHeadLds<64, 8>) : sizeof(GdnHeadLds<128, 8>));
+    return {"gdn_head_kernel", Hv, B, 1, 8 * Dv, (int)lds};
+}
+
+// The gated norm inside the launch, bf16 at aligned rows, and as many heads as the line above asks for.
 bool gdn_head_applies(const GdnArgs& A, const GdnPrep& P, int B, int Dk) {
     if (P.fin_gate == nullptr || !P.fin_wide || A.in_dtype != DFLASH_BF16) return false;
     if ((((uintptr_t)A.tape | (uintptr_t)A.state_out) & 15) != 0 || ((uintptr_t)P.v_out & 7) != 0) return false;       // stored in wider pieces than by the other form
-    if ((Dk != 64 && Dk != 128) || (A.Dv != 64 && A.Dv != 128)) return false;
-    const int elems = Dk * A.Dv;
-    // (128x64 from 16 heads: eight of ten steps 7.8 us with a workgroup per tile, 8.0 per head)
-    return B * A.Hv >= (elems == 64 * 64 ? 1 : elems == 128 * 128 ? 40 : Dk == 64 ? 4 : 16);
+    const int from = gdn_head_from(Dk, A.Dv);
+    return from > 0 && B * A.Hv >= from;
 }
 
 template <int DK, int TILES> static auto head_kernel(int heads) {
@@ -484,7 +498,8 @@ template <int DK, int TILES> static auto head_kernel(int heads) {
 template <int DK, int TILES>
 static int launch_head(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B) {
     LaunchBracket br(DFLASH_KERNEL_GDN_LAYER, st);
-    DFLASH_HIP_TRY(br.launch(head_kernel<DK, TILES>(B * A.Hv), dim3(A.Hv, B), dim3(128 * TILES), sizeof(GdnHeadLds<DK, TILES>), A, P));
+    const dflash_launch_shape g = gdn_head_shape(B, A.Hv, DK, A.Dv);
+    DFLASH_HIP_TRY(br.launch(head_kernel<DK, TILES>(B * A.Hv), dim3(g.grid_x, g.grid_y), dim3(g.threads), g.lds_bytes, A, P));
     return DFLASH_OK;
 }
 int launch_gdn_head(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B, int Dk) {

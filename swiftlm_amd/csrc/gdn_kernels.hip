@@ -1684,13 +1684,15 @@ static bool chunk_index_setup(GdnArgs& A, int B, int Dk) {
     return true;
 }
 
+template <int DK> static dflash_launch_shape gdn_layer_shape(bool bf, int B, int Hv, int Dv) {
+    return {"gdn_layer_kernel", Dv / kChunkRows, Hv, B, kThreads, (int)(bf ? sizeof(GdnChunkLds<DK, true, true>) : sizeof(GdnChunkLds<DK, false, true>))};
+}
 template <int DK>
 static int launch_gdn_layer(hipStream_t st, const GdnArgs& A, const GdnPrep& P, int B) {
     const bool bf = A.in_dtype == DFLASH_BF16;
-    const size_t lds = bf ? sizeof(GdnChunkLds<DK, true, true>) : sizeof(GdnChunkLds<DK, false, true>);
-    dim3 grid(A.Dv / kChunkRows, A.Hv, B);
+    const dflash_launch_shape g = gdn_layer_shape<DK>(bf, B, A.Hv, A.Dv);
     LaunchBracket br(DFLASH_KERNEL_GDN_LAYER, st);
-    DFLASH_HIP_TRY(br.launch(bf ? gdn_layer_kernel<DK, true> : gdn_layer_kernel<DK, false>, grid, dim3(kThreads), lds, A, P));
+    DFLASH_HIP_TRY(br.launch(bf ? gdn_layer_kernel<DK, true> : gdn_layer_kernel<DK, false>, dim3(g.grid_x, g.grid_y, g.grid_z), dim3(g.threads), g.lds_bytes, A, P));
     return DFLASH_OK;
 }
 
@@ -1931,4 +1933,16 @@ extern "C" int dflash_gdn_layer(void* stream, const void* mixed_qkv, const void*
     else rc = launch_gdn_layer<256>(st, A, P, B);
     if (rc || !gate || finish_inside) return rc;
     return dflash_gdn_finish(stream, y_out, gate, out_norm_weight, out, in_dtype, out_norm_eps, gate_kind, B, T, Hv, Dv);
+}
+
+extern "C" int dflash_profile_gdn_layer_launch(int in_dtype, int B, int Hv, int Dk, int Dv, dflash_launch_shape* shape) {
+    const bool bf = in_dtype == DFLASH_BF16;
+    if (!shape || (!bf && in_dtype != DFLASH_F16 && in_dtype != DFLASH_F32) || B <= 0 || Hv <= 0 || (long)B * Hv > 65535 || Dv <= 0 || Dv % kChunkRows != 0) return 0;
+    const int from = bf ? gdn_head_from(Dk, Dv) : 0;
+    if (from > 0 && B * Hv >= from) *shape = gdn_head_shape(B, Hv, Dk, Dv);
+    else if (Dk == 64) *shape = gdn_layer_shape<64>(bf, B, Hv, Dv);
+    else if (Dk == 128) *shape = gdn_layer_shape<128>(bf, B, Hv, Dv);
+    else if (Dk == 256) *shape = gdn_layer_shape<256>(bf, B, Hv, Dv);
+    else return 0;
+    return 1;
 }

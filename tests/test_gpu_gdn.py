@@ -454,16 +454,28 @@ def test_gdn_layer_equals_prepare_forward_finish_bitwise(gpu_lib, cfg, in_dt, ca
     np.testing.assert_allclose(host(r["out"]), O.gdn_finish(host(y), host(z), host(nw), 1e-6, "silu"), **tol)
 
 
+def layer_kernel(B, Hv, Dk, Dv):
+    """The kernel of a bf16 layer call with its norm inside, by the library's own account."""
+    from swiftlm_amd import _lib
+
+    shape = _lib.LaunchShape()
+    assert _lib.load().dflash_profile_gdn_layer_launch(_lib.BF16, B, Hv, Dk, Dv, shape) == 1
+    return shape.kernel.decode()
+
+
 # A workgroup per head: each size of head that has the form, at the smallest head count that takes it and one below (the form with a
 # workgroup per row tile), and where its stores begin to be written through; one step, fewer steps than taps, a ragged and a whole block;
 # several value heads per key head, two sequences; rows of y, tape and the state that only the other form stores.
 @pytest.mark.parametrize("B,Hk,Hv,Dk,Dv", [(1, 1, 1, 64, 64), (1, 1, 3, 64, 128), (2, 1, 2, 64, 128), (1, 5, 15, 128, 64), (2, 4, 8, 128, 64),
-                                           (1, 39, 39, 128, 128), (2, 10, 20, 128, 128), (1, 47, 47, 128, 64), (2, 12, 24, 128, 64)], ids=str)
+                                           (1, 39, 39, 128, 128), (2, 10, 20, 128, 128), (1, 47, 47, 128, 64), (2, 12, 24, 128, 64),
+                                           (1, 7, 7, 64, 128), (2, 2, 4, 64, 128), (1, 47, 47, 128, 128), (2, 12, 24, 128, 128)], ids=str)
 @pytest.mark.parametrize("T,carry", [(1, True), (2, False), (9, True), (16, False)], ids=str)
 def test_gdn_layer_with_a_workgroup_per_head_bitwise(gpu_lib, B, Hk, Hv, Dk, Dv, T, carry):
     from swiftlm_amd import DFlashKernels as K, _lib
     from swiftlm_amd.dflash_kernels import _ptr
 
+    per_head = B * Hv >= {(64, 64): 1, (64, 128): 8, (128, 64): 16, (128, 128): 48}[Dk, Dv]
+    assert layer_kernel(B, Hv, Dk, Dv) == ("gdn_head_kernel" if per_head else "gdn_layer_kernel")
     args, kw, _ = _layer_case(B + T + Dk + Dv, B, T, Hk, Hv, Dk, Dv)
     if not carry:
         args = (args[0], None) + args[2:]
@@ -502,11 +514,12 @@ def test_gdn_layer_with_a_workgroup_per_head_bitwise(gpu_lib, B, Hk, Hv, Dk, Dv,
 
 
 # The counters' bound is that of the form with a workgroup per row tile, Dv/16, and no output depends on them
-@pytest.mark.parametrize("Hk,Hv,Dk,Dv", [(2, 4, 64, 64), (2, 4, 64, 128), (8, 16, 128, 64), (20, 40, 128, 128)], ids=str)
+@pytest.mark.parametrize("Hk,Hv,Dk,Dv", [(2, 4, 64, 64), (4, 8, 64, 128), (8, 16, 128, 64), (24, 48, 128, 128)], ids=str)
 def test_gdn_layer_with_a_workgroup_per_head_arrivals(gpu_lib, Hk, Hv, Dk, Dv):
     from swiftlm_amd import DFlashKernels as K, _lib
     from swiftlm_amd.dflash_kernels import _ptr
 
+    assert layer_kernel(1, Hv, Dk, Dv) == "gdn_head_kernel"
     args, kw, want = _layer_case(Hv + Dk, 1, 7, Hk, Hv, Dk, Dv)
     status = torch.zeros(1, dtype=torch.int32, device="cuda")
     lib = _lib.load()
@@ -522,11 +535,13 @@ def test_gdn_layer_with_a_workgroup_per_head_arrivals(gpu_lib, Hk, Hv, Dk, Dv):
         lib.dflash_set_status_word(None)
 
 
-# A value that is not finite stays in its head and in the steps from its own on, as in the three calls
-def test_gdn_layer_with_a_workgroup_per_head_not_finite(gpu_lib):
+# A value that is not finite stays in its head and in the steps from its own on, as in the three calls (128x128 reads out in another way)
+@pytest.mark.parametrize("Hk,Hv,Dk,Dv", [(4, 8, 64, 64), (4, 8, 64, 128), (4, 16, 128, 64), (12, 48, 128, 128)], ids=str)
+def test_gdn_layer_with_a_workgroup_per_head_not_finite(gpu_lib, Hk, Hv, Dk, Dv):
     from swiftlm_amd import DFlashKernels as K
 
-    B, T, Hk, Hv, Dk, Dv = 1, 16, 4, 8, 64, 64
+    B, T = 1, 16
+    assert layer_kernel(B, Hv, Dk, Dv) == "gdn_head_kernel"
     args, kw, want = _layer_case(31, B, T, Hk, Hv, Dk, Dv)
     arrivals = torch.zeros(B * Hv, dtype=torch.int32, device="cuda")
     for bad in (float("inf"), float("nan")):
