@@ -499,7 +499,11 @@ template <int CH, int RPT> struct GdnStepOps {
     int on;
 };
 
-template <typename StateT, bool VEC_G, bool HAS_MASK, int DK, int LPR, int RPT>
+// THROUGH: outputs are written through.  So they are with a 16-bit state, and with an fp32 state where a compute unit has a second workgroup; where
+// none has, that loses (us in a graph, plain and through, T = 16, gate per channel, 32 heads of 128x128: one sequence 6.45 6.64, two 8.71 8.55, four
+// 13.4 12.4, four at Dk = 256 26.1 25.3; bf16 state, one 6.48 6.26, four 13.2 12.5, two heads of three steps 3.39 3.34).  Either half of it, y and
+// the tape or the state, is slower.
+template <typename StateT, bool VEC_G, bool HAS_MASK, int DK, int LPR, int RPT, bool THROUGH>
 __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
     constexpr int GR = kThreads / LPR, ROWS = RPT * GR;           // row groups; thread (group, j) has rows group, group + GR, ..
     constexpr int CH = DK / (4 * LPR);
@@ -531,10 +535,6 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
     const int j = tid % LPR;
     const int rloc = tid / LPR;
     StateT* s_out[RPT];
-    // Outputs are written through, but with an fp32 state where no compute unit has a second workgroup, which loses by it (us in a graph, plain and
-    // through, T = 16, gate per channel, 32 heads of 128x128: one sequence 6.45 6.64, two 8.71 8.55, four 13.4 12.4, four at Dk = 256 26.1 25.3;
-    // bf16 state, one 6.48 6.26, four 13.2 12.5, two heads of three steps 3.39 3.34).  Either half of it, y and the tape or the state, is slower.
-    const bool through = sizeof(StateT) == 2 || gridDim.x * gridDim.y > 256;
 
     // The state rows are the largest operand: their loads go out first.
     float4 s[RPT][CH];
@@ -767,7 +767,7 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
             const int t = i / ROWS, r = i % ROWS;
             if (row0 + r < A.Dv) {
                 const size_t o = (((size_t)b * A.T + t0 + t) * A.Hv + hv) * A.Dv + row0 + r;
-                if (through) {
+                if constexpr (THROUGH) {
                     store1_rt_agent(A.y, A.in_dtype, o, y_s[t][r]);
                     __hip_atomic_store(A.tape + o, t_s[t][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 } else {
@@ -784,7 +784,7 @@ __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
 #pragma unroll
             for (int c = 0; c < CH; ++c) {
                 StateT* const at = s_out[u] + c * 4 * LPR + 4 * j;
-                if (through) store4_through(at, s[u][c]);
+                if constexpr (THROUGH) store4_through(at, s[u][c]);
                 else store4(at, s[u][c]);
             }
         }
@@ -1737,13 +1737,18 @@ int gdn_device_setup() {
     return rc;
 }
 
+template <typename StateT, int DK, int LPR, int RPT, bool THROUGH> static auto steps_kernel(bool vec, bool masked) {
+    return vec ? (masked ? gated_delta_tape_kernel<StateT, true, true, DK, LPR, RPT, THROUGH> : gated_delta_tape_kernel<StateT, true, false, DK, LPR, RPT, THROUGH>)
+               : (masked ? gated_delta_tape_kernel<StateT, false, true, DK, LPR, RPT, THROUGH> : gated_delta_tape_kernel<StateT, false, false, DK, LPR, RPT, THROUGH>);
+}
 template <typename StateT, int DK, int LPR, int RPT = 1>
 static int launch_gdn_steps(hipStream_t st, const GdnArgs& A, int B, bool vec) {
     constexpr int rows = RPT * (kThreads / LPR);
     dim3 grid((A.Dv + rows - 1) / rows, B * A.Hv);
     LaunchBracket br(DFLASH_KERNEL_GDN_FORWARD, st);
-    auto kern = vec ? (A.mask ? gated_delta_tape_kernel<StateT, true, true, DK, LPR, RPT> : gated_delta_tape_kernel<StateT, true, false, DK, LPR, RPT>)
-                    : (A.mask ? gated_delta_tape_kernel<StateT, false, true, DK, LPR, RPT> : gated_delta_tape_kernel<StateT, false, false, DK, LPR, RPT>);
+    auto kern = steps_kernel<StateT, DK, LPR, RPT, sizeof(StateT) == 2>(vec, A.mask != nullptr);
+    if constexpr (sizeof(StateT) == 4 && LPR < 32)           // (more lanes to a row are taken where a compute unit has one workgroup)
+        if ((long)grid.x * grid.y > num_compute_units()) kern = steps_kernel<StateT, DK, LPR, RPT, true>(vec, A.mask != nullptr);
     DFLASH_HIP_TRY(br.launch(kern, grid, dim3(kThreads), 0, A));
     return DFLASH_OK;
 }

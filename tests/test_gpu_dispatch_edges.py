@@ -40,6 +40,27 @@ def test_step_kernel_lanes_per_row(gpu_lib, Dk, Hv, Dv, T):
     np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
 
 
+# ... and outputs written through where a compute unit has a second workgroup (fp32 state): as many workgroups as compute units, and a head more
+@pytest.mark.parametrize("Dk,tiles", [(128, 8), (64, 4), (256, 8), (96, 4)], ids=str)
+@pytest.mark.parametrize("more", [0, 1])
+@pytest.mark.parametrize("masked", [False, True])
+def test_step_kernel_stores(gpu_lib, Dk, tiles, more, masked):
+    from swiftlm_amd import DFlashKernels as K
+
+    rows = 32 if Dk == 96 else 16                      # of a workgroup
+    T, Hv, Dv = 5, torch.cuda.get_device_properties(0).multi_processor_count // tiles + more, rows * tiles
+    d = O.make_gdn_inputs(Dk + Hv, 1, T, 1, Hv, Dk, Dv, in_dtype="bf16", vec_gate=True)
+    mask = np.ones((1, T), np.float32) if masked else None
+    if masked:
+        mask[0, 2] = 0
+    y, s, tape = K.gated_delta_kernel_with_tape(*[dev(d[n], torch.bfloat16) for n in ("q", "k", "v", "g", "beta")], dev(d["state"]),
+                                                None if mask is None else dev(mask))
+    yw, sw, tw = O.gated_delta_ops_with_tape(d["q"], d["k"], d["v"], d["g"], d["beta"], d["state"], mask, dtype=np.float64)
+    np.testing.assert_allclose(host(s), sw, rtol=1e-4, atol=1e-6)
+    np.testing.assert_allclose(host(tape), tw, rtol=1e-4, atol=1e-5)
+    np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
+
+
 # ... and rows per thread: two where the one-row form takes several rounds (Dv beyond a whole tile of either)
 @pytest.mark.parametrize("Dk,Hv,Dv,vec", [(128, 65, 128, True), (128, 98, 120, False), (256, 33, 128, True), (256, 98, 120, False)], ids=lambda v: str(v))
 @pytest.mark.parametrize("T", [1, 2, 5, 16, 18])
