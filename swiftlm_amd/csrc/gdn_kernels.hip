@@ -118,6 +118,7 @@ struct ReplayArgs {
     int mask_dtype, tape_dtype, in_dtype;
     int steps, skip_if_full;
     int T_tape, Hk, Hv, Dv;
+    int small;               // fewer workgroups than compute units
 };
 
 constexpr int kReplayChunk = 16;  // steps staged in LDS at a time (8 for Dk = 256): one chunk covers the 16-token verify block
@@ -337,8 +338,10 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(Table P, ReplayAr
         const int r = row0 + rsub + RPP * i;
         // Written through by the replay of one layer (four sequences of 32 heads of 128x128 7.7 -> 6.8 us, one 3.60 -> 3.55).  A stack's states fit the
         // L2s, where the next step's forwards look for them: four steps of 16 layers take 605.9 to 607.0 us with plain stores, 609.3 to 612.2 through.
+        // Nor does it pay for a small state, Dk = 64 and not a workgroup to every compute unit (a replay, then its layer's forward, plain and through: 8 heads of
+        // 64x64 7.39 7.54, 32 7.50 7.65, two sequences of 32 7.84 7.80; 32 heads of 64x128 7.82 7.82; 8 of 128x128 8.45 8.34).
         if (owner && r < A.Dv) {
-            if constexpr (Table::kLayers == 1) store4_through(s_out + (size_t)r * DK + c4, s[i]);
+            if (Table::kLayers == 1 && !(DK <= 64 && NR == 1 && A.small)) store4_through(s_out + (size_t)r * DK + c4, s[i]);
             else store4(s_out + (size_t)r * DK + c4, s[i]);
         }
     }
@@ -360,9 +363,10 @@ __global__ __launch_bounds__(kThreads) void tape_replay_kernel(Table P, ReplayAr
 // 64x64 3.57 3.55.  A small table without windows is as fast (6.33 7.55 10.23 11.20 3.54), but 96 kernels more to load: the first call of
 // a process 26 -> 30 ms.
 template <typename StateT, bool VEC_G, int DK, int NR>
-static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, const ReplayArgs& A, int B, int n_layers) {
+static hipError_t launch_replay_layers(LaunchBracket& br, const ReplayTable& P, ReplayArgs A, int B, int n_layers) {
     constexpr int ROWS = kThreads / (DK / 4) * NR;
     dim3 grid((A.Dv + ROWS - 1) / ROWS, B * A.Hv, n_layers);
+    A.small = (long)grid.x * grid.y < num_compute_units();
     if (P.keep == 0 && n_layers > 1) {
         typedef ReplayAccept<DFLASH_MAX_BATCHED_LAYERS> Plain;
         return br.launch(tape_replay_kernel<StateT, VEC_G, DK, NR, Plain>, grid, dim3(kThreads), 0, static_cast<const Plain&>(P), A);

@@ -61,6 +61,29 @@ def test_step_kernel_stores(gpu_lib, Dk, tiles, more, masked):
     np.testing.assert_allclose(host(y), yw, rtol=2e-2, atol=2e-2)
 
 
+# Tape replay of one layer, whose state is written through where every compute unit has a workgroup, or Dk is above 64: both sides; nothing beside it
+@pytest.mark.parametrize("Dk,Dv", [(64, 64), (32, 128), (128, 32)], ids=str)
+@pytest.mark.parametrize("less", [0, 1])
+@pytest.mark.parametrize("state", ["f32", "bf16"])
+def test_replay_stores(gpu_lib, Dk, Dv, less, state):
+    from swiftlm_amd import DFlashKernels as K
+
+    T, Hv = 5, torch.cuda.get_device_properties(0).multi_processor_count // 4 - less           # four workgroups a head
+    sdt = {"f32": torch.float32, "bf16": torch.bfloat16}[state]
+    d = O.make_gdn_inputs(Dk + Hv, 1, T, 1, Hv, Dk, Dv, in_dtype="bf16")
+    tape = np.random.default_rng(Hv).standard_normal((1, T, Hv, Dv)).astype(np.float32)
+    k, g, s0 = dev(d["k"], torch.bfloat16), dev(d["g"], torch.bfloat16), dev(O.quantize(d["state"], state), sdt)
+    got = K.tape_replay_kernel(dev(tape), k, g, s0, None)
+    want = O.tape_replay_ops(tape, d["k"], d["g"], host(s0), dtype=np.float64, requant=None if state == "f32" else state)
+    # (bf16: rounded after every step; a sum of the other side of a tie is 2^-8 away, and five steps carry it on)
+    tol = dict(rtol=1e-4, atol=1e-6) if state == "f32" else dict(rtol=2e-2, atol=2e-2)
+    np.testing.assert_allclose(host(got), want, **tol)
+    # the replay of two layers writes plainly: the same bits
+    outs = [torch.empty_like(s0) for _ in range(2)]
+    K.tape_replay_batched([dev(tape)] * 2, [k] * 2, [g] * 2, [s0, s0.clone()], outs, T)
+    assert torch.equal(outs[0], got) and torch.equal(outs[1], got)
+
+
 # ... and rows per thread: two where the one-row form takes several rounds (Dv beyond a whole tile of either)
 @pytest.mark.parametrize("Dk,Hv,Dv,vec", [(128, 65, 128, True), (128, 98, 120, False), (256, 33, 128, True), (256, 98, 120, False)], ids=lambda v: str(v))
 @pytest.mark.parametrize("T", [1, 2, 5, 16, 18])
