@@ -50,11 +50,10 @@ namespace dflash {
 typedef short s16x4v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));   // (a select between two HIP uint4 is a select of addresses: the arrays end in scratch)
-// rows of v, y and the tape at any address that their elements may have: one load or store all the same (a HIP uint2 is a class, which
-// is not packed: it would claim 8 bytes)
+// rows of v at any address that their elements may have: one load all the same (a HIP uint2 is a class, which is not packed: it would
+// claim 8 bytes); y and the tape are stored by store_through(), which claims no more either
 struct __attribute__((packed, aligned(2))) Rows4x16 { u32x2v x; };
-struct __attribute__((packed, aligned(4))) Rows4x32 { f32x4v x; };
-static_assert(alignof(Rows4x16) == 2 && alignof(Rows4x32) == 4, "no more than the elements have");
+static_assert(alignof(Rows4x16) == 2, "no more than the elements have");
 
 template <int DK> struct GdnLongLds {
     static constexpr int LB = DK + 8;      // row pitch: 16 bytes of pad spread 16-byte reads of a column of rows over the banks

@@ -313,13 +313,18 @@ def test_combine_rows_in_flight(gpu_lib, D, N, S):
     attend(*tensors(N + D, 1, 3, 1, N, D), [N], D)
 
 
-def short_splits(B, Hq, Hk, N, D):
-    """Splits of the form with a workgroup per query head, 0 where the form with shared tiles runs; by the library's own account."""
+def first_launch(B, Hq, Hk, N, D):
     from swiftlm_amd import _lib
 
     shapes = (_lib.LaunchShape * 2)()
     assert _lib.load().dflash_profile_sdpa_launches(_lib.BF16, B, Hq, Hk, N, D, shapes) > 0
-    return shapes[0].grid_x // Hk if shapes[0].kernel == b"sdpa_short_kernel" else 0
+    return shapes[0]
+
+
+def short_splits(B, Hq, Hk, N, D):
+    """Splits of the form with a workgroup per query head, 0 where the form with shared tiles runs; by the library's own account."""
+    shape = first_launch(B, Hq, Hk, N, D)
+    return shape.grid_x // Hk if shape.kernel == b"sdpa_short_kernel" else 0
 
 
 # Short contexts in one launch, up to a line of keys that depends on the query heads (B * Hq), then a few splits of the same form, then
@@ -374,6 +379,7 @@ def test_short_parts_same_bits(gpu_lib, D, N):
     mask[:, :, 3:5, :min(N - 16, 40)] = float("-inf")
     run = lambda n, m: K.batched_sdpa_2pass(q[:n], k[:n], v[:n], 1.0 / math.sqrt(D), None if m is None else m[:n], return_lse=True)
     assert [short_splits(n, 32, 4, N, D) for n in (2, 3, 5)] == [1, 1, 1]
+    assert [first_launch(n, 32, 4, N, D).grid_y for n in (2, 3, 5)] == [8 * parts for parts in (4, 2, 1)]
     for m in (None, mask):
         few, some, many = run(2, m), run(3, m), run(5, m)
         for x, y, z in zip(few, some, many):
