@@ -213,6 +213,8 @@ __global__ __launch_bounds__(kChannelThreads) void gated_delta_channel_kernel(Gd
         }
         float* s_out = reinterpret_cast<float*>(A.state_out) + so;
         settle(s);
+        // written through, as y and the tape are (300 steps of 16 heads of 128x128 with the next stretch behind 38.1 -> 37.7 us, with a product of y as well
+        // 51.1 -> 50.6; 24 steps of 8 heads of 64x64 6.28 -> 6.22, 12.40 -> 12.17)
 #pragma unroll
         for (int i = 0; i < NB; ++i) store_through(s_out + 16 * i, s[i]);
         return;

@@ -506,7 +506,8 @@ template <int CH, int RPT> struct GdnStepOps {
 // THROUGH: outputs are written through.  So they are with a 16-bit state, and with an fp32 state where a compute unit has a second workgroup; where
 // none has, that loses (us in a graph, plain and through, T = 16, gate per channel, 32 heads of 128x128: one sequence 6.45 6.64, two 8.71 8.55, four
 // 13.4 12.4, four at Dk = 256 26.1 25.3; bf16 state, one 6.48 6.26, four 13.2 12.5, two heads of three steps 3.39 3.34).  Either half of it, y and
-// the tape or the state, is slower.
+// the tape or the state, is slower.  With the layer's next block behind, which reads the state, and a product of y, plain and through: bf16 state, one
+// sequence of 13 steps 17.24 17.12, four 27.30 26.75; fp32 state, four 29.6 28.5.
 template <typename StateT, bool VEC_G, bool HAS_MASK, int DK, int LPR, int RPT, bool THROUGH>
 __global__ __launch_bounds__(kThreads) void gated_delta_tape_kernel(GdnArgs A) {
     constexpr int GR = kThreads / LPR, ROWS = RPT * GR;           // row groups; thread (group, j) has rows group, group + GR, ..

@@ -309,7 +309,9 @@ __global__ __launch_bounds__(kLongThreads, DK == 256 ? 2 : 4) void gated_delta_l
         asm volatile("" : "+v"(gam), "+v"(beta), "+v"(vf), "+v"(G[0]), "+v"(G[1]), "+v"(G[2]), "+v"(G[3]));   // not sunk into the next interval
     };
     // One store each: row by row, two and four bytes per lane, they were eight.  Written through: 25 MB of a prompt of 1,000 steps lay dirty in
-    // the L2s, which the launch's end then wrote back (32 heads of 128x128, 64 steps 7.6 -> 7.2 us, 300 18.4 -> 17.3).
+    // the L2s, which the launch's end then wrote back (32 heads of 128x128, 64 steps 7.6 -> 7.2 us, 300 18.4 -> 17.3; with the next stretch behind, which reads
+    // the state, 17.5 -> 16.5, with a product that reads y as well 39.1 -> 38.4).  Few heads with only the next stretch behind lose (8 of 64x64, 40 steps
+    // 4.92 -> 5.02), but with a product of y behind, as in a model, they gain as much (11.01 -> 10.87).
     auto store_rows = [&](int m, int tc) {
         const uint32_t o = (((uint32_t)b * A.T + m * kChunkSteps) * A.Hv + hv) * A.Dv + row0 + 4 * g + __umul24(n, step);
         if (n < tc) {

@@ -35,8 +35,8 @@ namespace dflash {
 // 4g .. 4g+3.  S^T = K Q^T, then O^T += V^T P^T, with P^T taken from the accumulators of S^T as they are: lane (n, g) holds keys
 // 4g .. 4g+3 of each 16 keys, and V^T is gathered in that order by the transposing LDS read (16x16x16 for a tile of 16 keys).
 // 16-byte piece p of row r stands at p ^ (r % 16) (K, Q) or p ^ f(r) (V: four rows of 32 bytes each, read together, in different banks), which leaves
-// few conflicts (by the counters, with the merge's among them, 19 % of the LDS cycles over 512 keys of D = 128, 14 % over 4,112 of
-// D = 256, with V whole).  A wave's K slot is asked for again behind its scores, its V slot behind the product.
+// few conflicts (by the counters, with the merge's among them, 21 % of the LDS cycles over 512 keys of D = 128, V in four parts, 19 % over
+// 4,112 of D = 256, V whole).  A wave's K slot is asked for again behind its scores, its V slot behind the product.
 // ---------------------------------------------------------------------------
 constexpr int kShortWaves = 8;
 template <int D, int PS> struct SdpaShortLds {
